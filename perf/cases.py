@@ -1,0 +1,239 @@
+"""What a user of this package has it do, as cases that can be timed: layers and operators called through their public entry points.
+
+A case is a dict of plain values; `entry` says which entry point it goes through:
+
+  block   MoeBlock.forward of one mixture-of-experts layer (norm, router, dispatch, experts, combine), from a one-token
+          decode step to a prefill of some thousand tokens
+  ffn     FFN.forward, the dense gated feed-forward network over quantized weights
+  linear  LinearLayer.forward over one quantized matrix
+  load    a raw ggml tensor on the device taken to the reference's planes and dequantised
+
+Weights, router rows and activations are drawn as the benchmark and the tests of this repository draw them: weights
+N(0, 0.02) at 4096 columns (scaled with the square root of the reduction length elsewhere, so that activations keep their
+size), activations N(0, 1), quantised on the device with ggml's conventions.
+"""
+
+import math
+import os
+import sys
+
+import torch
+import torch.nn.functional as F
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "shark-platform_amd"))
+
+from sharktank_amd import types as ST  # noqa: E402
+from sharktank_amd.layers import FFN, LinearLayer, MoeBlock  # noqa: E402
+
+_DTYPES = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+_EPS = 1e-5
+# bytes of one weight: ggml's Q8_0 and Q4_1 blocks of 32, e4m3fn samples, plain tensors
+_WEIGHT_BYTES = {"q8_0": 34 / 32, "q4_1": 20 / 32, "fp8": 1.0, "f32": 4.0, "f16": 2.0, "bf16": 2.0}
+
+
+def _block(name, tokens, fmt, dtype, K, N, E=8, k=2, act="silu", skew=0.0, out_norm=False, act_quant=False):
+    case = dict(entry="block", tokens=tokens, fmt=fmt, dtype=dtype, K=K, N=N, E=E, k=k, act=act, skew=skew, out_norm=out_norm,
+                act_quant=act_quant)
+    return dict(case, name=name) if name else case
+
+
+def listed():
+    return [
+        # one token of one user: latency of a chain of short launches, two experts' weights read
+        _block("decode_1_q4_1_bf16", 1, "q4_1", "bf16", 4096, 14336),
+        # a decode step of a serving batch: every expert's weights are read for a handful of rows each
+        _block("decode_32_q8_0_f16", 32, "q8_0", "f16", 4096, 14336),
+        # a ragged batch between the two regimes: chunked prefill, or speculative tokens of many users
+        _block("batch_203_q4_1_bf16", 203, "q4_1", "bf16", 4096, 14336),
+        # prefill of one long prompt, the shape of the benchmark
+        _block("prefill_2048_q8_0_f16", 2048, "q8_0", "f16", 4096, 14336),
+        # prefill on the largest layer of the repository, with a routing that two experts dominate, erf-GELU and output norm
+        _block("prefill_1024_q4_1_skewed", 1024, "q4_1", "f16", 6144, 32768, act="gelu", skew=1.0, out_norm=True),
+        # prefill with fp8 weights and static fp8 quantizers on both activations
+        _block("prefill_4096_fp8_f16", 4096, "fp8", "f16", 4096, 14336, act_quant=True),
+        # a layer whose experts were left unquantized, a batch of short prompts (odd token count)
+        _block("prefill_515_dense_bf16", 515, "bf16", "bf16", 4096, 14336),
+        # many small experts, six per token, an FFN width that is not a multiple of 256
+        _block("prefill_400_fine_q8_0_bf16", 400, "q8_0", "bf16", 2048, 1408, E=64, k=6),
+        # the small fp32 layer that checks of a model against its reference run
+        _block("small_64_f32", 64, "f32", "f32", 512, 1024),
+        # the feed-forward network of a dense block, a decode step of seven sequences
+        dict(name="ffn_7_q8_0_f16", entry="ffn", tokens=7, fmt="q8_0", dtype="f16", K=4096, N=14336),
+        # one quantized projection of a model, a prefill chunk
+        dict(name="linear_300_q4_1_bf16", entry="linear", tokens=300, fmt="q4_1", dtype="bf16", K=4096, N=14336),
+        # a matrix of a ggml file brought to planes and to fp16 (loading a model, or handing it to plain torch code)
+        dict(name="load_q8_0_14336x4096", entry="load", fmt="q8_0", dtype="f16", K=4096, N=14336),
+    ]
+
+
+def _log(rng, lo, hi):
+    return math.exp(rng.uniform(math.log(lo), math.log(hi)))
+
+
+def _width(rng, lo, hi):
+    """A feature count as models have it: two in three multiples of 256, the rest multiples of 64."""
+    step = 256 if rng.random() < 2 / 3 else 64
+    return max(step, int(_log(rng, lo, hi) / step) * step)
+
+
+def draw(rng):
+    kind = rng.choices(["moe", "fine", "dense", "small", "ffn", "linear", "load"], [46, 12, 10, 8, 9, 9, 6])[0]
+    if kind == "moe":  # quantized layers of a few large experts, decode to prefill
+        fmt = rng.choice(["q8_0", "q4_1", "fp8"])
+        K, N, E = 256 * rng.randint(4, 24), _width(rng, 1024, 16384), rng.choice([4, 8, 16])
+        while E * N * K > 8 * 14336 * 6144:
+            E //= 2
+        k = rng.choice([1, 2, 2, 2, 4])
+        tokens = int(min(_log(rng, 1, 4097), 2.8e12 / (6 * k * N * K)))
+        return _block("", max(1, tokens), fmt, rng.choice(["f16", "bf16"]), K, N, E, k, rng.choice(["silu", "silu", "gelu"]),
+                      rng.choice([0.0, 0.0, 1.0]), rng.random() < 0.25, fmt == "fp8" and rng.random() < 0.5)
+    if kind == "fine":  # many small experts
+        return _block("", int(_log(rng, 1, 2049)), rng.choice(["q8_0", "q4_1"]), rng.choice(["f16", "bf16"]), 256 * rng.randint(4, 12),
+                      _width(rng, 512, 2816), rng.choice([32, 64]), rng.choice([4, 6]))
+    if kind == "dense":  # unquantized experts
+        dtype = rng.choice(["f16", "bf16"])
+        return _block("", int(_log(rng, 1, 2049)), dtype, dtype, 256 * rng.randint(4, 16), _width(rng, 1024, 14336))
+    if kind == "small":  # fp32 layers of the size tests use
+        return _block("", int(_log(rng, 8, 129)), "f32", "f32", 128 * rng.randint(2, 8), 128 * rng.randint(2, 12))
+    fmt, dtype = rng.choice(["q8_0", "q4_1"]), rng.choice(["f16", "bf16"])
+    K, N = 256 * rng.randint(4, 24), _width(rng, 1024, 16384)
+    if kind == "load":
+        return dict(entry="load", fmt=fmt, dtype=dtype, K=K, N=N)
+    return dict(entry=kind, tokens=int(_log(rng, 1, 2049)), fmt=fmt, dtype=dtype, K=K, N=N)
+
+
+# ---- what a program has in hand before the call ------------------------------------------------------------------------
+
+
+def _randn(gen, shape, scale=1.0):
+    return torch.randn(shape, generator=gen, device=gen.device, dtype=torch.float32).mul_(scale)
+
+
+def _q8_0(w):
+    wb = w.reshape(*w.shape[:-1], -1, 32)
+    d = wb.abs().amax(dim=-1, keepdim=True) / 127.0
+    return {"d": d.to(torch.float16), "qs": torch.round(wb / d.clamp_min(1e-30)).clamp_(-127, 127).to(torch.int8)}
+
+
+def _q4_1(w):
+    wb = w.reshape(*w.shape[:-1], -1, 32)
+    m = wb.amin(dim=-1, keepdim=True)
+    d = (wb.amax(dim=-1, keepdim=True) - m) / 15.0
+    q = torch.floor((wb - m) / d.clamp_min(1e-30) + 0.5).clamp_(0, 15).to(torch.uint8)
+    return {"d": d.to(torch.float16), "m": m.to(torch.float16), "qs": q[..., 0::2] | (q[..., 1::2] << 4)}
+
+
+def _weight(gen, name, shape, fmt):
+    """One weight tensor of a theta; a stacked one expert by expert, to bound the fp32 staging memory."""
+    scale = 0.02 * math.sqrt(4096 / shape[-1])
+    parts = shape[0] if len(shape) == 3 else 1
+    step = max(1, min(parts, (1 << 28) // (shape[-1] * shape[-2])))
+    pieces = []
+    for first in range(0, parts, step):
+        lead = [min(step, parts - first)] if len(shape) == 3 else []
+        w = _randn(gen, lead + shape[-2:], scale)
+        if fmt in _DTYPES:
+            pieces.append({"w": w.to(_DTYPES[fmt])})
+        elif fmt == "fp8":  # one scale per tensor: five standard deviations and a half at the largest e4m3 value
+            pieces.append({"qs": (w * (448.0 / (5.5 * scale))).clamp_(-448.0, 448.0).to(torch.float8_e4m3fn)})
+        else:
+            pieces.append((_q8_0 if fmt == "q8_0" else _q4_1)(w))
+    p = {n: torch.cat([x[n] for x in pieces]) if len(pieces) > 1 else pieces[0][n] for n in pieces[0]}
+    if fmt in _DTYPES:
+        return ST.DefaultPrimitiveTensor(name=name, data=p["w"])
+    if fmt == "fp8":
+        d = torch.tensor(5.5 * scale / 448.0, dtype=torch.float32, device=gen.device)
+        layout = ST.TensorScaledLayout(shape=shape, d=d, qs=p["qs"])
+    elif fmt == "q8_0":
+        layout = ST.BlockScaledLayout(shape, p["d"], p["qs"])
+    else:
+        layout = ST.BlockScaledI4Layout(shape, p["d"], p["qs"], m=p["m"], signed=False)
+    return ST.PlanarQuantizedTensor(name=name, shape=shape, layout=layout)
+
+
+def _plain(name, data):
+    return ST.DefaultPrimitiveTensor(name=name, data=data)
+
+
+def prepare(case, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    dtype, K, N, fmt = _DTYPES[case["dtype"]], case["K"], case["N"], case["fmt"]
+    if case["entry"] == "load":
+        p = (_q8_0 if fmt == "q8_0" else _q4_1)(_randn(gen, [N, K], 0.02 * math.sqrt(4096 / K)))
+        if fmt == "q4_1":  # ggml's nibble order: element i low, element i + 16 high
+            lin = torch.stack([p["qs"] & 15, p["qs"] >> 4], dim=-1).reshape(N, K // 32, 32)
+            planes = [p["d"].view(torch.uint8), p["m"].view(torch.uint8), lin[..., :16] | (lin[..., 16:] << 4)]
+        else:
+            planes = [p["d"].view(torch.uint8), p["qs"].view(torch.uint8)]
+        raw = torch.cat(planes, dim=-1).reshape(-1)
+        return {"case": case, "tensor": (ST.Q8_0 if fmt == "q8_0" else ST.Q4_1)(raw=raw, shape=[N, K], name="w")}
+    T = case["tokens"]
+    if case["entry"] == "linear":
+        layer = LinearLayer(ST.Theta({"weight": _weight(gen, "weight", [N, K], fmt)}))
+        return {"case": case, "layer": layer, "x": _randn(gen, [T, K]).to(dtype)}
+    if case["entry"] == "ffn":
+        theta = ST.Theta({f"ffn_{n}.weight": _weight(gen, f"ffn_{n}.weight", s, fmt)
+                          for n, s in (("gate", [N, K]), ("up", [N, K]), ("down", [K, N]))})
+        return {"case": case, "layer": FFN(theta), "x": _randn(gen, [1, T, K]).to(dtype)}
+    E = case["E"]
+    tensors = {f"ffn_{n}_exps.weight": _weight(gen, f"ffn_{n}_exps.weight", s, fmt)
+               for n, s in (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))}
+    h, router = _randn(gen, [1, T, K]), _randn(gen, [E, K], 0.02)
+    if case["skew"]:
+        # a direction that all tokens share carries a Zipf prior (p ~ 1 / rank) into the router's logits
+        u = _randn(gen, [K])
+        u /= u.norm()
+        h += 40.0 * u
+        logp = -case["skew"] * torch.log(torch.arange(1, E + 1, device=h.device, dtype=torch.float32))
+        router += (logp - logp.mean()).reshape(E, 1) * u / 40.0
+    tensors["ffn_gate_inp.weight"] = _plain("ffn_gate_inp.weight", router)
+    tensors["ffn_norm.weight"] = _plain("ffn_norm.weight", 1.0 + _randn(gen, [K], 0.1))
+    if case["out_norm"]:
+        tensors["layer_output_norm.weight"] = _plain("layer_output_norm.weight", 1.0 + _randn(gen, [K], 0.1))
+    if case["act_quant"]:  # calibrated scales: five and ten times the usual size of an element at the largest e4m3 value
+        for key, top in (("ffn_gate_exps.q_input", 5.0), ("ffn_down_exps.q_input", 16.0)):
+            rs = torch.tensor(top / 448.0, dtype=torch.float32, device=h.device)
+            tensors[key] = ST.StaticScaledQuantizer(name=key, scale=1.0 / rs, reciprocal_scale=rs, dtype=torch.float8_e4m3fn)
+    block = MoeBlock(ST.Theta(tensors), E, case["k"], _EPS, moe_activation=F.gelu if case["act"] == "gelu" else F.silu)
+    return {"case": case, "layer": block, "x": h.to(dtype)}
+
+
+def run(state):
+    if "tensor" in state:
+        planar = state["tensor"].to_planar()
+        layout = planar.unpack()
+        return [*layout.planes.values(), layout.dequant(_DTYPES[state["case"]["dtype"]])]
+    return state["layer"](state["x"])
+
+
+def work(case):
+    """Every weight of the experts that have rows (all of them, or as many as a uniform routing is expected to hit), the input
+    and the output once; the products of the three projections (two operations per multiply-add) and of the router."""
+    K, N, wb = case["K"], case["N"], _WEIGHT_BYTES[case["fmt"]]
+    es = 4 if case["dtype"] == "f32" else 2
+    if case["entry"] == "load":
+        return {"bytes": N * K * (2 * wb + es), "flops": 2 * N * K}
+    T = case["tokens"]
+    if case["entry"] == "linear":
+        return {"bytes": N * K * wb + T * (K + N) * es, "flops": 2 * T * N * K}
+    if case["entry"] == "ffn":
+        return {"bytes": 3 * N * K * wb + 2 * T * K * es, "flops": 6 * T * N * K}
+    E, k = case["E"], case["k"]
+    hit = E * (1.0 - (1.0 - k / E) ** T)
+    return {"bytes": 3 * hit * N * K * wb + 2 * T * K * es, "flops": 6 * T * k * N * K + 2 * T * E * K}
+
+
+def tolerance(case):
+    """About four times what two kernels of the package that add in different orders differ by on these ranges: results are
+    rounded to 16 bits, and a sum that lands on the other side of a rounding boundary moves one value by a whole step (a
+    quantised intermediate by a sixteenth of itself).  Plain fp32 layers: four times the error of one sum in sequence against
+    fp64.  Planes and dequantised values are whole."""
+    if case["entry"] == "load":
+        return "exact"
+    if case["dtype"] == "f32":
+        return {"rel": 2e-6, "max": 1e-5}
+    if case["dtype"] == "bf16":
+        return {"rel": 3e-3, "max": 0.09}
+    if case.get("act_quant"):
+        return {"rel": 1.2e-3, "max": 0.05}
+    return {"rel": 5e-4, "max": 0.012}
