@@ -20,7 +20,8 @@ import sys
 import torch
 import torch.nn.functional as F
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "shark-platform_amd"))
+# (imported with the root of the tree to be timed as the working folder)
+sys.path.insert(0, os.path.abspath("shark-platform_amd"))
 
 from sharktank_amd import types as ST  # noqa: E402
 from sharktank_amd.layers import FFN, LinearLayer, MoeBlock  # noqa: E402
