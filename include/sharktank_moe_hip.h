@@ -73,7 +73,7 @@ typedef enum {
                       * cannot rule such scales out does the same.) */
   STMOE_W_FP8 = 3,   /* TensorScaledLayout: qs e4m3fn [.,K], d = d_count scales of `dtype` (f32 or f16) */
   /* The same bytes re-ordered by stmoe_prepack() into the order the matrix-core kernels stream (every wavefront
-   * load is one contiguous kilobyte; see stmoe_prepack).  Plane sizes are unchanged. */
+   * load is one contiguous kilobyte; see stmoe_prepack).  Plane sizes are unchanged unless the shape is padded. */
   STMOE_W_Q8_0_PACKED = 4,
   STMOE_W_Q4_1_PACKED = 5,
   STMOE_W_FP8_PACKED = 6
@@ -159,7 +159,9 @@ int stmoe_fake_quant_fp8(const void* x, int dtype, const float* rscale, int64_t 
  * the odd ones the high half-word); block scales/offsets as [K/256][16 rows][8] fp16.  A pure permutation of bytes
  * (of nibbles for Q4_1): stmoe_unpack(stmoe_prepack(w)) == w bit for bit.  `planar` and `packed` describe the same
  * [experts, rows, cols] with formats X and X_PACKED and caller-owned planes of equal sizes; rows % 16 == 0 and
- * cols % 256 == 0.  The reference has no counterpart (its planes come from GGUF blocks,
+ * cols % 256 == 0.  `packed` may also have more rows per expert and more columns than `planar`: the rest is filled with
+ * zeros (an FFN whose width N is not a multiple of 256 pads the rows of its gate/up and the columns of its down matrix
+ * to one and is called with the padded width), and stmoe_unpack leaves the padding out.  The reference has no counterpart (its planes come from GGUF blocks,
  * sharktank/sharktank/types/gguf_interop/layouts.py:51-60,285-300, and are consumed row-major). */
 int stmoe_prepack(const stmoe_weight* planar, const stmoe_weight* packed_out, stmoe_stream_t stream);
 int stmoe_unpack(const stmoe_weight* packed, const stmoe_weight* planar_out, stmoe_stream_t stream);

@@ -336,7 +336,7 @@ static int launch_big_t(int mode, const GemmParams& p, int64_t max_rows, hipStre
 
 int launch_mfma_big(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
-  if (p.offsets && p.E >= 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma big kernel: at most 63 experts");
+  if (p.offsets && p.E > 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma big kernel: at most 64 experts");
   if (wtag != WF_Q8_0_P)
     return set_error(STMOE_ERR_UNSUPPORTED, "mfma big kernel: needs weights in the packed Q8_0 order");
   if (p.kred % 256 != 0 || p.lda % 8 != 0 || p.ldo % 4 != 0 || p.n_out % (mode == MODE_GATEUP ? 64 * STMOE_BIG_WN : 128 * STMOE_BIG_WN) != 0)
@@ -364,7 +364,7 @@ static int launch_narrow_t(int mode, const GemmParams& p, int64_t max_rows, hipS
 
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
-  if (p.offsets && p.E >= 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma narrow kernel: at most 63 experts");
+  if (p.offsets && p.E > 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma narrow kernel: at most 64 experts");
   if (p.kred % 256 != 0 || p.lda % 8 != 0 || p.ldo % 4 != 0 || p.n_out % (mode == MODE_GATEUP ? 16 * STMOE_NARROW_TI : 32 * STMOE_NARROW_TI) != 0)
     return set_error(STMOE_ERR_UNSUPPORTED, "mfma narrow kernel: needs K %% 256 == 0 and output features in whole tiles");
   {

@@ -91,10 +91,15 @@ struct BigPlan {
   int F, R, f0, f1, r0, r1, whole, rest, chunks;
 };
 // The offsets are fetched with one vector load (lane l holds offsets[l]) and read back with readlane: walking them with
-// scalar loads costs one memory latency per expert, twice per workgroup.  Needs E < 64 (checked by the launchers).
+// scalar loads costs one memory latency per expert, twice per workgroup.  At most 64 experts (checked
+// by the launchers): with 64 the last offset has no lane and is fetched where a walk gets that far (64 experts of
+// 2048 x 1408 with 37 rows each: layer 395 us on the 128 x 128 kernel, 338 us here).
 __device__ __forceinline__ int big_lane_offsets(const GemmParams& p) {
   const int lane = threadIdx.x & 63;
   return (p.offsets && lane <= p.E) ? p.offsets[lane] : 0;
+}
+__device__ __forceinline__ int big_offset(const GemmParams& p, int lane_off, int i) {
+  return i < 64 ? __builtin_amdgcn_readlane(lane_off, i) : p.offsets[i];
 }
 __device__ __forceinline__ BigPlan big_plan(const GemmParams& p, int lane_off, int BM, int n_tiles, int xcd, bool allow_split,
                                             bool absorb = false, int balance = 0) {
@@ -102,8 +107,9 @@ __device__ __forceinline__ BigPlan big_plan(const GemmParams& p, int lane_off, i
   pl.F = 0;
   pl.R = 0;
   if (p.offsets) {
-    for (int e = 0; e < p.E; ++e) {
-      const int rows = __builtin_amdgcn_readlane(lane_off, e + 1) - __builtin_amdgcn_readlane(lane_off, e);
+    for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0); e < p.E; ++e) {
+      const int end = big_offset(p, lane_off, e + 1), rows = end - b;
+      b = end;
       const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
       pl.F += x.main;
       pl.R += x.partial;
@@ -197,8 +203,8 @@ __device__ __forceinline__ bool big_unit(const GemmParams& p, int lane_off, int 
     return true;
   }
   if (!partial) {
-    for (int e = 0; e < p.E; ++e) {
-      const int b = __builtin_amdgcn_readlane(lane_off, e), rows = __builtin_amdgcn_readlane(lane_off, e + 1) - b;
+    for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0), rows; e < p.E; ++e, b += rows) {
+      rows = big_offset(p, lane_off, e + 1) - b;
       const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
       const int units = x.main * n_tiles;
       if (u < units) {
@@ -214,8 +220,8 @@ __device__ __forceinline__ bool big_unit(const GemmParams& p, int lane_off, int 
   }
   t.ntile = u / pl.R;
   int s = u - t.ntile * pl.R;
-  for (int e = 0; e < p.E; ++e) {
-    const int b = __builtin_amdgcn_readlane(lane_off, e), rows = __builtin_amdgcn_readlane(lane_off, e + 1) - b;
+  for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0), rows; e < p.E; ++e, b += rows) {
+    rows = big_offset(p, lane_off, e + 1) - b;
     if (big_expert_tiles(rows, BM, absorb, balance).partial) {
       if (s == 0) {
         t.e = e;

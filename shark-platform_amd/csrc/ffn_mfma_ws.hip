@@ -721,7 +721,7 @@ int mfma_ws_ticket_count() { return kWsTickets; }
 // run on a few CUs only, are split along the reduction.
 int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, float* partial, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
-  if (p.offsets && p.E >= 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma ws kernel: at most 63 experts");
+  if (p.offsets && p.E > 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma ws kernel: at most 64 experts");
   if (wtag != WF_Q8_0_P && wtag != WF_Q4_1_P && wtag != WF_FP8_F32D_P)
     return set_error(STMOE_ERR_UNSUPPORTED, "mfma ws kernel: needs weights in a packed streaming order");
   if (p.kred % 256 != 0 || p.lda % 8 != 0 || p.ldo % 8 != 0 || !aligned16(p.out) || p.n_out % (mode == MODE_GATEUP ? 128 : 256) != 0)

@@ -18,27 +18,57 @@
 
 namespace stmoe {
 
+// The packed form may have more rows per expert and more columns than the planar one (rows_p >= rows, cols_p >= cols): what it
+// holds beyond the planar tensor is zero (zero scales, offsets and samples, so the padding contributes zero to every product and
+// zero features).  An FFN whose width is not a multiple of 256 is packed that way: its gate/up rows and its down columns are
+// padded alike, and the matrix kernels see a width they take.  cols % 32 == 0 (16 for fp8) keeps every 16-byte piece of samples
+// whole; the scales of 256 columns are copied value by value where a planar row of them is not a multiple of 16 bytes.
+struct RepackShape {
+  int64_t rows, cols, rows_p, cols_p;
+};
 // kind 0: 1-byte samples, kind 1: Q4_1 nibbles, kind 2: fp16 block scales.  dir 0: pack, 1: unpack.
 template <int KIND, int DIR>
 __global__ void __launch_bounds__(256)
-repack_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, int64_t n16, int64_t cols) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // index of a 16-byte piece in packed order
+repack_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t n16, RepackShape sh) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;  // index of a 16-byte piece in packed order (below 2^32: 64 GB)
   if (i >= n16) return;
-  int64_t planar;  // index of the same 16-byte piece in planar order
-  if (KIND == 0) {
-    const int lane = (int)(i & 63), n = lane & 15, g = lane >> 4;
-    const int64_t blk = i >> 6, kbs = cols >> 6, rt = blk / kbs, kb = blk - rt * kbs;
-    planar = ((rt * 16 + n) * cols + kb * 64 + g * 16) >> 4;
-  } else if (KIND == 1) {
-    const int lane = (int)(i & 63), n = lane & 15, g = lane >> 4;
-    const int64_t blk = i >> 6, kbs = cols >> 7, rt = blk / kbs, kb = blk - rt * kbs;
-    planar = ((rt * 16 + n) * (cols >> 1) + kb * 64 + g * 16) >> 4;
-  } else {
-    const int n = (int)(i & 15);
-    const int64_t blk = i >> 4, cs = cols >> 8, rt = blk / cs, c = blk - rt * cs;
-    planar = ((rt * 16 + n) * (cols >> 5) + c * 8) >> 3;
+  // row tile and reduction offset of the piece
+  const uint32_t n = i & 15, g = (i & 63) >> 4;
+  const uint32_t blk = KIND == 2 ? i >> 4 : i >> 6;
+  const uint32_t steps = (uint32_t)sh.cols_p >> (KIND == 0 ? 6 : KIND == 1 ? 7 : 8);
+  const uint32_t rt = blk / steps, step = blk - rt * steps;
+  const uint32_t k0 = KIND == 0 ? step * 64 + g * 16 : KIND == 1 ? step * 128 + g * 32 : step * 256;
+  const uint32_t tiles = (uint32_t)(sh.rows_p >> 4), e = rt / tiles, r = (rt - e * tiles) * 16 + n;  // rows_p % 16 == 0
+  const bool inside = r < sh.rows && k0 < sh.cols;
+  const int64_t row = (int64_t)e * sh.rows + r;
+  if (KIND == 2) {
+    const int64_t first = row * (sh.cols >> 5) + (k0 >> 5);
+    const int64_t left = (sh.cols - (int64_t)k0) >> 5;  // scales of the planar row from here on
+    const uint16_t* sp = reinterpret_cast<const uint16_t*>(src);
+    uint16_t* dp = reinterpret_cast<uint16_t*>(dst);
+    if (DIR == 0) {
+      if (inside && (sh.cols & 255) == 0) {
+        dst[i] = src[first >> 3];
+      } else {
+        uint16_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = inside && j < left ? sp[first + j] : (uint16_t)0;
+        dst[i] = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
+      }
+    } else if (inside) {
+      if ((sh.cols & 255) == 0) {
+        dst[first >> 3] = src[i];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (j < left) dp[first + j] = sp[8 * (int64_t)i + j];
+      }
+    }
+    return;
   }
-  uint4 v = DIR == 0 ? src[planar] : src[i];
+  const int64_t planar = KIND == 0 ? (row * sh.cols + k0) >> 4 : (row * sh.cols + k0) >> 5;  // the same piece in planar order
+  if (DIR == 1 && !inside) return;
+  uint4 v = DIR == 1 ? src[i] : inside ? src[planar] : make_uint4(0, 0, 0, 0);
   if (KIND == 1) {  // nibbles of every dword: linear order <-> even elements low / odd elements high
     if (DIR == 0) v = make_uint4(q4_dword_to_packed(v.x), q4_dword_to_packed(v.y), q4_dword_to_packed(v.z), q4_dword_to_packed(v.w));
     else v = make_uint4(q4_dword_to_linear(v.x), q4_dword_to_linear(v.y), q4_dword_to_linear(v.z), q4_dword_to_linear(v.w));
@@ -48,12 +78,13 @@ repack_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, int64_t n1
 }
 
 template <int KIND>
-static int repack(const void* src, void* dst, int64_t bytes, int64_t cols, int dir, hipStream_t st) {
-  const int64_t n16 = bytes >> 4;
+static int repack(const void* src, void* dst, int64_t packed_bytes, const RepackShape& sh, int dir, hipStream_t st) {
+  const int64_t n16 = packed_bytes >> 4;
   if (n16 == 0) return STMOE_OK;
+  STMOE_REQUIRE(n16 < (int64_t)0xffffff00u, STMOE_ERR_SHAPE, "prepack: planes of 64 GB and more are not supported");
   dim3 grid((unsigned)((n16 + 255) / 256));
-  if (dir == 0) repack_kernel<KIND, 0><<<grid, 256, 0, st>>>((const uint4*)src, (uint4*)dst, n16, cols);
-  else repack_kernel<KIND, 1><<<grid, 256, 0, st>>>((const uint4*)src, (uint4*)dst, n16, cols);
+  if (dir == 0) repack_kernel<KIND, 0><<<grid, 256, 0, st>>>((const uint4*)src, (uint4*)dst, (uint32_t)n16, sh);
+  else repack_kernel<KIND, 1><<<grid, 256, 0, st>>>((const uint4*)src, (uint4*)dst, (uint32_t)n16, sh);
   return check_launch("repack");
 }
 
@@ -61,29 +92,32 @@ static int repack_weight(const stmoe_weight* src, const stmoe_weight* dst, int d
   const stmoe_weight* planar = dir == 0 ? src : dst;
   const stmoe_weight* packed = dir == 0 ? dst : src;
   STMOE_REQUIRE(src && dst, STMOE_ERR_NULL, "prepack: NULL descriptor");
-  STMOE_REQUIRE(planar->experts == packed->experts && planar->rows == packed->rows && planar->cols == packed->cols,
-                STMOE_ERR_SHAPE, "prepack: shapes differ");
-  STMOE_REQUIRE(planar->rows % 16 == 0 && planar->cols % 256 == 0, STMOE_ERR_SHAPE,
-                "prepack: needs rows %% 16 == 0 and cols %% 256 == 0 (got %lld x %lld)", (long long)planar->rows,
-                (long long)planar->cols);
+  STMOE_REQUIRE(planar->experts == packed->experts && planar->rows <= packed->rows && planar->cols <= packed->cols,
+                STMOE_ERR_SHAPE, "prepack: the packed form must have the planar one's shape or be padded beyond it");
+  STMOE_REQUIRE(packed->rows % 16 == 0 && packed->cols % 256 == 0, STMOE_ERR_SHAPE,
+                "prepack: needs rows %% 16 == 0 and cols %% 256 == 0 (got %lld x %lld)", (long long)packed->rows,
+                (long long)packed->cols);
+  STMOE_REQUIRE(planar->cols % (planar->format == STMOE_W_FP8 ? 16 : 32) == 0, STMOE_ERR_SHAPE,
+                "prepack: a planar row must hold whole blocks (got %lld columns)", (long long)planar->cols);
   STMOE_REQUIRE(src->qs && dst->qs && aligned16(src->qs) && aligned16(dst->qs), STMOE_ERR_ALIGN,
                 "prepack: qs planes must be non-NULL and 16-byte aligned");
-  const int64_t elems = planar->experts * planar->rows * planar->cols;
+  const int64_t elems = packed->experts * packed->rows * packed->cols;
+  const RepackShape sh{planar->rows, planar->cols, packed->rows, packed->cols};
   hipStream_t st = as_stream(stream);
   int rc;
   if (planar->format == STMOE_W_Q8_0 && packed->format == STMOE_W_Q8_0_PACKED) {
     STMOE_REQUIRE(src->d && dst->d, STMOE_ERR_NULL, "prepack: d plane is NULL");
-    if ((rc = repack<0>(src->qs, const_cast<void*>(dst->qs), elems, planar->cols, dir, st))) return rc;
-    return repack<2>(src->d, const_cast<void*>(dst->d), elems / 16, planar->cols, dir, st);
+    if ((rc = repack<0>(src->qs, const_cast<void*>(dst->qs), elems, sh, dir, st))) return rc;
+    return repack<2>(src->d, const_cast<void*>(dst->d), elems / 16, sh, dir, st);
   }
   if (planar->format == STMOE_W_Q4_1 && packed->format == STMOE_W_Q4_1_PACKED) {
     STMOE_REQUIRE(src->d && dst->d && src->m && dst->m, STMOE_ERR_NULL, "prepack: d/m plane is NULL");
-    if ((rc = repack<1>(src->qs, const_cast<void*>(dst->qs), elems / 2, planar->cols, dir, st))) return rc;
-    if ((rc = repack<2>(src->d, const_cast<void*>(dst->d), elems / 16, planar->cols, dir, st))) return rc;
-    return repack<2>(src->m, const_cast<void*>(dst->m), elems / 16, planar->cols, dir, st);
+    if ((rc = repack<1>(src->qs, const_cast<void*>(dst->qs), elems / 2, sh, dir, st))) return rc;
+    if ((rc = repack<2>(src->d, const_cast<void*>(dst->d), elems / 16, sh, dir, st))) return rc;
+    return repack<2>(src->m, const_cast<void*>(dst->m), elems / 16, sh, dir, st);
   }
   if (planar->format == STMOE_W_FP8 && packed->format == STMOE_W_FP8_PACKED) {
-    return repack<0>(src->qs, const_cast<void*>(dst->qs), elems, planar->cols, dir, st);  // the scale(s) are shared, not copied
+    return repack<0>(src->qs, const_cast<void*>(dst->qs), elems, sh, dir, st);  // the scale(s) are shared, not copied
   }
   return set_error(STMOE_ERR_UNSUPPORTED, "prepack: format pair %d -> %d has no packed order", src->format, dst->format);
 }

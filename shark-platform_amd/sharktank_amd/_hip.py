@@ -422,8 +422,11 @@ class DeviceWeight:
     def is_packed(self) -> bool:
         return self.format in (W_Q8_0_PACKED, W_Q4_1_PACKED, W_FP8_PACKED)
 
-    def can_prepack(self) -> bool:
-        return (self.format in _PACKED_OF and self.rows % 16 == 0 and self.cols % 256 == 0
+    def can_prepack(self, rows: Optional[int] = None, cols: Optional[int] = None) -> bool:
+        """Whether prepack(rows, cols) has a streaming order for this weight (rows, cols: the padded shape, if any)."""
+        rows, cols = rows or self.rows, cols or self.cols
+        return (self.format in _PACKED_OF and rows % 16 == 0 and cols % 256 == 0
+                and self.cols % (16 if self.format == W_FP8 else 32) == 0
                 and (self.format != W_FP8 or self.desc.dtype == F32) and self.q4_scales_in_range())
 
     def q4_scales_in_range(self) -> bool:
@@ -437,15 +440,21 @@ class DeviceWeight:
         d = self.keep[1]
         return bool(torch.isfinite(d).all()) and float(d.abs().max()) < Q4_1_PACKED_MAX_SCALE
 
-    def prepack(self) -> "DeviceWeight":
-        """The same weight in the streaming order of stmoe_prepack (new planes; this object is unchanged)."""
+    def prepack(self, rows: Optional[int] = None, cols: Optional[int] = None) -> "DeviceWeight":
+        """The same weight in the streaming order of stmoe_prepack (new planes; this object is unchanged).  With `rows` or
+        `cols` beyond the weight's own the packed form is padded with zeros to that shape."""
         qs, d, m = self.keep
         lib = load_library()
-        new_qs = torch.empty_like(qs)
+        rows, cols = rows or self.rows, cols or self.cols
         fp8 = self.format == W_FP8
-        new_d = d if fp8 else torch.empty_like(d)
-        new_m = None if m is None else torch.empty_like(m)
-        out = DeviceWeight(_PACKED_OF[self.format], self.experts, self.rows, self.cols, new_qs, new_d, new_m, self.desc.dtype)
+        if (rows, cols) == (self.rows, self.cols):
+            new_qs, new_d, new_m = torch.empty_like(qs), d if fp8 else torch.empty_like(d), None if m is None else torch.empty_like(m)
+        else:
+            lead, blocks = [self.experts, rows], cols if fp8 else cols // 32
+            new_qs = torch.empty(lead + ([blocks] if fp8 else [blocks, 16 if m is not None else 32]), dtype=qs.dtype, device=qs.device)
+            new_d = d if fp8 else torch.empty(lead + [blocks, 1], dtype=d.dtype, device=d.device)
+            new_m = None if m is None else torch.empty_like(new_d)
+        out = DeviceWeight(_PACKED_OF[self.format], self.experts, rows, cols, new_qs, new_d, new_m, self.desc.dtype)
         with torch.cuda.device(self.device):
             _check(lib.stmoe_prepack(self.ref, out.ref, _stream(self.device)))
         return out

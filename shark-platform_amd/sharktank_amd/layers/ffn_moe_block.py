@@ -13,7 +13,7 @@ import torch.nn.functional as F
 
 from .. import _hip
 from .. import ops
-from ..ops import device_weight, expert_dispatch, gather_experts
+from ..ops import device_weight, expert_dispatch, ffn_device_weights, gather_experts
 from ..utils import debugging
 from ..types import (DefaultPrimitiveTensor, DynamicScaledQuantizer, PlanarQuantizedTensor, QuantizedTensor,
                      StaticScaledQuantizer, Theta)
@@ -65,13 +65,15 @@ class PreGatherFFNMOE(ThetaLayer):
         self.prepack_weights = True
 
     def device_weights(self):
-        """C-ABI descriptors of the three stacked weights, built once (planes made contiguous once)."""
+        """C-ABI descriptors of the three stacked weights, built once (planes made contiguous once).  Their FFN width may be
+        padded for the fused calls (ffn_device_weights); the two halves called on their own hand the intermediate to a
+        quantizer in between and keep its true width."""
         if self._dw is None:
-            self._dw = (
-                device_weight(self.ffn_gate, stacked=True, prepack=self.prepack_weights),
-                device_weight(self.ffn_up, stacked=True, prepack=self.prepack_weights),
-                device_weight(self.ffn_down, stacked=True, prepack=self.prepack_weights),
-            )
+            weights = (self.ffn_gate, self.ffn_up, self.ffn_down)
+            if self.fusable:
+                self._dw = ffn_device_weights(*weights, stacked=True, prepack=self.prepack_weights)
+            else:
+                self._dw = tuple(device_weight(w, stacked=True, prepack=self.prepack_weights) for w in weights)
         return self._dw
 
     def pre_matmul_gather(self, inputs, weights, experts, einstring="mk,menk->men", dispatch=None):
@@ -205,8 +207,8 @@ class FFNMOE(ThetaLayer):
 
     def forward(self, h: torch.Tensor):
         if self._dw is None:
-            self._dw = tuple(device_weight(layer.weight, stacked=False, prepack=True)
-                             for layer in (self.ffn_gate, self.ffn_up, self.ffn_down))
+            self._dw = ffn_device_weights(*(layer.weight for layer in (self.ffn_gate, self.ffn_up, self.ffn_down)),
+                                          stacked=False, prepack=True)
         wg, wu, wd = self._dw
         x = h.reshape(-1, h.shape[-1])
         y = _hip.grouped_ffn(x, wg, wu, wd, _hip.ACT_SILU, None, None, 1)  # one expert owns every row: no offsets array

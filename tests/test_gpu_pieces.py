@@ -323,6 +323,52 @@ def test_prepack_round_trip_bit_exact(device, fmt):
         assert not torch.equal(planar.keep[0].view(torch.uint8), packed.keep[0].view(torch.uint8))
 
 
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("N,K,rows,cols", [(96, 512, 256, 512), (224, 256, 224, 768), (64, 352, 512, 512), (32, 32, 32, 256)])
+def test_prepack_padded_round_trip_and_zero_padding(device, fmt, N, K, rows, cols):
+    """A packed form larger than the planar tensor: unpacking it to the padded planar shape gives the planes with zeros
+    around them, unpacking it to the tensor's own shape gives the planes back, bit for bit."""
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    case = MC.build(MC.Case(T=4, K=K, N=N, E=3, fmt=fmt, seed=51))
+    planar = device_weight(MC.to_inference_tensor(fmt, case.planes["gate"], [3, N, K], "w", device), stacked=True)
+    packed = planar.prepack(rows, cols)
+    assert packed.is_packed and (packed.rows, packed.cols) == (rows, cols)
+    whole = packed.unpack()
+    own = _hip.DeviceWeight(planar.format, 3, N, K, *(None if t is None else torch.empty_like(t) if t.numel() > 1 else t for t in planar.keep),
+                            planar.desc.dtype)
+    _hip._check(_hip.load_library().stmoe_unpack(packed.ref, own.ref, torch.cuda.current_stream(device).cuda_stream))
+    for a, b, c in zip(planar.keep, own.keep, whole.keep):
+        if a is None or a.numel() == 1:  # (no offset plane; fp8's one scale is shared)
+            continue
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        want = torch.zeros(3, rows, c.numel() // (3 * rows), dtype=torch.uint8 if c.element_size() == 1 else torch.int16, device=device)
+        want[:, :N, : a.numel() // (3 * N)] = a.view(want.dtype).reshape(3, N, -1)
+        assert torch.equal(c.view(want.dtype).reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16), ("fp8", torch.float16)])
+@pytest.mark.parametrize("N", [32, 224, 288, 704])
+@pytest.mark.parametrize("T", [1, 20, 300])
+def test_block_with_padded_width_against_the_oracle(device, fmt, dtype, N, T):
+    """FFN widths around the multiples of 256 that the packed kernels take: the layer packs its weights with a padded width."""
+    from sharktank_amd.layers import MoeBlock
+
+    case = MC.build(MC.Case(T=T, K=512, N=N, fmt=fmt, dtype=dtype, seed=52))
+    block = MoeBlock(MC.make_theta(case, device), case.E, case.k, case.eps)
+    assert [w.is_packed for w in block.experts.device_weights()] == [True] * 3
+    h = case.planes["h"]
+    y, idx, _ = block(h.reshape(1, T, 512).to(device), return_routing=True)
+    want, want_idx, _ = MC.oracle_block(case)
+    assert torch.equal(idx.cpu().long(), want_idx)
+    # (the tolerance of the small layers: 1e-3 of the contribution in fp16; bf16 3e-3, single roundings show in short sums)
+    moe = want.float() - h.float()
+    err = float((y.reshape(T, 512).cpu().float() - want.float()).norm() / moe.norm())
+    step = 2.0 ** (-11 if dtype == torch.float16 else -8)  # the residual sum's own rounding, half a step of the output each way
+    assert err < (1e-3 if dtype == torch.float16 else 3e-3) + step * float(want.float().norm() / moe.norm()), err
+
+
 def test_prepack_layout_definition(device):
     """Spot-checks the documented order: lane 16*g + n of block (row tile rt, k block kb) holds row 16*rt+n,
     k = 64*kb + 16*g .. +15; scales of 8 consecutive blocks of a row are contiguous."""
