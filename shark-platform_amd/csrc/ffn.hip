@@ -49,6 +49,7 @@ static int check_weight(const stmoe_weight* w, const char* who, int64_t E, int64
 //          7 fp8 matrix cores, 128x128 tile kernel only (5 uses the 256x256 LDS-direct kernel where it applies),
 //          8 auto among the kernels that follow the reference's arithmetic step by step (never the fp8 matrix cores)
 //          9 MFMA 64 x 256 tile, the narrow form of 4 (a single matrix with a few hundred rows; packed formats)
+//         10 fp32 activations on the fp32 matrix cores
 // Automatic choice with fp8 weights and static quantizers on both activations: a prefill-sized launch with fp16
 // activations goes to the fp8 matrix cores (variant 5: both operands as bytes, the fp32 dot product scaled once; 1.8 times
 // faster than dequantise-then-multiply, and 6e-3 from it on the layer output at the Mixtral shape, inside the 2e-2 the fp8
@@ -122,7 +123,7 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     return rc != STMOE_ERR_UNSUPPORTED ? rc : set_error(STMOE_ERR_UNSUPPORTED, "grouped_ffn: no streaming kernel for a launch that builds its own dispatch");
   }
   if (variant == 0) {
-    if (dtype == STMOE_F32) variant = 1;
+    if (dtype == STMOE_F32) variant = 10;
     // (one matrix, with or without an offsets array around its rows)
     else if (p.E == 1) variant = max_rows <= (p.split_scratch ? kSkinnyMaxRowsSingleSplit : kSkinnyMaxRowsSingle) ? 3
                                  : narrow_pays(mode, p, max_rows) ? 9 : 6;
@@ -130,6 +131,11 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
                            max_rows <= kSkinnyMaxRows || max_rows <= skinny_max_avg_rows(p.E) * p.E)) variant = 3;
     // Everything else goes to the 256 x 256 kernel (which hands shapes it does not take down to the 128 x 128 one).
     else variant = 6;
+  }
+  if (variant == 10 && dtype == STMOE_F32) {
+    int rc = launch_f32(wtag, mode, p, max_rows, st);
+    if (rc != STMOE_ERR_UNSUPPORTED) return rc;
+    variant = 1;
   }
   if (variant == 9) {
     int rc = launch_mfma_narrow(dtype, wtag, mode, p, max_rows, st);

@@ -1,7 +1,7 @@
 // Generic grouped projection: one wavefront per (sorted row, output feature), fp32 FMA on the vector
-// ALU.  It covers every activation dtype x weight format combination, including fp32 activations that
-// have no MFMA path here, and serves as a second implementation against which the MFMA kernels are
-// cross-checked.
+// ALU.  It covers every activation dtype x weight format combination, the ones without a matrix-core
+// instantiation included (fp8 weights with fp16 scales), and serves as a second implementation against
+// which the MFMA kernels are cross-checked.
 #include "ffn_kernels.h"
 
 namespace stmoe {

@@ -681,3 +681,32 @@ def test_dynamic_and_per_axis_quantizers_of_the_intermediate(device, kind, throu
     want2 = O.grouped_ffn_moe(xq, want_idx, want_gate.to(torch.float16), wg, wu, wd, case.activation)
     assert O.rel_l2(out2, h + want2) < 3e-4
     assert not torch.equal(out2, plain_out), "the input quantizer left no trace in the output"
+
+
+@pytest.mark.parametrize("fmt", ["dense", "q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("T,K,N,E,k", [(1, 64, 32, 8, 2), (5, 96, 160, 3, 2), (40, 512, 96, 8, 2), (77, 352, 224, 4, 2), (150, 128, 320, 2, 2)])
+def test_f32_layers_against_the_general_kernel_and_fp64(device, fmt, T, K, N, E, k):
+    """fp32 activations: the matrix-core kernel (token tiles of 16, 32 and 64 rows, a last pass with fewer, reduction lengths
+    with a partial chunk of 64, feature counts with a partial tile of 32) against the general kernel and against fp64."""
+    import moe_cases as MC
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    case = MC.build(MC.Case(T=T, K=K, N=N, E=E, k=k, fmt=fmt, dtype=torch.float32, seed=900 + T))
+    idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:k] for t in range(T)]).to(torch.int32)
+    dws = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], shp, n, device), stacked=True)
+           for n, shp in (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))]
+    x = case.planes["h"].to(device)
+    _, offsets, perm, inv = _hip.dispatch_build(idx.to(device), E)
+    got = _hip.grouped_ffn(x, *dws, _hip.ACT_SILU, offsets, perm, k)
+    other = _hip.grouped_ffn(x, *dws, _hip.ACT_SILU, offsets, perm, k, variant=_hip.VARIANT_GENERIC)
+    wg, wu, wd = (w.double() for w in MC.dense_weights(case))
+    pairs = perm.cpu().long()
+    e, t = idx.reshape(-1)[pairs].long(), pairs // k
+    xs = case.planes["h"].double()[t]
+    z = torch.nn.functional.silu(torch.einsum("rk,rnk->rn", xs, wg[e])) * torch.einsum("rk,rnk->rn", xs, wu[e])
+    want = torch.einsum("rn,rkn->rk", z, wd[e])
+    # sums of up to 512 fp32 products: half a unit in the last place per addition at worst, three chained sums
+    tol = 3 * 512 ** 0.5 * 2.0 ** -24 * 4
+    for y in (got, other):
+        assert O.rel_l2(y.cpu().double(), want) < tol
