@@ -230,61 +230,47 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
 
   // The first expert's router-weight row chunks of this wavefront are requested before anything else, so that their
   // latency runs in parallel with the norm (they do not depend on it).  PRE chunks of 512 elements are kept in registers.
-  // Rows of at least NC * 512 elements (the usual case) take their first loads without a bounds test per load: loads
-  // under separate conditions are waited for one by one, those of a straight line are all in flight together.
+  // No load here has a condition of its own: past the row's end the last piece is read again and not used.  Loads under
+  // separate conditions are waited for one by one, those of a straight line are all in flight together (rows shorter than
+  // NC * 512 elements used to pay one memory latency per 512 elements: 7 tokens of 3328, launch 8.7 -> 6.8 us).
   // PRE = 8 (a whole row of 4096) for launches of at most 64 tokens and 4 up to 512 tokens (latency).  Launches of more
   // tokens, where throughput counts and the prefetch registers held through the norm would cost a quarter of the
   // workgroups a CU can hold, request the same 8 chunks only after the norm's registers are free (LATE), in front of the
   // barrier that ends the norm: all in flight together, where a loop over the chunks waits for them one by one.
   constexpr int NC = 8;
-  const bool long_row = K >= (int64_t)NC * 512;
   uint4 wpre[PRE ? PRE : 1];
-  auto prefetch = [&]() {
-    if (PRE > 0 && sizeof(T) == 2 && wave < E) {  // 16-bit rows (a chunk of 8 elements is one 16-byte load)
-      const T* wrow = wr + (int64_t)wave * K;
-      if (long_row) {
+  auto prefetch = [&](uint4 (&dst)[PRE ? PRE : 1], int e) {
+    if (PRE > 0 && sizeof(T) == 2 && e < E) {  // 16-bit rows (a chunk of 8 elements is one 16-byte load)
+      const T* wrow = wr + (int64_t)e * K;
 #pragma unroll
-        for (int j = 0; j < PRE; ++j) wpre[j] = *reinterpret_cast<const uint4*>(wrow + lane * 8 + j * 512);
-      } else {
-#pragma unroll
-        for (int j = 0; j < PRE; ++j) {
-          const int64_t k0 = (int64_t)lane * 8 + (int64_t)j * 512;
-          if (k0 < K) wpre[j] = *reinterpret_cast<const uint4*>(wrow + k0);
-        }
+      for (int j = 0; j < PRE; ++j) {
+        const int k0 = lane * 8 + j * 512;
+        dst[j] = *reinterpret_cast<const uint4*>(wrow + (k0 < (int)K ? k0 : (int)K - 8));
       }
     }
   };
-  if constexpr (!LATE) prefetch();
+  if constexpr (!LATE) prefetch(wpre, wave);
   if constexpr (FUSE_NORM) {
     // the row's elements tid + 512 j are read once and kept (NC of them) for the second pass; the norm weights are
     // requested before the reduction
     float xv[NC], nw[NC];
     float ss = 0.0f;
-    if (long_row) {
-      T xraw[NC];
-      W wraw[NC];
+    T xraw[NC];
+    W wraw[NC];
 #pragma unroll
-      for (int j = 0; j < NC; ++j) xraw[j] = xr[tid + j * 512];
+    for (int j = 0; j < NC; ++j) xraw[j] = xr[min(tid + j * 512, (int)K - 1)];
 #pragma unroll
-      for (int j = 0; j < NC; ++j) wraw[j] = norm_w[tid + j * 512];
+    for (int j = 0; j < NC; ++j) wraw[j] = norm_w[min(tid + j * 512, (int)K - 1)];
 #pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        xv[j] = Cvt<T>::to_f32(xraw[j]);
-        nw[j] = Cvt<W>::to_f32(wraw[j]);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        const int64_t i = tid + (int64_t)j * 512;
-        if (i < K) {
-          xv[j] = Cvt<T>::to_f32(xr[i]);
-          nw[j] = Cvt<W>::to_f32(norm_w[i]);
-        }
-      }
+    for (int j = 0; j < NC; ++j) {
+      xv[j] = Cvt<T>::to_f32(xraw[j]);
+      nw[j] = Cvt<W>::to_f32(wraw[j]);
     }
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
-      if (tid + (int64_t)j * 512 < K) ss = __fadd_rn(ss, __fmul_rn(xv[j], xv[j]));
+    for (int j = 0; j < NC; ++j) {
+      const float with = __fadd_rn(ss, __fmul_rn(xv[j], xv[j]));
+      ss = tid + j * 512 < (int)K ? with : ss;
+    }
     for (int64_t i = tid + (int64_t)NC * 512; i < K; i += 512) {
       const float v = Cvt<T>::to_f32(xr[i]);
       ss = __fadd_rn(ss, __fmul_rn(v, v));
@@ -317,26 +303,26 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
       for (int64_t i = (int64_t)tid * 8 + 4; i < K; i += 512 * 8)
         *reinterpret_cast<uint4*>(&xs[i]) = *reinterpret_cast<const uint4*>(&xr[i]);
   }
-  if constexpr (LATE) prefetch();
+  if constexpr (LATE) prefetch(wpre, wave);
   __syncthreads();
 
-  for (int e = wave; e < E; e += 8) {
+  // the logit of expert e, whose first PRE chunks (16-bit rows) are in `pre`
+  auto logit = [&](int e, const uint4 (&pre)[PRE ? PRE : 1]) {
     float acc = 0.0f;
     const T* wrow = wr + (int64_t)e * K;
-    auto chunk = [&](int64_t k0, const uint4* pre) {
+    auto chunk = [&](int64_t k0, const uint4* raw) {
       Vec8<T> xv, wv;
       xv.load(xs + k0);
-      if (pre) wv.from_raw(*pre);  // the prefetched chunk (16-bit rows, the wavefront's first expert)
+      if (raw) wv.from_raw(*raw);
       else wv.load(wrow + k0);
 #pragma unroll
       for (int jj = 0; jj < 8; ++jj) acc = __fadd_rn(acc, __fmul_rn(xv.v[jj], wv.v[jj]));
     };
-    const bool pre_ok = PRE > 0 && sizeof(T) == 2 && e == wave;
 #pragma unroll
     for (int j = 0; j < PRE; ++j) {  // chunks in increasing order, as the summation order requires
       const int64_t k0 = (int64_t)lane * 8 + (int64_t)j * 512;
       if (k0 < K) {
-        if (pre_ok) chunk(k0, &wpre[j]);
+        if constexpr (sizeof(T) == 2) chunk(k0, &pre[j]);
         else chunk(k0, nullptr);
       }
     }
@@ -356,42 +342,54 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
       lg_s[e] = l;
       if (logits_out) logits_out[t * E + e] = Cvt<T>::from_f32(l);
     }
+  };
+  if (E <= 8) {
+    if (wave < E) logit(wave, wpre);
+  } else {
+    // several experts per wavefront: the next one's chunks are on their way while this one's are summed
+    for (int e = wave; e < E; e += 8) {
+      uint4 wnext[PRE ? PRE : 1];
+      prefetch(wnext, e + 8);
+      logit(e, wpre);
+#pragma unroll
+      for (int j = 0; j < PRE; ++j) wpre[j] = wnext[j];
+    }
   }
   __syncthreads();
   if (wave != 0) return;
 
   // fp32 softmax, top-k of the probabilities (equal ones by increasing index), renormalised gates: same arithmetic and
   // order as router_topk_kernel, done by the first wavefront.  Lane e holds expert e: the exponentials and the divisions
-  // are computed side by side; everything whose order matters (the sum of the exponentials, the choice with its
-  // lower-index-first rule, the sum of the chosen probabilities) is the serial loop over values read from the lanes, which
-  // every lane runs alike.
-  const float l = lane < E ? lg_s[lane] : 0.0f;
-  float mx = __shfl(l, 0);
-  for (int e = 1; e < E; ++e) mx = fmaxf(mx, __shfl(l, e));
+  // are computed side by side; the sums, whose order matters, are serial loops over values read from the lanes
+  // (v_readlane), which every lane runs alike; the maxima are reductions inside the rows of 16 lanes.  (Read through the LDS
+  // crossbar one at a time, as (k + 2) E dependent reads, this tail took 18 us of the launch with 64 experts and top-6.)
+  const float l = lane < E ? lg_s[lane] : -INFINITY;
+  const float mx = wave_max(l);
   const float ex = softmax_exp(l - mx);
   float denom = 0.0f;
-  for (int e = 0; e < E; ++e) denom += __shfl(ex, e);
+  for (int e = 0; e < E; ++e) denom += lane_value(ex, e);
   const float pr = ex / denom;
+  // The j-th choice is the lowest lane that holds the largest probability left (probabilities are not negative; where a NaN
+  // logit has made all of them NaN, the lowest lane left).
+  const uint64_t experts = E == 64 ? ~0ull : (1ull << E) - 1ull;
   uint64_t taken = 0;
   float vsum = 0.0f;
   int my_best = 0;        // lane j: the j-th choice
   float my_bestv = 0.0f;
   for (int j = 0; j < k; ++j) {
-    int best = -1;
-    float bestv = 0.0f;
-    for (int e = 0; e < E; ++e) {
-      const float v = __shfl(pr, e);
-      if (!((taken >> e) & 1ull) && (best < 0 || v > bestv)) {
-        best = e;
-        bestv = v;
-      }
-    }
+    const bool left = ((experts & ~taken) >> lane) & 1ull;
+    const float bestv = wave_max(left ? pr : -1.0f);
+    uint64_t holders = __ballot(left && pr == bestv);
+    const bool all_nan = holders == 0;
+    if (all_nan) holders = experts & ~taken;
+    const int best = __builtin_ctzll(holders);
     taken |= 1ull << best;
+    const float v = all_nan ? NAN : bestv;
     if (lane == j) {
       my_best = best;
-      my_bestv = bestv;
+      my_bestv = v;
     }
-    vsum += bestv;
+    vsum += v;
   }
   if (lane < k) {
     idx_out[t * k + lane] = my_best;
@@ -600,7 +598,8 @@ static int launch_router_wg(const void* x, const void* norm_w, float eps, void* 
   if (T_tokens <= 64)
     router_wg_kernel<T, W, FUSE_NORM, 8, false><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
-  else if (T_tokens <= 512)
+  else if (T_tokens <= 512 || E > 16)  // (several experts per wavefront: the next one's row is worth its registers
+    // at any size; with the tail on v_readlane 400 tokens of 2048 with 64 experts take 17 us instead of 51, 26 tokens with 32 experts 11 instead of 25)
     router_wg_kernel<T, W, FUSE_NORM, 4, false><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   else
@@ -672,12 +671,11 @@ softmax_rows_kernel(const void* __restrict__ x, int x_dtype, int64_t rows, int64
   if (r >= rows) return;
   const int64_t base = r * cols;
   if (cols <= 64) {
-    const float l = lane < cols ? softmax_load(x, x_dtype, base + lane) : 0.0f;
-    float mx = __shfl(l, 0);
-    for (int e = 1; e < cols; ++e) mx = fmaxf(mx, __shfl(l, e));
+    const float l = lane < cols ? softmax_load(x, x_dtype, base + lane) : -INFINITY;
+    const float mx = wave_max(l);
     const float ex = softmax_exp(l - mx);
     float denom = 0.0f;
-    for (int e = 0; e < cols; ++e) denom += __shfl(ex, e);
+    for (int e = 0; e < cols; ++e) denom += lane_value(ex, e);
     if (lane < cols) softmax_store(out, o_dtype, base + lane, ex / denom);
     return;
   }

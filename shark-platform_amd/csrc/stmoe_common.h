@@ -178,12 +178,41 @@ __device__ __forceinline__ float rms_scale(float total, int64_t K, float eps) {
 // ---- wavefront helpers -----------------------------------------------------------------------------
 static constexpr int kWave = 64;
 
+// v of lane `src` (the same for every lane of the wavefront), without the LDS crossbar that __shfl goes through
+__device__ __forceinline__ float lane_value(float v, int src) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src)); }
+// v of lane (lane ^ MASK) by moves inside a row of 16 lanes (rotation by 8 is ^ 8; a mirrored half row is ^ 7, and ^ 3 on top
+// of it ^ 4).
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int MASK> __device__ __forceinline__ float lane_xor(float v) {
+  static_assert(MASK == 8 || MASK == 4 || MASK == 2 || MASK == 1, "inside a row of 16 lanes");
+  if constexpr (MASK == 8) return dpp_move<0x128>(v);                    // row_ror:8
+  else if constexpr (MASK == 4) return dpp_move<0x1b>(dpp_move<0x141>(v));  // row_half_mirror, then quad_perm [3,2,1,0]
+  else if constexpr (MASK == 2) return dpp_move<0x4e>(v);                // quad_perm [2,3,0,1]
+  else return dpp_move<0xb1>(v);                                         // quad_perm [1,0,3,2]
+}
 __device__ __forceinline__ float wave_xor_sum(float v) {
   // Fixed butterfly: partner distance 32, 16, 8, 4, 2, 1.  Each step adds a value and its partner's,
-  // which is commutative, so every lane ends with the same bits.
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off, kWave);
-  return v;
+  // which is commutative, so every lane ends with the same bits.  A swap of a register with itself leaves the even halves
+  // (quarters) of the wavefront in one result and the odd ones in the other: a value and its partner's in every lane.
+  typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
+  const pair_t h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(h.x) + __uint_as_float(h.y);
+  const pair_t q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(q.x) + __uint_as_float(q.y);
+  v = v + lane_xor<8>(v);
+  v = v + lane_xor<4>(v);
+  v = v + lane_xor<2>(v);
+  return v + lane_xor<1>(v);
+}
+// The largest of 64 values (NaN passed over), the same for every lane.
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, lane_xor<8>(v));
+  v = fmaxf(v, lane_xor<4>(v));
+  v = fmaxf(v, lane_xor<2>(v));
+  v = fmaxf(v, lane_xor<1>(v));
+  return fmaxf(fmaxf(lane_value(v, 0), lane_value(v, 16)), fmaxf(lane_value(v, 32), lane_value(v, 48)));
 }
 
 }  // namespace stmoe
