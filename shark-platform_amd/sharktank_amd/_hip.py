@@ -186,8 +186,29 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# A call of a few microseconds of GPU work is as fast as the host issues it, so the two things every wrapper does are kept
+# short: torch.cuda.device() resolves and wraps its argument in 3 us, torch.cuda.current_stream() builds a Stream object in
+# 3 more (a linear call 16 us, of which the launch itself takes 3).
+class _on_device:
+    """Makes the device of the operands the current one for the duration of a call."""
+
+    __slots__ = ("index", "previous")
+
+    def __init__(self, dev: torch.device):
+        self.index = dev.index
+
+    def __enter__(self):
+        self.previous = torch.cuda._exchange_device(self.index)
+
+    def __exit__(self, *exc):
+        if self.previous != self.index:
+            torch.cuda._maybe_exchange_device(self.previous)
+        return False
+
+
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The current stream of `dev` as a hipStream_t."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _contig(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -208,7 +229,7 @@ def dequant_block_scaled(d, qs, m, dtype: Optional[torch.dtype]) -> torch.Tensor
     block = qs_c.shape[-1]
     n_blocks = qs_c.numel() // block if block else 0
     out = torch.empty(qs_c.shape, dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_dequant_block_scaled(_ptr(d_c), _ptr(m_c), dtype_enum(d_c.dtype), _ptr(qs_c), n_blocks, block,
                                               _ptr(out), dtype_enum(out_dtype), _stream(dev)))
     return out
@@ -224,7 +245,7 @@ def dequant_block_scaled_i4(d, qs_packed, m, signed: bool, dtype: Optional[torch
     block = qs_c.shape[-1] * 2
     n_blocks = qs_c.numel() * 2 // block if block else 0
     out = torch.empty(tuple(qs_c.shape[:-1]) + (block,), dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_dequant_block_scaled_i4(_ptr(d_c), _ptr(m_c), dtype_enum(d_c.dtype), _ptr(qs_c), n_blocks, block,
                                                  int(bool(signed)), _ptr(out), dtype_enum(out_dtype), _stream(dev)))
     return out
@@ -237,7 +258,7 @@ def promote_i4_block(qs_packed, signed: bool) -> torch.Tensor:
     if qs_c.dtype not in (torch.uint8, torch.int8):
         raise AssertionError(f"Expected tensor to by uint8 or int8. Got: {qs_c.dtype}")
     out = torch.empty(tuple(qs_c.shape[:-1]) + (qs_c.shape[-1] * 2,), dtype=torch.int8 if signed else torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_promote_i4(_ptr(qs_c), qs_c.numel(), int(bool(signed)), _ptr(out), _stream(dev)))
     return out
 
@@ -253,7 +274,7 @@ def dequant_tensor_scaled(qs, d, m, dtype: torch.dtype) -> torch.Tensor:
         raise NotImplementedError("TensorScaledLayout dequant: offset and scale must have the same shape")
     out = torch.empty(qs_c.shape, dtype=dtype, device=dev)
     axis = _broadcast_axis(d_c, qs_c) if d_count != 1 else None
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         if axis is None:
             _check(lib.stmoe_dequant_tensor_scaled(_ptr(qs_c), dtype_enum(qs_c.dtype), _ptr(d_c), _ptr(m_c), dtype_enum(d_c.dtype),
                                                    1, n, _ptr(out), dtype_enum(dtype), _stream(dev)))
@@ -294,7 +315,7 @@ def quantize_fp8_per_axis(x: torch.Tensor, scale: torch.Tensor, axis: int) -> to
     for s_ in x_c.shape[axis + 1:]:
         inner *= s_
     out = torch.empty(x_c.shape, dtype=torch.float8_e4m3fn, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_quantize_fp8_per_axis(_ptr(x_c), dtype_enum(x_c.dtype), _ptr(s_c), dtype_enum(s_c.dtype), s_c.numel(),
                                                inner, x_c.numel(), _ptr(out), _stream(dev)))
     return out
@@ -306,7 +327,7 @@ def quantize_fp8(x: torch.Tensor, rscale: torch.Tensor) -> torch.Tensor:
     x_c = _contig(x)
     rs = _scale1(rscale)
     out = torch.empty(x_c.shape, dtype=torch.float8_e4m3fn, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_quantize_fp8(_ptr(x_c), dtype_enum(x_c.dtype), _ptr(rs), x_c.numel(), _ptr(out), _stream(dev)))
     return out
 
@@ -320,7 +341,7 @@ def dynamic_quantize_fp8(x: torch.Tensor):
     out = torch.empty(x_c.shape, dtype=torch.float8_e4m3fn, device=dev)
     sr = torch.empty(2, dtype=torch.float32, device=dev)
     scratch = torch.empty(int(lib.stmoe_dynamic_quantize_fp8_scratch_bytes()), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_dynamic_quantize_fp8(_ptr(x_c), dtype_enum(x_c.dtype), x_c.numel(), _ptr(out), _ptr(sr), _ptr(scratch),
                                               scratch.numel(), _stream(dev)))
     sr_t = sr.to(x_c.dtype)  # exact: both values were rounded to x's dtype on the device
@@ -334,7 +355,7 @@ def fake_quant_fp8(x: torch.Tensor, rscale: torch.Tensor) -> torch.Tensor:
     x_c = _contig(x)
     rs = _scale1(rscale)
     out = torch.empty_like(x_c)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_fake_quant_fp8(_ptr(x_c), dtype_enum(x_c.dtype), _ptr(rs), x_c.numel(), _ptr(out), _stream(dev)))
     return out
 
@@ -343,6 +364,8 @@ def _scale1(s: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """A reciprocal scale as one contiguous device fp32 value (None stays None)."""
     if s is None:
         return None
+    if s.dtype == torch.float32 and s.numel() == 1:
+        return s
     return s.to(torch.float32).reshape(1).contiguous()
 
 
@@ -356,7 +379,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, epsilon: float) -> torch.Ten
     K = x_c.shape[-1]
     T = x_c.numel() // K if K else 0
     out = torch.empty_like(x_c)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_rms_norm(_ptr(x_c), dtype_enum(x_c.dtype), _ptr(w_c), dtype_enum(w_c.dtype), T, K, float(epsilon),
                                   _ptr(out), _stream(dev)))
     return out
@@ -375,7 +398,7 @@ def router_topk(x: torch.Tensor, w_router: torch.Tensor, k: int, *, want_logits:
     idx64 = torch.empty((T, k), dtype=torch.int64, device=dev) if index_dtype == torch.int64 else None
     gate = torch.empty((T, k), dtype=x_c.dtype, device=dev)
     logits = torch.empty((T, E), dtype=x_c.dtype, device=dev) if want_logits else None
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_router_topk(_ptr(x_c), _ptr(w_c), dtype_enum(x_c.dtype), T, K, E, k, _ptr(logits), _ptr(idx), _ptr(idx64),
                                      _ptr(gate), _stream(dev)))
     return (idx64 if idx64 is not None else idx), gate, logits
@@ -391,7 +414,7 @@ def dispatch_build(idx: torch.Tensor, E: int):
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
     perm = torch.empty(n, dtype=torch.int32, device=dev)
     inv = torch.empty(n, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_dispatch_build(_ptr(idx_c), n, E, _ptr(counts), _ptr(offsets), _ptr(perm), _ptr(inv), _stream(dev)))
     return counts, offsets, perm, inv
 
@@ -456,7 +479,7 @@ class DeviceWeight:
             new_d = d if fp8 else torch.empty(lead + [blocks, 1], dtype=d.dtype, device=d.device)
             new_m = None if m is None else torch.empty_like(new_d)
         out = DeviceWeight(_PACKED_OF[self.format], self.experts, rows, cols, new_qs, new_d, new_m, self.desc.dtype)
-        with torch.cuda.device(self.device):
+        with _on_device(self.device):
             _check(lib.stmoe_prepack(self.ref, out.ref, _stream(self.device)))
         return out
 
@@ -468,7 +491,7 @@ class DeviceWeight:
         fp8 = planar_fmt == W_FP8
         out = DeviceWeight(planar_fmt, self.experts, self.rows, self.cols, torch.empty_like(qs), d if fp8 else torch.empty_like(d),
                            None if m is None else torch.empty_like(m), self.desc.dtype)
-        with torch.cuda.device(self.device):
+        with _on_device(self.device):
             _check(lib.stmoe_unpack(self.ref, out.ref, _stream(self.device)))
         return out
 
@@ -477,10 +500,11 @@ GGUF_Q8_0, GGUF_Q4_1 = 0, 1
 
 
 def gguf_ingest(raw: torch.Tensor, gguf_type: int, experts: int, rows: int, cols: int, *, packed: bool,
-                check_scales: bool = True) -> DeviceWeight:
+                check_scales: bool = True, row_shape=None) -> DeviceWeight:
     """Raw ggml blocks (uint8, on the device) -> a DeviceWeight with freshly allocated planes, planar (the reference's
     planes bit for bit) or in the streaming order of stmoe_prepack.  With `check_scales` a Q4_1 tensor whose block scales
-    the packed kernels cannot take (DeviceWeight.q4_scales_in_range) comes back planar even when `packed` is asked for."""
+    the packed kernels cannot take (DeviceWeight.q4_scales_in_range) comes back planar even when `packed` is asked for.
+    `row_shape`: the shape the experts * rows rows have in the planes (default [experts, rows])."""
     dev = _dev(raw)
     lib = load_library()
     raw_c = _contig(raw)
@@ -491,12 +515,13 @@ def gguf_ingest(raw: torch.Tensor, gguf_type: int, experts: int, rows: int, cols
     if cols % 32 != 0 or raw_c.numel() != nb * block_bytes:
         raise ValueError(f"raw buffer of {raw_c.numel()} bytes does not hold [{experts},{rows},{cols}] in {block_bytes}-byte blocks")
     q4 = gguf_type == GGUF_Q4_1
-    qs = torch.empty((experts, rows, cols // 32, 16 if q4 else 32), dtype=torch.uint8 if q4 else torch.int8, device=dev)
-    d = torch.empty((experts, rows, cols // 32, 1), dtype=torch.float16, device=dev)
+    lead = (experts, rows) if row_shape is None else tuple(row_shape)
+    qs = torch.empty(lead + (cols // 32, 16 if q4 else 32), dtype=torch.uint8 if q4 else torch.int8, device=dev)
+    d = torch.empty(lead + (cols // 32, 1), dtype=torch.float16, device=dev)
     m = torch.empty_like(d) if q4 else None
     fmt = W_Q4_1 if q4 else W_Q8_0
     out = DeviceWeight(_PACKED_OF[fmt] if packed else fmt, experts, rows, cols, qs, d, m)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_gguf_ingest(_ptr(raw_c), gguf_type, out.ref, _stream(dev)))
     if packed and check_scales and not out.q4_scales_in_range():
         return gguf_ingest(raw, gguf_type, experts, rows, cols, packed=False)  # see DeviceWeight.q4_scales_in_range
@@ -524,7 +549,7 @@ def grouped_ffn(x, w_gate: DeviceWeight, w_up: DeviceWeight, w_down: DeviceWeigh
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
     y = torch.empty((T * k, K), dtype=x_c.dtype, device=dev)
     xs, zs = _scale1(x_scale), _scale1(z_scale)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_grouped_ffn(_ptr(x_c), dtype_enum(x_c.dtype), T, K, N, E, k, w_gate.ref, w_up.ref, w_down.ref, act,
                                      _ptr(offsets), _ptr(perm), _ptr(xs), _ptr(zs), _ptr(y), _ptr(workspace), workspace.numel(), variant,
                                      _stream(dev)))
@@ -542,7 +567,7 @@ def grouped_gate_up(x, w_gate: DeviceWeight, w_up: DeviceWeight, act: int, offse
     workspace = torch.empty(max(grouped_ffn_workspace_bytes(T, k, K, N, x_c.dtype), 1), dtype=torch.uint8, device=dev)
     z = torch.empty((T * k, N), dtype=x_c.dtype, device=dev)
     xs = _scale1(x_scale)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_grouped_gate_up(_ptr(x_c), dtype_enum(x_c.dtype), T, K, N, E, k, w_gate.ref, w_up.ref, act, _ptr(offsets),
                                          _ptr(perm), _ptr(xs), _ptr(z), _ptr(workspace), workspace.numel(), variant, _stream(dev)))
     return z
@@ -556,7 +581,7 @@ def grouped_down(z, w_down: DeviceWeight, offsets, T: int, k: int, *, variant: i
     N, K, E = w_down.cols, w_down.rows, w_down.experts
     workspace = torch.empty(max(grouped_ffn_workspace_bytes(T, k, K, N, z_c.dtype), 1), dtype=torch.uint8, device=dev)
     y = torch.empty((T * k, K), dtype=z_c.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_grouped_down(_ptr(z_c), dtype_enum(z_c.dtype), T, K, N, E, k, w_down.ref, _ptr(offsets), _ptr(y),
                                       _ptr(workspace), workspace.numel(), variant, _stream(dev)))
     return y
@@ -572,7 +597,7 @@ def add_bias(y: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"add_bias: bias {list(bias.shape)} does not match rows of {cols} elements")
     rows = y_c.numel() // cols if cols else 0
     out = torch.empty(y_c.shape, dtype=torch.promote_types(y_c.dtype, b_c.dtype), device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_add_bias(_ptr(y_c), dtype_enum(y_c.dtype), _ptr(b_c), dtype_enum(b_c.dtype), rows, cols, _ptr(out),
                                   dtype_enum(out.dtype), _stream(dev)))
     return out
@@ -588,7 +613,7 @@ def softmax(x: torch.Tensor, dim: int = -1, dtype: Optional[torch.dtype] = None)
     cols = x_c.shape[-1]
     rows = x_c.numel() // cols if cols else 0
     out = torch.empty(x_c.shape, dtype=out_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_softmax(_ptr(x_c), dtype_enum(x_c.dtype), rows, cols, _ptr(out), dtype_enum(out_dtype), _stream(dev)))
     return out.movedim(-1, dim)
 
@@ -600,7 +625,7 @@ def grouped_mmt(a: torch.Tensor, w: "DeviceWeight", offsets, perm, T: int, k: in
     lib = load_library()
     a_c = _contig(a)
     out = torch.empty((T, k, w.rows), dtype=a_c.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_grouped_mmt(_ptr(a_c), dtype_enum(a_c.dtype), T, k, int(bool(a_per_pair)), w.ref, _ptr(offsets),
                                      _ptr(perm), _ptr(out), variant, _stream(dev)))
     return out
@@ -614,7 +639,7 @@ def scale_rows(y: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     K = y_c.shape[-1]
     rows = y_c.numel() // K if K else 0
     out = torch.empty_like(y_c)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_scale_rows(_ptr(y_c), _ptr(g_c), dtype_enum(y_c.dtype), rows, K, _ptr(out), _stream(dev)))
     return out
 
@@ -627,7 +652,7 @@ def combine(y_sorted, gate, inv, T: int, k: int, *, out_norm_w=None, eps: float 
     res_c = None if residual is None else _contig(residual)
     w_c = None if out_norm_w is None else _contig(out_norm_w)
     out = torch.empty((T, K), dtype=y_c.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_combine(_ptr(y_c), _ptr(g_c), _ptr(inv), dtype_enum(y_c.dtype), T, k, K, _ptr(w_c),
                                  dtype_enum(w_c.dtype) if w_c is not None else F32, float(eps), _ptr(res_c), _ptr(out), _stream(dev)))
     return out
@@ -640,15 +665,17 @@ def moe_forward_workspace_bytes(T: int, k: int, E: int, K: int, N: int, dtype: t
 def moe_forward(h, ffn_norm_w, out_norm_w, eps: float, w_router, w_gate: DeviceWeight, w_up: DeviceWeight, w_down: DeviceWeight,
                 act: int, k: int, *, variant: int = VARIANT_AUTO, workspace: Optional[torch.Tensor] = None, want_routing: bool = False,
                 out: Optional[torch.Tensor] = None, events=None, x_scale: Optional[torch.Tensor] = None,
-                z_scale: Optional[torch.Tensor] = None):
+                z_scale: Optional[torch.Tensor] = None, need: Optional[int] = None):
     """h [T,K] -> out [T,K] (and, if asked, idx int32 [T,k] and gate [T,k]).  `events`: optional ctypes array of
-    12 hipEvent_t handles that bracket the six stages (see stmoe_moe_forward_timed)."""
+    12 hipEvent_t handles that bracket the six stages (see stmoe_moe_forward_timed).  `need`: the workspace size of this
+    shape, if the caller has asked for it already."""
     dev = _dev(h, ffn_norm_w, out_norm_w, w_router)
-    lib = load_library()
-    h_c = _contig(h)
+    lib = _lib or load_library()
+    h_c = h.contiguous()
     T, K = h_c.shape
     N, E = w_gate.rows, w_gate.experts
-    need = moe_forward_workspace_bytes(T, k, E, K, N, h_c.dtype)
+    if need is None:
+        need = moe_forward_workspace_bytes(T, k, E, K, N, h_c.dtype)
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
     if out is None:
@@ -659,7 +686,7 @@ def moe_forward(h, ffn_norm_w, out_norm_w, eps: float, w_router, w_gate: DeviceW
     args = (_ptr(h_c), dtype_enum(h_c.dtype), T, K, N, E, k, _ptr(ffn_norm_w), _ptr(out_norm_w),
             dtype_enum(ffn_norm_w.dtype), float(eps), _ptr(w_router), w_gate.ref, w_up.ref, w_down.ref, act,
             _ptr(xs), _ptr(zs), _ptr(out), _ptr(idx), _ptr(gate), _ptr(workspace), workspace.numel(), variant, _stream(dev))
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         if events is None:
             _check(lib.stmoe_moe_forward(*args))
         else:
@@ -681,7 +708,7 @@ def moe_forward_static(h, ffn_norm_w, out_norm_w, eps: float, w_router, w_gate: 
     if not h.is_contiguous() or not out.is_contiguous():
         raise ValueError("moe_forward_static: h and out must be contiguous")
     T, K = h.shape
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _check(lib.stmoe_moe_forward_static(_ptr(h), dtype_enum(h.dtype), T, K, w_gate.rows, w_gate.experts, k, _ptr(ffn_norm_w),
                                             _ptr(out_norm_w), dtype_enum(ffn_norm_w.dtype), float(eps), _ptr(w_router), w_gate.ref,
                                             w_up.ref, w_down.ref, act, _ptr(x_scale), _ptr(z_scale), _ptr(out), _ptr(idx), _ptr(gate),
@@ -714,7 +741,7 @@ def mmt(a: torch.Tensor, w: DeviceWeight, *, variant: int = VARIANT_AUTO, worksp
     K = a_c.shape[-1]
     M = a_c.numel() // K if K else 0
     out = torch.empty(tuple(a_c.shape[:-1]) + (w.rows,), dtype=a_c.dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         stream = _stream(dev)
         ready = workspace is None  # a caller's buffer has an unknown history
         if workspace is None:
@@ -739,7 +766,7 @@ def probe_mfma(device, kind: int = 0, random_operands: bool = True, iters: int =
     dev = torch.device(device)
     sink = torch.zeros(1, dtype=torch.float32, device=dev)
     flop = ctypes.c_double(0.0)
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         for _ in range(warm_launches):
             _check(lib.stmoe_probe_mfma(kind, int(random_operands), iters, _ptr(sink), None, _stream(dev)))
         start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

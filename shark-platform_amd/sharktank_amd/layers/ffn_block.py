@@ -43,8 +43,9 @@ class FFN(ThetaLayer):
     def _fusable(self, h: torch.Tensor) -> bool:
         if not self.is_gated or self._act is None or h.dtype not in (torch.float16, torch.bfloat16, torch.float32):
             return False
-        layers = (self.ffn_gate, self.ffn_up, self.ffn_down)
-        return all(l.bias is None and l.q_input is None and not l.fake_quant for l in layers)
+        modules = self._modules
+        return all(l.bias is None and l.q_input is None and not l.fake_quant
+                   for l in (modules["ffn_gate"], modules["ffn_up"], modules["ffn_down"]))
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         if self._fusable(h):

@@ -52,8 +52,8 @@ class MoeBlock(ThetaLayer):
         """The router matrix in the activation dtype.  The cast copy is keyed by the source tensor's storage, so a theta
         whose router tensor is replaced or resized gets a fresh copy (an in-place update of the same storage needs
         `reset_caches()`)."""
-        src = unbox_tensor(self.ffn_gate_inp.weight)
-        key = (dtype, src.data_ptr(), tuple(src.shape), src.dtype, _tensor_version(src))
+        src = unbox_tensor(self._modules["ffn_gate_inp"].weight)
+        key = (dtype, src.data_ptr(), src.shape, src.dtype, _tensor_version(src))
         hit = self._router_w.get(dtype)
         if hit is None or hit[0] != key:
             hit = (key, src.to(dtype).contiguous())
@@ -78,31 +78,34 @@ class MoeBlock(ThetaLayer):
         batch_size, sequence_length, feature_dim = h.shape
         x = h.reshape(-1, feature_dim)
         T = x.shape[0]
-        wg, wu, wd = self.experts.device_weights()
+        # (sub-modules are read from their dictionary: the attribute lookup of torch modules costs a small forward 2 us)
+        modules = self._modules
+        experts, out_norm = modules["experts"], modules["layer_output_norm"]
+        wg, wu, wd = experts._dw or experts.device_weights()
         if wg.experts != self.expert_count:
             raise ValueError(f"expert_count {self.expert_count} != stacked weight experts {wg.experts}")
-        out_norm = self.layer_output_norm
         out_norm_w = unbox_tensor(out_norm.weight) if isinstance(out_norm, RMSNormLayer) else None
-        ffn_norm_w = unbox_tensor(self.ffn_norm.weight)
+        ffn_norm_w = unbox_tensor(modules["ffn_norm"].weight)
         if out_norm_w is not None and out_norm_w.dtype != ffn_norm_w.dtype:
             out_norm_w = out_norm_w.to(ffn_norm_w.dtype)  # the C ABI takes one dtype for both norm weights
         need = _hip.moe_forward_workspace_bytes(T, self.expert_used_count, self.expert_count, feature_dim, wg.rows, h.dtype)
         # The workspace grows to the largest forward seen and is then reused.  A HIP graph captured from a forward
         # replays into the workspace of that moment: capture after a warm-up call with the largest token count (or call
         # reserve_workspace first), so that no later, larger forward replaces the buffer under the graph.
-        if self._workspace is None or self._workspace.numel() < need or self._workspace.device != h.device:
-            self._workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=h.device)
-        if not self.experts.fusable:
+        workspace = self._workspace
+        if workspace is None or workspace.numel() < need or workspace.device != h.device:
+            workspace = self._workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=h.device)
+        if not experts.fusable:
             return self._forward_staged(h, x, ffn_norm_w, out_norm_w, return_routing)
-        xs, zs = self.experts.activation_scales()
+        xs, zs = experts.activation_scales()
         # With tracing or golden dumps switched on, the routing is fetched as well and recorded beside the output (the
         # kernels and the results are the same either way).
         tracing = debugging.flags.enable_tensor_trace or debugging.flags.save_goldens_path is not None
         res = _hip.moe_forward(
             x, ffn_norm_w, out_norm_w, self.rms_epsilon, self._router_weight(h.dtype),
-            wg, wu, wd, self.experts._act, self.expert_used_count,
-            variant=self.experts.kernel_variant, workspace=self._workspace, want_routing=return_routing or tracing,
-            x_scale=xs, z_scale=zs,
+            wg, wu, wd, experts._act, self.expert_used_count,
+            variant=experts.kernel_variant, workspace=workspace, want_routing=return_routing or tracing,
+            x_scale=xs, z_scale=zs, need=need,
         )
         if return_routing or tracing:
             out, idx, gate = res

@@ -13,7 +13,7 @@ from torch import Tensor
 from .. import _hip
 from ..types.gguf_interop import Q4_1, Q8_0
 from ..types.layouts import BlockScaledI4Layout, BlockScaledLayout, TensorScaledLayout
-from ..types.tensors import GatheredExpertsTensor, InferenceTensor, PrimitiveTensor, QuantizedTensor, unbox_tensor
+from ..types.tensors import GatheredExpertsTensor, InferenceTensor, PlanarQuantizedTensor, PrimitiveTensor, QuantizedTensor, unbox_tensor
 from ._registry import AllOfType
 from .signatures import *
 
@@ -76,13 +76,18 @@ def _tensor_version(t: torch.Tensor) -> int:
 def _planes_key(w):
     """What a cached descriptor of `w` depends on: the identity, shape and version of every plane.  (The version counts
     in-place changes made through torch; a plane rewritten through a raw pointer needs a fresh tensor object.)"""
-    if isinstance(w, torch.Tensor):
+    kind = type(w)
+    if kind is PlanarQuantizedTensor:
+        ts = w.layout.planes.values()
+    elif kind is Q8_0 or kind is Q4_1:
+        ts = (w.raw,)
+    elif isinstance(w, torch.Tensor):
         ts = (w,)
     elif isinstance(w, (Q8_0, Q4_1)):
         ts = (w.raw,)
     else:
-        ts = tuple(w.globals.values())
-    return tuple((t.data_ptr(), tuple(t.shape), t.dtype, _tensor_version(t)) for t in ts)
+        ts = w.globals.values()
+    return [(t.data_ptr(), t.shape, t.dtype, _tensor_version(t)) for t in ts]
 
 
 _TENSOR_CACHE = {}  # id(torch.Tensor) -> (weakref to it, {(stacked, prepack, dtype): (planes key, descriptor)})

@@ -25,10 +25,7 @@ def _device_planes(t, gguf_type: int):
     for s in lead:
         experts *= s
     rows, cols = (int(t.shape[-2]), int(t.shape[-1])) if len(t.shape) >= 2 else (1, int(t.shape[-1]))
-    dw = _hip.gguf_ingest(t.raw, gguf_type, experts, rows, cols, packed=False)
-    qs, d, m = dw.keep
-    plane_shape = list(t.shape[:-1]) + [cols // 32]
-    return qs.reshape(plane_shape + [-1]), d.reshape(plane_shape + [1]), None if m is None else m.reshape(plane_shape + [1])
+    return _hip.gguf_ingest(t.raw, gguf_type, experts, rows, cols, packed=False, row_shape=t.shape[:-1]).keep
 
 
 class Q8_0(QuantizedTensor):
