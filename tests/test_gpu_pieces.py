@@ -650,3 +650,25 @@ def test_fake_quant_every_16_bit_value_against_eager_torch(device, dtype):
         a, b = got_qs.view(torch.uint8), want_qs.view(torch.uint8)
         same = (a == b) | ((a & 0x7f) == 0x7f) & ((b & 0x7f) == 0x7f)  # (any NaN code for NaN)
         assert bool(same.all()), f"scale {s!r}: {int((~same).sum())} quantised samples differ, first at bits {int(bits[~same][0]) & 0xffff:#06x}"
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n_blocks", [1, 3, 255, 257, 1025])
+def test_dequant_of_ggml_blocks_at_every_alignment(device, n_blocks, out_dtype):
+    """Blocks of 32 with fp16 scales: the kernel that takes 8 elements at a time (counts on both sides of its workgroups) and,
+    for samples that do not begin on a whole piece, the general one, bit for bit against the oracle."""
+    g = torch.Generator().manual_seed(n_blocks)
+    d = (torch.randn(n_blocks, 1, generator=g).abs() * 0.01).to(torch.float16)  # (ggml's scales are not negative)
+    m = (torch.randn(n_blocks, 1, generator=g) * 0.1).to(torch.float16)
+    qs = torch.randint(-128, 128, (n_blocks, 32), generator=g, dtype=torch.int8)
+    q4 = torch.randint(0, 256, (n_blocks, 16), generator=g, dtype=torch.uint8)
+    bits = torch.int32 if out_dtype == torch.float32 else torch.int16
+    for shift in (0, 4, 2):
+        def shifted(t):
+            buf = torch.empty(t.numel() + shift, dtype=t.dtype, device=device)
+            buf[shift:] = t.reshape(-1).to(device)
+            return buf[shift:].reshape(t.shape)
+        got8 = _hip().dequant_block_scaled(d.to(device), shifted(qs), None, out_dtype).cpu()
+        assert torch.equal(got8.view(bits), O.dequant_block_scaled(d, qs, dtype=out_dtype).reshape(got8.shape).view(bits))
+        got4 = _hip().dequant_block_scaled_i4(d.to(device), shifted(q4), m.to(device), False, out_dtype).cpu()
+        assert torch.equal(got4.view(bits), O.dequant_block_scaled_i4(d, q4, m, dtype=out_dtype).reshape(got4.shape).view(bits))
