@@ -50,6 +50,7 @@ static int check_weight(const stmoe_weight* w, const char* who, int64_t E, int64
 //          8 auto among the kernels that follow the reference's arithmetic step by step (never the fp8 matrix cores)
 //          9 MFMA 64 x 256 tile, the narrow form of 4 (a single matrix with a few hundred rows; packed formats)
 //         10 fp32 activations on the fp32 matrix cores
+//         11 256-row tiles of unquantized 16-bit weights, both operands straight into LDS
 // Automatic choice with fp8 weights and static quantizers on both activations: a prefill-sized launch with fp16
 // activations goes to the fp8 matrix cores (variant 5: both operands as bytes, the fp32 dot product scaled once; 1.8 times
 // faster than dequantise-then-multiply, and 6e-3 from it on the layer output at the Mixtral shape, inside the 2e-2 the fp8
@@ -102,6 +103,19 @@ static bool narrow_pays(int mode, const GemmParams& p, int64_t rows) {
   if (p.n_out / features * ((rows + 255) / 256) > 256) return false;
   return p.split_scratch == nullptr || p.kred <= 6144;
 }
+// Unquantized 16-bit weights: the kernel that brings both operands straight into LDS, against the streaming kernel.  For the
+// gate/up projection it is the faster one at any number of rows (8 experts of 4096 x 14336, us, streaming / this one: 1 token
+// 111 / 85, 8 tokens 346 / 316, 64 tokens 444 / 329; of 1024 x 1024, 1 token 13 / 11; a single 14336 x 4096 pair 73 / 47).  The
+// down projection has a quarter of the units or less, and below some 190 of them the streaming kernel, which cuts the reduction,
+// keeps more CUs busy (2 tokens, 128 units: 108 / 118; 4 tokens, 256 units: 150 / 133; a single 4096 x 14336 matrix 44 / 96).
+// Beyond the streaming kernel's rows this one takes every launch (down, 100 tokens: 292 / 164).
+static bool dense_pays(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
+  if (!dense_takes(dtype, wtag, mode, p, rows)) return false;
+  if (mode == MODE_GATEUP || p.n_out / 128 * (p.offsets ? std::min<int64_t>(p.E, rows) : 1) >= 192) return true;
+  if (p.E == 1) return rows > kSkinnyMaxRowsSingleSplit;
+  return !(p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) && rows > kSkinnyMaxRows &&
+         rows > skinny_max_avg_rows(p.E) * p.E;
+}
 // fp8 activations x fp8 weights on the fp8 matrix cores: the 256 x 256 kernel for packed weights and launches with
 // enough rows to fill its tiles (variant 5), the 128 x 128 kernel otherwise (and always with variant 7).
 // Whether the 256 x 256 kernel takes a projection (its token rows must come without a gather: see fp8_ws_takes' caller).
@@ -125,6 +139,7 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
   if (variant == 0) {
     if (dtype == STMOE_F32) variant = 10;
     // (one matrix, with or without an offsets array around its rows)
+    else if (dense_pays(dtype, wtag, mode, p, max_rows)) variant = 11;
     else if (p.E == 1) variant = max_rows <= (p.split_scratch ? kSkinnyMaxRowsSingleSplit : kSkinnyMaxRowsSingle) ? 3
                                  : narrow_pays(mode, p, max_rows) ? 9 : 6;
     else if (p.offsets && ((p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) ||
@@ -136,6 +151,11 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     int rc = launch_f32(wtag, mode, p, max_rows, st);
     if (rc != STMOE_ERR_UNSUPPORTED) return rc;
     variant = 1;
+  }
+  if (variant == 11) {
+    int rc = launch_dense(dtype, wtag, mode, p, max_rows, st);
+    if (rc != STMOE_ERR_UNSUPPORTED) return rc;
+    variant = 2;
   }
   if (variant == 9) {
     int rc = launch_mfma_narrow(dtype, wtag, mode, p, max_rows, st);
@@ -497,6 +517,7 @@ static int moe_forward_impl(const void* h, int dtype, int64_t T, int64_t K, int6
   const bool gate_up_dispatches =
       fused_front && T > 1 && T * k <= 64 && E >= 2 && (variant == 0 || variant == 3) && (dtype == STMOE_F16 || dtype == STMOE_BF16) &&
       w_gate && w_up && weight_tag(w_gate) == weight_tag(w_up) && !(x_scale && !x_fq) &&
+      !(variant == 0 && w_gate->format == STMOE_W_DENSE && N % 64 == 0) &&  // (the unquantized kernel takes those)
       skinny_takes_grouped(dtype, weight_tag(w_gate), E, K, N, K, N);
   // the dispatch launch also clears the ticket words of the projections' split reductions (if this shape has any)
   const FfnWs fws = carve_ffn(T, k, K, N, dtype);

@@ -161,6 +161,8 @@ namespace stmoe {
 // STMOE_ERR_UNSUPPORTED when the family has no instantiation for the combination.
 int launch_generic(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_f32(int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
+bool dense_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows);
+int launch_dense(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_tile(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_big(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);

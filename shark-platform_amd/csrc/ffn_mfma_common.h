@@ -234,10 +234,11 @@ __device__ __forceinline__ bool big_unit(const GemmParams& p, int lane_off, int 
   }
   return false;
 }
-__device__ __forceinline__ bool big_tile_id(const GemmParams& p, int BM, int n_tiles, bool allow_split, BigTile& t, bool absorb = false) {
+__device__ __forceinline__ bool big_tile_id(const GemmParams& p, int BM, int n_tiles, bool allow_split, BigTile& t, bool absorb = false,
+                                            int balance = 0) {
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
   const int lane_off = big_lane_offsets(p);
-  const BigPlan pl = big_plan(p, lane_off, BM, n_tiles, xcd, allow_split, absorb);
+  const BigPlan pl = big_plan(p, lane_off, BM, n_tiles, xcd, allow_split, absorb, balance);
   int unit;
   if (j < pl.whole) {
     unit = j;
@@ -252,7 +253,7 @@ __device__ __forceinline__ bool big_tile_id(const GemmParams& p, int BM, int n_t
     t.nchunks = pl.chunks;
     t.chunk_slot = xcd * kBigChunkSlotsPerXcd + c;
   }
-  return big_unit(p, lane_off, BM, n_tiles, pl, unit, t, absorb);
+  return big_unit(p, lane_off, BM, n_tiles, pl, unit, t, absorb, balance);
 }
 // Item j of an XCD's work list: the whole units first, then the chunks of the split ones (the same numbering as the
 // workgroup index j of big_tile_id), from a plan and offsets fetched once: for workgroups that walk several items.

@@ -29,6 +29,7 @@ VARIANT_AUTO, VARIANT_GENERIC, VARIANT_MFMA_TILE, VARIANT_SKINNY, VARIANT_MFMA_B
 VARIANT_FP8_TILE = 7
 VARIANT_STEP_BY_STEP = 8  # automatic choice among the kernels that round where the reference rounds (never the fp8 matrix cores)
 VARIANT_MFMA_F32 = 10  # fp32 activations on the fp32 matrix cores (chosen automatically)
+VARIANT_DENSE = 11  # 16-bit weights of the activations' type, both operands straight into LDS (chosen automatically where it pays)
 VARIANT_MFMA_NARROW = 9  # 64 x 256 tiles: a single matrix with a few hundred rows (chosen automatically where it pays)
 
 _DTYPE_ENUM = {

@@ -710,3 +710,48 @@ def test_f32_layers_against_the_general_kernel_and_fp64(device, fmt, T, K, N, E,
     tol = 3 * 512 ** 0.5 * 2.0 ** -24 * 4
     for y in (got, other):
         assert O.rel_l2(y.cpu().double(), want) < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,N,act", [
+    ((1, 0, 15, 16), 64, 64, "silu"),               # one K step; fewer weight rows than one wide unit
+    ((17, 63, 64, 65), 128, 128, "gelu"),
+    ((127, 128, 129, 0), 192, 320, "silu"),         # the two unit shapes; 128-row units of a width 256 does not divide
+    ((192, 193, 256, 257), 256, 256, "silu"),       # three and four column blocks, a full tile, one row more
+    ((0, 513, 640, 3), 320, 192, "gelu"),           # several tiles per expert, of equal size and with a rest
+    ((70,) * 32, 128, 4096, "silu"),                # enough units for 256 weight rows each
+    ((300,), 512, 768, "silu"),                     # a single expert
+])
+def test_dense_16_bit_kernel_against_the_tile_kernel_and_fp64(device, rows, K, N, act, dtype):
+    """Unquantized weights: row counts on both sides of the column blocks, the token groups, the two unit shapes and the tile,
+    against fp64 and (the down projection adds in the same order) bit for bit against the 128 x 128 kernel."""
+    from sharktank_amd import _hip
+
+    E, T = len(rows), sum(rows)
+    g = torch.Generator().manual_seed(1000 + T)
+    x, wg, wu = (torch.randn(s, generator=g).to(dtype) for s in ([T, K], [E, N, K], [E, N, K]))
+    wg, wu = wg / K ** 0.5, wu / K ** 0.5
+    wd = (torch.randn([E, K, N], generator=g) / N ** 0.5).to(dtype)
+    dg, du, dd = (_hip.DeviceWeight(_hip.W_DENSE, E, w.shape[1], w.shape[2], w.to(device), None, None, _hip.dtype_enum(dtype)) for w in (wg, wu, wd))
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)].to(torch.int32).reshape(T, 1)
+    _, offsets, perm, _ = _hip.dispatch_build(idx.to(device), E)
+    act_id = _hip.ACT_SILU if act == "silu" else _hip.ACT_GELU_ERF
+    z = _hip.grouped_gate_up(x.to(device), dg, du, act_id, offsets, perm, 1, variant=_hip.VARIANT_DENSE)
+    pairs = perm.cpu().long()
+    xs, e = x[pairs].double(), idx.reshape(-1)[pairs].long()
+    want = torch.empty(T, N, dtype=torch.float64)
+    for ee in range(E):
+        a, b = xs[e == ee] @ wg[ee].double().T, xs[e == ee] @ wu[ee].double().T
+        # (four roundings to 16 bits on the way, of at most eps / 2 each)
+        want[e == ee] = (torch.nn.functional.silu(a) if act == "silu" else torch.nn.functional.gelu(a)) * b
+    eps = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert O.rel_l2(z.cpu().double(), want) < 2 * eps
+    down = {v: _hip.grouped_down(z, dd, offsets, T, 1, variant=v).cpu() for v in (_hip.VARIANT_DENSE, _hip.VARIANT_MFMA_TILE)}
+    bits = torch.int16
+    if N % 64 == 0 and K % 128 == 0:  # (narrower outputs run on the 128 x 128 kernel either way)
+        assert torch.equal(down[_hip.VARIANT_DENSE].view(bits), down[_hip.VARIANT_MFMA_TILE].view(bits))
+    auto = _hip.grouped_ffn(x.to(device), dg, du, dd, act_id, offsets, perm, 1)
+    y = torch.stack([wd[ee].double() @ zz for ee, zz in zip(e.tolist(), z.cpu().double())]) if T < 600 else None
+    if y is not None:
+        assert O.rel_l2(down[_hip.VARIANT_DENSE].double(), y) < eps
+        assert O.rel_l2(auto.cpu().double(), y) < 2 * eps  # (a z element may round the other way under another kernel)
