@@ -300,10 +300,9 @@ struct SkinnyExperts {
 // One pass of one work item: rows [r0, min(r0 + 16*MT, re)) of expert rows against the item's two weight tiles.
 // KS > 1: the KS wavefronts of a workgroup share the item, each takes a contiguous 1/KS of the chunks, and the partial
 // sums are added through LDS in a fixed order ((w0 + w1) + (w2 + w3)) by wavefront 0, which then writes the result.
-template <typename T, int WF, int MODE, int MT, int KS>
-__device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExperts& experts, const int64_t (&wrow)[2], int tile,
+template <typename T, int WF, int MODE, int MT, int KS, int NT>
+__device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExperts& experts, const int64_t (&wrow)[NT], int tile,
                                             int r0, int re, int64_t nch_total, int lane, bool pin_prefetch) {
-  constexpr int NT = 2;
   const int kw = KS > 1 ? (int)(threadIdx.x >> 6) : 0;
   const int64_t c_begin = KS > 1 ? nch_total * kw / KS : 0;
   const int64_t nch = KS > 1 ? nch_total * (kw + 1) / KS : nch_total;  // end of this wavefront's chunk range
@@ -334,12 +333,14 @@ __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExp
   SkinnyW<WF> w0[NT], w1[NT];
   w0[0].init(p.w0, wrow[0]);
   w1[0].init(p.w0, wrow[0]);
-  w0[1].init(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1]);
-  w1[1].init(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1]);
+  if constexpr (NT == 2) {
+    w0[1].init(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1]);
+    w1[1].init(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1]);
+  }
   SkinnyX<WF> x0[MT], x1[XDB ? MT : 1];
   auto load_w = [&](SkinnyW<WF>* w, int64_t c) {
     w[0].load(p.w0, wrow[0], c, g);
-    w[1].load(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1], c, g);
+    if constexpr (NT == 2) w[1].load(MODE == MODE_GATEUP ? p.w1 : p.w0, wrow[1], c, g);
   };
   auto load_x = [&](SkinnyX<WF>* x, int64_t c) {
 #pragma unroll
@@ -437,7 +438,7 @@ __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExp
     const int i = r0 + mt * 16 + n_in;
     if (i < re) {
       T* orow = reinterpret_cast<T*>(p.out) + out_row(p, i) * p.ldo;
-      if (MODE == MODE_GATEUP) {
+      if constexpr (MODE == MODE_GATEUP) {
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = gateup_epilogue<T>(p.act, acc[mt][0][r], acc[mt][1][r], 1.0f, fq);
@@ -445,7 +446,7 @@ __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExp
       } else {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-          *reinterpret_cast<uint2*>(orow + tile * 32 + t * 16 + 4 * g) =
+          *reinterpret_cast<uint2*>(orow + tile * 16 * NT + t * 16 + 4 * g) =
               make_uint2(pack2<T>(acc[mt][t][0], acc[mt][t][1]), pack2<T>(acc[mt][t][2], acc[mt][t][3]));
       }
     }
@@ -458,16 +459,17 @@ template <int WF> struct SkinnyUsesLds { static constexpr bool value = WF == WF_
 // Workgroups resident per CU (two wavefronts per SIMD: the double-buffered chunks need about 200 registers).
 template <int WF> struct SkinnyOcc { static constexpr int value = 2; };
 
-// KS == 1: `total_workers` wavefronts, one item each at a time.  KS == 4: `total_workers` workgroups, the four
+// KS == 1: `total_workers` wavefronts, one item each at a time.  KS > 1: `total_workers` workgroups, the KS
 // wavefronts of a workgroup split the reduction of one item (for launches with too few items to fill the chip).
-template <typename T, int WF, int MODE, int KS>
+// NT: weight tiles of an item (GATEUP 2: gate and up of 16 features; DOWN 2 or 1 of 16 features each).
+template <typename T, int WF, int MODE, int KS, int NT>
 __global__ void __launch_bounds__(256, SkinnyOcc<WF>::value)
 grouped_skinny_kernel(GemmParams p, int tiles_per_expert, int total_waves, bool pin_prefetch) {
+  static_assert(MODE == MODE_DOWN || NT == 2, "gate and up");
   const int lane = threadIdx.x & 63;
   const int n_in = lane & 15;
   const int wave_global = KS > 1 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int64_t nch = p.kred >> 8;
-
   // experts that received rows, in increasing id
   SkinnyExperts experts;
   experts.template init<MODE>(p, lane, blockIdx.x == 0 && threadIdx.x < 64);
@@ -478,20 +480,19 @@ grouped_skinny_kernel(GemmParams p, int tiles_per_expert, int total_waves, bool 
     int e, rb, re;
     experts.find(__builtin_amdgcn_readfirstlane(a_idx), e, rb, re);
 
-    // the two weight tiles of this item
-    int64_t wrow[2];
+    int64_t wrow[NT];
     if (MODE == MODE_GATEUP) {
       wrow[0] = (int64_t)e * p.w0.rows + tile * 16 + n_in;
-      wrow[1] = (int64_t)e * p.w1.rows + tile * 16 + n_in;
+      wrow[NT - 1] = (int64_t)e * p.w1.rows + tile * 16 + n_in;
     } else {
-      wrow[0] = (int64_t)e * p.w0.rows + tile * 32 + n_in;
-      wrow[1] = wrow[0] + 16;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wrow[t] = (int64_t)e * p.w0.rows + tile * 16 * NT + 16 * t + n_in;
     }
     // up to 16 rows: one 16-row token tile; otherwise passes of two tiles (one pass up to 32 rows)
     if (re - rb <= 16) {
-      skinny_pass<T, WF, MODE, 1, KS>(p, experts, wrow, tile, rb, re, nch, lane, pin_prefetch);
+      skinny_pass<T, WF, MODE, 1, KS, NT>(p, experts, wrow, tile, rb, re, nch, lane, pin_prefetch);
     } else {
-      for (int r0 = rb; r0 < re; r0 += 32) skinny_pass<T, WF, MODE, 2, KS>(p, experts, wrow, tile, r0, re, nch, lane, false);
+      for (int r0 = rb; r0 < re; r0 += 32) skinny_pass<T, WF, MODE, 2, KS, NT>(p, experts, wrow, tile, r0, re, nch, lane, false);
     }
   }
 }
@@ -679,18 +680,30 @@ static int pick_waves(int64_t items, int wg_per_cu) {
 template <typename T, int WF>
 static int launch_skinny_t(int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   const int tiles = (int)(mode == MODE_GATEUP ? p.n_out / 16 : p.n_out / 32);
-  // at most min(E, rows) experts receive rows; with so few items that four wavefronts per item still fit the chip,
-  // a workgroup shares each item and splits its reduction
+  // At most min(E, rows) experts receive rows.  With so few items that four wavefronts per item fit the chip, a workgroup shares
+  // each item and splits its reduction: down projections up to 1024 items (two rounds over the wavefronts that are resident),
+  // gate/up up to 768, where the second round is worth less than what it costs to start.  Measured (us, [4096, 14336] gate/up
+  // of one matrix, 896 items, Q8_0 / Q4_1): 7 rows split 29.4 / 27.6, whole items 25.5 / 23.4; 32 rows split 47.6 / 48.8, whole
+  // items through LDS 30.0 / 31.8; with 352 items split is the better one (9.7 / 12.0, 20 rows 14.5 / 16.1).
+  // A down projection whose items of 32 features are no more than half the CUs takes items of 16 instead (Q8_0, us, 32 / 16):
+  // [4096, 14336] 1 row 20.2 / 13.5, 8 rows 19.6 / 15.7, 32 rows 42.5 / 31.9; [1024, 4096] 8 rows 9.3 / 7.3; with 192 items 8 rows
+  // of [6144, 2048] 7.1 / 8.1.
   const int64_t active_bound = max_rows < p.E ? max_rows : p.E;
   const bool pin = max_rows <= 16;  // a handful of rows in the whole launch: the pinned, unconditional prefetch pays
   const int64_t items_bound = active_bound * tiles;
-  if (items_bound * 4 <= 2 * 1024 * SkinnyOcc<WF>::value && (p.kred >> 8) >= 4) {
+  // the most rows one expert can have: one per token (when the caller says how many tokens there are), else all of them
+  const int64_t rows_bound = p.expert_rows_bound > 0 && p.expert_rows_bound < max_rows ? p.expert_rows_bound : max_rows;
+  if (items_bound <= (mode == MODE_GATEUP ? 768 : 1024) && (p.kred >> 8) >= 4) {
     dim3 grid((unsigned)items_bound);
-    if (mode == MODE_GATEUP) grouped_skinny_kernel<T, WF, MODE_GATEUP, 4><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
-    else grouped_skinny_kernel<T, WF, MODE_DOWN, 4><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
+    if (mode == MODE_GATEUP) grouped_skinny_kernel<T, WF, MODE_GATEUP, 4, 2><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
+    else if (items_bound <= 128)
+      grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 1><<<dim3((unsigned)items_bound * 2), 256, 0, st>>>(p, tiles * 2, (int)items_bound * 2, pin);
+    else grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 2><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
     return check_launch("grouped_skinny(split)");
   }
-  {
+  // gate/up launches of up to 1024 items and one token tile per expert: a wavefront per item (one round)
+  const bool whole_items = mode == MODE_GATEUP && items_bound <= 1024 && rows_bound <= 16;
+  if (!whole_items) {
     // token rows shared through LDS: needs whole groups of four tiles and 32-bit token offsets.  The down projection
     // has four times fewer groups than the gate/up projection; with few rows per expert (one token tile, few loads to
     // share) it is better off with independent wavefronts.
@@ -700,8 +713,6 @@ static int launch_skinny_t(int mode, const GemmParams& p, int64_t max_rows, hipS
       const int64_t groups = (int64_t)(tiles / 4) * p.E, capacity = 256 * SkinnyLdsOcc<WF>::value;
       const int64_t per_wg = (groups + capacity - 1) / capacity;
       dim3 grid((unsigned)((groups + per_wg - 1) / per_wg));
-      // the most rows one expert can have: one per token (when the caller says how many tokens there are), else all of them
-      const int64_t rows_bound = p.expert_rows_bound > 0 && p.expert_rows_bound < max_rows ? p.expert_rows_bound : max_rows;
       if (rows_bound <= 32) {
         if (mode == MODE_GATEUP) grouped_skinny_lds_kernel<T, WF, MODE_GATEUP, 2><<<grid, 256, 0, st>>>(p, tiles);
         else grouped_skinny_lds_kernel<T, WF, MODE_DOWN, 2><<<grid, 256, 0, st>>>(p, tiles);
@@ -714,8 +725,8 @@ static int launch_skinny_t(int mode, const GemmParams& p, int64_t max_rows, hipS
   }
   const int waves = pick_waves((int64_t)tiles * p.E, SkinnyOcc<WF>::value);
   dim3 grid((unsigned)(waves / 4));
-  if (mode == MODE_GATEUP) grouped_skinny_kernel<T, WF, MODE_GATEUP, 1><<<grid, 256, 0, st>>>(p, tiles, waves, pin);
-  else grouped_skinny_kernel<T, WF, MODE_DOWN, 1><<<grid, 256, 0, st>>>(p, tiles, waves, pin);
+  if (mode == MODE_GATEUP) grouped_skinny_kernel<T, WF, MODE_GATEUP, 1, 2><<<grid, 256, 0, st>>>(p, tiles, waves, pin);
+  else grouped_skinny_kernel<T, WF, MODE_DOWN, 1, 2><<<grid, 256, 0, st>>>(p, tiles, waves, pin);
   return check_launch("grouped_skinny");
 }
 

@@ -755,3 +755,40 @@ def test_dense_16_bit_kernel_against_the_tile_kernel_and_fp64(device, rows, K, N
     if y is not None:
         assert O.rel_l2(down[_hip.VARIANT_DENSE].double(), y) < eps
         assert O.rel_l2(auto.cpu().double(), y) < 2 * eps  # (a z element may round the other way under another kernel)
+
+
+@pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16)])
+@pytest.mark.parametrize("rows,n_out", [(1, 4096), (16, 4096), (17, 4128), (32, 32), (32, 4096), (5, 1056)])
+def test_streamed_single_matrix_items_of_16_and_32_features(device, rows, n_out, fmt, dtype):
+    """A single matrix with few rows: items of 16 output features up to 4096 of them, of 32 beyond, one and two token tiles."""
+    import moe_cases as MC
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    g = torch.Generator().manual_seed(rows + n_out)
+    w = torch.randn(n_out, 1280, generator=g) * 0.03
+    planes = dict(zip(("d", "qs"), O.quantize_q8_0(w))) if fmt == "q8_0" else dict(zip(("d", "m", "qs"), O.quantize_q4_1(w)))
+    dw = device_weight(MC.to_inference_tensor(fmt, planes, [n_out, 1280], "w", device), stacked=False, prepack=True)
+    x = torch.randn(rows, 1280, generator=g).to(dtype).to(device)
+    got, tile = _hip.mmt(x, dw), _hip.mmt(x, dw, variant=_hip.VARIANT_MFMA_TILE)
+    # the same products in another order: a value moves by one unit of the last place where the sum sits at a rounding boundary
+    assert O.rel_l2(got.cpu().double(), tile.cpu().double()) < 2.0 ** (-11 if dtype == torch.float16 else -8) / 4
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17])
+@pytest.mark.parametrize("N", [12288, 12544, 16384, 16640])
+def test_streamed_gate_up_on_both_sides_of_its_splits(device, rows, N):
+    """Gate/up of 768 and 1024 items and one tile more: reduction split over a workgroup, whole items, items through LDS."""
+    import moe_cases as MC
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    g = torch.Generator().manual_seed(N + rows)
+    dws = []
+    for shape in ([N, 1024], [N, 1024], [1024, N]):
+        w = torch.randn(shape, generator=g) * 0.03
+        dws.append(device_weight(MC.to_inference_tensor("q8_0", dict(zip(("d", "qs"), O.quantize_q8_0(w))), shape, "w", device), stacked=False, prepack=True))
+    x = torch.randn(rows, 1024, generator=g).to(torch.float16).to(device)
+    got, tile = (_hip.grouped_ffn(x, *dws, _hip.ACT_SILU, None, None, 1, variant=v) for v in (_hip.VARIANT_AUTO, _hip.VARIANT_MFMA_TILE))
+    # (see above; the intermediate is rounded as well)
+    assert O.rel_l2(got.cpu().double(), tile.cpu().double()) < 2.0 ** -11 / 2
