@@ -96,11 +96,18 @@ static constexpr int64_t kSkinnyMaxRowsSingleSplit = 32;
 // fp32 partial tiles and their sum.  Measured ([out, in] Q8_0 fp16, narrow / split, us): [14336, 4096] 192 rows 42 / 58,
 // 256 rows 45 / 64 (0.67 PFLOP/s), 384 rows 81 / 73; [4096, 4096] 192 ... 1024 rows 33 ... 47 / 42 ... 67; [8192, 8192] 256
 // rows 75 / 69; [4096, 14336] 256 rows 123 / 86.  Without scratch the 256 x 256 kernel takes 1.15 us per step unsplit.
-static bool narrow_pays(int mode, const GemmParams& p, int64_t rows) {
+// Where tiles of 64 are more than the CUs, tiles of 128 features x 256 rows (1.0 us per K step) against the split: they pay once the
+// partial tiles, which grow with features x rows, cost more than the reduction that the split shortens; the 4-bit format converts
+// faster and pays sooner.  Measured (128-row tiles / split, us, Q4_1 bf16; Q8_0 fp16): [14336, 4096] 257 rows 65 / 62; 68 / 61, 300
+// rows 63 / 70; 68 / 65, 512 rows 67 / 78; 71 / 75; [8192, 4096] 513 rows 64 / 66; 68 / 65, 1024 rows 70 / 85; 75 / 82; [16384, 2048]
+// 300 rows 35 / 52; 38 / 50; [14336, 6144] 300 rows 91 / 89; 99 / 83, 512 rows 95 / 100; 101 / 96.
+static bool narrow_pays(int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (rows <= 128) return false;
-  const int64_t features = mode == MODE_GATEUP ? 32 : 64;
+  const int64_t features = (mode == MODE_GATEUP ? 32 : 64) * (narrow_wide(mode, p.n_out, rows) ? 2 : 1);
   if (p.n_out % features != 0) return false;
   if (p.n_out / features * ((rows + 255) / 256) > 256) return false;
+  if (narrow_wide(mode, p.n_out, rows))
+    return p.split_scratch && p.kred <= 6144 && p.n_out * (mode == MODE_GATEUP ? 2 : 1) * rows >= p.kred * (wtag == WF_Q4_1_P ? 1024 : 1600);
   return p.split_scratch == nullptr || p.kred <= 6144;
 }
 // Unquantized 16-bit weights: the kernel that brings both operands straight into LDS, against the streaming kernel.  For the
@@ -141,7 +148,7 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     // (one matrix, with or without an offsets array around its rows)
     else if (dense_pays(dtype, wtag, mode, p, max_rows)) variant = 11;
     else if (p.E == 1) variant = max_rows <= (p.split_scratch ? kSkinnyMaxRowsSingleSplit : kSkinnyMaxRowsSingle) ? 3
-                                 : narrow_pays(mode, p, max_rows) ? 9 : 6;
+                                 : narrow_pays(wtag, mode, p, max_rows) ? 9 : 6;
     else if (p.offsets && ((p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) ||
                            max_rows <= kSkinnyMaxRows || max_rows <= skinny_max_avg_rows(p.E) * p.E)) variant = 3;
     // Everything else goes to the 256 x 256 kernel (which hands shapes it does not take down to the 128 x 128 one).

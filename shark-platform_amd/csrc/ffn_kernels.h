@@ -165,6 +165,11 @@ bool dense_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t
 int launch_dense(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_tile(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_big(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
+// Whether the narrow tiles take 128 weight rows instead of 64: where tiles of 64 x 256 are more than the CUs.
+static inline bool narrow_wide(int mode, int64_t n_out, int64_t rows) {
+  const int64_t features = mode == MODE_GATEUP ? 32 : 64;
+  return n_out % (2 * features) == 0 && n_out / features * ((rows + 255) / 256) > 256;
+}
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, float* partial, hipStream_t st);
 size_t mfma_ws_partial_bytes();

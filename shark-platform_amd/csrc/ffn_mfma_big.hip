@@ -38,6 +38,9 @@ struct BigTagOff { static constexpr bool value = false; };
 // hundred rows: 256 rows of a [14336, 4096] matrix are 56 tiles of 256 x 256 but 224 of 64 x 256, which fill the CUs
 // without cutting the reduction (no fp32 partial tiles, no workspace).  A K step then has only four weight pieces: the
 // first four wavefronts load and convert one each, the others only send token rows.
+// TI = 4 (128 weight rows, a piece for every wavefront) is for the sizes at which tiles of 64 are more than the CUs, such as 257 to
+// 512 rows of that matrix: 300 rows in Q4_1 bf16 69.7 us with a split reduction, 63.7 here; of [16384, 2048] in Q8_0 52 and 36.
+// What bounds it is the 1.0 us of a K step (conversion, then 32 MFMAs per wavefront behind one barrier).
 template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI>
 __global__ void __launch_bounds__(64 * WN * WM, 1)
 grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
@@ -352,20 +355,19 @@ int launch_mfma_big(int act_dtype, int wtag, int mode, const GemmParams& p, int6
   return set_error(STMOE_ERR_UNSUPPORTED, "mfma big kernel: activation dtype %d", act_dtype);
 }
 
-// The narrow form: 64 weight rows x 256 token rows per workgroup (see the kernel's head).
-#ifndef STMOE_NARROW_TI
-#define STMOE_NARROW_TI 2
-#endif
+// The narrow form: 64 weight rows x 256 token rows per workgroup (see the kernel's head), or 128 where tiles of 64 would not fit
+// one round over the 256 CUs (narrow_pays says where either is chosen).
 template <typename T, int WF>
 static int launch_narrow_t(int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
-  if (mode == MODE_GATEUP) return launch_big_m<T, WF, MODE_GATEUP, 2, 4, 2, STMOE_NARROW_TI>(p, max_rows, st);
-  return launch_big_m<T, WF, MODE_DOWN, 2, 4, 2, STMOE_NARROW_TI>(p, max_rows, st);
+  const bool wide = narrow_wide(mode, p.n_out, max_rows);
+  if (mode == MODE_GATEUP) return wide ? launch_big_m<T, WF, MODE_GATEUP, 2, 4, 2, 4>(p, max_rows, st) : launch_big_m<T, WF, MODE_GATEUP, 2, 4, 2, 2>(p, max_rows, st);
+  return wide ? launch_big_m<T, WF, MODE_DOWN, 2, 4, 2, 4>(p, max_rows, st) : launch_big_m<T, WF, MODE_DOWN, 2, 4, 2, 2>(p, max_rows, st);
 }
 
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
   if (p.offsets && p.E > 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma narrow kernel: at most 64 experts");
-  if (p.kred % 256 != 0 || p.lda % 8 != 0 || p.ldo % 4 != 0 || p.n_out % (mode == MODE_GATEUP ? 16 * STMOE_NARROW_TI : 32 * STMOE_NARROW_TI) != 0)
+  if (p.kred % 256 != 0 || p.lda % 8 != 0 || p.ldo % 4 != 0 || p.n_out % (mode == MODE_GATEUP ? 32 : 64) != 0)
     return set_error(STMOE_ERR_UNSUPPORTED, "mfma narrow kernel: needs K %% 256 == 0 and output features in whole tiles");
   {
     const int64_t src_rows = p.perm ? (max_rows + p.k_top - 1) / p.k_top : max_rows;

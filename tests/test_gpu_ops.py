@@ -792,3 +792,25 @@ def test_streamed_gate_up_on_both_sides_of_its_splits(device, rows, N):
     got, tile = (_hip.grouped_ffn(x, *dws, _hip.ACT_SILU, None, None, 1, variant=v) for v in (_hip.VARIANT_AUTO, _hip.VARIANT_MFMA_TILE))
     # (see above; the intermediate is rounded as well)
     assert O.rel_l2(got.cpu().double(), tile.cpu().double()) < 2.0 ** -11 / 2
+
+
+@pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16), ("fp8", torch.float16)])
+@pytest.mark.parametrize("rows", [257, 300, 512, 700])
+def test_narrow_tiles_of_128_features(device, fmt, dtype, rows):
+    """A single matrix whose tiles of 64 features are more than the CUs: tiles of 128 (bit for bit against the 128 x 128 kernel: both
+    keep one running sum in the same order), and tiles of 64 where 128 does not divide its features; the gated form beside it."""
+    import moe_cases as MC
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows)).to(dtype).to(device)
+    for N in (8320, 8384):  # 130 and 131 tiles of 64, two or three tiles of rows
+        case = MC.build(MC.Case(T=4, K=256, N=N, E=1, k=1, fmt=fmt, dtype=dtype, seed=430))
+        dws = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], [1, N, 256], n, device), stacked=True, prepack=True) for n in ("gate", "up")]
+        narrow, tile = (_hip.mmt(x, dws[0], variant=v) for v in (_hip.VARIANT_MFMA_NARROW, _hip.VARIANT_MFMA_TILE))
+        assert torch.equal(narrow.view(torch.int16), tile.view(torch.int16))
+        idx = torch.zeros(rows, 1, dtype=torch.int32, device=device)
+        _, offsets, perm, _ = _hip.dispatch_build(idx, 1)
+        got, want = (_hip.grouped_gate_up(x, *dws, _hip.ACT_SILU, offsets, perm, 1, variant=v) for v in (_hip.VARIANT_MFMA_NARROW, _hip.VARIANT_MFMA_TILE))
+        # (the same sums; the gated product may be rounded once more or less on the way: one unit of the last place)
+        assert O.rel_l2(got.cpu().double(), want.cpu().double()) < 2.0 ** (-11 if dtype == torch.float16 else -8)
