@@ -435,6 +435,7 @@ class DeviceWeight:
         )
         self.format = fmt
         self.experts, self.rows, self.cols = experts, rows, cols
+        self.padded = False  # whether rows or cols are larger than those of the tensor it was made from (prepack)
 
     @property
     def ref(self):
@@ -480,6 +481,7 @@ class DeviceWeight:
             new_d = d if fp8 else torch.empty(lead + [blocks, 1], dtype=d.dtype, device=d.device)
             new_m = None if m is None else torch.empty_like(new_d)
         out = DeviceWeight(_PACKED_OF[self.format], self.experts, rows, cols, new_qs, new_d, new_m, self.desc.dtype)
+        out.padded = (rows, cols) != (self.rows, self.cols)
         with _on_device(self.device):
             _check(lib.stmoe_prepack(self.ref, out.ref, _stream(self.device)))
         return out
@@ -495,6 +497,13 @@ class DeviceWeight:
         with _on_device(self.device):
             _check(lib.stmoe_unpack(self.ref, out.ref, _stream(self.device)))
         return out
+
+
+def _ffn_variant(variant: int, w_gate: DeviceWeight) -> int:
+    """The kernel variant of a fused FFN call.  The automatic choice takes fp8 layers with static quantizers to the fp8 matrix
+    cores where the FFN width is a multiple of 256; a width that was padded to one (ops.ffn_device_weights) is none, so such a
+    layer keeps the kernels that dequantise, round and multiply as the reference does."""
+    return VARIANT_STEP_BY_STEP if variant == VARIANT_AUTO and w_gate.padded else variant
 
 
 GGUF_Q8_0, GGUF_Q4_1 = 0, 1
@@ -552,8 +561,8 @@ def grouped_ffn(x, w_gate: DeviceWeight, w_up: DeviceWeight, w_down: DeviceWeigh
     xs, zs = _scale1(x_scale), _scale1(z_scale)
     with _on_device(dev):
         _check(lib.stmoe_grouped_ffn(_ptr(x_c), dtype_enum(x_c.dtype), T, K, N, E, k, w_gate.ref, w_up.ref, w_down.ref, act,
-                                     _ptr(offsets), _ptr(perm), _ptr(xs), _ptr(zs), _ptr(y), _ptr(workspace), workspace.numel(), variant,
-                                     _stream(dev)))
+                                     _ptr(offsets), _ptr(perm), _ptr(xs), _ptr(zs), _ptr(y), _ptr(workspace), workspace.numel(),
+                                     _ffn_variant(variant, w_gate), _stream(dev)))
     return y
 
 
@@ -686,7 +695,8 @@ def moe_forward(h, ffn_norm_w, out_norm_w, eps: float, w_router, w_gate: DeviceW
     xs, zs = _scale1(x_scale), _scale1(z_scale)
     args = (_ptr(h_c), dtype_enum(h_c.dtype), T, K, N, E, k, _ptr(ffn_norm_w), _ptr(out_norm_w),
             dtype_enum(ffn_norm_w.dtype), float(eps), _ptr(w_router), w_gate.ref, w_up.ref, w_down.ref, act,
-            _ptr(xs), _ptr(zs), _ptr(out), _ptr(idx), _ptr(gate), _ptr(workspace), workspace.numel(), variant, _stream(dev))
+            _ptr(xs), _ptr(zs), _ptr(out), _ptr(idx), _ptr(gate), _ptr(workspace), workspace.numel(), _ffn_variant(variant, w_gate),
+            _stream(dev))
     with _on_device(dev):
         if events is None:
             _check(lib.stmoe_moe_forward(*args))
@@ -713,7 +723,7 @@ def moe_forward_static(h, ffn_norm_w, out_norm_w, eps: float, w_router, w_gate: 
         _check(lib.stmoe_moe_forward_static(_ptr(h), dtype_enum(h.dtype), T, K, w_gate.rows, w_gate.experts, k, _ptr(ffn_norm_w),
                                             _ptr(out_norm_w), dtype_enum(ffn_norm_w.dtype), float(eps), _ptr(w_router), w_gate.ref,
                                             w_up.ref, w_down.ref, act, _ptr(x_scale), _ptr(z_scale), _ptr(out), _ptr(idx), _ptr(gate),
-                                            variant, _stream(dev)))
+                                            _ffn_variant(variant, w_gate), _stream(dev)))
     return out
 
 

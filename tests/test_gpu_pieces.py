@@ -369,6 +369,29 @@ def test_block_with_padded_width_against_the_oracle(device, fmt, dtype, N, T):
     assert err < (1e-3 if dtype == torch.float16 else 3e-3) + step * float(want.float().norm() / moe.norm()), err
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N", [320, 704, 1408])
+@pytest.mark.parametrize("T", [159, 160, 400])
+def test_fp8_block_with_padded_width_and_quantizers(device, dtype, N, T):
+    """Static quantizers on both activations of an fp8 layer whose width was padded, on both sides of the 320 pairs from which
+    widths that are multiples of 256 go to the fp8 matrix cores: these widths do not, whatever they were padded to."""
+    from sharktank_amd.layers import MoeBlock
+
+    case = MC.build(MC.Case(T=T, K=512, N=N, fmt="fp8", dtype=dtype, act_quant=True, seed=53))
+    block = MoeBlock(MC.make_theta(case, device), case.E, case.k, case.eps)
+    assert all(w.is_packed and w.padded for w in block.experts.device_weights())
+    h = case.planes["h"].reshape(1, T, 512)
+    y, idx, _ = block(h.to(device), return_routing=True)
+    block.experts.kernel_variant = _hip().VARIANT_STEP_BY_STEP
+    assert torch.equal(y.view(torch.int16), block(h.to(device)).view(torch.int16))
+    want, want_idx, _ = MC.oracle_block(case)
+    assert torch.equal(idx.cpu().long(), want_idx)
+    moe = want.float() - case.planes["h"].float()
+    err = float((y.reshape(T, 512).cpu().float() - want.float()).norm() / moe.norm())
+    step = 2.0 ** (-11 if dtype == torch.float16 else -8)  # the residual sum's own rounding, half a step of the output each way
+    assert err < (1e-3 if dtype == torch.float16 else 3e-3) + step * float(want.float().norm() / moe.norm()), err
+
+
 def test_prepack_layout_definition(device):
     """Spot-checks the documented order: lane 16*g + n of block (row tile rt, k block kb) holds row 16*rt+n,
     k = 64*kb + 16*g .. +15; scales of 8 consecutive blocks of a row are contiguous."""
