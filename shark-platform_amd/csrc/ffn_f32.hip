@@ -7,9 +7,14 @@
 // 32 features where they divide), its four wavefronts a quarter of the reduction each: a layer of 8 x 1024 x 512 has 512 such
 // items, 2048 wavefronts, whose loads are all in flight after two steps.  The quarters are added through LDS in a fixed order.
 // Measured (8 experts, top-2, gate/up + down, us; general kernel / this one): 64 tokens of 512 x 1024 71 + 33 / 17 + 11; the
-// whole layer 110 / 37 us, of which the host takes 31.  109 tokens of 896 x 1280: layer 325 / 72 us; 101 tokens of 256 x 1152
+// whole layer 110 / 38 us, of which the host takes 31.  109 tokens of 896 x 1280: layer 325 / 69 us; 101 tokens of 256 x 1152
 // 154 / 47.  At 10 tokens of 768 x 1536 the gate/up launch reads 3.3 TB/s; with 25 rows per expert and more the time goes into the
 // multiplications (32 cycles each for 16 x 16 x 4).  Eight wavefronts per item instead of four: no change.
+// Order of the sums: the matrix instruction rounds after every product, so one running sum per quarter was up to 3.6 times as far
+// from fp64 as the general kernel, whose 64 lanes hold short sums (K = 4096: rms error 9.6 / 2.7 times 2^-24 of the result's rms;
+// K = 512: 3.5 / 1.6).  A chunk of 64 elements is eight sums of 8 products, added in pairs: 1.9 and 1.4, below the general kernel at
+// every K from 64 to 4096.  The additions run beside the other wavefront's products: layers of the sizes above 0 to 4 % slower, a
+// product of 2000 x 1024 x 1024 6 % faster.
 //
 // Operands: weight rows are the MFMA "A" rows, token rows the "B" columns; one step multiplies 4 reduction elements, one per
 // lane group.  The operands only have to agree on which element a lane holds, so a lane loads what is contiguous for it:
@@ -90,12 +95,26 @@ __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, const int64
     float v[NT][16];
 #pragma unroll
     for (int t = 0; t < NT; ++t) w[t].values(v[t]);
+    // A chunk's sixteen instructions are eight chains of two, which start at zero and are added in pairs; the chunk's sum then
+    // goes to the running one.
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int mt = 0; mt < MT; ++mt) {
+        floatx4_t half[2];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][s], x[mt][s >> 2][s & 3], acc[mt][t], 0, 0, 0);
+        for (int h = 0; h < 2; ++h) {
+          floatx4_t c[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][8 * h + 2 * i], x[mt][2 * h + (i >> 1)][(2 * i) & 3], (floatx4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][8 * h + 2 * i + 1], x[mt][2 * h + (i >> 1)][(2 * i + 1) & 3], c[i], 0, 0, 0);
+          half[h] = (c[0] + c[1]) + (c[2] + c[3]);
+        }
+        acc[mt][t] += half[0] + half[1];
+        // (finished here: sunk behind the next chunk's loads, the adds would keep the chains of all tiles in registers)
+        asm volatile("" : "+v"(acc[mt][t]));
+      }
   };
   if (c_begin < c_end) {
     // Both operands one chunk ahead while the registers allow it (four token tiles: the weights only).  Requests are

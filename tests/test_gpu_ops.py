@@ -712,6 +712,21 @@ def test_f32_layers_against_the_general_kernel_and_fp64(device, fmt, T, K, N, E,
         assert O.rel_l2(y.cpu().double(), want) < tol
 
 
+@pytest.mark.parametrize("K", [64, 128, 512, 1024, 2048, 4096])
+def test_f32_products_are_no_further_from_fp64_than_the_general_kernel(device, K):
+    """Rounding error of the fp32 matrix-core kernel's sums against that of the general kernel, whose lanes add 1/64 of the
+    products each (tiles of 64, 32 and 16 rows, dense weights)."""
+    from sharktank_amd import _hip
+
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(112, K, generator=g), torch.randn(256, K, generator=g) / K ** 0.5
+    want = x.double() @ w.double().T
+    dw = _hip.DeviceWeight(_hip.W_DENSE, 1, 256, K, w.to(device), None, None, _hip.F32)
+    err = {v: O.rel_l2(_hip.mmt(x.to(device), dw, variant=v).cpu().double(), want) for v in (_hip.VARIANT_AUTO, _hip.VARIANT_GENERIC)}
+    # a mean over 28672 rounding errors: 1 % of itself, so 5 % are room enough
+    assert err[_hip.VARIANT_AUTO] < 1.05 * err[_hip.VARIANT_GENERIC], err
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,K,N,act", [
     ((1, 0, 15, 16), 64, 64, "silu"),               # one K step; fewer weight rows than one wide unit
