@@ -177,7 +177,7 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
           const floatx4_t ga = acc[ti][tj], ua = acc[ti + TI / 2][tj];
           const float gq[4] = {ga[0], ga[1], ga[2], ga[3]}, uq[4] = {ua[0], ua[1], ua[2], ua[3]};
           uint2* dst = reinterpret_cast<uint2*>(orow + ti * 16);
-          if (p.act == STMOE_ACT_SILU) *dst = gateup_quad<T, STMOE_ACT_SILU>(gq, uq, fq);
+          if (p.act == STMOE_ACT_SILU) *dst = gateup_quad<T, ACT_SILU_IEEE>(gq, uq, fq);
           else *dst = gateup_quad<T, STMOE_ACT_GELU_ERF>(gq, uq, fq);
         }
       } else {

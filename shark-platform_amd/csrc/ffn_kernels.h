@@ -106,9 +106,14 @@ template <typename T> __device__ __forceinline__ float gateup_epilogue(int act, 
 // hardware exp2 / rcp (about 1 ulp of fp32 each, far below the rounding to the 16-bit activation dtype that
 // follows); for fp16 the last product is a packed fp16 multiply, which rounds the exact product once like the fp32
 // multiply followed by the conversion.
+// ACT_SILU_IEEE: SiLU with expf and a division instead (the kernel of unquantized weights, which waits for memory: it gives the
+// bits of the 128 x 128 kernel).
+enum : int { ACT_SILU_IEEE = 0x100 };
 template <int ACT> __device__ __forceinline__ float act_fast(float v) {
   if constexpr (ACT == STMOE_ACT_SILU)
     return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v * -1.44269504088896340736f));
+  else if constexpr (ACT == ACT_SILU_IEEE)
+    return act_silu(v);
   else
     return act_gelu_erf(v);
 }

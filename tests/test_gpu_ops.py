@@ -751,7 +751,8 @@ def test_dense_16_bit_kernel_against_the_tile_kernel_and_fp64(device, rows, K, N
     idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))[torch.randperm(T, generator=g)].to(torch.int32).reshape(T, 1)
     _, offsets, perm, _ = _hip.dispatch_build(idx.to(device), E)
     act_id = _hip.ACT_SILU if act == "silu" else _hip.ACT_GELU_ERF
-    z = _hip.grouped_gate_up(x.to(device), dg, du, act_id, offsets, perm, 1, variant=_hip.VARIANT_DENSE)
+    z, z_tile = (_hip.grouped_gate_up(x.to(device), dg, du, act_id, offsets, perm, 1, variant=v) for v in (_hip.VARIANT_DENSE, _hip.VARIANT_MFMA_TILE))
+    assert torch.equal(z.view(torch.int16), z_tile.view(torch.int16))  # (the same sums, and the activation function as precise)
     pairs = perm.cpu().long()
     xs, e = x[pairs].double(), idx.reshape(-1)[pairs].long()
     want = torch.empty(T, N, dtype=torch.float64)
