@@ -90,35 +90,47 @@ static constexpr int kBigChunkSlotsPerXcd = 32;  // rest * chunks <= 32
 struct BigPlan {
   int F, R, f0, f1, r0, r1, whole, rest, chunks;
 };
-// The offsets are fetched with one vector load (lane l holds offsets[l]) and read back with readlane: walking them with
-// scalar loads costs one memory latency per expert, twice per workgroup.  At most 64 experts (checked
-// by the launchers): with 64 the last offset has no lane and is fetched where a walk gets that far (64 experts of
-// 2048 x 1408 with 37 rows each: layer 395 us on the 128 x 128 kernel, 338 us here).
+// The offsets are fetched with one vector load (lane l holds offsets[l]); walking them with scalar loads costs one memory
+// latency per expert, twice per workgroup.  At most 64 experts (checked by the launchers): with 64 the last offset has no
+// lane and comes with a load of its own.
 __device__ __forceinline__ int big_lane_offsets(const GemmParams& p) {
   const int lane = threadIdx.x & 63;
   return (p.offsets && lane <= p.E) ? p.offsets[lane] : 0;
 }
-__device__ __forceinline__ int big_offset(const GemmParams& p, int lane_off, int i) {
-  return i < 64 ? __builtin_amdgcn_readlane(lane_off, i) : p.offsets[i];
+// Every lane counts the token tiles of its own expert, one scan numbers them and a ballot finds the expert of a unit.  A walk over
+// the experts, one after the other, cost every unit some 700 cycles per expert: gate/up of 64 experts of 2048 x 512 at 400 tokens,
+// two units per CU, 60 us (69 on the 128 x 128 kernel), here 31; the down projection 71 (36) and 27; 8 experts 2 to 4 us less.
+struct BigLanes {
+  int begin, rows;   // this lane's expert (rows 0: no expert)
+  int main;          // its main tiles
+  int main_end;      // main tiles of the experts up to and including this one
+  uint64_t partial;  // experts that have a partial tile
+  uint64_t even;     // experts whose main tiles are of equal size
+};
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8: sums inside each row of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15: rows 1 and 3 take the row before along
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31: rows 2 and 3 take the first half along
+  return v;
 }
-__device__ __forceinline__ BigPlan big_plan(const GemmParams& p, int lane_off, int BM, int n_tiles, int xcd, bool allow_split,
-                                            bool absorb = false, int balance = 0) {
-  BigPlan pl;
-  pl.F = 0;
-  pl.R = 0;
+__device__ __forceinline__ BigLanes big_lanes(const GemmParams& p, int lane_off, int lane, int BM, bool absorb, int balance) {
+  int begin = 0, rows = lane == 0 ? (int)p.fixed_rows : 0;
   if (p.offsets) {
-    for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0); e < p.E; ++e) {
-      const int end = big_offset(p, lane_off, e + 1), rows = end - b;
-      b = end;
-      const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
-      pl.F += x.main;
-      pl.R += x.partial;
-    }
-  } else {
-    const BigExpertTiles x = big_expert_tiles((int)p.fixed_rows, BM, absorb, balance);
-    pl.F = x.main;
-    pl.R = x.partial;
+    int end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);  // (lane 63 reads lane 0: no expert unless there are 64)
+    if (p.E == 64) end = lane == 63 ? p.offsets[64] : end;
+    begin = lane_off;
+    rows = lane < p.E ? end - begin : 0;
   }
+  const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
+  return BigLanes{begin, rows, x.main, wave_inclusive_sum(x.main), __ballot(x.partial != 0), __ballot(x.even)};
+}
+__device__ __forceinline__ BigPlan big_plan(const BigLanes& l, int n_tiles, int xcd, bool allow_split) {
+  BigPlan pl;
+  pl.F = __builtin_amdgcn_readlane(l.main_end, 63);
+  pl.R = __popcll(l.partial);
   const int UF = pl.F * n_tiles, UR = pl.R * n_tiles;
   pl.f0 = (int)((int64_t)UF * xcd / 8);
   pl.f1 = (int)((int64_t)UF * (xcd + 1) / 8);
@@ -162,10 +174,10 @@ __device__ __forceinline__ void big_set_tail(int b, int rows, int BM, int s, boo
   t.tail_rows = min(kBigTailRows, rows - first);
 }
 // Rows of main tile s of an expert (first row b, `rows` rows) and the tail rows it takes along.
-__device__ __forceinline__ void big_main_tile(int b, int rows, int BM, int s, const BigExpertTiles& x, bool absorb, BigTile& t) {
-  if (x.even) {
-    t.row_begin = b + (int)((int64_t)rows * s / x.main);
-    t.row_end = b + (int)((int64_t)rows * (s + 1) / x.main);
+__device__ __forceinline__ void big_main_tile(int b, int rows, int BM, int s, int main, bool even, bool absorb, BigTile& t) {
+  if (even) {
+    t.row_begin = b + (int)((int64_t)rows * s / main);
+    t.row_end = b + (int)((int64_t)rows * (s + 1) / main);
     t.tail_begin = 0;
     t.tail_rows = 0;
   } else {
@@ -174,106 +186,58 @@ __device__ __forceinline__ void big_main_tile(int b, int rows, int BM, int s, co
     big_set_tail(b, rows, BM, s, absorb, t);
   }
 }
-__device__ __forceinline__ bool big_unit(const GemmParams& p, int lane_off, int BM, int n_tiles, const BigPlan& pl, int unit, BigTile& t,
-                                         bool absorb = false, int balance = 0) {
-  int u;
-  bool partial;
+__device__ __forceinline__ bool big_unit(const BigLanes& l, int BM, int n_tiles, const BigPlan& pl, int unit, BigTile& t, bool absorb) {
   t.tail_begin = 0;
   t.tail_rows = 0;
   if (unit < pl.f1 - pl.f0) {
-    u = pl.f0 + unit;
-    partial = false;
-  } else if (unit - (pl.f1 - pl.f0) < pl.r1 - pl.r0) {
-    u = pl.r0 + unit - (pl.f1 - pl.f0);
-    partial = true;
-  } else {
-    return false;
-  }
-  if (!p.offsets) {
-    t.e = 0;
-    if (partial) {
-      t.ntile = u;
-      t.row_begin = (int)(p.fixed_rows / BM) * BM;
-      t.row_end = (int)p.fixed_rows;
-    } else {
-      int s;
-      big_full_unit(u, pl.F, n_tiles, s, t.ntile);
-      big_main_tile(0, (int)p.fixed_rows, BM, s, big_expert_tiles((int)p.fixed_rows, BM, absorb, balance), absorb, t);
-    }
+    int u = pl.f0 + unit;
+    const int e = __builtin_ctzll(__ballot(l.main_end * n_tiles > u));  // (u < F n_tiles: there is one)
+    const int b = __builtin_amdgcn_readlane(l.begin, e), rows = __builtin_amdgcn_readlane(l.rows, e);
+    const int main = __builtin_amdgcn_readlane(l.main, e);
+    u -= (__builtin_amdgcn_readlane(l.main_end, e) - main) * n_tiles;
+    int s;
+    big_full_unit(u, main, n_tiles, s, t.ntile);
+    t.e = e;
+    big_main_tile(b, rows, BM, s, main, (l.even >> e) & 1, absorb, t);
     return true;
   }
-  if (!partial) {
-    for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0), rows; e < p.E; ++e, b += rows) {
-      rows = big_offset(p, lane_off, e + 1) - b;
-      const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
-      const int units = x.main * n_tiles;
-      if (u < units) {
-        int s;
-        big_full_unit(u, x.main, n_tiles, s, t.ntile);
-        t.e = e;
-        big_main_tile(b, rows, BM, s, x, absorb, t);
-        return true;
-      }
-      u -= units;
-    }
-    return false;
-  }
+  if (unit - (pl.f1 - pl.f0) >= pl.r1 - pl.r0) return false;
+  const int u = pl.r0 + unit - (pl.f1 - pl.f0);
   t.ntile = u / pl.R;
-  int s = u - t.ntile * pl.R;
-  for (int e = 0, b = __builtin_amdgcn_readlane(lane_off, 0), rows; e < p.E; ++e, b += rows) {
-    rows = big_offset(p, lane_off, e + 1) - b;
-    if (big_expert_tiles(rows, BM, absorb, balance).partial) {
-      if (s == 0) {
-        t.e = e;
-        t.row_begin = b + rows / BM * BM;
-        t.row_end = b + rows;
-        return true;
-      }
-      --s;
-    }
-  }
-  return false;
+  const int s = u - t.ntile * pl.R;  // the s-th expert that has a partial tile
+  const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(l.partial >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)l.partial, 0u));
+  const int e = __builtin_ctzll(__ballot(before == s) & l.partial);
+  const int b = __builtin_amdgcn_readlane(l.begin, e), rows = __builtin_amdgcn_readlane(l.rows, e);
+  t.e = e;
+  t.row_begin = b + rows / BM * BM;
+  t.row_end = b + rows;
+  return true;
 }
+// Item j of an XCD's work list: the whole units first, then the chunks of the split ones.
+__device__ __forceinline__ bool big_item(const BigLanes& l, int BM, int n_tiles, const BigPlan& pl, int xcd, int j, BigTile& t,
+                                         bool absorb = false) {
+  int unit;
+  if (j < pl.whole) {
+    unit = j;
+    t.chunk = 0;
+    t.nchunks = 1;
+    t.chunk_slot = 0;
+  } else {
+    const int c = j - pl.whole;
+    if (c >= pl.rest * pl.chunks) return false;
+    unit = pl.whole + c / pl.chunks;
+    t.chunk = c % pl.chunks;
+    t.nchunks = pl.chunks;
+    t.chunk_slot = xcd * kBigChunkSlotsPerXcd + c;
+  }
+  return big_unit(l, BM, n_tiles, pl, unit, t, absorb);
+}
+// The item of a workgroup that takes one.
 __device__ __forceinline__ bool big_tile_id(const GemmParams& p, int BM, int n_tiles, bool allow_split, BigTile& t, bool absorb = false,
                                             int balance = 0) {
-  const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-  const int lane_off = big_lane_offsets(p);
-  const BigPlan pl = big_plan(p, lane_off, BM, n_tiles, xcd, allow_split, absorb, balance);
-  int unit;
-  if (j < pl.whole) {
-    unit = j;
-    t.chunk = 0;
-    t.nchunks = 1;
-    t.chunk_slot = 0;
-  } else {
-    const int c = j - pl.whole;
-    if (c >= pl.rest * pl.chunks) return false;
-    unit = pl.whole + c / pl.chunks;
-    t.chunk = c % pl.chunks;
-    t.nchunks = pl.chunks;
-    t.chunk_slot = xcd * kBigChunkSlotsPerXcd + c;
-  }
-  return big_unit(p, lane_off, BM, n_tiles, pl, unit, t, absorb, balance);
-}
-// Item j of an XCD's work list: the whole units first, then the chunks of the split ones (the same numbering as the
-// workgroup index j of big_tile_id), from a plan and offsets fetched once: for workgroups that walk several items.
-__device__ __forceinline__ bool big_item(const GemmParams& p, int lane_off, int BM, int n_tiles, const BigPlan& pl, int xcd, int j, BigTile& t,
-                                         bool absorb = false, int balance = 0) {
-  int unit;
-  if (j < pl.whole) {
-    unit = j;
-    t.chunk = 0;
-    t.nchunks = 1;
-    t.chunk_slot = 0;
-  } else {
-    const int c = j - pl.whole;
-    if (c >= pl.rest * pl.chunks) return false;
-    unit = pl.whole + c / pl.chunks;
-    t.chunk = c % pl.chunks;
-    t.nchunks = pl.chunks;
-    t.chunk_slot = xcd * kBigChunkSlotsPerXcd + c;
-  }
-  return big_unit(p, lane_off, BM, n_tiles, pl, unit, t, absorb, balance);
+  const int xcd = blockIdx.x & 7;
+  const BigLanes l = big_lanes(p, big_lane_offsets(p), threadIdx.x & 63, BM, absorb, balance);
+  return big_item(l, BM, n_tiles, big_plan(l, n_tiles, xcd, allow_split), xcd, blockIdx.x >> 3, t, absorb);
 }
 // Grid size that covers every XCD's share for at most `slots_bound` token tiles (a split adds up to 24 workgroups).
 static inline int big_grid(int n_tiles, int slots_bound, bool allow_split) {

@@ -220,7 +220,8 @@ grouped_mfma_ws_kernel(WsArgs args) {
   const int n_tiles = ka.n_tiles;
   float* const partial = ka.partial;
   const int xcd = blockIdx.x & 7, wg = blockIdx.x >> 3, wgs = ka.wgs_per_xcd;
-  const BigPlan pl = big_plan(p, lane_off, BM, n_tiles, xcd, partial != nullptr, true, kBalance);
+  const BigLanes lanes = big_lanes(p, lane_off, lane, BM, true, kBalance);
+  const BigPlan pl = big_plan(lanes, n_tiles, xcd, partial != nullptr);
   // Which item of round `round` (wgs consecutive items of the XCD's list) this workgroup takes: its own index shifted
   // by half a round plus one per round.  Neighbouring items differ systematically in cost (in a block of 32 full units the
   // first half belongs to an expert's first token tile, which carries most ride-along rows; partial units cycle through
@@ -228,7 +229,7 @@ grouped_mfma_ws_kernel(WsArgs args) {
   // collect one kind: the launch ends when the slowest workgroup does.
   const int slot = (wg + round * ((wgs >> 1) + 1)) % wgs;
   BigTile tile;
-  if (!big_item(p, lane_off, BM, n_tiles, pl, xcd, round * wgs + slot, tile, true, kBalance)) return;
+  if (!big_item(lanes, BM, n_tiles, pl, xcd, round * wgs + slot, tile, true)) return;
   const int e = tile.e, row_begin = tile.row_begin, row_end = tile.row_end, ntile = tile.ntile;
   const int rows_here = row_end - row_begin;
   // this workgroup's K steps: all of them, or one chunk of a split unit

@@ -376,3 +376,38 @@ def test_random_shapes_automatic_choice_against_vector_alu_kernel(device):
         alu = hip.grouped_ffn(x, *dws, act, offsets, perm, k, variant=hip.VARIANT_GENERIC)
         err = O.rel_l2(auto.float().cpu(), alu.float().cpu())
         assert torch.isfinite(auto.float()).all() and err < (2e-3 if dtype == torch.float16 else 1.2e-2), f"{what}: rel-L2 {err:.3e}"
+
+
+@pytest.mark.parametrize("E,K,N", [(33, 256, 768), (63, 256, 768), (64, 256, 768), (64, 1536, 256)])
+def test_many_experts_on_the_256_row_kernels(device, E, K, N):
+    """Row counts with every kind of token tile (none, a few rows, full, full with ride-along rows, two of equal size, a partial one
+    behind full ones) on up to 64 experts, with units left over that are split (K = 1536): the prefill kernel against the 128 x 128
+    kernel, the kernel of unquantized weights bit for bit against it."""
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    g = torch.Generator().manual_seed(E)
+    kinds = [0, 1, 17, 40, 256, 260, 470, 300, 0, 700]
+    rows = [kinds[int(i)] for i in torch.randint(0, len(kinds), (E - 2,), generator=g)] + [3, 290]  # (the last expert has a partial tile)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).to(torch.int32)
+    T = idx.numel()
+    idx = idx[torch.randperm(T, generator=g)].reshape(T, 1).to(device)
+    x = torch.randn(T, K, generator=g).to(torch.float16).to(device)
+    case = MC.build(MC.Case(T=4, K=K, N=N, E=E, k=1, fmt="q8_0", seed=E))
+    shapes = (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))
+    packed = [device_weight(MC.to_inference_tensor("q8_0", case.planes[n], s, n, device), stacked=True, prepack=True) for n, s in shapes]
+    dense = [_hip.DeviceWeight(_hip.W_DENSE, *s, w.contiguous().to(device), None, None, _hip.F16) for (_, s), w in zip(shapes, MC.dense_weights(case))]
+    _, offsets, perm, _ = _hip.dispatch_build(idx, E)
+    assert offsets.cpu().tolist() == [0, *torch.tensor(rows).cumsum(0).tolist()]
+    for dws, variant in ((packed, _hip.VARIANT_MFMA_WS), (dense, _hip.VARIANT_DENSE)):
+        z, z_tile = (_hip.grouped_gate_up(x, dws[0], dws[1], _hip.ACT_GELU_ERF, offsets, perm, 1, variant=v) for v in (variant, _hip.VARIANT_MFMA_TILE))
+        y, y_tile = (_hip.grouped_down(z_tile, dws[2], offsets, T, 1, variant=v) for v in (variant, _hip.VARIANT_MFMA_TILE))
+        for got, want in ((z, z_tile), (y, y_tile)):
+            if dws is dense:
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+            else:
+                # A split reduction adds in another order: gate, up, the activation and the product may each round the other way, one
+                # unit of the last place (2^-10) each, of the value or of the sum that cancelled to it.
+                size = torch.maximum(want.float().abs(), want.float().pow(2).mean(dim=1, keepdim=True).sqrt())
+                worst = ((got.float() - want.float()).abs() / size).amax(dim=1)
+                assert float(worst.max()) < 4 * 2.0 ** -10, int(worst.argmax())
