@@ -718,8 +718,21 @@ size_t mfma_ws_partial_bytes() { return big_partial_bytes(256, 256) + kWsTickets
 size_t mfma_ws_tickets_offset() { return big_partial_bytes(256, 256); }
 int mfma_ws_ticket_count() { return kWsTickets; }
 
-// `partial`: optional fp32 scratch of mfma_ws_partial_bytes() bytes; with it the last units of a launch, which would
-// run on a few CUs only, are split along the reduction.
+// Whether the last units of a launch, which would run on a few CUs only, are split along the reduction.  A K step saved is worth
+// 1.0 us (Q8_0, fp8) or 1.2 us (Q4_1); the fp32 partial tiles and their sum cost 15 us where a few units are split and 30 and more
+// where they are many.  So short reductions are left whole, and those up to 3072 where the launch has more than one unit per 24
+// reduction elements (its most: every expert with rows may have a tile of its own).  Measured (split / whole, us, [out, in] of one, 8
+// and 64 experts): Q8_0 [1024, 512] 8 experts 1024 tokens 39 / 19; [1024, 1280] 200 rows 28 / 28; [1024, 1536] 200 rows 29 / 32, 8 experts
+// 1024 tokens 48 / 39; [2048, 3072] 200 rows 35 / 55; Q4_1 [1024, 1024] 8 experts 1024 tokens 44 / 32; [1024, 1280] 200 rows 30 / 33.
+// Over 64 to 3000 tokens and 1024 to 4096 outputs, split took 0.97 to 3.0 times as long as whole where the rule leaves whole.
+static bool ws_split_pays(int wtag, int mode, const GemmParams& p, int64_t max_rows) {
+  if (p.kred <= (wtag == WF_Q4_1_P ? 1024 : 1280)) return false;
+  const int64_t tiles = p.n_out / (mode == MODE_GATEUP ? 128 : 256);
+  const int64_t units = tiles * ((max_rows + 255) / 256 + (p.offsets ? std::min<int64_t>(p.E, max_rows) : 0));
+  return p.kred > 3072 || units * 24 <= p.kred;
+}
+
+// `partial`: optional fp32 scratch of mfma_ws_partial_bytes() bytes for split units.
 int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, float* partial, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
   if (p.offsets && p.E > 64) return set_error(STMOE_ERR_UNSUPPORTED, "mfma ws kernel: at most 64 experts");
@@ -733,6 +746,7 @@ int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64
     if (src_rows * p.lda * 2 >= (int64_t)1 << 32)
       return set_error(STMOE_ERR_UNSUPPORTED, "mfma ws kernel: activations span 4 GB or more");
   }
+  if (!ws_split_pays(wtag, mode, p, max_rows)) partial = nullptr;
   if (act_dtype == STMOE_F16) {
     if (wtag == WF_Q8_0_P) return launch_ws_t<f16_t, WF_Q8_0_P>(mode, p, max_rows, partial, st);
     if (wtag == WF_Q4_1_P) return launch_ws_t<f16_t, WF_Q4_1_P>(mode, p, max_rows, partial, st);
