@@ -22,11 +22,6 @@ __all__ = ["device_weight", "expert_dispatch", "ffn_device_weights", "gather_exp
 _FLOAT_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
-def padded_width(n: int) -> int:
-    """The FFN width the packed matrix kernels run a width of `n` at: the next multiple of 256."""
-    return (n + 255) // 256 * 256
-
-
 def device_weight(w, *, stacked: bool, prepack: bool = False, pad=(None, None)) -> _hip.DeviceWeight:
     """C-ABI descriptor of a weight tensor.  `stacked`: [E, rows, cols]; otherwise a single [rows, cols] matrix.
     Planes are made contiguous once here (GGUF-derived planes are strided views of the raw blocks).  With
@@ -46,6 +41,21 @@ def device_weight(w, *, stacked: bool, prepack: bool = False, pad=(None, None)) 
     return dw
 
 
+def padded_ffn_width(gate, up, down):
+    """The width a gated FFN (gate, up [.., N, K]; down [.., K, N]) is packed at when N, not being a multiple of 256, keeps its
+    planes out of the streaming order: the next multiple, or None where the planes stay as they are.  Every reason that shapes give
+    is looked at here, before anything is built: weights that disagree about the width (the calls refuse those), a K that keeps
+    gate and up out of that order whatever N is, or rows of the down matrix that do not hold whole blocks."""
+    n, k = int(gate.shape[-2]), int(gate.shape[-1])
+    width = (n + 255) // 256 * 256
+    if width == n or k % 256 != 0 or not all(isinstance(w, QuantizedTensor) for w in (gate, up, down)):
+        return None
+    if list(up.shape) != list(gate.shape) or list(down.shape) != [*gate.shape[:-2], k, n]:
+        return None
+    block = 16 if isinstance(down, PlanarQuantizedTensor) and type(down.layout) is TensorScaledLayout else 32
+    return width if n % block == 0 else None
+
+
 def ffn_device_weights(gate, up, down, *, stacked: bool, prepack: bool, build=device_weight):
     """Descriptors of the three matrices of a gated FFN (gate, up [.., N, K]; down [.., K, N]) for the fused calls.  A width N
     that is not a multiple of 256 keeps the planes out of the streaming order, so they are packed with N padded to one: the
@@ -54,9 +64,8 @@ def ffn_device_weights(gate, up, down, *, stacked: bool, prepack: bool, build=de
     width no tile divides, run on the general 128 x 128 kernel.  Whole call, planar / padded: Q4_1 FFN 3072 x 3904 at 1098
     rows 283 / 103 us; Q8_0 FFN 3072 x 12416 at 148 rows 262 / 134; Q8_0 layer 2048 x 2368 at 12 tokens 64 / 31; 16 experts
     of 5120 x 3456 in Q4_1 at 98 tokens 314 / 195; the narrowest measured (64 experts of 640, a fifth of it padding) 200 / 170."""
-    n = int(gate.shape[-2])
-    width = padded_width(n)
-    if prepack and width != n and isinstance(gate, QuantizedTensor):
+    width = padded_ffn_width(gate, up, down) if prepack else None
+    if width is not None:
         packed = tuple(build(w, stacked=stacked, prepack=True, pad=pad)
                        for w, pad in ((gate, (width, None)), (up, (width, None)), (down, (None, width))))
         if all(dw.is_packed for dw in packed):

@@ -145,3 +145,27 @@ def test_unused_reference_alternatives_are_named():
     ffn = PreGatherFFNMOE(_tiny_theta())
     with pytest.raises(NotImplementedError, match="unused by forward"):
         ffn.one_hot_matmul(None, None, None)
+
+
+def _ffn_weights(K, N, N_up=None, N_down=None, d_dtype=torch.float16):
+    def q8(rows, cols):
+        layout = ST.BlockScaledLayout([rows, cols], torch.ones(rows, cols // 32, 1, dtype=d_dtype), torch.zeros(rows, cols // 32, 32, dtype=torch.int8))
+        return ST.PlanarQuantizedTensor(shape=[rows, cols], layout=layout)
+
+    return q8(N, K), q8(N_up or N, K), q8(K, N_down or N)
+
+
+@pytest.mark.parametrize("K,N,width", [(256, 256, None), (256, 704, 768), (256, 160, 256), (256, 320, 512),
+                                       (288, 288, None), (2880, 2880, None), (512, 2880, 3072)])
+def test_ffn_widths_that_are_padded(K, N, width):
+    from sharktank_amd.ops.hip_impls import padded_ffn_width
+
+    assert padded_ffn_width(*_ffn_weights(K, N)) == width
+
+
+def test_ffn_weights_of_different_widths_are_not_padded_to_one():
+    """Gate, up and down of widths that round up to the same multiple of 256 do not fit each other; the calls must get to see that."""
+    from sharktank_amd.ops.hip_impls import padded_ffn_width
+
+    assert padded_ffn_width(*_ffn_weights(256, 704, N_up=736)) is None
+    assert padded_ffn_width(*_ffn_weights(256, 704, N_down=736)) is None
