@@ -11,14 +11,13 @@ packed matrix kernels through `ops.linear`.
 
 from __future__ import annotations
 
-from functools import partial
 from typing import Callable
 
 import torch
 import torch.nn.functional as F
 
 from .. import _hip, ops
-from ..ops.hip_impls import cached_device_weight, ffn_device_weights
+from ..ops import ffn_device_weights
 from .base import Theta, ThetaLayer
 from .ffn_moe_block import activation_enum
 from .linear import LinearLayer
@@ -50,7 +49,7 @@ class FFN(ThetaLayer):
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         if self._fusable(h):
             wg, wu, wd = ffn_device_weights(self.ffn_gate.weight, self.ffn_up.weight, self.ffn_down.weight, stacked=False,
-                                            prepack=True, build=partial(cached_device_weight, cast_to=h.dtype))
+                                            prepack=True, cache=True, cast_to=h.dtype)
             x = h.reshape(-1, h.shape[-1])
             T = x.shape[0]
             if T == 0:

@@ -7,6 +7,8 @@ Anything not implemented returns `NotImplemented`, which surfaces as the referen
 
 from __future__ import annotations
 
+from functools import partial
+
 import torch
 from torch import Tensor
 
@@ -56,21 +58,45 @@ def padded_ffn_width(gate, up, down):
     return width if n % block == 0 else None
 
 
-def ffn_device_weights(gate, up, down, *, stacked: bool, prepack: bool, build=device_weight):
+def ffn_device_weights(gate, up, down, *, stacked: bool, prepack: bool, cache: bool = False, cast_to: torch.dtype = None):
     """Descriptors of the three matrices of a gated FFN (gate, up [.., N, K]; down [.., K, N]) for the fused calls.  A width N
-    that is not a multiple of 256 keeps the planes out of the streaming order, so they are packed with N padded to one: the
-    padded features of the intermediate come out as zeros and meet zero columns of the down matrix.  All three are padded or
-    none (the calls take one width).  Unpadded, the down matrix stays planar and its product, and the gate/up product of a
-    width no tile divides, run on the general 128 x 128 kernel.  Whole call, planar / padded: Q4_1 FFN 3072 x 3904 at 1098
-    rows 283 / 103 us; Q8_0 FFN 3072 x 12416 at 148 rows 262 / 134; Q8_0 layer 2048 x 2368 at 12 tokens 64 / 31; 16 experts
-    of 5120 x 3456 in Q4_1 at 98 tokens 314 / 195; the narrowest measured (64 experts of 640, a fifth of it padding) 200 / 170."""
+    that is not a multiple of 256 keeps the planes out of the streaming order, so they are packed with N padded to one
+    (padded_ffn_width): the padded features of the intermediate come out as zeros and meet zero columns of the down matrix.  All
+    three are padded or none (the calls take one width).  Unpadded, the down matrix stays planar and its product, and the gate/up
+    product of a width no tile divides, run on the general 128 x 128 kernel.  Whole call, planar / padded: Q4_1 FFN 3072 x 3904 at
+    1098 rows 283 / 103 us; Q8_0 FFN 3072 x 12416 at 148 rows 262 / 134; Q8_0 layer 2048 x 2368 at 12 tokens 64 / 31; 16 experts
+    of 5120 x 3456 in Q4_1 at 98 tokens 314 / 195; 8 experts of 1024 x 320 in Q8_0 at 1, 128 and 2048 tokens 21 / 18, 58 / 36 and
+    80 / 76.  With `cache` the descriptors are kept with the weights (cached_device_weight, `cast_to` as there)."""
+    weights = (gate, up, down)
+    build = partial(cached_device_weight, cast_to=cast_to) if cache else device_weight
     width = padded_ffn_width(gate, up, down) if prepack else None
     if width is not None:
-        packed = tuple(build(w, stacked=stacked, prepack=True, pad=pad)
-                       for w, pad in ((gate, (width, None)), (up, (width, None)), (down, (None, width))))
-        if all(dw.is_packed for dw in packed):
-            return packed
-    return tuple(build(w, stacked=stacked, prepack=prepack) for w in (gate, up, down))
+        pads = ((width, None), (width, None), (None, width))
+        if cache:
+            stores = [_descriptor_store(w) for w in weights]
+            slots = [(stacked, True, cast_to, pad) for pad in pads]
+            # (a weight that an earlier call found to be not packable: its entry holds no descriptor)
+            kept = [store.get(slot) for store, slot in zip(stores, slots)]
+            refused = any(hit is not None and hit[1] is None and hit[0] == _planes_key(w) for hit, w in zip(kept, weights))
+        else:
+            refused = False
+        packed = []
+        while not refused and len(packed) < 3:
+            dw = build(weights[len(packed)], stacked=stacked, prepack=True, pad=pads[len(packed)])
+            if dw.is_packed:
+                packed.append(dw)
+                continue
+            # Only the values can still say no (Q4_1 block scales outside the packed kernels' range).  What was built for the padded
+            # width is given back, and the weight that said no is remembered.
+            refused = True
+            if cache:
+                for w, store, slot in zip(weights[:len(packed)], stores, slots):
+                    store.pop(slot, None)
+                i = len(packed)
+                stores[i][slots[i]] = (_planes_key(weights[i]), None)
+        if not refused:
+            return tuple(packed)
+    return tuple(build(w, stacked=stacked, prepack=prepack) for w in weights)
 
 
 def _tensor_version(t: torch.Tensor) -> int:
@@ -99,14 +125,11 @@ def _planes_key(w):
     return [(t.data_ptr(), t.shape, t.dtype, _tensor_version(t)) for t in ts]
 
 
-_TENSOR_CACHE = {}  # id(torch.Tensor) -> (weakref to it, {(stacked, prepack, dtype): (planes key, descriptor)})
+_TENSOR_CACHE = {}  # id(torch.Tensor) -> (weakref to it, its _descriptor_store)
 
 
-def cached_device_weight(w, *, stacked: bool, prepack: bool = True, cast_to: torch.dtype = None, pad=(None, None)) -> _hip.DeviceWeight:
-    """device_weight(w) built once per weight and kept with it: the planes are made contiguous and (where the shape allows)
-    re-ordered into the kernels' streaming order on the first call; later calls with unchanged planes reuse the result.
-    InferenceTensors carry their descriptors themselves; plain torch tensors are tracked through weak references.  `cast_to`
-    (dense weights only) is the dtype the kernels need, cast once as well."""
+def _descriptor_store(w) -> dict:
+    """Where the descriptors of a weight are kept: {(stacked, prepack, dtype, padding): (planes key, descriptor)}."""
     if isinstance(w, torch.Tensor):
         ent = _TENSOR_CACHE.get(id(w))
         if ent is None or ent[0]() is not w:
@@ -115,9 +138,16 @@ def cached_device_weight(w, *, stacked: bool, prepack: bool = True, cast_to: tor
             wid = id(w)
             ent = (weakref.ref(w, lambda _, wid=wid: _TENSOR_CACHE.pop(wid, None)), {})
             _TENSOR_CACHE[wid] = ent
-        store = ent[1]
-    else:
-        store = w.__dict__.setdefault("_stmoe_descriptors", {})
+        return ent[1]
+    return w.__dict__.setdefault("_stmoe_descriptors", {})
+
+
+def cached_device_weight(w, *, stacked: bool, prepack: bool = True, cast_to: torch.dtype = None, pad=(None, None)) -> _hip.DeviceWeight:
+    """device_weight(w) built once per weight and kept with it: the planes are made contiguous and (where the shape allows)
+    re-ordered into the kernels' streaming order on the first call; later calls with unchanged planes reuse the result.
+    InferenceTensors carry their descriptors themselves; plain torch tensors are tracked through weak references.  `cast_to`
+    (dense weights only) is the dtype the kernels need, cast once as well."""
+    store = _descriptor_store(w)
     slot, key = (stacked, prepack, cast_to, pad), _planes_key(w)
     hit = store.get(slot)
     if hit is None or hit[0] != key:

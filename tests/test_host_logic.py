@@ -169,3 +169,33 @@ def test_ffn_weights_of_different_widths_are_not_padded_to_one():
 
     assert padded_ffn_width(*_ffn_weights(256, 704, N_up=736)) is None
     assert padded_ffn_width(*_ffn_weights(256, 704, N_down=736)) is None
+
+
+@pytest.mark.parametrize("refusing", [0, 1, 2, None])
+def test_a_refused_padding_is_given_back_and_remembered(monkeypatch, refusing):
+    """A weight whose values keep it out of the streaming order (Q4_1 block scales): the other two keep no padded copy beside the
+    descriptors that are used, and later calls build nothing."""
+    from types import SimpleNamespace
+
+    from sharktank_amd.ops import hip_impls
+
+    weights = _ffn_weights(256, 704)
+    built = []
+
+    def device_weight(w, *, stacked, prepack=False, pad=(None, None)):
+        i = next(i for i, x in enumerate(weights) if x is w)
+        built.append((i, pad))
+        return SimpleNamespace(is_packed=i != refusing, pad=pad, weight=i)
+
+    monkeypatch.setattr(hip_impls, "device_weight", device_weight)
+    first = hip_impls.ffn_device_weights(*weights, stacked=False, prepack=True, cache=True)
+    n_built = len(built)
+    assert hip_impls.ffn_device_weights(*weights, stacked=False, prepack=True, cache=True) == first and len(built) == n_built
+    assert [d.weight for d in first] == [0, 1, 2]
+    if refusing is None:
+        assert [d.pad for d in first] == [(768, None), (768, None), (None, 768)] and n_built == 3
+    else:
+        assert [d.pad for d in first] == [(None, None)] * 3 and n_built == 3 + refusing + 1
+    for w, used in zip(weights, first):  # (nothing is kept that is not used)
+        kept = [d for _, d in hip_impls._descriptor_store(w).values() if d is not None]
+        assert kept == [used]
