@@ -47,10 +47,12 @@ def padded_ffn_width(gate, up, down):
     """The width a gated FFN (gate, up [.., N, K]; down [.., K, N]) is packed at when N, not being a multiple of 256, keeps its
     planes out of the streaming order: the next multiple, or None where the planes stay as they are.  Every reason that shapes give
     is looked at here, before anything is built: weights that disagree about the width (the calls refuse those), a K that keeps
-    gate and up out of that order whatever N is, or rows of the down matrix that do not hold whole blocks."""
+    gate and up out of that order whatever N is, rows of the down matrix that do not hold whole blocks, and padding of more than
+    0.6 N (N = 128 runs at twice its width: 8 experts of 2048 x 128 at 700 tokens 67 us instead of 63, 64 experts of 2048 x 64 at
+    128 tokens 55 instead of 50; from 0.6 down nothing was slower by more than a tenth, and most calls a third faster)."""
     n, k = int(gate.shape[-2]), int(gate.shape[-1])
     width = (n + 255) // 256 * 256
-    if width == n or k % 256 != 0 or not all(isinstance(w, QuantizedTensor) for w in (gate, up, down)):
+    if width == n or 5 * width > 8 * n or k % 256 != 0 or not all(isinstance(w, QuantizedTensor) for w in (gate, up, down)):
         return None
     if list(up.shape) != list(gate.shape) or list(down.shape) != [*gate.shape[:-2], k, n]:
         return None

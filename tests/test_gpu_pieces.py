@@ -349,15 +349,18 @@ def test_prepack_padded_round_trip_and_zero_padding(device, fmt, N, K, rows, col
 
 
 @pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16), ("fp8", torch.float16)])
-@pytest.mark.parametrize("N", [32, 224, 288, 704])
+@pytest.mark.parametrize("N", [32, 128, 160, 224, 288, 320, 704])
 @pytest.mark.parametrize("T", [1, 20, 300])
 def test_block_with_padded_width_against_the_oracle(device, fmt, dtype, N, T):
-    """FFN widths around the multiples of 256 that the packed kernels take: the layer packs its weights with a padded width."""
+    """FFN widths around the multiples of 256 that the packed kernels take: the layer packs its weights with a padded width unless
+    that is more than 1.6 times its own (gate and up of 32, 128 and 288 are packed as they are, the down matrix stays planar)."""
     from sharktank_amd.layers import MoeBlock
 
     case = MC.build(MC.Case(T=T, K=512, N=N, fmt=fmt, dtype=dtype, seed=52))
     block = MoeBlock(MC.make_theta(case, device), case.E, case.k, case.eps)
-    assert [w.is_packed for w in block.experts.device_weights()] == [True] * 3
+    padded = N not in (32, 128, 288)
+    assert [w.is_packed for w in block.experts.device_weights()] == [True, True, padded]
+    assert [w.padded for w in block.experts.device_weights()] == [padded] * 3
     h = case.planes["h"]
     y, idx, _ = block(h.reshape(1, T, 512).to(device), return_routing=True)
     want, want_idx, _ = MC.oracle_block(case)

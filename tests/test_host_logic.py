@@ -155,7 +155,7 @@ def _ffn_weights(K, N, N_up=None, N_down=None, d_dtype=torch.float16):
     return q8(N, K), q8(N_up or N, K), q8(K, N_down or N)
 
 
-@pytest.mark.parametrize("K,N,width", [(256, 256, None), (256, 704, 768), (256, 160, 256), (256, 320, 512),
+@pytest.mark.parametrize("K,N,width", [(256, 256, None), (256, 704, 768), (256, 160, 256), (256, 128, None), (256, 320, 512), (256, 288, None),
                                        (288, 288, None), (2880, 2880, None), (512, 2880, 3072)])
 def test_ffn_widths_that_are_padded(K, N, width):
     from sharktank_amd.ops.hip_impls import padded_ffn_width
