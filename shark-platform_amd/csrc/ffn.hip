@@ -110,15 +110,22 @@ static bool narrow_pays(int wtag, int mode, const GemmParams& p, int64_t rows) {
     return p.split_scratch && p.kred <= 6144 && p.n_out * (mode == MODE_GATEUP ? 2 : 1) * rows >= p.kred * (wtag == WF_Q4_1_P ? 1024 : 1600);
   return p.split_scratch == nullptr || p.kred <= 6144;
 }
-// Unquantized 16-bit weights: the kernel that brings both operands straight into LDS, against the streaming kernel.  For the
-// gate/up projection it is the faster one at any number of rows (8 experts of 4096 x 14336, us, streaming / this one: 1 token
-// 111 / 85, 8 tokens 346 / 316, 64 tokens 444 / 329; of 1024 x 1024, 1 token 13 / 11; a single 14336 x 4096 pair 73 / 47).  The
-// down projection has a quarter of the units or less, and below some 190 of them the streaming kernel, which cuts the reduction,
-// keeps more CUs busy (2 tokens, 128 units: 108 / 118; 4 tokens, 256 units: 150 / 133; a single 4096 x 14336 matrix 44 / 96).
-// Beyond the streaming kernel's rows this one takes every launch (down, 100 tokens: 292 / 164).
+// Unquantized 16-bit weights: the kernel that brings both operands straight into LDS, against the streaming kernel inside that one's
+// window.  For the gate/up projection it is the faster one (8 experts of 4096 x 14336, us, streaming / this one: 1 token 111 / 85, 8
+// tokens 346 / 316, 64 tokens 444 / 329; of 1024 x 1024, 1 token 13 / 11; a single 14336 x 4096 pair 73 / 47) unless the launch is at
+// most 64 units of 64 features with a long reduction, which the streaming kernel cuts, and no expert has more than 64 rows (8 experts of
+// 4096 x 256 at 16 tokens 18 / 23, 4 of 4096 x 1024 at 2 tokens 18 / 22, at 64 tokens 20 / 23; with 3072 elements 0.8 to 1.1 times as long, with 96 units
+// 0.7).  The down projection has a quarter of the units or less, and below some 190 of them the streaming kernel keeps more CUs busy (2
+// tokens, 128 units: 108 / 118; 4 tokens, 256 units: 150 / 133; a single 4096 x 14336 matrix 44 / 96).  Beyond the streaming kernel's
+// rows this one takes every launch (down, 100 tokens: 292 / 164).
+static bool dense_pays_gate_up(int64_t K, int64_t N, int64_t experts, int64_t rows_of_one) {
+  return K <= 3072 || N / 64 * experts > 64 || rows_of_one > 64;
+}
 static bool dense_pays(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (!dense_takes(dtype, wtag, mode, p, rows)) return false;
-  if (mode == MODE_GATEUP || p.n_out / 128 * (p.offsets ? std::min<int64_t>(p.E, rows) : 1) >= 192) return true;
+  const int64_t experts = p.offsets ? std::min<int64_t>(p.E, rows) : 1;
+  if (mode == MODE_GATEUP) return dense_pays_gate_up(p.kred, p.n_out, experts, p.expert_rows_bound > 0 ? std::min(p.expert_rows_bound, rows) : rows);
+  if (p.n_out / 128 * experts >= 192) return true;
   if (p.E == 1) return rows > kSkinnyMaxRowsSingleSplit;
   return !(p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) && rows > kSkinnyMaxRows &&
          rows > skinny_max_avg_rows(p.E) * p.E;
@@ -524,7 +531,7 @@ static int moe_forward_impl(const void* h, int dtype, int64_t T, int64_t K, int6
   const bool gate_up_dispatches =
       fused_front && T > 1 && T * k <= 64 && E >= 2 && (variant == 0 || variant == 3) && (dtype == STMOE_F16 || dtype == STMOE_BF16) &&
       w_gate && w_up && weight_tag(w_gate) == weight_tag(w_up) && !(x_scale && !x_fq) &&
-      !(variant == 0 && w_gate->format == STMOE_W_DENSE && N % 64 == 0) &&  // (the unquantized kernel takes those)
+      !(variant == 0 && w_gate->format == STMOE_W_DENSE && N % 64 == 0 && dense_pays_gate_up(K, N, std::min<int64_t>(E, T * k), T)) &&  // (the unquantized kernel takes those)
       skinny_takes_grouped(dtype, weight_tag(w_gate), E, K, N, K, N);
   // the dispatch launch also clears the ticket words of the projections' split reductions (if this shape has any)
   const FfnWs fws = carve_ffn(T, k, K, N, dtype);

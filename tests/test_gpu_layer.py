@@ -179,6 +179,13 @@ def test_fp8_matrix_core_path_is_exact_up_to_dequant_rounding(device, variant_na
     assert O.rel_l2(got, want_pairs) < 1e-3
 
 
+@pytest.mark.parametrize("T", [3, 32, 64, 65])
+def test_narrow_unquantized_layer_with_a_long_reduction(device, T):
+    """32 units of 64 features at most: up to 64 tokens the streaming kernel (which builds its own dispatch up to 64 pairs), from 65 on
+    the kernel of unquantized weights."""
+    check_case(MC.Case(T=T, K=3328, N=256, fmt="dense", dtype=torch.float16, seed=60 + T), device)
+
+
 def test_gelu_and_output_norm(device):
     """Grok-style block: exact-erf GELU and a layer_output_norm (sharktank/sharktank/models/grok/grok.py:102-109)."""
     case = MC.Case(T=80, K=384, N=512, fmt="q4_1", dtype=torch.float16, act="gelu", out_norm=True, seed=22)
