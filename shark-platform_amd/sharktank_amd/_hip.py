@@ -774,8 +774,8 @@ def probe_mfma(device, kind: int = 0, random_operands: bool = True, iters: int =
     timed with events on the current stream.  The untimed launches in front (some tens of milliseconds) let the chip's
     power management settle: a short burst after idle runs at a clock the chip does not hold."""
     lib = load_library()
-    dev = torch.device(device)
-    sink = torch.zeros(1, dtype=torch.float32, device=dev)
+    sink = torch.zeros(1, dtype=torch.float32, device=device)
+    dev = sink.device  # (with its index, also where `device` names none)
     flop = ctypes.c_double(0.0)
     with _on_device(dev):
         for _ in range(warm_launches):

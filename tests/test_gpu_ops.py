@@ -830,3 +830,10 @@ def test_narrow_tiles_of_128_features(device, fmt, dtype, rows):
         got, want = (_hip.grouped_gate_up(x, *dws, _hip.ACT_SILU, offsets, perm, 1, variant=v) for v in (_hip.VARIANT_MFMA_NARROW, _hip.VARIANT_MFMA_TILE))
         # (the same sums; the gated product may be rounded once more or less on the way: one unit of the last place)
         assert O.rel_l2(got.cpu().double(), want.cpu().double()) < 2.0 ** (-11 if dtype == torch.float16 else -8)
+
+
+def test_probe_takes_a_device_without_an_index(device):
+    from sharktank_amd import _hip
+
+    for dev in ("cuda", torch.device("cuda"), device):
+        assert _hip.probe_mfma(dev, iters=100, launches=1, warm_launches=1) > 0
