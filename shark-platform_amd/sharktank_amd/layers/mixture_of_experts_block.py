@@ -81,7 +81,7 @@ class MoeBlock(ThetaLayer):
         # (sub-modules are read from their dictionary: the attribute lookup of torch modules costs a small forward 2 us)
         modules = self._modules
         experts, out_norm = modules["experts"], modules["layer_output_norm"]
-        wg, wu, wd = experts._dw or experts.device_weights()
+        wg, wu, wd = experts.device_weights()
         if wg.experts != self.expert_count:
             raise ValueError(f"expert_count {self.expert_count} != stacked weight experts {wg.experts}")
         out_norm_w = unbox_tensor(out_norm.weight) if isinstance(out_norm, RMSNormLayer) else None

@@ -186,6 +186,26 @@ def test_narrow_unquantized_layer_with_a_long_reduction(device, T):
     check_case(MC.Case(T=T, K=3328, N=256, fmt="dense", dtype=torch.float16, seed=60 + T), device)
 
 
+def test_a_subclass_that_overrides_device_weights_is_asked_every_time(device):
+    from sharktank_amd.layers import MoeBlock, PreGatherFFNMOE
+
+    case = MC.build(MC.Case(T=8, K=256, N=256, fmt="q8_0", dtype=torch.float16, seed=61))
+    block = MoeBlock(MC.make_theta(case, device), case.E, case.k, case.eps)
+
+    class Counting(PreGatherFFNMOE):
+        calls = 0
+
+        def device_weights(self):
+            self.calls += 1
+            return super().device_weights()
+
+    block.experts.__class__ = Counting
+    h = case.planes["h"].reshape(1, 8, 256).to(device)
+    for n in (1, 2, 3):
+        block(h)
+        assert block.experts.calls == n
+
+
 def test_gelu_and_output_norm(device):
     """Grok-style block: exact-erf GELU and a layer_output_norm (sharktank/sharktank/models/grok/grok.py:102-109)."""
     case = MC.Case(T=80, K=384, N=512, fmt="q4_1", dtype=torch.float16, act="gelu", out_norm=True, seed=22)
