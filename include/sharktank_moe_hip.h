@@ -161,8 +161,10 @@ int stmoe_fake_quant_fp8(const void* x, int dtype, const float* rscale, int64_t 
  * [experts, rows, cols] with formats X and X_PACKED and caller-owned planes of equal sizes; rows % 16 == 0 and
  * cols % 256 == 0.  `packed` may also have more rows per expert and more columns than `planar`: the rest is filled with
  * zeros (an FFN whose width N is not a multiple of 256 pads the rows of its gate/up and the columns of its down matrix
- * to one and is called with the padded width), and stmoe_unpack leaves the padding out.  The reference has no counterpart (its planes come from GGUF blocks,
- * sharktank/sharktank/types/gguf_interop/layouts.py:51-60,285-300, and are consumed row-major). */
+ * to one and is called with the padded width; an fp8 layer with static quantizers whose caller wants the arithmetic of its own
+ * width passes variant 8, see stmoe_grouped_ffn), and stmoe_unpack leaves the padding out.  Planes of 64 GB and more are refused.
+ * The reference has no counterpart (its planes come from GGUF blocks, sharktank/sharktank/types/gguf_interop/layouts.py:51-60,285-300,
+ * and are consumed row-major). */
 int stmoe_prepack(const stmoe_weight* planar, const stmoe_weight* packed_out, stmoe_stream_t stream);
 int stmoe_unpack(const stmoe_weight* packed, const stmoe_weight* planar_out, stmoe_stream_t stream);
 

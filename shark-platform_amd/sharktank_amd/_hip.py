@@ -423,6 +423,11 @@ def dispatch_build(idx: torch.Tensor, E: int):
 Q4_1_PACKED_MAX_SCALE = 64.0
 
 
+def packable_size(fmt: int, experts: int, rows: int, cols: int) -> bool:
+    """Whether stmoe_prepack takes planes of this size: it counts 16-byte pieces in 32 bits, so from 64 GB on they stay planar."""
+    return experts * rows * cols // (2 if fmt in (W_Q4_1, W_Q4_1_PACKED) else 1) // 16 < 0xFFFFFF00
+
+
 class DeviceWeight:
     """An expert-stacked weight `[E, rows, cols]` as the C ABI sees it; keeps its planes alive."""
 
@@ -451,7 +456,7 @@ class DeviceWeight:
     def can_prepack(self, rows: Optional[int] = None, cols: Optional[int] = None) -> bool:
         """Whether prepack(rows, cols) has a streaming order for this weight (rows, cols: the padded shape, if any)."""
         rows, cols = rows or self.rows, cols or self.cols
-        return (self.format in _PACKED_OF and rows % 16 == 0 and cols % 256 == 0
+        return (self.format in _PACKED_OF and packable_size(self.format, self.experts, rows, cols) and rows % 16 == 0 and cols % 256 == 0
                 and self.cols % (16 if self.format == W_FP8 else 32) == 0
                 and (self.format != W_FP8 or self.desc.dtype == F32) and self.q4_scales_in_range())
 

@@ -199,3 +199,16 @@ def test_a_refused_padding_is_given_back_and_remembered(monkeypatch, refusing):
     for w, used in zip(weights, first):  # (nothing is kept that is not used)
         kept = [d for _, d in hip_impls._descriptor_store(w).values() if d is not None]
         assert kept == [used]
+
+
+def test_planes_of_64_gb_stay_planar():
+    """stmoe_prepack refuses them, so a weight of that size must not be sent there."""
+    from sharktank_amd import _hip
+
+    w = object.__new__(_hip.DeviceWeight)
+    w.format, w.experts, w.rows, w.cols = _hip.W_Q8_0, 64, 32768, 32768 - 256
+    assert w.can_prepack()
+    assert not w.can_prepack(cols=32768)
+    w.cols = 32768
+    assert not w.can_prepack()
+    assert _hip.packable_size(_hip.W_Q4_1, 64, 32768, 32768) and not _hip.packable_size(_hip.W_Q4_1, 128, 32768, 32768)
