@@ -288,7 +288,8 @@ int stmoe_softmax(const void* x, int x_dtype, int64_t rows, int64_t cols, void* 
 /* Weighted combine (ffn_moe_block.py:73-74) and the layer tail (mixture_of_experts_block.py:86-90):
  *   o[t,:] = sum_j round(gate[t,j] * y[inv[t*k+j],:])   (slot order, fp32 sum, rounded to `dtype`)
  *   o = rms_norm(o; out_norm_w, eps) if out_norm_w != NULL     (layer_output_norm)
- *   out[t,:] = residual[t,:] + o[t,:] if residual != NULL      (h + moe_output)   */
+ *   out[t,:] = residual[t,:] + o[t,:] if residual != NULL      (h + moe_output)
+ * Rows are read and written in pieces of 16 bytes; out_norm_w may have any alignment (16-byte aligned ones are read faster). */
 int stmoe_combine(const void* y_sorted, const void* gate, const int32_t* inv, int dtype, int64_t T, int k,
                   int64_t K, const void* out_norm_w /*nullable*/, int w_dtype, float eps,
                   const void* residual /*nullable*/, void* out, stmoe_stream_t stream);

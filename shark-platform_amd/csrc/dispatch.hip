@@ -220,7 +220,7 @@ template <typename T> struct Row8 {
 template <typename T, typename W, int THREADS, bool NORM>
 __global__ void __launch_bounds__(THREADS)
 combine_kernel(const T* __restrict__ y, const T* __restrict__ gate, const int32_t* __restrict__ inv, int k,
-               int64_t K, const W* __restrict__ norm_w, float eps, const T* __restrict__ residual,
+               int64_t K, const W* __restrict__ norm_w, bool norm_w_aligned, float eps, const T* __restrict__ residual,
                T* __restrict__ out) {
   __shared__ float partial[THREADS / 64];
   const int64_t t = blockIdx.x;
@@ -297,7 +297,12 @@ combine_kernel(const T* __restrict__ y, const T* __restrict__ gate, const int32_
     auto finish = [&](int64_t i, Row8<T>& v) {
       Row8<T> h;
       Row8<W> nw;
-      nw.load(norm_w + i);
+      if (norm_w_aligned) {
+        nw.load(norm_w + i);
+      } else {  // (a view into a flat buffer of weights)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) nw.v[q] = Cvt<W>::to_f32(norm_w[i + q]);
+      }
       if (residual) h.load(residual + t * K + i);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -432,7 +437,8 @@ extern "C" int stmoe_combine(const void* y_sorted, const void* gate, const int32
   // rows beyond 2048 (2048 tokens of 4096: 12.3 us against 13.3); fewer tokens are done sooner with 256 (32 tokens 4.9 / 5.2)
 #define STMOE_COMBINE_T(TT, WW, THREADS, NORM)                                                                          \
   combine_kernel<TT, WW, THREADS, NORM><<<g, THREADS, 0, st>>>((const TT*)y_sorted, (const TT*)gate, inv, k, K,         \
-                                                               (const WW*)out_norm_w, eps, (const TT*)residual, (TT*)out)
+                                                               (const WW*)out_norm_w, aligned16(out_norm_w), eps,       \
+                                                               (const TT*)residual, (TT*)out)
 #define STMOE_COMBINE(TT, WW)                                                   \
   do {                                                                          \
     if (out_norm_w) STMOE_COMBINE_T(TT, WW, 512, true);                         \

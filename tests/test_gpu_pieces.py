@@ -296,6 +296,41 @@ def test_combine_with_output_norm_and_residual(device):
         assert O.rel_l2(got_full, want_full) < tol
 
 
+@pytest.mark.parametrize("w_shift", [0, 1])
+@pytest.mark.parametrize("dtype,w_dtype", [(torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("K", [2048, 2056, 4104, 8192, 8200])  # rows of one, two and three steps, kept in registers or not
+@pytest.mark.parametrize("T,k", [(1, 1), (64, 3), (65, 5), (7, 4)])
+def test_combine_row_lengths_slots_and_norm_alignment(device, T, k, K, dtype, w_dtype, w_shift):
+    """Both thread counts, rows that wait in registers for their norm and rows that pass through the output, batches of four slots
+    with a rest, and norm weights that start in the middle of a 16-byte piece."""
+    hip = _hip()
+    g = torch.Generator().manual_seed(K + k)
+    y = torch.randn(T * k, K, generator=g).to(dtype)
+    gate = torch.rand(T, k, generator=g).to(dtype)
+    inv = torch.randperm(T * k, generator=g).to(torch.int32)
+    h = torch.randn(T, K, generator=g).to(dtype)
+    w = (torch.ones(K + w_shift) + 0.1 * torch.randn(K + w_shift, generator=g)).to(w_dtype)
+    down = y[inv.long()].reshape(T, k, K)
+    o = torch.zeros(T, K)
+    for j in range(k):  # products rounded, added in fp32 in slot order
+        o += (gate[:, j:j + 1] * down[:, j]).float()
+    o = o.to(dtype)
+    dev = [t.to(device) for t in (y, gate, inv)]
+    w_dev = w.to(device)[w_shift:]
+    assert w_dev.data_ptr() % 16 == w_shift * w.element_size()
+    bits = torch.int16
+    assert torch.equal(hip.combine(*dev, T, k).cpu().view(bits), o.view(bits))
+    assert torch.equal(hip.combine(*dev, T, k, residual=h.to(device)).cpu().view(bits), (h + o).view(bits))
+    normed = O.rms_norm(o, w[w_shift:], 1e-5)
+    step = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for residual in (None, h):
+        got = hip.combine(*dev, T, k, out_norm_w=w_dev, eps=1e-5, residual=None if residual is None else residual.to(device)).cpu().float()
+        want = normed.float() if residual is None else (residual + normed.to(dtype)).float()
+        # the sum of squares is added in another order: a value (and the residual sum it enters) may round the other way once each
+        size = torch.maximum(want.abs(), normed.float().abs())
+        assert float(((got - want).abs() / size.clamp_min(1e-4)).max()) <= 2 * step
+
+
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8", "dense"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("T", [1, 7, 16, 32, 45])
