@@ -210,8 +210,8 @@ struct SingleTokenDispatch {
   int32_t *counts, *offsets, *perm, *inv;
 };
 
-template <typename T, typename W, bool FUSE_NORM, int PRE, bool LATE>
-__global__ void __launch_bounds__(512, (PRE && !LATE) ? 4 : 8)
+template <typename T, typename W, bool FUSE_NORM, int PRE>
+__global__ void __launch_bounds__(512, PRE ? 4 : 8)
 router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float eps, T* __restrict__ xn,
                  const T* __restrict__ wr, int64_t K, int E, int k, T* __restrict__ logits_out,
                  int32_t* __restrict__ idx_out, int64_t* __restrict__ idx64_out, T* __restrict__ gate_out,
@@ -233,10 +233,9 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
   // No load here has a condition of its own: past the row's end the last piece is read again and not used.  Loads under
   // separate conditions are waited for one by one, those of a straight line are all in flight together (rows shorter than
   // NC * 512 elements used to pay one memory latency per 512 elements: 7 tokens of 3328, launch 8.7 -> 6.8 us).
-  // PRE = 8 (a whole row of 4096) for launches of at most 64 tokens and 4 up to 512 tokens (latency).  Launches of more
-  // tokens, where throughput counts and the prefetch registers held through the norm would cost a quarter of the
-  // workgroups a CU can hold, request the same 8 chunks only after the norm's registers are free (LATE), in front of the
-  // barrier that ends the norm: all in flight together, where a loop over the chunks waits for them one by one.
+  // PRE = 8 (a whole row of 4096) for launches of at most 64 tokens, 4 up to 512 tokens and wherever a wavefront has several
+  // experts (latency).  Other launches of more tokens, where throughput counts and the prefetch registers held through the norm
+  // would cost half of the workgroups a CU can hold, have PRE = 0 and read the rows in the loop over the chunks.
   constexpr int NC = 8;
   uint4 wpre[PRE ? PRE : 1];
   auto prefetch = [&](uint4 (&dst)[PRE ? PRE : 1], int e) {
@@ -249,7 +248,7 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
       }
     }
   };
-  if constexpr (!LATE) prefetch(wpre, wave);
+  prefetch(wpre, wave);
   if constexpr (FUSE_NORM) {
     // the row's elements tid + 512 j are read once and kept (NC of them) for the second pass; the norm weights are
     // requested before the reduction
@@ -303,7 +302,6 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
       for (int64_t i = (int64_t)tid * 8 + 4; i < K; i += 512 * 8)
         *reinterpret_cast<uint4*>(&xs[i]) = *reinterpret_cast<const uint4*>(&xr[i]);
   }
-  if constexpr (LATE) prefetch(wpre, wave);
   __syncthreads();
 
   // the logit of expert e, whose first PRE chunks (16-bit rows) are in `pre`
@@ -596,14 +594,14 @@ static int launch_router_wg(const void* x, const void* norm_w, float eps, void* 
   const size_t lds = ((K * sizeof(T) + 15) / 16) * 16 + (64 + 8 + 64) * sizeof(float);
   if (lds > 64 * 1024) return set_error(STMOE_ERR_UNSUPPORTED, "router: K=%lld does not fit the per-token LDS row", (long long)K);
   if (T_tokens <= 64)
-    router_wg_kernel<T, W, FUSE_NORM, 8, false><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
+    router_wg_kernel<T, W, FUSE_NORM, 8><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   else if (T_tokens <= 512 || E > 16)  // (several experts per wavefront: the next one's row is worth its registers
     // at any size; with the tail on v_readlane 400 tokens of 2048 with 64 experts take 17 us instead of 51, 26 tokens with 32 experts 11 instead of 25)
-    router_wg_kernel<T, W, FUSE_NORM, 4, false><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
+    router_wg_kernel<T, W, FUSE_NORM, 4><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   else
-    router_wg_kernel<T, W, FUSE_NORM, 0, true><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
+    router_wg_kernel<T, W, FUSE_NORM, 0><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   return check_launch("router_wg");
 }
