@@ -731,15 +731,17 @@ def test_f32_products_are_no_further_from_fp64_than_the_general_kernel(device, K
 @pytest.mark.parametrize("rows,K,N,act", [
     ((1, 0, 15, 16), 64, 64, "silu"),               # one K step; fewer weight rows than one wide unit
     ((17, 63, 64, 65), 128, 128, "gelu"),
-    ((127, 128, 129, 0), 192, 320, "silu"),         # the two unit shapes; 128-row units of a width 256 does not divide
+    ((127, 128, 129, 0), 256, 320, "silu"),         # the two unit shapes; 128-row units of a width 256 does not divide
     ((192, 193, 256, 257), 256, 256, "silu"),       # three and four column blocks, a full tile, one row more
-    ((0, 513, 640, 3), 320, 192, "gelu"),           # several tiles per expert, of equal size and with a rest
+    ((0, 513, 640, 3), 384, 192, "gelu"),           # several tiles per expert with a rest of 1 and of 128 rows
+    ((385, 511, 0), 128, 192, "silu"),              # two tiles of equal size (a remainder of 129 and of 255 rows)
+    ((650, 700), 256, 128, "gelu"),                 # three
     ((70,) * 32, 128, 4096, "silu"),                # enough units for 256 weight rows each
     ((300,), 512, 768, "silu"),                     # a single expert
 ])
 def test_dense_16_bit_kernel_against_the_tile_kernel_and_fp64(device, rows, K, N, act, dtype):
     """Unquantized weights: row counts on both sides of the column blocks, the token groups, the two unit shapes and the tile,
-    against fp64 and (the down projection adds in the same order) bit for bit against the 128 x 128 kernel."""
+    against fp64 and (both add in the same order) bit for bit against the 128 x 128 kernel."""
     from sharktank_amd import _hip
 
     E, T = len(rows), sum(rows)
@@ -764,13 +766,14 @@ def test_dense_16_bit_kernel_against_the_tile_kernel_and_fp64(device, rows, K, N
     assert O.rel_l2(z.cpu().double(), want) < 2 * eps
     down = {v: _hip.grouped_down(z, dd, offsets, T, 1, variant=v).cpu() for v in (_hip.VARIANT_DENSE, _hip.VARIANT_MFMA_TILE)}
     bits = torch.int16
-    if N % 64 == 0 and K % 128 == 0:  # (narrower outputs run on the 128 x 128 kernel either way)
-        assert torch.equal(down[_hip.VARIANT_DENSE].view(bits), down[_hip.VARIANT_MFMA_TILE].view(bits))
+    assert N % 64 == 0 and (K % 128 == 0 or K == 64)  # (K = 64: the down projection has no tile and runs on the 128 x 128 kernel)
+    assert torch.equal(down[_hip.VARIANT_DENSE].view(bits), down[_hip.VARIANT_MFMA_TILE].view(bits))
     auto = _hip.grouped_ffn(x.to(device), dg, du, dd, act_id, offsets, perm, 1)
-    y = torch.stack([wd[ee].double() @ zz for ee, zz in zip(e.tolist(), z.cpu().double())]) if T < 600 else None
-    if y is not None:
-        assert O.rel_l2(down[_hip.VARIANT_DENSE].double(), y) < eps
-        assert O.rel_l2(auto.cpu().double(), y) < 2 * eps  # (a z element may round the other way under another kernel)
+    y = torch.empty(T, K, dtype=torch.float64)
+    for ee in range(E):
+        y[e == ee] = z.cpu().double()[e == ee] @ wd[ee].double().T
+    assert O.rel_l2(down[_hip.VARIANT_DENSE].double(), y) < eps
+    assert O.rel_l2(auto.cpu().double(), y) < 2 * eps  # (a z element may round the other way under another kernel)
 
 
 @pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16)])

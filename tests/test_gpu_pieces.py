@@ -112,7 +112,9 @@ def test_rms_norm(device, dtype):
                                      # more than 512 tokens (launches that fill the chip several times over), rows longer
                                      # than the per-token LDS row of the one-workgroup-per-token kernel
                                      (700, 4096, 8, 2), (1100, 6144, 8, 2), (600, 1024, 16, 4), (512 * 66 + 5, 512, 8, 2),
-                                     (520, 8192 + 512, 8, 2)])
+                                     (520, 8192 + 512, 8, 2),
+                                     # several experts per wavefront, below and above 64 and 512 tokens
+                                     (40, 1024, 17, 3), (70, 2048, 24, 4), (33, 2048, 64, 6), (600, 1024, 33, 6), (700, 512, 64, 6)])
 def test_router_bit_exact(device, dtype, T, K, E, k):
     g = torch.Generator().manual_seed(5)
     x = torch.randn(T, K, generator=g).to(dtype)
@@ -129,6 +131,26 @@ def test_router_bit_exact(device, dtype, T, K, E, k):
     ref_idx, _, _ = O.route(O.router_logits(x, wr), k)
     mism = int((ref_idx != want_idx).any(dim=1).sum())
     assert mism <= max(1, T // 100), f"{mism} of {T} tokens route differently from torch.matmul logits"
+
+
+@pytest.mark.parametrize("E", [5, 24, 64])
+@pytest.mark.parametrize("T", [4, 520])
+def test_router_rows_with_nan_and_infinite_logits(device, E, T):
+    """A NaN logit (or an infinite one, whose distance to the maximum is a NaN) makes every probability of its row a NaN: the choice is
+    then the lowest experts in order, with NaN gates, and the other rows are routed as if it were not there."""
+    K, k = 256, 4
+    g = torch.Generator().manual_seed(E)
+    x, wr = torch.randn(T, K, generator=g).to(torch.float16), (torch.randn(E, K, generator=g) * 0.02).to(torch.float16)
+    bad = torch.arange(T) % 4 == 1
+    x[1::8, 7] = float("nan")
+    x[5::8, 7] = float("inf")
+    wr[:, 7] = wr[:, 7].abs() + 0.01  # (an infinite element gives infinite logits)
+    idx, gate, _ = _hip().router_topk(x.to(device), wr.to(device), k)
+    idx, gate = idx.cpu().long(), gate.cpu()
+    assert torch.equal(idx[bad], torch.arange(k).expand(int(bad.sum()), k)) and bool(gate[bad].isnan().all())
+    want_idx, want_gate, _ = O.route(O.router_logits_ordered(x[~bad], wr.float()), k)
+    assert torch.equal(idx[~bad], want_idx)
+    assert O.rel_l2(gate[~bad], want_gate) < 2e-3
 
 
 @pytest.mark.parametrize("T", [3, 700])
