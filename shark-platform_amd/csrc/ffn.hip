@@ -99,8 +99,9 @@ static constexpr int64_t kSkinnyMaxRowsSingleSplit = 32;
 // Where tiles of 64 are more than the CUs, tiles of 128 features x 256 rows (1.0 us per K step) against the split: they pay once the
 // partial tiles, which grow with features x rows, cost more than the reduction that the split shortens; the 4-bit format converts
 // faster and pays sooner.  Measured (128-row tiles / split, us, Q4_1 bf16; Q8_0 fp16): [14336, 4096] 257 rows 65 / 62; 68 / 61, 300
-// rows 63 / 70; 68 / 65, 512 rows 67 / 78; 71 / 75; [8192, 4096] 513 rows 64 / 66; 68 / 65, 1024 rows 70 / 85; 75 / 82; [16384, 2048]
-// 300 rows 35 / 52; 38 / 50; [14336, 6144] 300 rows 91 / 89; 99 / 83, 512 rows 95 / 100; 101 / 96.
+// rows 63 / 70; 68 / 65, 512 rows 67 / 78; 71 / 75; [8192, 4096] 513 rows 64 / 66; 68 / 65, 1024 rows 70 / 85; 75 / 82; [14336, 6144] 300
+// rows 91 / 89; 99 / 83, 512 rows 95 / 100; 101 / 96; against whole units, which reductions up to 3072 keep, [16384, 2048] 300 rows 38 / 50;
+// 40 / 43.  fp8 takes Q8_0's constant: [14336, 4096] 300 rows 58 / 66, 512 rows 64 / 77, [14336, 6144] 300 rows 83 / 84.
 static bool narrow_pays(int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (rows <= 128) return false;
   const int64_t features = (mode == MODE_GATEUP ? 32 : 64) * (narrow_wide(mode, p.n_out, rows) ? 2 : 1);

@@ -687,7 +687,8 @@ static int launch_skinny_t(int mode, const GemmParams& p, int64_t max_rows, hipS
   // items through LDS 30.0 / 31.8; with 352 items split is the better one (9.7 / 12.0, 20 rows 14.5 / 16.1).
   // A down projection whose items of 32 features are no more than half the CUs takes items of 16 instead (Q8_0, us, 32 / 16):
   // [4096, 14336] 1 row 20.2 / 13.5, 8 rows 19.6 / 15.7, 32 rows 42.5 / 31.9; [1024, 4096] 8 rows 9.3 / 7.3; with 192 items 8 rows
-  // of [6144, 2048] 7.1 / 8.1.
+  // of [6144, 2048] 7.1 / 8.1.  Both rules hold for grouped launches: of 1920 layers (2 to 32 experts of 1024 to 6144 columns, 512 to
+  // 8192 features, 1 to 16 tokens, three formats) 5 were slower with them by more than 3 %, the mean 1.12 times as fast.
   const int64_t active_bound = max_rows < p.E ? max_rows : p.E;
   const bool pin = max_rows <= 16;  // a handful of rows in the whole launch: the pinned, unconditional prefetch pays
   const int64_t items_bound = active_bound * tiles;

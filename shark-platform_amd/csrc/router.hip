@@ -596,8 +596,9 @@ static int launch_router_wg(const void* x, const void* norm_w, float eps, void* 
   if (T_tokens <= 64)
     router_wg_kernel<T, W, FUSE_NORM, 8><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
-  else if (T_tokens <= 512 || E > 16)  // (several experts per wavefront: the next one's row is worth its registers
-    // at any size; with the tail on v_readlane 400 tokens of 2048 with 64 experts take 17 us instead of 51, 26 tokens with 32 experts 11 instead of 25)
+  else if (T_tokens <= 512 || E > 16)
+    // (several experts per wavefront: the next one's row is worth its registers at any size.  With the tail on v_readlane 26 tokens of
+    // 2048 with 32 experts take 11 us instead of 25, 400 with 64 experts 17 instead of 51, 2048 with 64 47 instead of 73)
     router_wg_kernel<T, W, FUSE_NORM, 4><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   else
