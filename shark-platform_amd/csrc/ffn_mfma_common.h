@@ -117,15 +117,16 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
   return v;
 }
 __device__ __forceinline__ BigLanes big_lanes(const GemmParams& p, int lane_off, int lane, int BM, bool absorb, int balance) {
-  int begin = 0, rows = lane == 0 ? (int)p.fixed_rows : 0;
-  if (p.offsets) {
-    int end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);  // (lane 63 reads lane 0: no expert unless there are 64)
-    if (p.E == 64) end = lane == 63 ? p.offsets[64] : end;
-    begin = lane_off;
-    rows = lane < p.E ? end - begin : 0;
+  if (!p.offsets) {  // one expert: the same in every lane
+    const int rows = (int)p.fixed_rows;
+    const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
+    return BigLanes{0, rows, x.main, x.main, x.partial ? 1ull : 0ull, x.even ? 1ull : 0ull};
   }
+  int end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);  // (lane 63 reads lane 0: no expert unless there are 64)
+  if (p.E == 64) end = lane == 63 ? p.offsets[64] : end;
+  const int rows = lane < p.E ? end - lane_off : 0;
   const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance);
-  return BigLanes{begin, rows, x.main, wave_inclusive_sum(x.main), __ballot(x.partial != 0), __ballot(x.even)};
+  return BigLanes{lane_off, rows, x.main, wave_inclusive_sum(x.main), __ballot(x.partial != 0), __ballot(x.even)};
 }
 __device__ __forceinline__ BigPlan big_plan(const BigLanes& l, int n_tiles, int xcd, bool allow_split) {
   BigPlan pl;
