@@ -14,8 +14,9 @@
 //   wavefronts: 4 x 2 (64 x 64 of BN = 256) up to 128 rows, 2 x 4 (128 x 64) above; the rows of a unit are spread evenly over
 //     the token groups in multiples of 16 and only the column blocks that hold rows are multiplied.
 //   The reduction runs in the order of the 128 x 128 kernel: the sums are the same bits.
-// Measured (8 experts of 4096 x 14336, top-2, bf16; gate/up + down, us; 128 x 128 kernel / this one): 100 tokens 423 + 271 /
-// 329 + 164, 515 tokens 645 + 308 / 374 + 197 (5 TB/s of weights), 2048 tokens 1897 + 824 / 1002 + 537 (0.95 PFLOP/s).
+// Measured (8 experts of 4096 x 14336, top-2, bf16; gate/up + down, us; 128 x 128 kernel / this one): 100 tokens 421 + 279 /
+// 329 + 195, 515 tokens 640 + 313 / 376 + 212 (5 TB/s of weights), 2048 tokens 1916 + 823 / 1025 + 537 (0.92 PFLOP/s; SiLU
+// by expf and a division, as the 128 x 128 kernel computes it, is 20 us of the 1025: on the hardware exp2 and reciprocal 1002).
 #include "ffn_mfma_common.h"
 
 namespace stmoe {
