@@ -724,8 +724,11 @@ int mfma_ws_ticket_count() { return kWsTickets; }
 // reduction elements (its most: every expert with rows may have a tile of its own).  Measured (split / whole, us, [out, in] of one, 8
 // and 64 experts): Q8_0 [1024, 512] 8 experts 1024 tokens 39 / 19; [1024, 1280] 200 rows 28 / 28; [1024, 1536] 200 rows 29 / 32, 8 experts
 // 1024 tokens 48 / 39; [2048, 3072] 200 rows 35 / 55; Q4_1 [1024, 1024] 8 experts 1024 tokens 44 / 32; [1024, 1280] 200 rows 30 / 33.
-// Over 64 to 3000 tokens and 1024 to 4096 outputs, split took 0.97 to 3.0 times as long as whole where the rule leaves whole.
+// Over 64 to 3000 tokens and 1024 to 4096 outputs, split took 0.97 to 3.0 times as long as whole where the rule leaves whole.  A single
+// matrix with at most 128 rows has few units and small partial tiles and is always split (Q4_1 [1024, 1024] 33 rows 12.9 / 18.2, 96 rows
+// 17.6 / 21.1; Q8_0 [1024, 1280] 33 rows 12.3 / 16.2).
 static bool ws_split_pays(int wtag, int mode, const GemmParams& p, int64_t max_rows) {
+  if (!p.offsets && max_rows <= 128) return true;
   if (p.kred <= (wtag == WF_Q4_1_P ? 1024 : 1280)) return false;
   const int64_t tiles = p.n_out / (mode == MODE_GATEUP ? 128 : 256);
   const int64_t units = tiles * ((max_rows + 255) / 256 + (p.offsets ? std::min<int64_t>(p.E, max_rows) : 0));
