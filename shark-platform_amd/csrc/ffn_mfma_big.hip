@@ -63,7 +63,10 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
 
   BigTile tile;
   if (!big_tile_id(p, BM, n_tiles, false, tile)) return;
-  const int e = tile.e, row_begin = tile.row_begin, row_end = tile.row_end, ntile = tile.ntile;
+  int e = tile.e, row_begin = tile.row_begin, row_end = tile.row_end, ntile = tile.ntile;
+  // (What the compiler can tell about these values from the lookup moves the scheduling of the K loop: with it the narrow Q4_1 tiles of
+  // 64 features take 0.05 us more per step, 31.5 instead of 28.6 us for 200 rows of [2048, 3072].)
+  asm volatile("" : "+s"(e), "+s"(row_begin), "+s"(row_end), "+s"(ntile));
   const int rows_here = row_end - row_begin;
 
   // ---- producer assignment ---------------------------------------------------------------------------
