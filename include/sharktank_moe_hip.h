@@ -328,7 +328,7 @@ int stmoe_moe_forward_timed(const void* h, int dtype, int64_t T, int64_t K, int6
  * stmoe_moe_forward_workspace_bytes() exceeds that size (prefill-sized batches) are refused with STMOE_ERR_WORKSPACE.
  * All calls on one GPU share the array: calls that overlap on one GPU (two streams, two threads) race; serialise them.
  * The first call on a device looks the array's address up (hipGetSymbolAddress): make it outside graph capture. */
-#define STMOE_STATIC_SCRATCH_BYTES (16u << 20)
+#define STMOE_STATIC_SCRATCH_BYTES (17u << 20)
 int stmoe_moe_forward_static(const void* h, int dtype, int64_t T, int64_t K, int64_t N, int E, int k,
                              const void* ffn_norm_w, const void* out_norm_w, int w_dtype, float eps,
                              const void* w_router, const stmoe_weight* w_gate, const stmoe_weight* w_up,

@@ -115,7 +115,7 @@ SIGNATURES = {
     "stmoe_mmt": (c_int, [c_void_p, c_int, c_int64, POINTER(StmoeWeight), c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p]),
     "stmoe_probe_mfma": (c_int, [c_int, c_int, c_int, c_void_p, POINTER(ctypes.c_double), c_void_p]),
 }
-STATIC_SCRATCH_BYTES = 16 << 20  # STMOE_STATIC_SCRATCH_BYTES
+STATIC_SCRATCH_BYTES = 17 << 20  # STMOE_STATIC_SCRATCH_BYTES
 
 _lib = None
 

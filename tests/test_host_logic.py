@@ -212,3 +212,17 @@ def test_planes_of_64_gb_stay_planar():
     w.cols = 32768
     assert not w.can_prepack()
     assert _hip.packable_size(_hip.W_Q4_1, 64, 32768, 32768) and not _hip.packable_size(_hip.W_Q4_1, 128, 32768, 32768)
+
+
+def test_padded_layers_that_fitted_the_built_in_workspace_still_do():
+    """A layer of a padded width is called with that width: what its own width needed of 16 MiB must not become too much."""
+    from sharktank_amd import _hip
+
+    for dtype in (torch.float16, torch.float32):
+        for T, k in ((1, 2), (64, 2), (128, 1), (21, 6), (200, 1)):
+            for K in (256, 2048, 8192):
+                need = lambda n: _hip.moe_forward_workspace_bytes(T, k, 8, K, n, dtype)
+                for n in range(32, 1 << 18, 1024 + 32):
+                    if need(n) > 16 << 20:
+                        break
+                    assert need((n + 255) // 256 * 256) <= _hip.STATIC_SCRATCH_BYTES, (T, k, K, n)
