@@ -68,7 +68,7 @@ class PreGatherFFNMOE(ThetaLayer):
         """C-ABI descriptors of the three stacked weights, built once (planes made contiguous once).  Their FFN width may be
         padded for the fused calls (ffn_device_weights); the two halves called on their own hand the intermediate to a
         quantizer in between and keep its true width."""
-        if self._dw is None:
+        if self._dw is None or (self._dw[0].padded and not self.fusable):  # (a quantizer may have been replaced since)
             weights = (self.ffn_gate, self.ffn_up, self.ffn_down)
             if self.fusable:
                 self._dw = ffn_device_weights(*weights, stacked=True, prepack=self.prepack_weights)

@@ -452,6 +452,26 @@ def test_fp8_block_with_padded_width_and_quantizers(device, dtype, N, T):
     assert err < (1e-3 if dtype == torch.float16 else 3e-3) + step * float(want.float().norm() / moe.norm()), err
 
 
+def test_padded_layer_whose_quantizer_is_replaced_by_a_per_axis_one(device):
+    """The intermediate meets the quantizer of its own width, also where the layer had packed its weights for fused calls before."""
+    from sharktank_amd import types as ST
+    from sharktank_amd.layers import MoeBlock
+
+    N = 704
+    case = MC.build(MC.Case(T=40, K=512, N=N, fmt="q8_0", dtype=torch.float16, act_quant=True, seed=54))
+    h = case.planes["h"].reshape(1, 40, 512).to(device)
+    scale = (torch.rand(N, generator=torch.Generator().manual_seed(3)) + 0.5) * 200.0
+    q = ST.StaticScaledQuantizer(name="ffn_down_exps.q_input", scale=scale.to(device), reciprocal_scale=(1.0 / scale).to(device), axis=-1,
+                                 dtype=torch.float8_e4m3fn)
+    used, fresh = (MoeBlock(MC.make_theta(case, device), case.E, case.k, case.eps) for _ in range(2))
+    used(h)
+    assert all(w.padded for w in used.experts.device_weights())
+    for block in (used, fresh):
+        block.experts.q_intermediate = q
+    assert torch.equal(used(h).view(torch.int16), fresh(h).view(torch.int16))
+    assert not any(w.padded for w in used.experts.device_weights())
+
+
 def test_prepack_layout_definition(device):
     """Spot-checks the documented order: lane 16*g + n of block (row tile rt, k block kb) holds row 16*rt+n,
     k = 64*kb + 16*g .. +15; scales of 8 consecutive blocks of a row are contiguous."""
