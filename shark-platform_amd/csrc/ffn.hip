@@ -131,6 +131,52 @@ static bool dense_pays(int dtype, int wtag, int mode, const GemmParams& p, int64
   return !(p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) && rows > kSkinnyMaxRows &&
          rows > skinny_max_avg_rows(p.E) * p.E;
 }
+// Packed weights and some dozen rows per expert: the kernel that converts weights in the registers of the wavefronts that multiply them
+// (launch_mfma_reg; units of 64 rows x 256 weight rows, the units after the last whole round over the CUs cut in two if the halves fit
+// one round).  Against the prefill kernel, whose units cost nearly the same with 30 rows as with 250, it is the faster one while experts
+// have one unit's rows on average (us, prefill kernel / this one, gate/up and down, 8 experts of 4096 x 14336): Q4_1 bf16 25 rows 220 / 161
+// and 115 / 80, 51 rows 238 / 190 and 119 / 98, 63 rows 247 / 261 and 131 / 159; Q4_1 fp16 25 rows 208 / 124 and 110 / 62, 51 rows 220 / 163
+// and 117 / 84; Q8_0 fp16 25 rows 194 / 169 and 107 / 78, 51 rows 207 / 191 and 117 / 92; 64 experts of 2048 x 1536 at 28 rows (Q4_1 fp16)
+// 98 / 75 and 55 / 44; with a routing that gives one expert a third of the pairs 0.95 to 1.4 times as fast.  Beyond that it still is where
+// all its units fit one round (down: 8 of [1024, 2048] at 200 rows 42 / 18, 16 of [2048, 4096] at 100 rows 65 / 47, 4 of [4096, 8192]
+// at 75 rows 56 / 48; gate/up of 8 x 1024 x 2048 at 100 rows 24 / 20) and the reduction is not as long as 14336 (63 rows above).
+// Against the streaming kernel it takes down projections whose half units fill three quarters of the CUs and whose reduction is long
+// enough to pay for the start of a unit (two rows per expert on average and 3072 elements: 8 of [4096, 14336], Q8_0 / Q4_1 fp16, 2 rows
+// 74 / 69 and 68 / 52, 8 rows 80 / 78 and 78 / 55, 16 rows 108 / 78 and 107 / 60; 16 of [3072, 6144] Q4_1 bf16 5 rows 61 / 57; 32 of
+// [2048, 2816] 6 rows 36 / 38), or half of them if experts have more than one token tile (4 of [4096, 8192]: 10 rows 26 / 29, 20 rows
+// 38 / 32, 32 rows 58 / 36).
+// A single matrix: its half units run at the pace of their reduction, whatever their number, where the prefill kernel cuts the reduction
+// in four and the narrow tiles re-read the token rows ([out, in], other kernels / this one, Q8_0 fp16; Q4_1 bf16): [14336, 4096] 33 rows
+// 28 / 22; 31 / 26, 128 rows 42 / 27; 43 / 31, 160 rows 40 / 41; 39 / 48; [4096, 4096] 64 rows 21 / 21; 25 / 27, 100 rows 27 / 22;
+// 31 / 28, 256 rows 38 / 23; 37 / 28, 512 rows 39 / 29; 42 / 31; [4096, 14336] 128 rows 54 / 65; 68 / 83, 160 rows 76 / 65; 88 / 84, 512 rows
+// 96 / 82; 103 / 96; [8192, 8192] 64 rows 33 / 41; 40 / 50, 160 rows 56 / 41; 64 / 53, 256 rows 67 / 49; 72 / 57; [2048, 1024] 33 rows
+// 12 / 8; 13 / 9.  From 129 rows on reductions up to 2048 stay on the narrow tiles, which give the bits of an unsplit prefill launch
+// (13 / 10 at 300 rows).
+static bool reg_pays(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
+  if (!reg_takes(dtype, wtag, mode, p, rows)) return false;
+  const int64_t tiles = p.n_out / (mode == MODE_GATEUP ? 128 : 256);  // units per token tile
+  if (p.E == 1) {
+    const int64_t units = (rows + kRegUnitRows - 1) / kRegUnitRows * tiles;
+    if (rows <= kSkinnyMaxRowsSingleSplit || p.kred < 1024 || units > 128) return false;
+    if (rows <= 64) return p.kred <= 2048 || (p.kred <= 4096 && tiles >= 32);
+    return rows > 128 ? p.kred > 2048 : p.kred <= 4096;
+  }
+  if (!p.offsets) return false;
+  const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||
+                       rows <= skinny_max_avg_rows(p.E) * p.E;
+  if (streams) {
+    const int64_t halves = 2 * tiles * std::min<int64_t>(p.E, rows);
+    return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * (int64_t)p.E) || (halves >= 128 && rows > 16 * (int64_t)p.E));
+  }
+  if (p.kred < 1024) return false;
+  // (short reductions over several rounds of units: a unit's start, 5 us that nothing hides, counts; the formats that convert faster gain
+  // less: 64 experts of 2048 x 1536, Q8_0 bf16 37 rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
+  if (wtag != WF_Q4_1_P && p.kred <= 2048 && tiles * p.E > 256 && rows > 24 * (int64_t)p.E) return false;
+  if (rows <= 52 * (int64_t)p.E) return true;
+  // (an expert's rows vary: by a seventh for a uniform routing of this many)
+  const int64_t units = (rows * 8 / 7 / p.E + kRegUnitRows - 1) / kRegUnitRows * tiles * p.E;
+  return p.kred <= 8192 && units <= 256;
+}
 // fp8 activations x fp8 weights on the fp8 matrix cores: the 256 x 256 kernel for packed weights and launches with
 // enough rows to fill its tiles (variant 5), the 128 x 128 kernel otherwise (and always with variant 7).
 // Whether the 256 x 256 kernel takes a projection (its token rows must come without a gather: see fp8_ws_takes' caller).
@@ -155,6 +201,7 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     if (dtype == STMOE_F32) variant = 10;
     // (one matrix, with or without an offsets array around its rows)
     else if (dense_pays(dtype, wtag, mode, p, max_rows)) variant = 11;
+    else if (reg_pays(dtype, wtag, mode, p, max_rows)) variant = 12;
     else if (p.E == 1) variant = max_rows <= (p.split_scratch ? kSkinnyMaxRowsSingleSplit : kSkinnyMaxRowsSingle) ? 3
                                  : narrow_pays(wtag, mode, p, max_rows) ? 9 : 6;
     else if (p.offsets && ((p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) ||
@@ -174,6 +221,11 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
   }
   if (variant == 9) {
     int rc = launch_mfma_narrow(dtype, wtag, mode, p, max_rows, st);
+    if (rc != STMOE_ERR_UNSUPPORTED) return rc;
+    variant = 6;
+  }
+  if (variant == 12) {
+    int rc = launch_mfma_reg(dtype, wtag, mode, p, max_rows, st);
     if (rc != STMOE_ERR_UNSUPPORTED) return rc;
     variant = 6;
   }

@@ -580,6 +580,39 @@ def test_ffn_mfma_ws_kernel_formats(device, dtype, fmt):
     assert O.rel_l2(outs[hip.VARIANT_MFMA_WS], outs[hip.VARIANT_MFMA_TILE]) < tol
 
 
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,E,act", [(256, 256, 8, "silu"), (2048, 1280, 8, "gelu"), (3584, 512, 8, "silu"), (256, 768, 64, "silu")])
+def test_ffn_mfma_reg_kernel(device, fmt, dtype, N, K, E, act):
+    """The kernel that converts weights in the registers of the wavefronts that multiply them, forced: experts without rows, with one row,
+    on both sides of its 16-row tiles and its 64-row units; reductions of 1 to 14 chunks (the register sets' three and the LDS stages' four
+    with every remainder); launches of half units only, of whole ones only (gate/up of N = 2048: 20 units per XCD) and of a round of whole
+    ones with halves behind it (N = 3584: 35)."""
+    hip = _hip()
+    from sharktank_amd.ops import device_weight
+
+    rows = [0, 1, 16, 17, 33, 64, 65, 130] if E == 8 else [i % 7 for i in range(E)]
+    T = sum(rows)
+    tol = 1e-3 if dtype == torch.float16 else 8e-3
+    case = MC.build(MC.Case(T=T, K=K, N=N, E=E, k=1, fmt=fmt, dtype=dtype, act=act, seed=70))
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(71))
+    idx = torch.tensor([e for e, n in enumerate(rows) for _ in range(n)])[order].reshape(T, 1)
+    want = O.grouped_ffn_moe(case.planes["h"], idx, torch.ones(T, 1, dtype=dtype), *MC.dense_weights(case), case.activation)
+    dws = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], shp, n, device), stacked=True, prepack=True)
+           for n, shp in (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))]
+    assert all(w.is_packed for w in dws)
+    _, offsets, perm, inv = hip.dispatch_build(idx.to(torch.int32).to(device), E)
+    act_id = hip.ACT_SILU if act == "silu" else hip.ACT_GELU_ERF
+    outs = {}
+    for variant in (hip.VARIANT_MFMA_REG, hip.VARIANT_MFMA_TILE):
+        y = hip.grouped_ffn(case.planes["h"].to(device), *dws, act_id, offsets, perm, 1, variant=variant)
+        outs[variant] = hip.combine(y, torch.ones(T, 1, dtype=dtype, device=device), inv, T, 1).cpu()
+        assert O.rel_l2(outs[variant], want) < tol
+    # the worst row as well: a row or a unit that another one overwrote would hide in the mean
+    diff, size = outs[hip.VARIANT_MFMA_REG].double() - want.double(), want.double().norm(dim=1)
+    assert float((diff.norm(dim=1) / size).max()) < 4 * tol
+
+
 def _raw_blocks(fmt: str, shape, seed: int):
     """Random bit patterns in ggml block structs: the scales are arbitrary fp16 bits (NaNs included), so a conversion
     anywhere on the way would show."""
