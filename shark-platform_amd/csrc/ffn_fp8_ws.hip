@@ -5,8 +5,10 @@
 // then only reads LDS operands and issues MFMAs.
 //
 //   256 x 256 workgroup tile (GATEUP: 128 gate + the same 128 up rows), 8 wavefronts of 128 weight rows x 64 token
-//   rows, K stage 64 (one v_mfma_scale_f32_32x32x64_f8f6f4 deep), five stages of 16 KB weights + 16 KB tokens = 160 KB,
-//   loads issued four stages ahead, one barrier per stage.
+//   rows, K stage 64 (one v_mfma_scale_f32_32x32x64_f8f6f4 deep), four stages of 16 KB weights + 16 KB tokens + 2 KB
+//   ride-along tokens = 136 KB, loads issued three stages ahead (four are no faster), one barrier per stage.
+//   ride-along rows: an expert with a few rows more than c full tiles would need a partial tile for them, whose units load all
+//            256 rows and leave most matrix cores idle; each full tile takes up to 32 of them along instead (tail_rows).
 //   weights: a packed 1 KB piece (16 rows x 64 k; lane 16 g + n holds row n, k = 16 g .. + 15) lands in LDS as it is;
 //            MFMA lane (r, h) supplies row r, samples 32 h .. 32 h + 31: pieces' units 2 h and 2 h + 1 of row r % 16,
 //            16 consecutive lanes read 256 consecutive bytes.
@@ -20,7 +22,7 @@
 //            quantise the gated intermediate to e4m3fn for the down projection.
 //   What bounds it: at 256 flop per operand byte the tile needs 32 KB per stage from L2 / HBM; with the operand loads
 //   alone (no MFMA) the launch takes two thirds of its full time and with the MFMAs alone 60 %, i.e. the two overlap only
-//   partly: the bytes in flight are capped by the LDS (4 stages of 32 KB), which covers the load latency under load only
+//   partly: the bytes in flight (3 or 4 stages of 32 KB, no difference) cover the load latency under load only
 //   just.  Reading the next stage's operands from LDS ahead of the barrier (software pipelining) changed nothing.
 #include "ffn_mfma_common.h"
 
@@ -38,6 +40,22 @@ __device__ __forceinline__ intx8_t join8(const u32x4_t& lo, const u32x4_t& hi) {
 // is flipped with bit 2 of the row; 8 consecutive rows reading the same logical unit then touch 32 distinct banks.
 __device__ __forceinline__ int x_unit(int row, int u) { return u ^ ((row >> 2) & 1); }
 
+// vm_load16_to_lds for a base that vector instructions have just written to scalar registers: a memory instruction may read those only
+// five wait states later, and the compiler's hazard handling does not look into inline assembly.
+__device__ __forceinline__ void f8_load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_addr) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+  const void* b = reinterpret_cast<const void*>((uint64_t)lo | ((uint64_t)hi << 32));
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(b), "s"(lds_addr) : "memory", "m0");
+}
+// The same for the first 16 lanes only (256 bytes), without a branch around it.  Every lane of the wavefront must be active.
+__device__ __forceinline__ void f8_load16_to_lds_16_lanes(const void* base, uint32_t byte_off, uint32_t lds_addr) {
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, 0xffff\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte_off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+
 struct F8Args {
   GemmParams p;
   int n_tiles;
@@ -47,18 +65,21 @@ struct F8Args {
 // One entry of a workgroup's unit table: what lane r of the table holds for the workgroup's r-th unit.
 struct F8Unit {
   int e, ntile, row_begin, row_end;
+  int tail_begin, tail_rows;  // rows of the expert that ride along with this full tile (0: none)
 };
+// Rows that a full token tile takes along: one MFMA column block.
+static constexpr int kF8TailRows = 32;
 
 // The launch's units in the order of big_unit (ffn_mfma_common.h: an XCD takes an eighth of the main list, expert by
 // expert and feature tile by feature tile with an expert's token tiles of one feature tile next to each other, then an
 // eighth of the partial token tiles), looked up for a different item in every lane: the loop over the experts is the
 // same for all lanes (row counts come from readlane), each lane keeps what matches its own item.  `lane_off`: lane l holds
 // the first row of expert l (lane E: the row total).  Returns whether the lane's item exists.
-__device__ __forceinline__ bool f8_unit_of_lane(int lane_off, int E, int BM, int n_tiles, int xcd, int item, int balance, F8Unit& out) {
+__device__ __forceinline__ bool f8_unit_of_lane(int lane_off, int E, int BM, int n_tiles, int xcd, int item, int balance, bool absorb, F8Unit& out) {
   int F = 0, R = 0;
   for (int e = 0; e < E; ++e) {
     const int rows = __builtin_amdgcn_readlane(lane_off, e + 1) - __builtin_amdgcn_readlane(lane_off, e);
-    const BigExpertTiles x = big_expert_tiles(rows, BM, false, balance);
+    const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance, kF8TailRows);
     F += x.main;
     R += x.partial;
   }
@@ -72,10 +93,10 @@ __device__ __forceinline__ bool f8_unit_of_lane(int lane_off, int E, int BM, int
   const int p_ntile = R > 0 ? u / max(R, 1) : 0;
   int p_s = u - p_ntile * R;
   bool found = false;
-  out.e = 0; out.ntile = 0; out.row_begin = 0; out.row_end = 0;
+  out.e = 0; out.ntile = 0; out.row_begin = 0; out.row_end = 0; out.tail_begin = 0; out.tail_rows = 0;
   for (int e = 0; e < E; ++e) {
     const int b = __builtin_amdgcn_readlane(lane_off, e), rows = __builtin_amdgcn_readlane(lane_off, e + 1) - b;
-    const BigExpertTiles x = big_expert_tiles(rows, BM, false, balance);
+    const BigExpertTiles x = big_expert_tiles(rows, BM, absorb, balance, kF8TailRows);
     if (in_main) {
       const int units = x.main * n_tiles;
       if (!found && u < units) {
@@ -88,6 +109,11 @@ __device__ __forceinline__ bool f8_unit_of_lane(int lane_off, int E, int BM, int
         } else {
           out.row_begin = b + s * BM;
           out.row_end = out.row_begin + BM;
+          const int first = rows / BM * BM + kF8TailRows * s;
+          if (big_tail_absorbed(rows, BM, absorb, kF8TailRows) && first < rows) {
+            out.tail_begin = b + first;
+            out.tail_rows = min(kF8TailRows, rows - first);
+          }
         }
         found = true;
       }
@@ -117,8 +143,7 @@ __global__ void __launch_bounds__(512, 1)
 grouped_fp8_ws_kernel(F8Args args) {
   constexpr int BN = 256, BM = 256, KS = 64;      // K samples (= bytes per row) per stage
   constexpr int WSTAGE = BN * KS, XSTAGE = BM * KS;  // bytes
-  constexpr int STAGE = WSTAGE + XSTAGE, D = 5;   // stages in LDS
-  constexpr int LOADS = 4;                        // LDS-direct loads per wavefront and stage: 2 weight pieces + 2 x 16 token rows
+  constexpr int STAGE = WSTAGE + XSTAGE + kF8TailRows * KS, D = 4;  // stages in LDS
   constexpr int kBalance = 1;
   extern __shared__ __align__(16) uint8_t lds8[];
   const GemmParams& p = args.p;
@@ -130,9 +155,17 @@ grouped_fp8_ws_kernel(F8Args args) {
   const int nst = (int)(p.kred >> 6);
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds8);
   const uint32_t w_lds = lds0 + 2 * wave * 1024, x_lds = lds0 + WSTAGE + 32 * wave * KS;
+  const uint32_t t_lds = lds0 + WSTAGE + XSTAGE + 4 * wave * KS;
   const uint32_t lane16 = lane * 16;
   // bytes from one K stage of a token row to the next: 64 in a plain row, a whole block of rows in the blocked layout
   const uint32_t x_stage_bytes = p.a_block_rows ? (uint32_t)(p.a_block_rows * KS) : (uint32_t)KS;
+
+  // Launches without ride-along rows walk their units with an instance that knows nothing of them: their loads and the branches around
+  // them cost 4 % (2048 rows of one expert, gate/up 239 -> 249 us).
+  auto walk = [&](auto tails_tag) __attribute__((always_inline)) {
+  constexpr bool TAILS = decltype(tails_tag)::value != 0;
+  // LDS-direct loads per wavefront and stage: 2 weight pieces, 2 x 16 token rows and 4 ride-along rows
+  constexpr int LOADS = TAILS ? 5 : 4;
 
   // ---- operands: lane (r, h) supplies row r, samples 32 h .. 32 h + 31 ------------------------------------
   const int wn = wave & 1, wm = wave >> 1;
@@ -143,7 +176,16 @@ grouped_fp8_ws_kernel(F8Args args) {
   const uint8_t* const b_rd = lds8 + WSTAGE + xrow * KS;
   const int bu0 = x_unit(xrow, 2 * h32) << 4, bu1 = x_unit(xrow, 2 * h32 + 1) << 4;  // rows xrow and xrow + 32 swizzle alike
   floatx16_t acc[4][2];
-
+  // Ride-along rows.  The four wavefronts that share a weight half (128 rows) take 32 of its rows each against all of the unit's ride-along
+  // rows: one MFMA per stage, GATEUP 16 gate rows and the same 16 up rows, so that both sums of a feature meet in one lane.
+  floatx16_t tacc;
+  auto compute_tail = [&](int slot) __attribute__((always_inline)) {
+    const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? ((r32 >> 4) * 7 + wm) * 1024 : wm * 2048);
+    const uint8_t* bp = b_rd + slot * STAGE + (BM - wm * 64) * KS;  // (rows BM + r32: swizzled like xrow)
+    const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
+    const intx8_t bf = join8(*reinterpret_cast<const u32x4_t*>(bp + bu0), *reinterpret_cast<const u32x4_t*>(bp + bu1));
+    tacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf, tacc, 0, 0, 0, 127, 0, 127);
+  };
   auto compute = [&](auto both_tag, int slot) __attribute__((always_inline)) {
     constexpr bool BOTH = decltype(both_tag)::value;  // rows in both 32-row token blocks
     const uint8_t* bp = b_rd + slot * STAGE;
@@ -169,54 +211,75 @@ grouped_fp8_ws_kernel(F8Args args) {
   // 1 / out_rs once; per element q = v * inv refined by one residual step (fma(-q, rs, v) * inv + q), which is the
   // correctly rounded quotient except in rare last-bit cases that the following rounding to T absorbs
   const float out_inv = p.out_scale ? __builtin_amdgcn_rcpf(out_rs) : 0.0f;
+  struct Scales {
+    float s0, s1;
+  };
+  auto scales_of = [&](const F8Unit& un) __attribute__((always_inline)) {
+    return Scales{xsc * reinterpret_cast<const float*>(p.w0.d)[p.w0.d_count > 1 ? un.e : 0],
+                  MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(p.w1.d)[p.w1.d_count > 1 ? un.e : 0] : 0.0f};
+  };
+  // four consecutive features `col`.. of output row `orow_i`: gate and up sums (GATEUP), or the sums `g` (DOWN)
+  auto store_quad = [&](auto act_tag, int64_t orow_i, int64_t col, const float(&g)[4], const float(&u)[4], const Scales& sc) __attribute__((always_inline)) {
+    constexpr int ACT = decltype(act_tag)::value;
+    const int64_t orow = orow_i * p.ldo;
+    if (MODE == MODE_GATEUP) {
+      float gq[4], uq[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        gq[q] = g[q] * sc.s0;
+        uq[q] = u[q] * sc.s1;
+      }
+      if (p.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
+        float t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[q])));
+          const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[q])));
+          const float q0 = v * out_inv;
+          const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
+          t[q] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
+        }
+        int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
+        qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
+        const int64_t at = p.out_block_rows ? ((col >> 6) * p.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
+        *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(p.out) + at) = qv;
+      } else {
+        *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
+      }
+    } else {
+      *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) =
+          make_uint2(pack2<T>(g[0] * sc.s0, g[1] * sc.s0), pack2<T>(g[2] * sc.s0, g[3] * sc.s0));
+    }
+  };
   auto epilogue = [&](auto tj_tag, auto act_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
     constexpr int tj = decltype(tj_tag)::value;
-    constexpr int ACT = decltype(act_tag)::value;
-    const float s0 = xsc * reinterpret_cast<const float*>(p.w0.d)[p.w0.d_count > 1 ? un.e : 0];
-    const float s1 = MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(p.w1.d)[p.w1.d_count > 1 ? un.e : 0] : 0.0f;
+    const Scales sc = scales_of(un);
     if (tj * 32 + r32 < my_rows) {
       const int64_t orow_i = out_row(p, un.row_begin + wm * rpg + tj * 32 + r32);
-      const int64_t orow = orow_i * p.ldo;
-      if (MODE == MODE_GATEUP) {
 #pragma unroll
-        for (int ti = 0; ti < 2; ++ti)
+      for (int ti = 0; ti < (MODE == MODE_GATEUP ? 2 : 4); ++ti)
 #pragma unroll
-          for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
-            const int64_t col = (int64_t)un.ntile * (BN / 2) + wn * 64 + ti * 32 + 8 * b + 4 * h32;
-            float gq[4], uq[4];
+        for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
+          const int64_t col = (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 2 : BN) + wn * (MODE == MODE_GATEUP ? 64 : 128) + ti * 32 + 8 * b + 4 * h32;
+          const floatx16_t &c = acc[ti][tj], &d = acc[MODE == MODE_GATEUP ? ti + 2 : ti][tj];
+          const float g[4] = {c[4 * b], c[4 * b + 1], c[4 * b + 2], c[4 * b + 3]}, u[4] = {d[4 * b], d[4 * b + 1], d[4 * b + 2], d[4 * b + 3]};
+          store_quad(act_tag, orow_i, col, g, u, sc);
+          __builtin_amdgcn_sched_barrier(0);  // one quad at a time: the accumulators leave no room for more
+        }
+    }
+  };
+  auto tail_epilogue = [&](auto act_tag, const F8Unit& un) __attribute__((always_inline)) {
+    const Scales sc = scales_of(un);
+    if (r32 < un.tail_rows) {
+      const int64_t orow_i = out_row(p, un.tail_begin + r32);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              gq[q] = acc[ti][tj][4 * b + q] * s0;
-              uq[q] = acc[ti + 2][tj][4 * b + q] * s1;
-            }
-            if (p.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
-              float t[4];
-#pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[q])));
-                const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[q])));
-                const float q0 = v * out_inv;
-                const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
-                t[q] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
-              }
-              int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
-              qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
-              const int64_t at = p.out_block_rows ? ((col >> 6) * p.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
-              *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(p.out) + at) = qv;
-            } else {
-              *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
-            }
-          }
-      } else {
-#pragma unroll
-        for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const int64_t col = (int64_t)un.ntile * BN + wn * 128 + ti * 32 + 8 * b + 4 * h32;
-            const floatx16_t& c = acc[ti][tj];
-            *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) =
-                make_uint2(pack2<T>(c[4 * b] * s0, c[4 * b + 1] * s0), pack2<T>(c[4 * b + 2] * s0, c[4 * b + 3] * s0));
-          }
+      for (int b = 0; b < (MODE == MODE_GATEUP ? 2 : 4); ++b) {
+        const int64_t col = MODE == MODE_GATEUP ? (int64_t)un.ntile * (BN / 2) + wn * 64 + wm * 16 + 8 * b + 4 * h32
+                                                : (int64_t)un.ntile * BN + wn * 128 + wm * 32 + 8 * b + 4 * h32;
+        constexpr int UP = MODE == MODE_GATEUP ? 8 : 0;
+        const float g[4] = {tacc[4 * b], tacc[4 * b + 1], tacc[4 * b + 2], tacc[4 * b + 3]};
+        const float u[4] = {tacc[UP + 4 * b], tacc[UP + 4 * b + 1], tacc[UP + 4 * b + 2], tacc[UP + 4 * b + 3]};
+        store_quad(act_tag, orow_i, col, g, u, sc);
       }
     }
   };
@@ -241,11 +304,12 @@ grouped_fp8_ws_kernel(F8Args args) {
     F8Unit mine;
     const int round = round0 + lane;
     const int place = (wg + round * ((wgs >> 1) + 1)) % wgs;
-    const bool have = f8_unit_of_lane(lane_off, E, BM, n_tiles, xcd, round * wgs + place, kBalance, mine);
+    const bool have = f8_unit_of_lane(lane_off, E, BM, n_tiles, xcd, round * wgs + place, kBalance, TAILS, mine);
     // (the items of later rounds come later in the list: the lanes that hold a unit are lanes 0 .. n_units - 1)
     const int n_units = __builtin_popcountll(__ballot(have));
     if (n_units == 0) return;
     const int t_en = mine.e | (mine.ntile << 8), t_rb = mine.row_begin, t_re = mine.row_end;
+    const int t_tb = mine.tail_begin, t_tr = mine.tail_rows;
     auto unit_at = [&](int i) {
       F8Unit un;
       const int en = __builtin_amdgcn_readlane(t_en, i);
@@ -253,13 +317,15 @@ grouped_fp8_ws_kernel(F8Args args) {
       un.ntile = en >> 8;
       un.row_begin = __builtin_amdgcn_readlane(t_rb, i);
       un.row_end = __builtin_amdgcn_readlane(t_re, i);
+      un.tail_begin = __builtin_amdgcn_readlane(t_tb, i);
+      un.tail_rows = __builtin_amdgcn_readlane(t_tr, i);
       return un;
     };
     const int total = n_units * nst;  // K stages of this batch of units
 
     // ---- the load side: stage `gl` of the batch = stage `sl` of unit `ul` ------------------------------------
     const uint8_t* wq[2] = {nullptr, nullptr};
-    uint32_t xoff[2] = {0, 0};
+    uint32_t xoff[2] = {0, 0}, toff = 0;
     int ul = -1, sl = nst, gl = 0;
     auto issue_next = [&]() __attribute__((always_inline)) {
       if (sl == nst) {  // first stage of the next unit: its operand addresses
@@ -292,12 +358,18 @@ grouped_fp8_ws_kernel(F8Args args) {
           const int r = min((lr >> 6) * rpg + min(lr & 63, rpg - 1), rows_here - 1);
           xoff[j] = (uint32_t)((int64_t)(un.row_begin + r) * (p.a_block_rows ? KS : p.lda) + (x_unit(lr, lane & 3) << 4));
         }
+        if constexpr (TAILS) {  // (a unit without ride-along rows: its own rows again, never used)
+          const int tr = 4 * wave + ((lane & 15) >> 2);
+          const int i = un.tail_rows > 0 ? un.tail_begin + min(tr, un.tail_rows - 1) : un.row_begin + min(tr, rows_here - 1);
+          toff = (uint32_t)((int64_t)i * (p.a_block_rows ? KS : p.lda) + (x_unit(tr, lane & 3) << 4));
+        }
       }
       const uint32_t slot = (uint32_t)(gl % D) * STAGE;
-      vm_load16_to_lds(wq[0], lane16 + (uint32_t)sl * 1024, w_lds + slot);
-      vm_load16_to_lds(wq[1], lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
+      f8_load16_to_lds(wq[0], lane16 + (uint32_t)sl * 1024, w_lds + slot);
+      f8_load16_to_lds(wq[1], lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
       vm_load16_to_lds(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
       vm_load16_to_lds(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
+      if constexpr (TAILS) f8_load16_to_lds_16_lanes(p.a, toff + (uint32_t)sl * x_stage_bytes, t_lds + slot);
       ++sl;
       ++gl;
     };
@@ -317,35 +389,65 @@ grouped_fp8_ws_kernel(F8Args args) {
         for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) tacc[q] = 0.0f;
+      auto stages = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
 #pragma unroll 1
-      for (int st = 0; st < nst; ++st, ++g) {
-        // the loads of the D - 2 stages after this one may still be in flight when this stage is needed; the batch's
-        // last stages have nothing behind them to issue
-        if (g + D - 1 < total) {
-          vm_wait<(D - 2) * LOADS>();
-          __syncthreads();  // everybody's loads of this stage have landed; everybody is done with the stage before
-          issue_next();     // into the slot of the stage before
-        } else {
-          vm_wait<0>();
-          __syncthreads();
+        for (int st = 0; st < nst; ++st, ++g) {
+          // the loads of the D - 2 stages after this one may still be in flight when this stage is needed; the batch's
+          // last stages have nothing behind them to issue
+          if (g + D - 1 < total) {
+            vm_wait<(D - 2) * LOADS>();
+            __syncthreads();  // everybody's loads of this stage have landed; everybody is done with the stage before
+            issue_next();     // into the slot of the stage before
+          } else {
+            vm_wait<0>();
+            __syncthreads();
+          }
+          if constexpr (decltype(both_tag)::value >= 0) compute(both_tag, slot);
+          if constexpr (decltype(tail_tag)::value != 0) compute_tail(slot);
+          slot = slot == D - 1 ? 0 : slot + 1;
         }
-        if (my_rows > 32) compute(F8Int<1>{}, slot);
-        else if (my_rows > 0) compute(F8Int<0>{}, slot);
-        slot = slot == D - 1 ? 0 : slot + 1;
+      };
+      if (TAILS && un.tail_rows > 0) {
+        if constexpr (TAILS) {
+          stages(F8Int<1>{}, F8Int<1>{});
+          epilogues(F8Int<1>{}, un, rpg, my_rows);
+          if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) tail_epilogue(EpiAct<STMOE_ACT_SILU>{}, un);
+          else tail_epilogue(EpiAct<STMOE_ACT_GELU_ERF>{}, un);
+        }
+      } else if (my_rows > 32) {
+        stages(F8Int<1>{}, F8Int<0>{});
+        epilogues(F8Int<1>{}, un, rpg, my_rows);
+      } else if (my_rows > 0) {
+        stages(F8Int<0>{}, F8Int<0>{});
+        epilogues(F8Int<0>{}, un, rpg, my_rows);
+      } else {
+        stages(F8Int<-1>{}, F8Int<0>{});
       }
-      if (my_rows > 32) epilogues(F8Int<1>{}, un, rpg, my_rows);
-      else if (my_rows > 0) epilogues(F8Int<0>{}, un, rpg, my_rows);
     }
     // (a further batch, if the workgroup has more than 64 units, starts with empty LDS stages: every load has landed and
     // the last barrier is passed by all before the next stage 0 is written... after one more barrier)
     __syncthreads();
-  }
+  }  };
+  // Ride-along rows save their expert's partial tile and cost the full tiles an MFMA per nine and their loads: a unit that carries them
+  // takes 10-15 % longer.  They are taken along where that saves a round over the CUs (8 experts of 4096 x 14336, 4096 tokens: gate/up 16
+  // rounds to 14, 1107 / 1050 us, down 3 to 2, 617 / 512; down at 1000 tokens is one round either way: 206 / 227).
+  const int lane_end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);
+  const int lane_rows = lane < E ? lane_end - lane_off : 0;
+  auto rounds = [&](bool absorb) {
+    const BigExpertTiles x = big_expert_tiles(lane_rows, BM, absorb, kBalance, kF8TailRows);
+    const int units = __builtin_amdgcn_readlane(wave_inclusive_sum(x.main + x.partial), 63) * n_tiles;
+    return (units + 8 * wgs - 1) / (8 * wgs);
+  };
+  if (rounds(true) < rounds(false)) walk(F8Int<1>{});
+  else walk(F8Int<0>{});
 }
 
 template <typename T, int MODE>
 static int launch_fp8_ws_m(const GemmParams& p, int64_t max_rows, hipStream_t st) {
   constexpr int BN = 256, BM = 256;
-  constexpr size_t lds_bytes = (size_t)5 * (BN + BM) * 64;
+  constexpr size_t lds_bytes = (size_t)4 * (BN + BM + kF8TailRows) * 64;
   static std::atomic<uint64_t> lds_ready{0};
   auto kern = grouped_fp8_ws_kernel<T, MODE>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_ready, "fp8 ws kernel")) return rc;

@@ -47,9 +47,10 @@ struct BigTile {
 // instead lets every full token tile of such an expert take up to kBigTailRows of the tail rows along: full tile s of
 // the expert's c full tiles takes tail rows [16 s, 16 s + 16).  A tail is absorbed when it fits: 0 < tail <= 16 c.
 static constexpr int kBigTailRows = 16;
-__device__ __forceinline__ bool big_tail_absorbed(int rows, int BM, bool absorb) {
+// (`per_tile`: the rows that one full tile takes along, kBigTailRows unless a kernel says otherwise)
+__device__ __forceinline__ bool big_tail_absorbed(int rows, int BM, bool absorb, int per_tile = kBigTailRows) {
   const int c = rows / BM, t = rows - c * BM;
-  return absorb && t > 0 && t <= kBigTailRows * c;
+  return absorb && t > 0 && t <= per_tile * c;
 }
 // Token tiles of an expert with `rows` rows.  Usually rows / BM full tiles and, if rows remain that no full tile takes
 // along, one partial tile, which is listed with the other experts' partial tiles at the end of the launch.  With `balance`
@@ -65,13 +66,13 @@ struct BigExpertTiles {
   int partial;  // 1: a partial tile in the list of partial tiles
   bool even;    // main tiles are the equal-sized ones: tile s = rows [s rows / main, (s + 1) rows / main)
 };
-__device__ __forceinline__ BigExpertTiles big_expert_tiles(int rows, int BM, bool absorb, int balance) {
+__device__ __forceinline__ BigExpertTiles big_expert_tiles(int rows, int BM, bool absorb, int balance, int per_tile = kBigTailRows) {
   const int c = rows / BM, t = rows - c * BM;
   BigExpertTiles x;
   x.main = c;
   x.partial = 0;
   x.even = false;
-  if (t == 0 || big_tail_absorbed(rows, BM, absorb)) return x;
+  if (t == 0 || big_tail_absorbed(rows, BM, absorb, per_tile)) return x;
   if (2 * t > BM && (balance == 2 ? c > 0 : balance == 1 && c == 1)) {
     x.main = c + 1;
     x.even = true;

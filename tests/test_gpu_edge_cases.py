@@ -168,6 +168,39 @@ def test_fp8_matrix_core_kernels_agree(device, dtype, E, k, T, K, N, routing):
     assert O.rel_l2(a, want) < 6e-2 and O.rel_l2(b, want) < 6e-2
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,act", [(256, 3840, "silu"), (7680, 256, "gelu")])
+def test_fp8_full_tiles_take_ride_along_rows(device, dtype, K, N, act):
+    """Experts a few rows above whole tiles of the 256 x 256 fp8 kernel: 1 row on one tile, 32 and 96 rows on two and three tiles (the most
+    they take: 32 each), one expert with too few rows for a tile and one with none.  30 feature tiles (of the gate/up launch, then of the
+    down launch) make 210 units with ride-along rows and 300 without, one round over the CUs instead of two, which is when they ride along."""
+    from sharktank_amd import _hip as hip
+    from sharktank_amd.ops import device_weight
+
+    rows = [257, 0, 544, 864, 5]
+    E, T = len(rows), sum(rows)
+    case = MC.build(MC.Case(T=T, K=K, N=N, E=E, k=1, fmt="fp8", dtype=dtype, act=act, act_quant=True, seed=95))
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(96))
+    idx = torch.tensor([e for e, n in enumerate(rows) for _ in range(n)])[order].reshape(T, 1)
+    x, xs, zs = case.planes["h"], case.planes["x_rscale"], case.planes["z_rscale"]
+    want = O.grouped_ffn_moe(x, idx, torch.ones(T, 1, dtype=dtype), *MC.dense_weights(case), case.activation, x_rscale=xs, z_rscale=zs)
+    dws = [device_weight(MC.to_inference_tensor("fp8", case.planes[n], shp, n, device), stacked=True, prepack=True)
+           for n, shp in (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))]
+    _, offsets, perm, inv = hip.dispatch_build(idx.to(torch.int32).to(device), E)
+    act_id = hip.ACT_SILU if act == "silu" else hip.ACT_GELU_ERF
+    outs = {}
+    for variant in (hip.VARIANT_FP8_MFMA, hip.VARIANT_FP8_TILE):
+        y = hip.grouped_ffn(x.to(device), *dws, act_id, offsets, perm, 1, variant=variant, x_scale=xs.to(device), z_scale=zs.to(device))
+        outs[variant] = hip.combine(y, torch.ones(T, 1, dtype=dtype, device=device), inv, T, 1).cpu()
+    a, b = outs[hip.VARIANT_FP8_MFMA], outs[hip.VARIANT_FP8_TILE]
+    tol = 2e-3 if dtype == torch.float16 else 1.5e-2
+    assert O.rel_l2(a, b) < tol and O.rel_l2(a, want) < 6e-2
+    # every row by itself: an element of the intermediate on the other side of an e4m3 boundary moves by 1/16, a row that another one
+    # overwrote would be off by its whole size
+    diff, size = a.double() - b.double(), b.double().norm(dim=1)
+    assert float((diff.norm(dim=1) / size).max()) < 0.1
+
+
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_streaming_kernel_two_row_tiles_in_one_pass(device, fmt, dtype):
