@@ -101,14 +101,18 @@ static constexpr int64_t kSkinnyMaxRowsSingleSplit = 32;
 // faster and pays sooner.  Measured (128-row tiles / split, us, Q4_1 bf16; Q8_0 fp16): [14336, 4096] 257 rows 65 / 62; 68 / 61, 300
 // rows 63 / 70; 68 / 65, 512 rows 67 / 78; 71 / 75; [8192, 4096] 513 rows 64 / 66; 68 / 65, 1024 rows 70 / 85; 75 / 82; [14336, 6144] 300
 // rows 91 / 89; 99 / 83, 512 rows 95 / 100; 101 / 96; against whole units, which reductions up to 3072 keep, [16384, 2048] 300 rows 38 / 50;
-// 40 / 43.  fp8 takes Q8_0's constant: [14336, 4096] 300 rows 58 / 66, 512 rows 64 / 77, [14336, 6144] 300 rows 83 / 84.
+// 40 / 43.  With equal token tiles of at most 192 rows they pay earlier ([14336, 4096], 128-row tiles / split: 270 rows Q4_1 bf16 57 / 64, Q8_0
+// fp16 55 / 62, fp8 49 / 60, 384 rows Q8_0 59 / 69, fp8 53 / 67).  fp8 takes Q8_0's constant: [14336, 4096] 300 rows 58 / 66, 512 rows 64 / 77, [14336, 6144] 300 rows 83 / 84.
 static bool narrow_pays(int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (rows <= 128) return false;
   const int64_t features = (mode == MODE_GATEUP ? 32 : 64) * (narrow_wide(mode, p.n_out, rows) ? 2 : 1);
   if (p.n_out % features != 0) return false;
   if (p.n_out / features * ((rows + 255) / 256) > 256) return false;
-  if (narrow_wide(mode, p.n_out, rows))
-    return p.split_scratch && p.kred <= 6144 && p.n_out * (mode == MODE_GATEUP ? 2 : 1) * rows >= p.kred * (wtag == WF_Q4_1_P ? 1024 : 1600);
+  if (narrow_wide(mode, p.n_out, rows)) {
+    const int64_t row_tiles = (rows + 255) / 256;
+    const bool equal = !p.offsets && (rows + row_tiles - 1) / row_tiles <= 192;  // (see launch_mfma_narrow)
+    return p.split_scratch && p.kred <= 6144 && p.n_out * (mode == MODE_GATEUP ? 2 : 1) * rows >= p.kred * (equal ? 900 : wtag == WF_Q4_1_P ? 1024 : 1600);
+  }
   return p.split_scratch == nullptr || p.kred <= 6144;
 }
 // Unquantized 16-bit weights: the kernel that brings both operands straight into LDS, against the streaming kernel inside that one's

@@ -41,7 +41,14 @@ struct BigTagOff { static constexpr bool value = false; };
 // TI = 4 (128 weight rows, a piece for every wavefront) is for the sizes at which tiles of 64 are more than the CUs, such as 257 to
 // 512 rows of that matrix: 300 rows in Q4_1 bf16 69.7 us with a split reduction, 63.7 here; of [16384, 2048] in Q8_0 52 and 36.
 // What bounds it is the 1.0 us of a K step (conversion, then 32 MFMAs per wavefront behind one barrier).
-template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI>
+//
+// TJ: 16-row column blocks of a wavefront.  TJ = 3 is for a single matrix whose token tiles, made equal, have at most 192 rows (129 to 192
+// rows, and 257 to 384, which would be a tile of 256 and a rest): the tile's rows are spread over the four token-row groups in multiples
+// of 16 (tile row grp * rpg + i lives in LDS row grp * 64 + i), so that every wavefront has 3 blocks to multiply instead of some four and
+// some none, and the launch, one round, ends with tiles of 150 rows instead of 256.  [14336, 4096] at 300 rows, us: Q4_1 bf16 64 -> 60, fp8
+// 58 -> 51, Q8_0 fp16 72 -> 59; [14336, 2048] Q8_0 39 -> 31; [8192, 4096] Q4_1 41 -> 38.  With both counts of blocks in
+// one kernel the full tiles were up to 10 % slower (Q8_0, 256 rows 41 -> 45).
+template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI, int TJ>
 __global__ void __launch_bounds__(64 * WN * WM, 1)
 grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
   constexpr int NTHR = 64 * WN * WM;
@@ -62,12 +69,14 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
   const int wn = wave / WM, wm = wave % WM;
 
   BigTile tile;
-  if (!big_tile_id(p, BM, n_tiles, false, tile)) return;
+  constexpr bool SPREAD = TJ < 4;
+  if (!big_tile_id(p, BM, n_tiles, false, tile, false, SPREAD ? 3 : 0)) return;
   int e = tile.e, row_begin = tile.row_begin, row_end = tile.row_end, ntile = tile.ntile;
   // (What the compiler can tell about these values from the lookup moves the scheduling of the K loop: with it the narrow Q4_1 tiles of
   // 64 features take 0.05 us more per step, 31.5 instead of 28.6 us for 200 rows of [2048, 3072].)
   asm volatile("" : "+s"(e), "+s"(row_begin), "+s"(row_end), "+s"(ntile));
   const int rows_here = row_end - row_begin;
+  const int rpg = SPREAD ? min(16 * TJ, ((rows_here + WM - 1) / WM + 15) / 16 * 16) : 64;
 
   // ---- producer assignment ---------------------------------------------------------------------------
   const int g = lane >> 4, n_in = lane & 15;
@@ -96,7 +105,7 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
 #pragma unroll
   for (int j = 0; j < XPIECES; ++j) {
     const int lr = (tid >> 3) + XROWS_PER_PASS * j;  // LDS row
-    const int r = min(lr, rows_here - 1);
+    const int r = min(SPREAD ? (lr >> 6) * rpg + min(lr & 63, rpg - 1) : lr, rows_here - 1);
     const int i = row_begin + r;
     const int64_t src = p.perm ? (int64_t)(p.perm[i] / p.k_top) : (int64_t)i;
     xoff[j] = (uint32_t)((src * p.lda + (((tid & 7) ^ (lr & 7)) << 3)) * 2);
@@ -153,25 +162,26 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
   // ---- consumer -----------------------------------------------------------------------------------------
   // wavefront tile: GATEUP gate rows wn*64..+63 (LDS rows wn*64..) and the same up rows (LDS rows BN/2 + wn*64..);
   //                 DOWN rows wn*128..+127.  Token rows wm*64..+63.
-  floatx4_t acc[TI][4];
+  floatx4_t acc[TI][TJ];
 #pragma unroll
   for (int a = 0; a < TI; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
-  const bool active = rows_here > wm * 64;  // wavefronts whose token rows are all past the end skip their MFMAs
+    for (int b = 0; b < TJ; ++b) acc[a][b] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+  const int my_rows = min(rpg, rows_here - wm * rpg);  // token rows of this wavefront's group
+  const bool active = my_rows > 0;                     // wavefronts whose token rows are all past the end skip their MFMAs
 
   auto compute = [&](auto parity_tag, int xstage, int ks) {
     constexpr int PAR = decltype(parity_tag)::value;
     const uint16_t* bp = b_rd[ks] + xstage * XSTAGE;
-    u32x4_t bf[4];
+    u32x4_t bf[TJ];
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) bf[tj] = *reinterpret_cast<const u32x4_t*>(bp + tj * 16 * BIG_LS);
+    for (int tj = 0; tj < TJ; ++tj) bf[tj] = *reinterpret_cast<const u32x4_t*>(bp + tj * 16 * BIG_LS);
 #pragma unroll
     for (int ti = 0; ti < TI; ++ti) {
       const int row_off = MODE == MODE_GATEUP ? (ti < TI / 2 ? 0 : BN / 2) + (ti % (TI / 2)) * 16 : ti * 16;
       const u32x4_t af = *reinterpret_cast<const u32x4_t*>(a_rd[ks] + PAR * WSTAGE + row_off * BIG_LS);
 #pragma unroll
-      for (int tj = 0; tj < 4; ++tj) acc[ti][tj] = mfma16b<T>(af, bf[tj], acc[ti][tj]);
+      for (int tj = 0; tj < TJ; ++tj) acc[ti][tj] = mfma16b<T>(af, bf[tj], acc[ti][tj]);
     }
   };
 
@@ -280,9 +290,9 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
     constexpr int ACT = decltype(act_tag)::value;
     const FakeQuant fq = fq_scale(p);
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-      const int r = wm * 64 + tj * 16 + n_in;
-      if (r < rows_here) {
+    for (int tj = 0; tj < TJ; ++tj) {
+      const int r = wm * rpg + tj * 16 + n_in;
+      if (tj * 16 + n_in < my_rows) {
         T* orow = reinterpret_cast<T*>(p.out) + out_row(p, row_begin + r) * p.ldo + (int64_t)ntile * (BN / 2) + wn * (WROWS / 2) + 4 * g;
 #pragma unroll
         for (int ti = 0; ti < TI / 2; ++ti) {
@@ -298,9 +308,9 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
     else store_gateup(EpiAct<STMOE_ACT_GELU_ERF>{});
   } else {
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-      const int r = wm * 64 + tj * 16 + n_in;
-      if (r < rows_here) {
+    for (int tj = 0; tj < TJ; ++tj) {
+      const int r = wm * rpg + tj * 16 + n_in;
+      if (tj * 16 + n_in < my_rows) {
         T* orow = reinterpret_cast<T*>(p.out) + out_row(p, row_begin + r) * p.ldo;
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti)
@@ -311,12 +321,12 @@ grouped_mfma_big_kernel(GemmParams p, int n_tiles) {
   }
 }
 
-template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI = 8>
+template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI = 8, int TJ = 4>
 static int launch_big_m(const GemmParams& p, int64_t max_rows, hipStream_t st) {
   constexpr int BN = 16 * TI * WN, BM = 64 * WM;
   constexpr size_t lds_bytes = (size_t)(2 * BN + 3 * BM) * BIG_LS * 2;
   static std::atomic<uint64_t> lds_ready{0};
-  auto kern = grouped_mfma_big_kernel<T, WF, MODE, WN, WM, STAGES, TI>;
+  auto kern = grouped_mfma_big_kernel<T, WF, MODE, WN, WM, STAGES, TI, TJ>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_ready, "mfma big kernel")) return rc;
   const int n_tiles = (int)(MODE == MODE_GATEUP ? p.n_out / (BN / 2) : p.n_out / BN);
   const int experts = p.offsets ? p.E : 1;
@@ -360,11 +370,18 @@ int launch_mfma_big(int act_dtype, int wtag, int mode, const GemmParams& p, int6
 
 // The narrow form: 64 weight rows x 256 token rows per workgroup (see the kernel's head), or 128 where tiles of 64 would not fit
 // one round over the 256 CUs (narrow_pays says where either is chosen).
+template <typename T, int WF, int MODE>
+static int launch_narrow_m(const GemmParams& p, int64_t max_rows, hipStream_t st) {
+  const bool wide = narrow_wide(MODE, p.n_out, max_rows);
+  // (without offsets the rows, and with them the tiles, are known here)
+  const int64_t tiles = (max_rows + 255) / 256;
+  if (!p.offsets && p.fixed_rows == max_rows && (max_rows + tiles - 1) / tiles <= 192)
+    return wide ? launch_big_m<T, WF, MODE, 2, 4, 2, 4, 3>(p, max_rows, st) : launch_big_m<T, WF, MODE, 2, 4, 2, 2, 3>(p, max_rows, st);
+  return wide ? launch_big_m<T, WF, MODE, 2, 4, 2, 4>(p, max_rows, st) : launch_big_m<T, WF, MODE, 2, 4, 2, 2>(p, max_rows, st);
+}
 template <typename T, int WF>
 static int launch_narrow_t(int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
-  const bool wide = narrow_wide(mode, p.n_out, max_rows);
-  if (mode == MODE_GATEUP) return wide ? launch_big_m<T, WF, MODE_GATEUP, 2, 4, 2, 4>(p, max_rows, st) : launch_big_m<T, WF, MODE_GATEUP, 2, 4, 2, 2>(p, max_rows, st);
-  return wide ? launch_big_m<T, WF, MODE_DOWN, 2, 4, 2, 4>(p, max_rows, st) : launch_big_m<T, WF, MODE_DOWN, 2, 4, 2, 2>(p, max_rows, st);
+  return mode == MODE_GATEUP ? launch_narrow_m<T, WF, MODE_GATEUP>(p, max_rows, st) : launch_narrow_m<T, WF, MODE_DOWN>(p, max_rows, st);
 }
 
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {

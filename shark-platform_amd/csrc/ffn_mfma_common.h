@@ -60,7 +60,8 @@ __device__ __forceinline__ bool big_tail_absorbed(int rows, int BM, bool absorb,
 // full tile and its expert's partial tile, half a launch apart, both fetch it from memory).  balance = 1 does that for
 // experts with one full tile, balance = 2 for any number of full tiles (650 rows: 3 x 217 instead of 256 + 256 + 138),
 // which pays where a tile with fewer rows is a faster unit (Q8_0: Mixtral layer at 4096 tokens 2 % faster) and costs
-// where the loaders set the pace of a unit whatever its rows (Q4_1: Grok-shape skewed prefill 2.4 % slower).
+// where the loaders set the pace of a unit whatever its rows (Q4_1: Grok-shape skewed prefill 2.4 % slower).  balance = 3 does it whatever
+// the remainder: for launches of one round, which end with their largest tile.
 struct BigExpertTiles {
   int main;     // tiles in the main list (full tiles, or the equal-sized ones)
   int partial;  // 1: a partial tile in the list of partial tiles
@@ -73,7 +74,7 @@ __device__ __forceinline__ BigExpertTiles big_expert_tiles(int rows, int BM, boo
   x.partial = 0;
   x.even = false;
   if (t == 0 || big_tail_absorbed(rows, BM, absorb, per_tile)) return x;
-  if (2 * t > BM && (balance == 2 ? c > 0 : balance == 1 && c == 1)) {
+  if (balance == 3 ? c > 0 : 2 * t > BM && (balance == 2 ? c > 0 : balance == 1 && c == 1)) {
     x.main = c + 1;
     x.even = true;
   } else {

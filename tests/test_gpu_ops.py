@@ -835,6 +835,27 @@ def test_narrow_tiles_of_128_features(device, fmt, dtype, rows):
         assert O.rel_l2(got.cpu().double(), want.cpu().double()) < 2.0 ** (-11 if dtype == torch.float16 else -8)
 
 
+@pytest.mark.parametrize("fmt,dtype", [("q8_0", torch.float16), ("q4_1", torch.bfloat16), ("fp8", torch.float16)])
+@pytest.mark.parametrize("rows", [1, 49, 192, 193, 257, 384, 385])
+def test_narrow_tiles_of_equal_rows(device, fmt, dtype, rows):
+    """Narrow tiles of at most 192 rows spread their rows over the four token-row groups: on both sides of every change of the tiling, bit
+    for bit against the 128 x 128 kernel (one running sum per output in the same order), 64 and 128 features per tile, plain and gated."""
+    import moe_cases as MC
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    K = 512
+    x = torch.randn(rows, K, generator=torch.Generator().manual_seed(rows)).to(dtype).to(device)
+    for N in (512, 16640):  # tiles of 64 features; 260 of them are more than the CUs from the first row on: tiles of 128
+        case = MC.build(MC.Case(T=4, K=K, N=N, E=1, k=1, fmt=fmt, dtype=dtype, seed=440))
+        dws = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], [1, N, K], n, device), stacked=True, prepack=True) for n in ("gate", "up")]
+        narrow, tile = (_hip.mmt(x, dws[0], variant=v) for v in (_hip.VARIANT_MFMA_NARROW, _hip.VARIANT_MFMA_TILE))
+        assert torch.equal(narrow.view(torch.int16), tile.view(torch.int16))
+        got, want = (_hip.grouped_gate_up(x, *dws, _hip.ACT_SILU, None, None, 1, variant=v) for v in (_hip.VARIANT_MFMA_NARROW, _hip.VARIANT_MFMA_TILE))
+        # (the same sums; the gated product may be rounded once more or less on the way: one unit of the last place)
+        assert O.rel_l2(got.cpu().double(), want.cpu().double()) < 2.0 ** (-11 if dtype == torch.float16 else -8)
+
+
 def test_probe_takes_a_device_without_an_index(device):
     from sharktank_amd import _hip
 
