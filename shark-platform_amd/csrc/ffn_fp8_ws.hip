@@ -40,19 +40,11 @@ __device__ __forceinline__ intx8_t join8(const u32x4_t& lo, const u32x4_t& hi) {
 // is flipped with bit 2 of the row; 8 consecutive rows reading the same logical unit then touch 32 distinct banks.
 __device__ __forceinline__ int x_unit(int row, int u) { return u ^ ((row >> 2) & 1); }
 
-// vm_load16_to_lds for a base that vector instructions have just written to scalar registers: a memory instruction may read those only
-// five wait states later, and the compiler's hazard handling does not look into inline assembly.
-__device__ __forceinline__ void f8_load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
-  const void* b = reinterpret_cast<const void*>((uint64_t)lo | ((uint64_t)hi << 32));
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(b), "s"(lds_addr) : "memory", "m0");
-}
-// The same for the first 16 lanes only (256 bytes), without a branch around it.  Every lane of the wavefront must be active.
+// vm_load16_to_lds for the first 16 lanes only (256 bytes), without a branch around it.  Every lane of the wavefront must be active.
 __device__ __forceinline__ void f8_load16_to_lds_16_lanes(const void* base, uint32_t byte_off, uint32_t lds_addr) {
   lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, 0xffff\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte_off), "s"(base), "s"(lds_addr)
+  asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, 0xffff\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte_off), "s"(base), "s"(lds_addr),
+               "n"(kBaseFromVector)
                : "memory", "m0");
 }
 
@@ -365,10 +357,10 @@ grouped_fp8_ws_kernel(F8Args args) {
         }
       }
       const uint32_t slot = (uint32_t)(gl % D) * STAGE;
-      f8_load16_to_lds(wq[0], lane16 + (uint32_t)sl * 1024, w_lds + slot);
-      f8_load16_to_lds(wq[1], lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
-      vm_load16_to_lds(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
-      vm_load16_to_lds(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
+      vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[0]), lane16 + (uint32_t)sl * 1024, w_lds + slot);
+      vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[1]), lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
+      vm_load16_to_lds<kBaseFromVector>(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
+      vm_load16_to_lds<kBaseFromVector>(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
       if constexpr (TAILS) f8_load16_to_lds_16_lanes(p.a, toff + (uint32_t)sl * x_stage_bytes, t_lds + slot);
       ++sl;
       ++gl;

@@ -264,10 +264,21 @@ static inline int reserve_lds(const void* kernel, size_t bytes, std::atomic<uint
 }
 
 // ---- hand-issued vector-memory operations ------------------------------------------------------------
+// A wave-uniform pointer in scalar registers, where the compiler cannot prove it uniform by itself.
+__device__ __forceinline__ const void* uniform_ptr(const void* p) {
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+  return reinterpret_cast<const void*>((uint64_t)lo | ((uint64_t)hi << 32));
+}
 // Lane l's 16 bytes at base + byte_off land at LDS byte address lds_addr + 16*l (base and lds_addr wave-uniform).
-__device__ __forceinline__ void vm_load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_addr) {
+// NOP: a memory instruction may read scalar registers that a vector instruction has written (v_readfirstlane, or v_readlane where the
+// compiler had put the base aside) only five wait states later, and the compiler's hazard handling does not look into inline assembly.
+// Kernels whose bases pass through vector instructions wait here (kBaseFromVector); those that compute them with scalar ones
+// do not (waiting costs the loaders of the Q4_1 prefill kernel 2 %), and a test looks through the built code for a base that is read early.
+static constexpr int kBaseFromVector = 4;
+template <int NOP = 0> __device__ __forceinline__ void vm_load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_addr) {
   lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);  // the compiler cannot always prove it uniform
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(lds_addr)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(lds_addr), "n"(NOP)
                : "memory", "m0");
 }
 template <int N> __device__ __forceinline__ void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }

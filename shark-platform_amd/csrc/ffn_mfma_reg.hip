@@ -63,14 +63,6 @@ template <> struct RegTile<WF_Q4_1_P> {
   }
 };
 
-// vm_load16_to_lds for a base that vector instructions have just written to scalar registers (v_readfirstlane, or v_readlane where the
-// compiler had put it aside): such registers may be read by a memory instruction only five wait states later, and the compiler's
-// hazard handling does not look into inline assembly.
-__device__ __forceinline__ void reg_load16_to_lds(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(lds_addr)
-               : "memory", "m0");
-}
 __device__ __forceinline__ u32x4_t reg_ld16(const uint8_t* base, uint32_t off) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + off));
 }
@@ -258,12 +250,9 @@ grouped_mfma_reg_kernel(RegArgs args) {
         xoff[j] = (uint32_t)((src * p.lda + (((lane & 31) ^ reg_x_swizzle<WF>(lr)) << 3)) * 2);
       }
       auto load_x = [&](int slot, int c) {
-        const uint64_t addr = reinterpret_cast<uint64_t>(p.a) + (uint32_t)c * 512u;  // (wave-uniform: goes into scalar registers)
-        const uint32_t addr_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
-        const uint32_t addr_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
-        const void* src = reinterpret_cast<const void*>((uint64_t)addr_lo | ((uint64_t)addr_hi << 32));
+        const void* src = uniform_ptr(reinterpret_cast<const uint8_t*>(p.a) + (uint32_t)c * 512u);
 #pragma unroll
-        for (int j = 0; j < NTJ; ++j) reg_load16_to_lds(src, xoff[j], lds0 + slot * STAGE + (16 * j + 2 * wave) * 512);
+        for (int j = 0; j < NTJ; ++j) vm_load16_to_lds<kBaseFromVector>(src, xoff[j], lds0 + slot * STAGE + (16 * j + 2 * wave) * 512);
       };
 #pragma unroll
       for (int c = 0; c < D - 1; ++c) load_x(c, min(c, last));

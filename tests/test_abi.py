@@ -108,3 +108,57 @@ def test_hand_scheduled_kernels_get_no_scratch_accesses_from_the_compiler():
         assert r["VGPRs Spill"] == "0", (n, r)
         if "grouped_mfma_ws_kernel" in n:
             assert int(r["VGPRs"]) <= 168, (n, r)  # 12 wavefronts per CU
+
+
+def test_hand_issued_loads_wait_for_their_base(tmp_path):
+    """A vector-memory instruction may read a scalar register that a vector instruction wrote only five wait states later.  The compiler
+    sees to that for its own instructions, not for those inside inline assembly.  In the built library no vector-memory instruction
+    reads such a register too early, and in the kernels whose bases pass through vector instructions (or come back from a scalar spill,
+    the same thing) every load into LDS carries the wait states itself, so that no register allocation can break one."""
+    import re
+    import shutil
+    import subprocess
+
+    from sharktank_amd import _hip
+
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    lib = str(tmp_path / "lib.so")
+    shutil.copy(_hip.library_path(), lib)
+    subprocess.run([objdump, "--offloading", lib], check=True, stdout=subprocess.DEVNULL, cwd=tmp_path)
+    memory = re.compile(r"(?:global|buffer|scratch)_\w+ .*?s\[(\d+):(\d+)\]")
+    vector_write = re.compile(r"v_(?:readlane_b32|readfirstlane_b32|cmp\w*) s(?:(\d+)|\[(\d+):(\d+)\]),")
+    scalar_write = re.compile(r"s_\w+ s(?:(\d+)|\[(\d+):(\d+)\]),")
+    span = lambda m: [int(m[1])] if m[1] else range(int(m[2]), int(m[3]) + 1)  # noqa: E731
+    waiting, bad = {"grouped_fp8_ws_kernel": 0, "grouped_mfma_reg_kernel": 0}, []
+    for obj in sorted(tmp_path.glob("*gfx950")):
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(obj)], check=True, capture_output=True, text=True).stdout
+        if "global_load_lds_dwordx4" not in text:  # (the kernels that issue loads by hand all have some of these)
+            continue
+        written, last_nop = {}, 0  # scalar register -> wait states since a vector instruction wrote it; those of a directly preceding s_nop
+        kernel = None
+        for line in text.splitlines():
+            if not line.startswith("\t"):  # (a label: what precedes it in the listing still counts, as if fallen through)
+                if line.endswith(">:") and "L0" not in line:
+                    kernel = next((k for k in waiting if k in line), None)
+                continue
+            ins = line.split("//")[0].strip()
+            if kernel and ins.startswith("global_load_lds_dwordx4"):
+                waiting[kernel] += 1
+                if last_nop < 5:
+                    bad.append((kernel, ins))
+            m = memory.match(ins)
+            if m and any(written.get(r, 5) < 5 for r in span((None, None, m[1], m[2]))):
+                bad.append(ins)
+            nop = re.match(r"s_nop (\w+)", ins)
+            last_nop = int(nop[1], 0) + 1 if nop else 0
+            written = {r: n + max(last_nop, 1) for r, n in written.items() if n < 5}
+            m = vector_write.match(ins)
+            if m:
+                written.update((r, 0) for r in span(m))
+            m = scalar_write.match(ins)
+            if m:
+                for r in span(m):
+                    written.pop(r, None)
+    assert all(waiting.values()) and not bad, (waiting, len(bad), bad[:5])
