@@ -423,8 +423,11 @@ grouped_fp8_ws_kernel(F8Args args) {
     __syncthreads();
   }  };
   // Ride-along rows save their expert's partial tile and cost the full tiles an MFMA per nine and their loads: a unit that carries them
-  // takes 10-15 % longer.  They are taken along where that saves a round over the CUs (8 experts of 4096 x 14336, 4096 tokens: gate/up 16
-  // rounds to 14, 1107 / 1050 us, down 3 to 2, 617 / 512; down at 1000 tokens is one round either way: 206 / 227).
+  // takes 10-15 % longer, every other one of the launch some 4 %.  They are taken along where that saves an eighth of the rounds over the
+  // CUs or more (8 experts of 4096 x 14336, 4096 tokens: gate/up 16 rounds to 14, 1107 / 1050 us, down 3 to 2, 617 / 512).  Over 3500
+  // launches of 4 to 16 experts, 1024 to 6144 x 1024 to 16384, what they save of the whole layer (median, worst): gate/up one round of 2
+  // 15, 7 %; of 4 4, -4 %; of 6 2, -2 %; of 8 2, -3 %; of 9 0, -3 %; of 14 and more -2, -6 %; two of 16 1, -1 %; down one of 2 10, -4 %; of
+  // 3 5, 0 %; of 4 to 6 2 to 4, 1 %.
   const int lane_end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);
   const int lane_rows = lane < E ? lane_end - lane_off : 0;
   auto rounds = [&](bool absorb) {
@@ -432,7 +435,7 @@ grouped_fp8_ws_kernel(F8Args args) {
     const int units = __builtin_amdgcn_readlane(wave_inclusive_sum(x.main + x.partial), 63) * n_tiles;
     return (units + 8 * wgs - 1) / (8 * wgs);
   };
-  if (rounds(true) < rounds(false)) walk(F8Int<1>{});
+  if (8 * rounds(true) <= 7 * rounds(false)) walk(F8Int<1>{});
   else walk(F8Int<0>{});
 }
 
