@@ -141,45 +141,67 @@ static bool dense_pays(int dtype, int wtag, int mode, const GemmParams& p, int64
 // have one unit's rows on average (us, prefill kernel / this one, gate/up and down, 8 experts of 4096 x 14336): Q4_1 bf16 25 rows 220 / 161
 // and 115 / 80, 51 rows 238 / 190 and 119 / 98, 63 rows 247 / 261 and 131 / 159; Q4_1 fp16 25 rows 208 / 124 and 110 / 62, 51 rows 220 / 163
 // and 117 / 84; Q8_0 fp16 25 rows 194 / 169 and 107 / 78, 51 rows 207 / 191 and 117 / 92; 64 experts of 2048 x 1536 at 28 rows (Q4_1 fp16)
-// 98 / 75 and 55 / 44; with a routing that gives one expert a third of the pairs 0.95 to 1.4 times as fast.  Beyond that it still is where
-// all its units fit one round (down: 8 of [1024, 2048] at 200 rows 42 / 18, 16 of [2048, 4096] at 100 rows 65 / 47, 4 of [4096, 8192]
-// at 75 rows 56 / 48; gate/up of 8 x 1024 x 2048 at 100 rows 24 / 20) and the reduction is not as long as 14336 (63 rows above).
+// 98 / 75 and 55 / 44.  Beyond that it still is where all its units fit one round (down: 8 of [1024, 2048] at 200 rows 42 / 18, 16 of
+// [2048, 4096] at 100 rows 65 / 47, 4 of [4096, 8192] at 75 rows 56 / 48; gate/up of 8 x 1024 x 2048 at 100 rows 24 / 20) and the
+// reduction is not as long as 14336 (63 rows above).
 // Against the streaming kernel it takes down projections whose half units fill three quarters of the CUs and whose reduction is long
 // enough to pay for the start of a unit (two rows per expert on average and 3072 elements: 8 of [4096, 14336], Q8_0 / Q4_1 fp16, 2 rows
 // 74 / 69 and 68 / 52, 8 rows 80 / 78 and 78 / 55, 16 rows 108 / 78 and 107 / 60; 16 of [3072, 6144] Q4_1 bf16 5 rows 61 / 57; 32 of
 // [2048, 2816] 6 rows 36 / 38), or half of them if experts have more than one token tile (4 of [4096, 8192]: 10 rows 26 / 29, 20 rows
 // 38 / 32, 32 rows 58 / 36).
+// Over 16000 whole layers (4 to 64 experts, 1024 to 6144 x 512 to 16384, 2 to 260 rows per expert, all formats in fp16 and bf16, routings
+// uniform or Zipf) it saves 9 % of the layer's time on average; 6 to 7 % of the launches it takes are slower by more than 1 %
+// (worst 16 % under a uniform routing, 18 % where one expert gets a third of the rows), scattered among others that gain: which experts
+// spill out of a round the totals that the rule sees do not tell.  reg_loses holds what lost as a group (what leaving it to the other
+// kernels gives, of the layer's time, mean and extremes).
+static bool reg_loses(int dtype, int wtag, int mode, int64_t kred, int64_t units, int64_t halves, int64_t E, int64_t rows, bool streams) {
+  const bool fast = wtag == WF_Q4_1_P && dtype == STMOE_F16;  // (the format that converts fastest gains in the first two)
+  // fewer than four rows per expert: under an uneven routing some experts have none and the halves no longer fill the CUs (16 and
+  // 8 experts: Zipf 8 and 5 %, -6 .. 29, uniform nothing, -8 .. 15; with 4 experts there is nothing to win)
+  if (streams) return !fast && rows < 4 * E && (E >= 16 ? halves <= 256 : E >= 8 && halves < 224);
+  // units for a quarter of the CUs and a long reduction, which the prefill kernel cuts in four (4 experts 9 %, -12 .. 35, 8 experts from
+  // 11264 elements on 6 %, -11 .. 27, below that 3 and, under Zipf, -1 %; with 16 nothing)
+  if (!fast && E <= 8 && units <= 64 && kred > (E <= 4 ? 8192 : 11264) && rows <= 52 * E) return true;
+  if (E < 32 || units <= 224 || units > 256) return false;
+  // one round of whole units that is nearly full, over many experts: some have more than 64 rows and spill into a second round
+  // (32 and 64 experts 7 %, -6 .. 14) ...
+  if (rows > (E >= 64 ? 47 : 51) * E && rows <= 64 * E) return true;
+  // ... or the reduction is short and its start, 5 us that nothing hides, counts (with the line above, 32 and 64 experts
+  // 3 and 5 %, -9 .. 27)
+  return wtag != WF_Q4_1_P && mode == MODE_GATEUP && kred <= 2560;
+}
+static bool reg_pays_grouped(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
+  const int64_t E = p.E, units = p.n_out / (mode == MODE_GATEUP ? 128 : 256) * E;  // units: with one token tile per expert
+  const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||
+                       rows <= skinny_max_avg_rows(p.E) * E;
+  const int64_t halves = 2 * (units / E) * std::min<int64_t>(E, rows);
+  if (reg_loses(dtype, wtag, mode, p.kred, units, halves, E, rows, streams)) return false;
+  if (streams) return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * E) || (halves >= 128 && rows > 16 * E));
+  if (p.kred < 1024) return false;
+  // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 37
+  // rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
+  if (wtag != WF_Q4_1_P && p.kred <= 2048 && units > 256 && rows > 24 * E) return false;
+  if (rows <= 52 * E) return true;
+  // (an expert's rows vary: by a seventh for a uniform routing of this many)
+  return p.kred <= 8192 && (rows * 8 / 7 / E + kRegUnitRows - 1) / kRegUnitRows * units <= 256;
+}
 // A single matrix: its half units run at the pace of their reduction, whatever their number, where the prefill kernel cuts the reduction
 // in four and the narrow tiles re-read the token rows ([out, in], other kernels / this one, Q8_0 fp16; Q4_1 bf16): [14336, 4096] 33 rows
 // 28 / 22; 31 / 26, 128 rows 42 / 27; 43 / 31, 160 rows 40 / 41; 39 / 48; [4096, 4096] 64 rows 21 / 21; 25 / 27, 100 rows 27 / 22;
 // 31 / 28, 256 rows 38 / 23; 37 / 28, 512 rows 39 / 29; 42 / 31; [4096, 14336] 128 rows 54 / 65; 68 / 83, 160 rows 76 / 65; 88 / 84, 512 rows
 // 96 / 82; 103 / 96; [8192, 8192] 64 rows 33 / 41; 40 / 50, 160 rows 56 / 41; 64 / 53, 256 rows 67 / 49; 72 / 57; [2048, 1024] 33 rows
 // 12 / 8; 13 / 9.  From 129 rows on reductions up to 2048 stay on the narrow tiles, which give the bits of an unsplit prefill launch
-// (13 / 10 at 300 rows).
+// (13 / 10 at 300 rows).  Over 1100 products of 33 to 2048 rows, 1024 to 6144 x 1024 to 16384, Q8_0 and Q4_1 in both types, none that comes
+// here is slower; median gain 27 to 56 % by format, at more than 1024 rows (narrow matrices) as at 64.  The gate/up pair of a dense
+// network follows the same line (3600 networks, all formats: none slower by more than 4 %, 2200 faster).
 static bool reg_pays(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (!reg_takes(dtype, wtag, mode, p, rows)) return false;
+  if (p.E > 1) return p.offsets && reg_pays_grouped(dtype, wtag, mode, p, rows);
   const int64_t tiles = p.n_out / (mode == MODE_GATEUP ? 128 : 256);  // units per token tile
-  if (p.E == 1) {
-    const int64_t units = (rows + kRegUnitRows - 1) / kRegUnitRows * tiles;
-    if (rows <= kSkinnyMaxRowsSingleSplit || p.kred < 1024 || units > 128) return false;
-    if (rows <= 64) return p.kred <= 2048 || (p.kred <= 4096 && tiles >= 32);
-    return rows > 128 ? p.kred > 2048 : p.kred <= 4096;
-  }
-  if (!p.offsets) return false;
-  const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||
-                       rows <= skinny_max_avg_rows(p.E) * p.E;
-  if (streams) {
-    const int64_t halves = 2 * tiles * std::min<int64_t>(p.E, rows);
-    return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * (int64_t)p.E) || (halves >= 128 && rows > 16 * (int64_t)p.E));
-  }
-  if (p.kred < 1024) return false;
-  // (short reductions over several rounds of units: a unit's start, 5 us that nothing hides, counts; the formats that convert faster gain
-  // less: 64 experts of 2048 x 1536, Q8_0 bf16 37 rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
-  if (wtag != WF_Q4_1_P && p.kred <= 2048 && tiles * p.E > 256 && rows > 24 * (int64_t)p.E) return false;
-  if (rows <= 52 * (int64_t)p.E) return true;
-  // (an expert's rows vary: by a seventh for a uniform routing of this many)
-  const int64_t units = (rows * 8 / 7 / p.E + kRegUnitRows - 1) / kRegUnitRows * tiles * p.E;
-  return p.kred <= 8192 && units <= 256;
+  const int64_t units = (rows + kRegUnitRows - 1) / kRegUnitRows * tiles;
+  if (rows <= kSkinnyMaxRowsSingleSplit || p.kred < 1024 || units > 128) return false;
+  if (rows <= 64) return p.kred <= 2048 || (p.kred <= 4096 && tiles >= 32);
+  return rows > 128 ? p.kred > 2048 : p.kred <= 4096;
 }
 // fp8 activations x fp8 weights on the fp8 matrix cores: the 256 x 256 kernel for packed weights and launches with
 // enough rows to fill its tiles (variant 5), the 128 x 128 kernel otherwise (and always with variant 7).

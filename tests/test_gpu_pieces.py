@@ -613,6 +613,62 @@ def test_ffn_mfma_reg_kernel(device, fmt, dtype, N, K, E, act):
     assert float((diff.norm(dim=1) / size).max()) < 4 * tol
 
 
+def _random_weight(fmt, shape, gen, device):
+    """A packed weight of random planes, made on the device (no reference for it: for launches that are compared with each other)."""
+    from sharktank_amd import types as ST
+    from sharktank_amd.ops import device_weight
+
+    blocks = [*shape[:-1], shape[-1] // 32]
+    scale = lambda top: (torch.rand(blocks + [1], generator=gen, device=device) * top).to(torch.float16)  # noqa: E731
+    if fmt == "q8_0":
+        qs = torch.randint(-127, 128, blocks + [32], generator=gen, device=device, dtype=torch.int8)
+        layout = ST.BlockScaledLayout(shape, scale(1e-3), qs)
+    elif fmt == "q4_1":
+        qs = torch.randint(0, 256, blocks + [16], generator=gen, device=device, dtype=torch.uint8)
+        layout = ST.BlockScaledI4Layout(shape, scale(1e-2), qs, m=-scale(5e-2), signed=False)
+    else:
+        qs = torch.randn(shape, generator=gen, device=device).mul_(100).clamp_(-448, 448).to(torch.float8_e4m3fn)
+        layout = ST.TensorScaledLayout(shape=shape, d=torch.tensor(1e-4, device=device), qs=qs)
+    dw = device_weight(ST.PlanarQuantizedTensor(name="w", shape=shape, layout=layout), stacked=True, prepack=True)
+    assert dw.is_packed
+    return dw
+
+
+@pytest.mark.parametrize("mode,fmt,dtype,E,k,T,kred,n_out,choice", [
+    # one round of whole units over many experts: a short reduction; in Q4_1, with rows for a second round
+    ("gate_up", "q8_0", torch.bfloat16, 32, 4, 300, 1024, 1024, "ws"),
+    ("gate_up", "q4_1", torch.bfloat16, 32, 4, 420, 1024, 1024, "ws"),
+    # units for a quarter of the CUs and a long reduction; few rows on many experts
+    ("down", "fp8", torch.float16, 4, 2, 67, 8448, 1024, "ws"),
+    ("down", "q4_1", torch.bfloat16, 16, 2, 16, 3328, 1792, "skinny"),
+    # inside the lines
+    ("gate_up", "q4_1", torch.bfloat16, 32, 4, 300, 1024, 1024, "reg"),
+    ("gate_up", "q4_1", torch.bfloat16, 8, 2, 203, 1024, 2048, "reg"),
+    ("gate_up", "q8_0", torch.float16, 8, 2, 120, 1024, 2048, "reg"),
+    ("down", "q4_1", torch.float16, 8, 2, 16, 3072, 4096, "reg"),
+    ("down", "q4_1", torch.float16, 16, 2, 16, 3328, 1792, "reg"),
+    ("down", "q8_0", torch.float16, 8, 2, 100, 9984, 1024, "reg"),
+])
+def test_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k, T, kred, n_out, choice):
+    """The automatic choice on both sides of the lines around the register kernel, told by the bits: the kernels add in different orders."""
+    hip = _hip()
+    gen = torch.Generator(device=device).manual_seed(91)
+    idx = torch.stack([torch.arange(k) + t for t in range(T)]).remainder(E).to(torch.int32).to(device)
+    _, offsets, perm, _ = hip.dispatch_build(idx, E)
+    w = _random_weight(fmt, [E, n_out, kred], gen, device)
+    a = torch.randn(T if mode == "gate_up" else T * k, kred, generator=gen, device=device).to(dtype)
+
+    def run(variant):
+        if mode == "gate_up":
+            return hip.grouped_gate_up(a, w, w, hip.ACT_SILU, offsets, perm, k, variant=variant).view(torch.int16)
+        return hip.grouped_down(a, w, offsets, T, k, variant=variant).view(torch.int16)
+
+    variants = {"reg": hip.VARIANT_MFMA_REG, "ws": hip.VARIANT_MFMA_WS, "skinny": hip.VARIANT_SKINNY}
+    auto = run(hip.VARIANT_AUTO)
+    assert torch.equal(auto, run(variants[choice]))
+    assert not torch.equal(auto, run(variants["reg" if choice != "reg" else "ws"]))
+
+
 def _raw_blocks(fmt: str, shape, seed: int):
     """Random bit patterns in ggml block structs: the scales are arbitrary fp16 bits (NaNs included), so a conversion
     anywhere on the way would show."""
