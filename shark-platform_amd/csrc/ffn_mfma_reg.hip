@@ -8,7 +8,9 @@
 // through LDS and no weight is converted twice.
 //
 //   chunk     256 reduction elements.  Weights: three register sets, requested three chunks ahead piece by piece as a set's registers
-//             come free; token rows: four LDS stages, filled three chunks ahead by direct loads, one barrier per chunk.
+//             come free; token rows: four LDS stages, filled three chunks ahead by direct loads, one barrier per chunk.  At a barrier
+//             the loads of two chunks could be in flight; the compiler's wait for the weights, which does not count the token loads,
+//             leaves 2 NTJ fewer (of 16 + 8 in a Q4_1 unit of two tiles and 64 rows, of 8 + 8 in a half unit).
 //   step      32 elements: the MFMAs of step s, the conversion of the weights of step s + 1 and the LDS reads of its token fragments
 //             are interleaved (the next chunk's first step included, so the barrier does not empty the matrix pipe).
 //   half unit the units after the last whole round over the workgroups are cut into two of 128 weight rows if the halves fit one round
@@ -17,7 +19,7 @@
 // What bounds it: at 25 rows per expert HBM (gate/up of 8 x 4096 x 14336, Q8_0 fp16 169 us = 5.9 TB/s, Q4_1 fp16 124 us = 4.7 TB/s), in
 // bf16 the vector instructions of the exact fp16 -> bf16 conversion (161 us); with more rows the issue slots of a SIMD, which its two
 // wavefronts' conversions and MFMAs share (51 rows 191, 163 and 190 us), and the requests of the CU's vector-memory path: leaving out the
-// scale loads, 256 bytes each, gave 7-10 %, leaving out the token loads 5-12 %.  Tried without gain: workgroups of four wavefronts, two per
+// scale loads, 256 bytes each, gave 7-10 %.  Tried without gain: workgroups of four wavefronts, two per
 // CU (token rows cross L2 twice: down 58 -> 80 us); sixteen wavefronts of one tile (128 registers: spills); the loads of a unit running
 // ahead into the next one (5-10 % for units of 8 chunks, 0-15 % slower for longer ones: the registers it needs are the third weight set).
 #include "ffn_mfma_common.h"
@@ -33,6 +35,30 @@ struct RegArgs {
 };
 
 static constexpr int kRegMaxTiles = kRegUnitRows / 16;  // 16-row token tiles of a unit
+static constexpr int kRegSets = 3, kRegStages = 4;      // register sets of weights, LDS stages of token rows
+
+// Vector-memory instructions that may be in flight when the token rows of the next chunk have to be there: what a wavefront issues after
+// them, `x` token loads and `w` weight loads a chunk.
+static constexpr int reg_wait(int x, int w) { return (kRegStages - 2) * x + (kRegSets - 1) * w; }
+// Whether every chunk's token rows have landed where they are read, for reductions of 1 to 9 chunks, in the order in which the kernel
+// issues its loads.  Loads return in the order of their issue.  At a barrier all but reg_wait() of those issued have landed, and the
+// weights of the chunk, which the compiler waits for at touch().  The refills of a register set in the chunks after the last whole
+// round over the sets are dead, and the compiler may drop them: they don't count as issued.
+static constexpr bool reg_tokens_landed(int x, int w) {
+  for (int chunks = 1; chunks <= 9; ++chunks) {
+    int issued = 0, x_end[16] = {}, w_end[16] = {};
+    w_end[0] = issued += w;
+    for (int c = 0; c < kRegStages - 1; ++c) x_end[c] = issued += x;
+    for (int c = 1; c < kRegSets; ++c) w_end[c] = issued += w;
+    for (int c = 0; c <= chunks; ++c) {  // the barrier in front of chunk c, then what chunk c issues up to the next one
+      const int landed = issued - reg_wait(x, w) > w_end[c] ? issued - reg_wait(x, w) : w_end[c];
+      if (landed < x_end[c]) return false;
+      x_end[c + kRegStages - 1] = issued += x;
+      if (c < chunks / kRegSets * kRegSets) w_end[c + kRegSets] = issued += w;
+    }
+  }
+  return true;
+}
 
 // A 16-row weight tile in the packed streaming order.  LOADS: load instructions per chunk.
 template <int WF> struct RegTile;
@@ -148,6 +174,12 @@ template <> struct RegData<WF_Q4_1_P> {
     return out;
   }
 };
+// The number of the lane within its wavefront, computed where it is asked for.
+__device__ __forceinline__ int lane_again() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+  return l;
+}
 // 16-byte unit of a token row that lane group g needs for MFMA step s (rows of 256 elements = 32 units)
 template <int WF> __device__ __forceinline__ int reg_x_unit(int s, int g) {
   return IsQ4<WF>::value ? 16 * (s >> 2) + 4 * g + (s & 3) : 8 * (s >> 1) + 2 * g + (s & 1);
@@ -204,10 +236,9 @@ grouped_mfma_reg_kernel(RegArgs args) {
 
     auto unit = [&](auto nt_tag, auto ntj_tag) {
       constexpr int NT = decltype(nt_tag)::value, NTJ = decltype(ntj_tag)::value;
-      constexpr int S = 3, WL = RegTile<WF>::LOADS * NT;
+      constexpr int S = kRegSets, D = kRegStages, WL = RegTile<WF>::LOADS * NT;
       constexpr int STAGE = 16 * NTJ * 512;
-      constexpr int D = 4;
-      constexpr int XWAIT = (D - 2) * NTJ + (S - 1 < D - 1 ? S - 1 : D - 1) * WL;
+      static_assert(reg_tokens_landed(NTJ, WL), "a chunk's token rows may be read before they have landed");
       // vector instructions that convert one weight fragment, for the issue order of a step
       constexpr int VALU_STEP = (WF == WF_FP8_F32D_P ? 14 : IsQ4<WF>::value ? 17 : 16) + (__is_same(T, f16_t) || WF == WF_FP8_F32D_P ? 0 : 12);
       // weight tiles of this wavefront
@@ -277,9 +308,10 @@ grouped_mfma_reg_kernel(RegArgs args) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) af[set][t] = wc[t].template frag<T>(wt[t], s, g);
       };
-      // the weights of chunk c + 1 and this wavefront's share of its token rows have landed, then everybody's
+      // The weights of chunk c + 1 and this wavefront's share of its token rows have landed, then everybody's.  The compiler adds its own
+      // wait for the weights at touch(), which counts weight loads only: it lets (S - 1) WL be in flight, (D - 2) NTJ fewer than would do.
       auto arrive = [&](RegData<WF>(&wn)[NT]) __attribute__((always_inline)) {
-        vm_wait<XWAIT>();
+        vm_wait<reg_wait(NTJ, WL)>();
 #pragma unroll
         for (int t = 0; t < NT; ++t) wn[t].touch();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -326,20 +358,21 @@ grouped_mfma_reg_kernel(RegArgs args) {
       for (int j = 0; j < NTJ; ++j) read_x(0, 0, j);
       convert(0, w[0], 0);
       __builtin_amdgcn_sched_barrier(0);
-      // whole rounds over the register sets, then what is left: one loop without exits in its body, so that the compiler's
-      // count of the weight loads in flight is exact at every wait
+      // whole rounds over the register sets, then what is left: one loop without exits in its body, so that the compiler knows at
+      // every wait how many weight loads are in flight
       for (int r = nch / S; r > 0; --r) {
 #pragma unroll
         for (int i = 0; i < S; ++i) chunk(w[i], w[(i + 1) % S]);
       }
       const int left = nch % S;
       if (left > 0) chunk(w[0], w[1]);
-      if constexpr (S > 2) {
-        if (left > 1) chunk(w[1], w[2]);
-      }
+      if (left > 1) chunk(w[1], w[2]);
       vm_wait<0>();
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS is free for the next unit (and the exchange below)
-      const int r0 = row_begin + n_in;
+      // (Q8_0 in bf16 has the longest conversion and two registers too few for the epilogue's addresses through the K loop: there the
+      // lane's number is computed again.  The other instances have them to spare, and Q4_1 in fp16 would be 1 % slower for it)
+      const int out_lane = WF == WF_Q8_0_P && !__is_same(T, f16_t) ? lane_again() : lane;
+      const int r0 = row_begin + (out_lane & 15), c0 = 4 * (out_lane >> 4);
       if constexpr (MODE == MODE_GATEUP) {
         if constexpr (NT == 1) {  // the up sums travel to the wavefront that has the gate sums
           if (wave >= 4) {
@@ -362,7 +395,7 @@ grouped_mfma_reg_kernel(RegArgs args) {
               __builtin_amdgcn_sched_barrier(0);  // (one tile at a time: the accumulators leave no room for more)
               if (r < row_end) {
                 const float gq[4] = {acc[0][j][0], acc[0][j][1], acc[0][j][2], acc[0][j][3]}, uq[4] = {up[0], up[1], up[2], up[3]};
-                *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + out_row(p, r) * p.ldo + col[0] + 4 * g) = gateup_quad<T, ACT>(gq, uq, fq);
+                *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + out_row(p, r) * p.ldo + col[0] + c0) = gateup_quad<T, ACT>(gq, uq, fq);
               }
             }
           };
@@ -375,7 +408,7 @@ grouped_mfma_reg_kernel(RegArgs args) {
         for (int j = 0; j < NTJ; ++j) {
           const int r = r0 + 16 * j;
           if (r < row_end) {
-            T* orow = reinterpret_cast<T*>(p.out) + out_row(p, r) * p.ldo + 4 * g;
+            T* orow = reinterpret_cast<T*>(p.out) + out_row(p, r) * p.ldo + c0;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
               *reinterpret_cast<uint2*>(orow + col[t]) =
