@@ -154,28 +154,29 @@ static bool dense_pays(int dtype, int wtag, int mode, const GemmParams& p, int64
 // (worst 16 % under a uniform routing, 18 % where one expert gets a third of the rows), scattered among others that gain: which experts
 // spill out of a round the totals that the rule sees do not tell.  reg_loses holds what lost as a group (what leaving it to the other
 // kernels gives, of the layer's time, mean and extremes).
-static bool reg_loses(int dtype, int wtag, int mode, int64_t kred, int64_t units, int64_t halves, int64_t E, int64_t rows, bool streams) {
+static bool reg_loses(int dtype, int wtag, int mode, const GemmParams& p, int64_t units, int64_t halves, int64_t rows, bool streams) {
+  const int64_t E = p.E;
   const bool fast = wtag == WF_Q4_1_P && dtype == STMOE_F16;  // (the format that converts fastest gains in the first two)
   // fewer than four rows per expert: under an uneven routing some experts have none and the halves no longer fill the CUs (16 and
   // 8 experts: Zipf 8 and 5 %, -6 .. 29, uniform nothing, -8 .. 15; with 4 experts there is nothing to win)
   if (streams) return !fast && rows < 4 * E && (E >= 16 ? halves <= 256 : E >= 8 && halves < 224);
-  // units for a quarter of the CUs and a long reduction, which the prefill kernel cuts in four (4 experts 9 %, -12 .. 35, 8 experts from
-  // 11264 elements on 6 %, -11 .. 27, below that 3 and, under Zipf, -1 %; with 16 nothing)
-  if (!fast && E <= 8 && units <= 64 && kred > (E <= 4 ? 8192 : 11264) && rows <= 52 * E) return true;
+  // units for a quarter of the CUs and a long reduction, which the prefill kernel cuts in four where it has scratch (4 experts 9 %,
+  // -12 .. 35, 8 experts from 11264 elements on 6 %, -11 .. 27, below that 3 and, under Zipf, -1 %; with 16 nothing)
+  if (!fast && p.split_scratch && E <= 8 && units <= 64 && p.kred > (E <= 4 ? 8192 : 11264) && rows <= 52 * E) return true;
   if (E < 32 || units <= 224 || units > 256) return false;
   // one round of whole units that is nearly full, over many experts: some have more than 64 rows and spill into a second round
   // (32 and 64 experts 7 %, -6 .. 14) ...
   if (rows > (E >= 64 ? 47 : 51) * E && rows <= 64 * E) return true;
   // ... or the reduction is short and its start, 5 us that nothing hides, counts (with the line above, 32 and 64 experts
   // 3 and 5 %, -9 .. 27)
-  return wtag != WF_Q4_1_P && mode == MODE_GATEUP && kred <= 2560;
+  return wtag != WF_Q4_1_P && mode == MODE_GATEUP && p.kred <= 2560;
 }
 static bool reg_pays_grouped(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   const int64_t E = p.E, units = p.n_out / (mode == MODE_GATEUP ? 128 : 256) * E;  // units: with one token tile per expert
   const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||
                        rows <= skinny_max_avg_rows(p.E) * E;
   const int64_t halves = 2 * (units / E) * std::min<int64_t>(E, rows);
-  if (reg_loses(dtype, wtag, mode, p.kred, units, halves, E, rows, streams)) return false;
+  if (reg_loses(dtype, wtag, mode, p, units, halves, rows, streams)) return false;
   if (streams) return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * E) || (halves >= 128 && rows > 16 * E));
   if (p.kred < 1024) return false;
   // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 37

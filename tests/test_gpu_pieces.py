@@ -669,6 +669,21 @@ def test_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k,
     assert not torch.equal(auto, run(variants["reg" if choice != "reg" else "ws"]))
 
 
+def test_register_kernel_without_scratch_for_split_reductions(device):
+    """A grouped product has no scratch, so the prefill kernel cannot cut its reduction: few units with a long one stay on the register
+    kernel, which the same shape leaves where there is scratch (above)."""
+    hip = _hip()
+    E, k, T, kred, n_out = 4, 2, 67, 8448, 1024
+    gen = torch.Generator(device=device).manual_seed(92)
+    idx = torch.stack([torch.arange(k) + t for t in range(T)]).remainder(E).to(torch.int32).to(device)
+    _, offsets, perm, _ = hip.dispatch_build(idx, E)
+    w = _random_weight("fp8", [E, n_out, kred], gen, device)
+    a = torch.randn(T, kred, generator=gen, device=device).to(torch.float16)
+    auto, reg, ws = (hip.grouped_mmt(a, w, offsets, perm, T, k, a_per_pair=False, variant=v).view(torch.int16)
+                     for v in (hip.VARIANT_AUTO, hip.VARIANT_MFMA_REG, hip.VARIANT_MFMA_WS))
+    assert torch.equal(auto, reg) and not torch.equal(auto, ws)
+
+
 def _raw_blocks(fmt: str, shape, seed: int):
     """Random bit patterns in ggml block structs: the scales are arbitrary fp16 bits (NaNs included), so a conversion
     anywhere on the way would show."""
