@@ -44,7 +44,7 @@ def test_empty_batch(device):
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
 def test_prefill_with_experts_that_get_no_rows(device, fmt):
     """600 tokens all routed to experts 2 and 5 of 8: two experts with 600 rows (three token tiles, the last one
-    partial), six without rows; the launch is small enough that units are split along the reduction."""
+    partial), six without rows."""
     case = MC.build(MC.Case(T=600, K=512, N=768, E=8, k=2, fmt=fmt, dtype=torch.float16, seed=71))
     idx = torch.tensor([[2, 5]]).repeat(600, 1)
     idx[::2] = torch.tensor([5, 2])

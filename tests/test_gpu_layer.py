@@ -478,13 +478,13 @@ def test_prefill_front_end_equals_staged_calls(device, dtype, T, K, E, k, norm_i
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("fmt,T,K,N", [("fp8", 40, 512, 768), ("fp8", 300, 512, 768), ("q8_0", 1100, 2048, 512), ("fp8", 700, 512, 256)])
+@pytest.mark.parametrize("fmt,T,K,N", [("fp8", 40, 512, 768), ("fp8", 300, 512, 768), ("q8_0", 1100, 2048, 512), ("q8_0", 2300, 3328, 512), ("fp8", 700, 512, 256)])
 def test_fused_activation_quantizers_equal_separate_passes(device, fmt, dtype, T, K, N):
     """Static e4m3fn quantizers of the experts' input and of the gated intermediate are applied where those tensors are
     produced (the norm launch writes the fake-quantised rows, the gate/up kernels write the fake-quantised intermediate).
     The result must have the bits of the same forward with each quantizer as a pass of its own over the finished tensor
-    (stmoe_fake_quant_fp8, itself bit-exact against the oracle): the streaming kernel, the prefill kernels with ride-along
-    rows and split units, and both front-end kernels are covered by the shapes."""
+    (stmoe_fake_quant_fp8, itself bit-exact against the oracle): the streaming kernel, the register kernel (1100 tokens), the
+    prefill kernels with ride-along rows and split units (2300 tokens), and both front-end kernels are covered by the shapes."""
     from sharktank_amd import _hip
     from sharktank_amd.layers import MoeBlock
     from sharktank_amd.types import unbox_tensor

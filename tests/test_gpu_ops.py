@@ -120,19 +120,21 @@ def test_quantized_linear_few_hundred_rows_splits_the_reduction(device, fmt, dty
     assert need > 0 and int(lib.stmoe_mmt_workspace_bytes(32)) == 0
     ws = torch.full((need,), 0xA5, dtype=torch.uint8, device=device)  # stale contents must not matter
     tol = 1e-3 if dtype == torch.float16 else 8e-3
-    # (the 256 x 256 kernel is named: from 129 rows on the automatic choice takes this matrix to 64 x 256 tiles, which need
-    # no split; up to 128 rows it is the automatic choice)
-    ws_kernel = _hip.VARIANT_MFMA_WS if M > 128 else _hip.VARIANT_AUTO
+    # (the 256 x 256 kernel is named: the automatic choice takes this matrix to the register kernel up to 128 rows and to 64 x 256 tiles
+    # from 129 on, neither of which splits)
+    ws_kernel = _hip.VARIANT_MFMA_WS
     plain = _hip.mmt(x.to(device), dw, workspace=torch.empty(0, dtype=torch.uint8, device=device), variant=ws_kernel)
     assert O.rel_l2(plain.cpu(), ref) < tol
     first = _hip.mmt(x.to(device), dw, workspace=ws, variant=ws_kernel)
     second = _hip.mmt(x.to(device), dw, workspace=ws, variant=ws_kernel)
-    default = _hip.mmt(x.to(device), dw)
+    own = _hip.mmt(x.to(device), dw, variant=ws_kernel)  # the binding's own buffer
     assert O.rel_l2(first.cpu(), ref) < tol
-    assert torch.equal(first.view(torch.int16), second.view(torch.int16))
-    # the binding's own buffer: the split sums again, or (narrow tiles) one running sum per output like `plain`
-    assert torch.equal(default.view(torch.int16), (first if M <= 128 else plain).view(torch.int16))
+    assert torch.equal(first.view(torch.int16), second.view(torch.int16)) and torch.equal(first.view(torch.int16), own.view(torch.int16))
+    assert not torch.equal(first.view(torch.int16), plain.view(torch.int16))  # (the reduction was split)
     assert O.rel_l2(first.float().cpu(), plain.float().cpu()) < (5e-4 if dtype == torch.float16 else 4e-3)
+    # (narrow tiles keep one running sum per output like `plain`)
+    auto = _hip.mmt(x.to(device), dw)
+    assert torch.equal(auto.view(torch.int16), (_hip.mmt(x.to(device), dw, variant=_hip.VARIANT_MFMA_REG) if M <= 128 else plain).view(torch.int16))
 
 
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
@@ -213,7 +215,11 @@ def test_quantized_linear_split_reduction_under_hip_graph_capture(device):
     dw = device_weight(it, stacked=True, prepack=True)
     g = torch.Generator().manual_seed(78)
     inputs = [(torch.randn(M, K, generator=g) * 0.5).to(torch.float16).to(device) for _ in range(3)]
-    eager = [_hip.mmt(x, dw) for x in inputs]  # (also the warm-up that capture needs)
+    # (the prefill kernel is named: the automatic choice takes this matrix to the register kernel, which does not split)
+    split = lambda x, **kw: _hip.mmt(x, dw, variant=_hip.VARIANT_MFMA_WS, **kw)  # noqa: E731
+    eager = [split(x) for x in inputs]  # (also the warm-up that capture needs)
+    unsplit = split(inputs[0], workspace=torch.empty(0, dtype=torch.uint8, device=device))
+    assert not torch.equal(eager[0].view(torch.int16), unsplit.view(torch.int16))
     torch.cuda.synchronize()
     static_in = torch.empty_like(inputs[0])
     graph = torch.cuda.CUDAGraph()
@@ -222,7 +228,7 @@ def test_quantized_linear_split_reduction_under_hip_graph_capture(device):
     with torch.cuda.stream(side):
         static_in.copy_(inputs[0])
         with torch.cuda.graph(graph, stream=side):
-            static_out = _hip.mmt(static_in, dw)
+            static_out = split(static_in)
     torch.cuda.current_stream().wait_stream(side)
     for rep in range(2):
         for x, want in zip(inputs, eager):
@@ -231,7 +237,7 @@ def test_quantized_linear_split_reduction_under_hip_graph_capture(device):
             got = static_out.clone()
             torch.cuda.synchronize()
             assert torch.equal(got.view(torch.int16), want.view(torch.int16))
-            again = _hip.mmt(x, dw)  # eager work between the replays
+            again = split(x)  # eager work between the replays
             assert torch.equal(again.view(torch.int16), want.view(torch.int16))
 
 
@@ -418,7 +424,7 @@ def test_quantized_matmul_descriptor_is_built_once_and_packed(device):
 
 
 @pytest.mark.parametrize("fmt", ["q8_0", "q4_1"])
-@pytest.mark.parametrize("M", [1, 32, 33, 100, 2048])  # 33, 100: the prefill kernel with its reductions split (scratch appended to the workspace)
+@pytest.mark.parametrize("M", [1, 32, 33, 100, 2048])  # 33 (down), 100: the prefill kernel with its reductions split (scratch appended to the workspace)
 def test_ffn_layer_llama_shape(device, fmt, M):
     """FFN (sharktank/sharktank/layers/ffn_block.py:21-51) at a Llama-8B shape, hidden 4096, FFN 14336, quantized weights:
     the gated form on the fused kernels against the closed form down(silu(gate x) * up x) of the oracle, row by row."""

@@ -613,6 +613,39 @@ def test_ffn_mfma_reg_kernel(device, fmt, dtype, N, K, E, act):
     assert float((diff.norm(dim=1) / size).max()) < 4 * tol
 
 
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_register_kernel_single_matrix_and_scattered_rows(device, fmt, dtype):
+    """The register kernel outside the grouped FFN, forced: a single matrix and its gate/up pair without offsets, on both sides of its
+    16-row tiles and 64-row units, and a grouped product whose output rows go back to pair order.  Against the 128 x 128 kernel: the same
+    products in another order, a value moves by one unit of the last place where its sum sits at a rounding boundary (a gated one may
+    be rounded the other way three times)."""
+    hip = _hip()
+    from sharktank_amd.ops import device_weight
+
+    K, N, E, k, T = 768, 512, 5, 2, 90
+    ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    case = MC.build(MC.Case(T=4, K=K, N=N, E=E, k=1, fmt=fmt, dtype=dtype, seed=97))
+    stacked = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], [E, N, K], n, device), stacked=True, prepack=True) for n in ("gate", "up")]
+    single = MC.build(MC.Case(T=4, K=K, N=N, E=1, k=1, fmt=fmt, dtype=dtype, seed=98))
+    pair = [device_weight(MC.to_inference_tensor(fmt, single.planes[n], [1, N, K], n, device), stacked=True, prepack=True) for n in ("gate", "up")]
+    gen = torch.Generator().manual_seed(99)
+
+    def worst_row(run):
+        reg, tile = (run(v).cpu().double().reshape(-1, N) for v in (hip.VARIANT_MFMA_REG, hip.VARIANT_MFMA_TILE))
+        return float(((reg - tile).norm(dim=1) / tile.norm(dim=1)).max())
+
+    for rows in (1, 16, 17, 64, 65, 200):
+        x = torch.randn(rows, K, generator=gen).to(dtype).to(device)
+        assert worst_row(lambda v: hip.mmt(x, pair[0], variant=v)) < ulp
+        assert worst_row(lambda v: hip.grouped_gate_up(x, *pair, hip.ACT_SILU, None, None, 1, variant=v)) < 3 * ulp
+    idx = torch.stack([torch.randperm(E, generator=gen)[:k] for _ in range(T)])
+    _, offsets, perm, _ = hip.dispatch_build(idx.to(torch.int32).to(device), E)
+    for per_pair in (False, True):
+        a = torch.randn(T * k if per_pair else T, K, generator=gen).to(dtype).to(device)
+        assert worst_row(lambda v: hip.grouped_mmt(a, stacked[0], offsets, perm, T, k, a_per_pair=per_pair, variant=v)) < ulp
+
+
 def _random_weight(fmt, shape, gen, device):
     """A packed weight of random planes, made on the device (no reference for it: for launches that are compared with each other)."""
     from sharktank_amd import types as ST
