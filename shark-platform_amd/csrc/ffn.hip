@@ -51,6 +51,8 @@ static int check_weight(const stmoe_weight* w, const char* who, int64_t E, int64
 //          9 MFMA 64 x 256 tile, the narrow form of 4 (a single matrix with a few hundred rows; packed formats)
 //         10 fp32 activations on the fp32 matrix cores
 //         11 256-row tiles of unquantized 16-bit weights, both operands straight into LDS
+//         12 units of 256 weight rows x 64 token rows, weights converted in the registers of the wavefronts that multiply
+//            them (some dozen rows per expert, single matrices of a few hundred rows; packed formats)
 // Automatic choice with fp8 weights and static quantizers on both activations: a prefill-sized launch with fp16
 // activations goes to the fp8 matrix cores (variant 5: both operands as bytes, the fp32 dot product scaled once; 1.8 times
 // faster than dequantise-then-multiply, and 6e-3 from it on the layer output at the Mixtral shape, inside the 2e-2 the fp8
@@ -71,7 +73,8 @@ static int effective_variant(int variant, int dtype, int64_t rows, int64_t K, in
 // the streaming kernel when no expert can get more than 32 rows (token count <= 32), when the launch has at most 128 rows
 // in all (such launches get no scratch for split reductions, without which the prefill kernel leaves most CUs idle), or
 // when experts get 16 rows or fewer on average (28 with at most 4 experts); everything else goes to the
-// specialised-wavefront prefill kernel.  Measured on the Mixtral layer (top-2, Q8_0 fp16, whole layer, us; streaming /
+// specialised-wavefront prefill kernel.  (On both sides of that line packed formats go to the register kernel where it pays,
+// reg_pays; 16-bit weights to a kernel of their own, dense_pays.)  Measured on the Mixtral layer (top-2, Q8_0 fp16, whole layer, us; streaming /
 // prefill kernel with split scratch): 8 experts at 64 / 80 / 96 / 128 / 160 tokens 297 / 340 / 360 / 436 / 559 against
 // 307 / 310 / 315 / 321 / 331 (Q4_1 bf16: 285 / 330 / 358 / 434 / 565 against 332 / 334 / 335 / 339 / 346); 4 experts at
 // 48 / 56 / 64 / 80 tokens 168 / 172 / 235 / 295 against 183 / 184 / 186 / 190; 2 experts at 40 / 64 tokens 171 / 185

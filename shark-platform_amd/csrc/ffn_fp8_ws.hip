@@ -22,8 +22,9 @@
 //            quantise the gated intermediate to e4m3fn for the down projection.
 //   What bounds it: at 256 flop per operand byte the tile needs 32 KB per stage from L2 / HBM; with the operand loads
 //   alone (no MFMA) the launch takes two thirds of its full time and with the MFMAs alone 60 %, i.e. the two overlap only
-//   partly: the bytes in flight (3 or 4 stages of 32 KB, no difference) cover the load latency under load only
-//   just.  Reading the next stage's operands from LDS ahead of the barrier (software pipelining) changed nothing.
+//   partly.  More bytes in flight change nothing (3 or 4 stages of 32 KB ahead), nor does reading the next stage's operands from LDS
+//   ahead of the barrier.  What keeps them apart has not been taken apart further; all eight wavefronts read their operands behind one
+//   barrier per stage.
 #include "ffn_mfma_common.h"
 
 namespace stmoe {
@@ -155,273 +156,274 @@ grouped_fp8_ws_kernel(F8Args args) {
   // Launches without ride-along rows walk their units with an instance that knows nothing of them: their loads and the branches around
   // them cost 4 % (2048 rows of one expert, gate/up 239 -> 249 us).
   auto walk = [&](auto tails_tag) __attribute__((always_inline)) {
-  constexpr bool TAILS = decltype(tails_tag)::value != 0;
-  // LDS-direct loads per wavefront and stage: 2 weight pieces, 2 x 16 token rows and 4 ride-along rows
-  constexpr int LOADS = TAILS ? 5 : 4;
+    constexpr bool TAILS = decltype(tails_tag)::value != 0;
+    // LDS-direct loads per wavefront and stage: 2 weight pieces, 2 x 16 token rows and 4 ride-along rows
+    constexpr int LOADS = TAILS ? 5 : 4;
 
-  // ---- operands: lane (r, h) supplies row r, samples 32 h .. 32 h + 31 ------------------------------------
-  const int wn = wave & 1, wm = wave >> 1;
-  const int r32 = lane & 31, h32 = lane >> 5;
-  // weight row r of a 32-row block: piece r / 16, lane position 16 g + r % 16 for g = 2 h, 2 h + 1
-  const uint8_t* const a_rd = lds8 + (MODE == MODE_GATEUP ? wn * 4 : wn * 8) * 1024 + (r32 >> 4) * 1024 + ((32 * h32 + (r32 & 15)) << 4);
-  const int xrow = wm * 64 + r32;
-  const uint8_t* const b_rd = lds8 + WSTAGE + xrow * KS;
-  const int bu0 = x_unit(xrow, 2 * h32) << 4, bu1 = x_unit(xrow, 2 * h32 + 1) << 4;  // rows xrow and xrow + 32 swizzle alike
-  floatx16_t acc[4][2];
-  // Ride-along rows.  The four wavefronts that share a weight half (128 rows) take 32 of its rows each against all of the unit's ride-along
-  // rows: one MFMA per stage, GATEUP 16 gate rows and the same 16 up rows, so that both sums of a feature meet in one lane.
-  floatx16_t tacc;
-  auto compute_tail = [&](int slot) __attribute__((always_inline)) {
-    const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? ((r32 >> 4) * 7 + wm) * 1024 : wm * 2048);
-    const uint8_t* bp = b_rd + slot * STAGE + (BM - wm * 64) * KS;  // (rows BM + r32: swizzled like xrow)
-    const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
-    const intx8_t bf = join8(*reinterpret_cast<const u32x4_t*>(bp + bu0), *reinterpret_cast<const u32x4_t*>(bp + bu1));
-    tacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf, tacc, 0, 0, 0, 127, 0, 127);
-  };
-  auto compute = [&](auto both_tag, int slot) __attribute__((always_inline)) {
-    constexpr bool BOTH = decltype(both_tag)::value;  // rows in both 32-row token blocks
-    const uint8_t* bp = b_rd + slot * STAGE;
-    intx8_t bf[2];
-#pragma unroll
-    for (int q = 0; q < (BOTH ? 2 : 1); ++q)
-      bf[q] = join8(*reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu0), *reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu1));
-#pragma unroll
-    for (int ti = 0; ti < 4; ++ti) {
-      // 32-row block ti of the wavefront: GATEUP blocks 0, 1 are gate rows, 2, 3 the matching up rows (pieces 8 ..)
-      const int piece_off = MODE == MODE_GATEUP ? (ti < 2 ? 0 : 8) + (ti & 1) * 2 : ti * 2;
-      const uint8_t* ap = a_rd + slot * STAGE + piece_off * 1024;
+    // ---- operands: lane (r, h) supplies row r, samples 32 h .. 32 h + 31 ------------------------------------
+    const int wn = wave & 1, wm = wave >> 1;
+    const int r32 = lane & 31, h32 = lane >> 5;
+    // weight row r of a 32-row block: piece r / 16, lane position 16 g + r % 16 for g = 2 h, 2 h + 1
+    const uint8_t* const a_rd = lds8 + (MODE == MODE_GATEUP ? wn * 4 : wn * 8) * 1024 + (r32 >> 4) * 1024 + ((32 * h32 + (r32 & 15)) << 4);
+    const int xrow = wm * 64 + r32;
+    const uint8_t* const b_rd = lds8 + WSTAGE + xrow * KS;
+    const int bu0 = x_unit(xrow, 2 * h32) << 4, bu1 = x_unit(xrow, 2 * h32 + 1) << 4;  // rows xrow and xrow + 32 swizzle alike
+    floatx16_t acc[4][2];
+    // Ride-along rows.  The four wavefronts that share a weight half (128 rows) take 32 of its rows each against all of the unit's ride-along
+    // rows: one MFMA per stage, GATEUP 16 gate rows and the same 16 up rows, so that both sums of a feature meet in one lane.
+    floatx16_t tacc;
+    auto compute_tail = [&](int slot) __attribute__((always_inline)) {
+      const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? ((r32 >> 4) * 7 + wm) * 1024 : wm * 2048);
+      const uint8_t* bp = b_rd + slot * STAGE + (BM - wm * 64) * KS;  // (rows BM + r32: swizzled like xrow)
       const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
+      const intx8_t bf = join8(*reinterpret_cast<const u32x4_t*>(bp + bu0), *reinterpret_cast<const u32x4_t*>(bp + bu1));
+      tacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf, tacc, 0, 0, 0, 127, 0, 127);
+    };
+    auto compute = [&](auto both_tag, int slot) __attribute__((always_inline)) {
+      constexpr bool BOTH = decltype(both_tag)::value;  // rows in both 32-row token blocks
+      const uint8_t* bp = b_rd + slot * STAGE;
+      intx8_t bf[2];
 #pragma unroll
       for (int q = 0; q < (BOTH ? 2 : 1); ++q)
-        acc[ti][q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf[q], acc[ti][q], 0, 0, 0, 127, 0, 127);
-    }
-  };
-
-  // ---- epilogue: scale by the activations' reciprocal scale times the weights' scale ---------------------
-  const float xsc = p.x_scale[0];
-  const float out_rs = p.out_scale ? p.out_scale[0] : 0.0f;
-  // 1 / out_rs once; per element q = v * inv refined by one residual step (fma(-q, rs, v) * inv + q), which is the
-  // correctly rounded quotient except in rare last-bit cases that the following rounding to T absorbs
-  const float out_inv = p.out_scale ? __builtin_amdgcn_rcpf(out_rs) : 0.0f;
-  struct Scales {
-    float s0, s1;
-  };
-  auto scales_of = [&](const F8Unit& un) __attribute__((always_inline)) {
-    return Scales{xsc * reinterpret_cast<const float*>(p.w0.d)[p.w0.d_count > 1 ? un.e : 0],
-                  MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(p.w1.d)[p.w1.d_count > 1 ? un.e : 0] : 0.0f};
-  };
-  // four consecutive features `col`.. of output row `orow_i`: gate and up sums (GATEUP), or the sums `g` (DOWN)
-  auto store_quad = [&](auto act_tag, int64_t orow_i, int64_t col, const float(&g)[4], const float(&u)[4], const Scales& sc) __attribute__((always_inline)) {
-    constexpr int ACT = decltype(act_tag)::value;
-    const int64_t orow = orow_i * p.ldo;
-    if (MODE == MODE_GATEUP) {
-      float gq[4], uq[4];
+        bf[q] = join8(*reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu0), *reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu1));
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        gq[q] = g[q] * sc.s0;
-        uq[q] = u[q] * sc.s1;
+      for (int ti = 0; ti < 4; ++ti) {
+        // 32-row block ti of the wavefront: GATEUP blocks 0, 1 are gate rows, 2, 3 the matching up rows (pieces 8 ..)
+        const int piece_off = MODE == MODE_GATEUP ? (ti < 2 ? 0 : 8) + (ti & 1) * 2 : ti * 2;
+        const uint8_t* ap = a_rd + slot * STAGE + piece_off * 1024;
+        const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
+#pragma unroll
+        for (int q = 0; q < (BOTH ? 2 : 1); ++q)
+          acc[ti][q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf[q], acc[ti][q], 0, 0, 0, 127, 0, 127);
       }
-      if (p.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
-        float t[4];
+    };
+
+    // ---- epilogue: scale by the activations' reciprocal scale times the weights' scale ---------------------
+    const float xsc = p.x_scale[0];
+    const float out_rs = p.out_scale ? p.out_scale[0] : 0.0f;
+    // 1 / out_rs once; per element q = v * inv refined by one residual step (fma(-q, rs, v) * inv + q), which is the
+    // correctly rounded quotient except in rare last-bit cases that the following rounding to T absorbs
+    const float out_inv = p.out_scale ? __builtin_amdgcn_rcpf(out_rs) : 0.0f;
+    struct Scales {
+      float s0, s1;
+    };
+    auto scales_of = [&](const F8Unit& un) __attribute__((always_inline)) {
+      return Scales{xsc * reinterpret_cast<const float*>(p.w0.d)[p.w0.d_count > 1 ? un.e : 0],
+                    MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(p.w1.d)[p.w1.d_count > 1 ? un.e : 0] : 0.0f};
+    };
+    // four consecutive features `col`.. of output row `orow_i`: gate and up sums (GATEUP), or the sums `g` (DOWN)
+    auto store_quad = [&](auto act_tag, int64_t orow_i, int64_t col, const float(&g)[4], const float(&u)[4], const Scales& sc) __attribute__((always_inline)) {
+      constexpr int ACT = decltype(act_tag)::value;
+      const int64_t orow = orow_i * p.ldo;
+      if (MODE == MODE_GATEUP) {
+        float gq[4], uq[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[q])));
-          const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[q])));
-          const float q0 = v * out_inv;
-          const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
-          t[q] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
+          gq[q] = g[q] * sc.s0;
+          uq[q] = u[q] * sc.s1;
         }
-        int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
-        qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
-        const int64_t at = p.out_block_rows ? ((col >> 6) * p.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
-        *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(p.out) + at) = qv;
+        if (p.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
+          float t[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[q])));
+            const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[q])));
+            const float q0 = v * out_inv;
+            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
+            t[q] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
+          }
+          int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
+          qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
+          const int64_t at = p.out_block_rows ? ((col >> 6) * p.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
+          *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(p.out) + at) = qv;
+        } else {
+          *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
+        }
       } else {
-        *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
+        *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) =
+            make_uint2(pack2<T>(g[0] * sc.s0, g[1] * sc.s0), pack2<T>(g[2] * sc.s0, g[3] * sc.s0));
       }
-    } else {
-      *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) =
-          make_uint2(pack2<T>(g[0] * sc.s0, g[1] * sc.s0), pack2<T>(g[2] * sc.s0, g[3] * sc.s0));
-    }
-  };
-  auto epilogue = [&](auto tj_tag, auto act_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
-    constexpr int tj = decltype(tj_tag)::value;
-    const Scales sc = scales_of(un);
-    if (tj * 32 + r32 < my_rows) {
-      const int64_t orow_i = out_row(p, un.row_begin + wm * rpg + tj * 32 + r32);
+    };
+    auto epilogue = [&](auto tj_tag, auto act_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
+      constexpr int tj = decltype(tj_tag)::value;
+      const Scales sc = scales_of(un);
+      if (tj * 32 + r32 < my_rows) {
+        const int64_t orow_i = out_row(p, un.row_begin + wm * rpg + tj * 32 + r32);
 #pragma unroll
-      for (int ti = 0; ti < (MODE == MODE_GATEUP ? 2 : 4); ++ti)
+        for (int ti = 0; ti < (MODE == MODE_GATEUP ? 2 : 4); ++ti)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
-          const int64_t col = (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 2 : BN) + wn * (MODE == MODE_GATEUP ? 64 : 128) + ti * 32 + 8 * b + 4 * h32;
-          const floatx16_t &c = acc[ti][tj], &d = acc[MODE == MODE_GATEUP ? ti + 2 : ti][tj];
-          const float g[4] = {c[4 * b], c[4 * b + 1], c[4 * b + 2], c[4 * b + 3]}, u[4] = {d[4 * b], d[4 * b + 1], d[4 * b + 2], d[4 * b + 3]};
+          for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
+            const int64_t col = (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 2 : BN) + wn * (MODE == MODE_GATEUP ? 64 : 128) + ti * 32 + 8 * b + 4 * h32;
+            const floatx16_t &c = acc[ti][tj], &d = acc[MODE == MODE_GATEUP ? ti + 2 : ti][tj];
+            const float g[4] = {c[4 * b], c[4 * b + 1], c[4 * b + 2], c[4 * b + 3]}, u[4] = {d[4 * b], d[4 * b + 1], d[4 * b + 2], d[4 * b + 3]};
+            store_quad(act_tag, orow_i, col, g, u, sc);
+            __builtin_amdgcn_sched_barrier(0);  // one quad at a time: the accumulators leave no room for more
+          }
+      }
+    };
+    auto tail_epilogue = [&](auto act_tag, const F8Unit& un) __attribute__((always_inline)) {
+      const Scales sc = scales_of(un);
+      if (r32 < un.tail_rows) {
+        const int64_t orow_i = out_row(p, un.tail_begin + r32);
+#pragma unroll
+        for (int b = 0; b < (MODE == MODE_GATEUP ? 2 : 4); ++b) {
+          const int64_t col = MODE == MODE_GATEUP ? (int64_t)un.ntile * (BN / 2) + wn * 64 + wm * 16 + 8 * b + 4 * h32
+                                                  : (int64_t)un.ntile * BN + wn * 128 + wm * 32 + 8 * b + 4 * h32;
+          constexpr int UP = MODE == MODE_GATEUP ? 8 : 0;
+          const float g[4] = {tacc[4 * b], tacc[4 * b + 1], tacc[4 * b + 2], tacc[4 * b + 3]};
+          const float u[4] = {tacc[UP + 4 * b], tacc[UP + 4 * b + 1], tacc[UP + 4 * b + 2], tacc[UP + 4 * b + 3]};
           store_quad(act_tag, orow_i, col, g, u, sc);
-          __builtin_amdgcn_sched_barrier(0);  // one quad at a time: the accumulators leave no room for more
-        }
-    }
-  };
-  auto tail_epilogue = [&](auto act_tag, const F8Unit& un) __attribute__((always_inline)) {
-    const Scales sc = scales_of(un);
-    if (r32 < un.tail_rows) {
-      const int64_t orow_i = out_row(p, un.tail_begin + r32);
-#pragma unroll
-      for (int b = 0; b < (MODE == MODE_GATEUP ? 2 : 4); ++b) {
-        const int64_t col = MODE == MODE_GATEUP ? (int64_t)un.ntile * (BN / 2) + wn * 64 + wm * 16 + 8 * b + 4 * h32
-                                                : (int64_t)un.ntile * BN + wn * 128 + wm * 32 + 8 * b + 4 * h32;
-        constexpr int UP = MODE == MODE_GATEUP ? 8 : 0;
-        const float g[4] = {tacc[4 * b], tacc[4 * b + 1], tacc[4 * b + 2], tacc[4 * b + 3]};
-        const float u[4] = {tacc[UP + 4 * b], tacc[UP + 4 * b + 1], tacc[UP + 4 * b + 2], tacc[UP + 4 * b + 3]};
-        store_quad(act_tag, orow_i, col, g, u, sc);
-      }
-    }
-  };
-  auto epilogues = [&](auto both_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
-    constexpr bool BOTH = decltype(both_tag)::value;
-    if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) {
-      epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
-      if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
-    } else {
-      epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
-      if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
-    }
-  };
-  // Rows per token-row group of 64 LDS rows: the rows of a partial tile are spread over the four groups in multiples of 16.
-  auto rows_per_group = [](int rows_here) { return min(64, ((rows_here + 3) / 4 + 15) / 16 * 16); };
-
-  // ---- the workgroup's units, up to 64 at a time -----------------------------------------------------------
-  // Round r of the walk takes the item of the XCD's list at place (wg + r (wgs / 2 + 1)) mod wgs of that round (see
-  // grouped_mfma_ws_kernel: neighbouring items differ systematically in cost and a workgroup that kept its place in every
-  // round would collect one kind).  Lane r of the table holds round r's unit.
-  for (int round0 = 0;; round0 += 64) {
-    F8Unit mine;
-    const int round = round0 + lane;
-    const int place = (wg + round * ((wgs >> 1) + 1)) % wgs;
-    const bool have = f8_unit_of_lane(lane_off, E, BM, n_tiles, xcd, round * wgs + place, kBalance, TAILS, mine);
-    // (the items of later rounds come later in the list: the lanes that hold a unit are lanes 0 .. n_units - 1)
-    const int n_units = __builtin_popcountll(__ballot(have));
-    if (n_units == 0) return;
-    const int t_en = mine.e | (mine.ntile << 8), t_rb = mine.row_begin, t_re = mine.row_end;
-    const int t_tb = mine.tail_begin, t_tr = mine.tail_rows;
-    auto unit_at = [&](int i) {
-      F8Unit un;
-      const int en = __builtin_amdgcn_readlane(t_en, i);
-      un.e = en & 0xff;
-      un.ntile = en >> 8;
-      un.row_begin = __builtin_amdgcn_readlane(t_rb, i);
-      un.row_end = __builtin_amdgcn_readlane(t_re, i);
-      un.tail_begin = __builtin_amdgcn_readlane(t_tb, i);
-      un.tail_rows = __builtin_amdgcn_readlane(t_tr, i);
-      return un;
-    };
-    const int total = n_units * nst;  // K stages of this batch of units
-
-    // ---- the load side: stage `gl` of the batch = stage `sl` of unit `ul` ------------------------------------
-    const uint8_t* wq[2] = {nullptr, nullptr};
-    uint32_t xoff[2] = {0, 0}, toff = 0;
-    int ul = -1, sl = nst, gl = 0;
-    auto issue_next = [&]() __attribute__((always_inline)) {
-      if (sl == nst) {  // first stage of the next unit: its operand addresses
-        ++ul;
-        sl = 0;
-        const F8Unit un = unit_at(ul);
-        const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int rtl = 2 * wave + j;  // row tile of 16 inside the 256 weight rows of the stage
-          int64_t row0;
-          const WeightView* wv;
-          if (MODE == MODE_GATEUP) {
-            const bool up = rtl >= BN / 32;
-            wv = up ? &p.w1 : &p.w0;
-            row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * (BN / 2) + (rtl % (BN / 32)) * 16;
-          } else {
-            wv = &p.w0;
-            row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * BN + rtl * 16;
-          }
-          const uint64_t addr = reinterpret_cast<uint64_t>(wv->qs + (row0 >> 4) * (p.kred >> 6) * 1024);  // K block 0 of the row tile
-          // wave-uniform by construction; say so to the compiler (the address goes into scalar registers)
-          // (the builtin returns a signed int: go through uint32_t, or the low half sign-extends into the high one)
-          const uint32_t addr_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
-          const uint32_t addr_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
-          wq[j] = reinterpret_cast<const uint8_t*>((uint64_t)addr_lo | ((uint64_t)addr_hi << 32));
-          // token rows: lane l fills LDS row 32 wave + 16 j + l / 4 with the 16 bytes that belong at position l % 4
-          // (x_unit is an involution: position -> logical unit); LDS rows without a tile row re-read a valid one
-          const int lr = 32 * wave + 16 * j + (lane >> 2);
-          const int r = min((lr >> 6) * rpg + min(lr & 63, rpg - 1), rows_here - 1);
-          xoff[j] = (uint32_t)((int64_t)(un.row_begin + r) * (p.a_block_rows ? KS : p.lda) + (x_unit(lr, lane & 3) << 4));
-        }
-        if constexpr (TAILS) {  // (a unit without ride-along rows: its own rows again, never used)
-          const int tr = 4 * wave + ((lane & 15) >> 2);
-          const int i = un.tail_rows > 0 ? un.tail_begin + min(tr, un.tail_rows - 1) : un.row_begin + min(tr, rows_here - 1);
-          toff = (uint32_t)((int64_t)i * (p.a_block_rows ? KS : p.lda) + (x_unit(tr, lane & 3) << 4));
         }
       }
-      const uint32_t slot = (uint32_t)(gl % D) * STAGE;
-      vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[0]), lane16 + (uint32_t)sl * 1024, w_lds + slot);
-      vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[1]), lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
-      vm_load16_to_lds<kBaseFromVector>(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
-      vm_load16_to_lds<kBaseFromVector>(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
-      if constexpr (TAILS) f8_load16_to_lds_16_lanes(p.a, toff + (uint32_t)sl * x_stage_bytes, t_lds + slot);
-      ++sl;
-      ++gl;
     };
-
-    // every wavefront loads its share of every stage and meets every barrier, with or without token rows of its own
-#pragma unroll 1
-    for (int st = 0; st < min(D - 1, total); ++st) issue_next();
-    int slot = 0, g = 0;
-#pragma unroll 1
-    for (int u = 0; u < n_units; ++u) {
-      const F8Unit un = unit_at(u);
-      const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
-      const int my_rows = min(rpg, rows_here - wm * rpg);
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.0f;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) tacc[q] = 0.0f;
-      auto stages = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
-#pragma unroll 1
-        for (int st = 0; st < nst; ++st, ++g) {
-          // the loads of the D - 2 stages after this one may still be in flight when this stage is needed; the batch's
-          // last stages have nothing behind them to issue
-          if (g + D - 1 < total) {
-            vm_wait<(D - 2) * LOADS>();
-            __syncthreads();  // everybody's loads of this stage have landed; everybody is done with the stage before
-            issue_next();     // into the slot of the stage before
-          } else {
-            vm_wait<0>();
-            __syncthreads();
-          }
-          if constexpr (decltype(both_tag)::value >= 0) compute(both_tag, slot);
-          if constexpr (decltype(tail_tag)::value != 0) compute_tail(slot);
-          slot = slot == D - 1 ? 0 : slot + 1;
-        }
-      };
-      if (TAILS && un.tail_rows > 0) {
-        if constexpr (TAILS) {
-          stages(F8Int<1>{}, F8Int<1>{});
-          epilogues(F8Int<1>{}, un, rpg, my_rows);
-          if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) tail_epilogue(EpiAct<STMOE_ACT_SILU>{}, un);
-          else tail_epilogue(EpiAct<STMOE_ACT_GELU_ERF>{}, un);
-        }
-      } else if (my_rows > 32) {
-        stages(F8Int<1>{}, F8Int<0>{});
-        epilogues(F8Int<1>{}, un, rpg, my_rows);
-      } else if (my_rows > 0) {
-        stages(F8Int<0>{}, F8Int<0>{});
-        epilogues(F8Int<0>{}, un, rpg, my_rows);
+    auto epilogues = [&](auto both_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
+      constexpr bool BOTH = decltype(both_tag)::value;
+      if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) {
+        epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
+        if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
       } else {
-        stages(F8Int<-1>{}, F8Int<0>{});
+        epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
+        if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
       }
+    };
+    // Rows per token-row group of 64 LDS rows: the rows of a partial tile are spread over the four groups in multiples of 16.
+    auto rows_per_group = [](int rows_here) { return min(64, ((rows_here + 3) / 4 + 15) / 16 * 16); };
+
+    // ---- the workgroup's units, up to 64 at a time -----------------------------------------------------------
+    // Round r of the walk takes the item of the XCD's list at place (wg + r (wgs / 2 + 1)) mod wgs of that round (see
+    // grouped_mfma_ws_kernel: neighbouring items differ systematically in cost and a workgroup that kept its place in every
+    // round would collect one kind).  Lane r of the table holds round r's unit.
+    for (int round0 = 0;; round0 += 64) {
+      F8Unit mine;
+      const int round = round0 + lane;
+      const int place = (wg + round * ((wgs >> 1) + 1)) % wgs;
+      const bool have = f8_unit_of_lane(lane_off, E, BM, n_tiles, xcd, round * wgs + place, kBalance, TAILS, mine);
+      // (the items of later rounds come later in the list: the lanes that hold a unit are lanes 0 .. n_units - 1)
+      const int n_units = __builtin_popcountll(__ballot(have));
+      if (n_units == 0) return;
+      const int t_en = mine.e | (mine.ntile << 8), t_rb = mine.row_begin, t_re = mine.row_end;
+      const int t_tb = mine.tail_begin, t_tr = mine.tail_rows;
+      auto unit_at = [&](int i) {
+        F8Unit un;
+        const int en = __builtin_amdgcn_readlane(t_en, i);
+        un.e = en & 0xff;
+        un.ntile = en >> 8;
+        un.row_begin = __builtin_amdgcn_readlane(t_rb, i);
+        un.row_end = __builtin_amdgcn_readlane(t_re, i);
+        un.tail_begin = __builtin_amdgcn_readlane(t_tb, i);
+        un.tail_rows = __builtin_amdgcn_readlane(t_tr, i);
+        return un;
+      };
+      const int total = n_units * nst;  // K stages of this batch of units
+
+      // ---- the load side: stage `gl` of the batch = stage `sl` of unit `ul` ------------------------------------
+      const uint8_t* wq[2] = {nullptr, nullptr};
+      uint32_t xoff[2] = {0, 0}, toff = 0;
+      int ul = -1, sl = nst, gl = 0;
+      auto issue_next = [&]() __attribute__((always_inline)) {
+        if (sl == nst) {  // first stage of the next unit: its operand addresses
+          ++ul;
+          sl = 0;
+          const F8Unit un = unit_at(ul);
+          const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int rtl = 2 * wave + j;  // row tile of 16 inside the 256 weight rows of the stage
+            int64_t row0;
+            const WeightView* wv;
+            if (MODE == MODE_GATEUP) {
+              const bool up = rtl >= BN / 32;
+              wv = up ? &p.w1 : &p.w0;
+              row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * (BN / 2) + (rtl % (BN / 32)) * 16;
+            } else {
+              wv = &p.w0;
+              row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * BN + rtl * 16;
+            }
+            const uint64_t addr = reinterpret_cast<uint64_t>(wv->qs + (row0 >> 4) * (p.kred >> 6) * 1024);  // K block 0 of the row tile
+            // wave-uniform by construction; say so to the compiler (the address goes into scalar registers)
+            // (the builtin returns a signed int: go through uint32_t, or the low half sign-extends into the high one)
+            const uint32_t addr_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
+            const uint32_t addr_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
+            wq[j] = reinterpret_cast<const uint8_t*>((uint64_t)addr_lo | ((uint64_t)addr_hi << 32));
+            // token rows: lane l fills LDS row 32 wave + 16 j + l / 4 with the 16 bytes that belong at position l % 4
+            // (x_unit is an involution: position -> logical unit); LDS rows without a tile row re-read a valid one
+            const int lr = 32 * wave + 16 * j + (lane >> 2);
+            const int r = min((lr >> 6) * rpg + min(lr & 63, rpg - 1), rows_here - 1);
+            xoff[j] = (uint32_t)((int64_t)(un.row_begin + r) * (p.a_block_rows ? KS : p.lda) + (x_unit(lr, lane & 3) << 4));
+          }
+          if constexpr (TAILS) {  // (a unit without ride-along rows: its own rows again, never used)
+            const int tr = 4 * wave + ((lane & 15) >> 2);
+            const int i = un.tail_rows > 0 ? un.tail_begin + min(tr, un.tail_rows - 1) : un.row_begin + min(tr, rows_here - 1);
+            toff = (uint32_t)((int64_t)i * (p.a_block_rows ? KS : p.lda) + (x_unit(tr, lane & 3) << 4));
+          }
+        }
+        const uint32_t slot = (uint32_t)(gl % D) * STAGE;
+        vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[0]), lane16 + (uint32_t)sl * 1024, w_lds + slot);
+        vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[1]), lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
+        vm_load16_to_lds<kBaseFromVector>(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
+        vm_load16_to_lds<kBaseFromVector>(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
+        if constexpr (TAILS) f8_load16_to_lds_16_lanes(p.a, toff + (uint32_t)sl * x_stage_bytes, t_lds + slot);
+        ++sl;
+        ++gl;
+      };
+
+      // every wavefront loads its share of every stage and meets every barrier, with or without token rows of its own
+#pragma unroll 1
+      for (int st = 0; st < min(D - 1, total); ++st) issue_next();
+      int slot = 0, g = 0;
+#pragma unroll 1
+      for (int u = 0; u < n_units; ++u) {
+        const F8Unit un = unit_at(u);
+        const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
+        const int my_rows = min(rpg, rows_here - wm * rpg);
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) tacc[q] = 0.0f;
+        auto stages = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
+#pragma unroll 1
+          for (int st = 0; st < nst; ++st, ++g) {
+            // the loads of the D - 2 stages after this one may still be in flight when this stage is needed; the batch's
+            // last stages have nothing behind them to issue
+            if (g + D - 1 < total) {
+              vm_wait<(D - 2) * LOADS>();
+              __syncthreads();  // everybody's loads of this stage have landed; everybody is done with the stage before
+              issue_next();     // into the slot of the stage before
+            } else {
+              vm_wait<0>();
+              __syncthreads();
+            }
+            if constexpr (decltype(both_tag)::value >= 0) compute(both_tag, slot);
+            if constexpr (decltype(tail_tag)::value != 0) compute_tail(slot);
+            slot = slot == D - 1 ? 0 : slot + 1;
+          }
+        };
+        if (TAILS && un.tail_rows > 0) {
+          if constexpr (TAILS) {
+            stages(F8Int<1>{}, F8Int<1>{});
+            epilogues(F8Int<1>{}, un, rpg, my_rows);
+            if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) tail_epilogue(EpiAct<STMOE_ACT_SILU>{}, un);
+            else tail_epilogue(EpiAct<STMOE_ACT_GELU_ERF>{}, un);
+          }
+        } else if (my_rows > 32) {
+          stages(F8Int<1>{}, F8Int<0>{});
+          epilogues(F8Int<1>{}, un, rpg, my_rows);
+        } else if (my_rows > 0) {
+          stages(F8Int<0>{}, F8Int<0>{});
+          epilogues(F8Int<0>{}, un, rpg, my_rows);
+        } else {
+          stages(F8Int<-1>{}, F8Int<0>{});
+        }
+      }
+      // (a further batch, if the workgroup has more than 64 units, starts with empty LDS stages: every load has landed and
+      // the last barrier is passed by all before the next stage 0 is written... after one more barrier)
+      __syncthreads();
     }
-    // (a further batch, if the workgroup has more than 64 units, starts with empty LDS stages: every load has landed and
-    // the last barrier is passed by all before the next stage 0 is written... after one more barrier)
-    __syncthreads();
-  }  };
+  };
   // Ride-along rows save their expert's partial tile and cost the full tiles an MFMA per nine and their loads: a unit that carries them
   // takes 10-15 % longer, every other one of the launch some 4 %.  They are taken along where that saves an eighth of the rounds over the
   // CUs or more (8 experts of 4096 x 14336, 4096 tokens: gate/up 16 rounds to 14, 1107 / 1050 us, down 3 to 2, 617 / 512).  Over 3500

@@ -296,6 +296,16 @@ __device__ __forceinline__ void vm_load_u16_to_reg(uint32_t& dst, const void* ba
 }
 template <typename V> __device__ __forceinline__ void vm_landed(V& v) { asm volatile("" : "+v"(v)::"memory"); }
 
+// Weights that are read once: past the caches' usual replacement.
+__device__ __forceinline__ u32x4_t ld_stream16(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+}
+// fp16 pair -> T pair (identity for fp16; fp16 -> fp32 -> bf16 with round-to-nearest-even for bf16)
+template <typename T> __device__ __forceinline__ uint32_t h2_to_T(uint32_t h2) {
+  if constexpr (__is_same(T, f16_t)) return h2;
+  else return pack2<bf16_t>(f16_bits_to_f32(h2 & 0xffffu), f16_bits_to_f32(h2 >> 16));
+}
+
 // ---- packed weight pieces -----------------------------------------------------------------------------
 // Per K step (64 reduction elements) and row tile (16 rows), lane (n = lane % 16, g = lane / 16) fetches the samples
 // of row n, k = 16*g .. 16*g + 15 and their block scale, and later converts them to 16 values of T (8 dwords) that

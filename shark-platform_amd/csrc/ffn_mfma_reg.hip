@@ -89,22 +89,14 @@ template <> struct RegTile<WF_Q4_1_P> {
   }
 };
 
-__device__ __forceinline__ u32x4_t reg_ld16(const uint8_t* base, uint32_t off) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + off));
-}
-template <typename T> __device__ __forceinline__ uint32_t reg_h2_to_T(uint32_t h2) {
-  if constexpr (__is_same(T, f16_t)) return h2;
-  else return pack2<bf16_t>(f16_bits_to_f32(h2 & 0xffffu), f16_bits_to_f32(h2 >> 16));
-}
-
 // A chunk of a weight tile as lane (n = lane % 16, g = lane / 16) holds it: row n, the elements given at `frag`.
 template <int WF> struct RegData;
 template <> struct RegData<WF_Q8_0_P> {
   u32x4_t q[4], d;
   // the part of chunk c that can be requested during MFMA step s, when the weights of step s + 1 are being converted
   __device__ __forceinline__ void load(const RegTile<WF_Q8_0_P>& t, int c, int lane, int s) {
-    if (s & 1) q[s >> 1] = reg_ld16(t.q + (int64_t)c * 4096 + (s >> 1) * 1024, lane * 16);
-    if (s == 7) d = reg_ld16(t.d + (int64_t)c * 256, (lane & 15) * 16);
+    if (s & 1) q[s >> 1] = ld_stream16(t.q + (int64_t)c * 4096 + (s >> 1) * 1024 + lane * 16);
+    if (s == 7) d = ld_stream16(t.d + (int64_t)c * 256 + (lane & 15) * 16);
   }
   __device__ __forceinline__ void touch() { asm volatile("" : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]), "+v"(d)); }
   // MFMA step s covers elements 64 (s / 2) + 16 g + 8 (s % 2) .. + 7
@@ -118,8 +110,8 @@ template <> struct RegData<WF_Q8_0_P> {
       const uint32_t u = q[i][2 * h + j] ^ 0x80808080u;
       const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
       const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
-      out[2 * j] = reg_h2_to_T<T>(as_u32((as_half2(lo) - bias) * dd));
-      out[2 * j + 1] = reg_h2_to_T<T>(as_u32((as_half2(hi) - bias) * dd));
+      out[2 * j] = h2_to_T<T>(as_u32((as_half2(lo) - bias) * dd));
+      out[2 * j + 1] = h2_to_T<T>(as_u32((as_half2(hi) - bias) * dd));
     }
     return out;
   }
@@ -127,7 +119,7 @@ template <> struct RegData<WF_Q8_0_P> {
 template <> struct RegData<WF_FP8_F32D_P> {
   u32x4_t q[4];
   __device__ __forceinline__ void load(const RegTile<WF_FP8_F32D_P>& t, int c, int lane, int s) {
-    if (s & 1) q[s >> 1] = reg_ld16(t.q + (int64_t)c * 4096 + (s >> 1) * 1024, lane * 16);
+    if (s & 1) q[s >> 1] = ld_stream16(t.q + (int64_t)c * 4096 + (s >> 1) * 1024 + lane * 16);
   }
   __device__ __forceinline__ void touch() { asm volatile("" : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3])); }
   template <typename T> __device__ __forceinline__ u32x4_t frag(const RegTile<WF_FP8_F32D_P>& t, int s, int) const {
@@ -147,10 +139,10 @@ template <> struct RegData<WF_FP8_F32D_P> {
 template <> struct RegData<WF_Q4_1_P> {
   u32x4_t q[2], d, m;
   __device__ __forceinline__ void load(const RegTile<WF_Q4_1_P>& t, int c, int lane, int s) {
-    if ((s & 3) == 3) q[s >> 2] = reg_ld16(t.q + (int64_t)c * 2048 + (s >> 2) * 1024, lane * 16);
+    if ((s & 3) == 3) q[s >> 2] = ld_stream16(t.q + (int64_t)c * 2048 + (s >> 2) * 1024 + lane * 16);
     if (s == 7) {
-      d = reg_ld16(t.d + (int64_t)c * 256, (lane & 15) * 16);
-      m = reg_ld16(t.m + (int64_t)c * 256, (lane & 15) * 16);
+      d = ld_stream16(t.d + (int64_t)c * 256 + (lane & 15) * 16);
+      m = ld_stream16(t.m + (int64_t)c * 256 + (lane & 15) * 16);
     }
   }
   __device__ __forceinline__ void touch() { asm volatile("" : "+v"(q[0]), "+v"(q[1]), "+v"(d), "+v"(m)); }
@@ -170,7 +162,7 @@ template <> struct RegData<WF_Q4_1_P> {
     q4_dword_dequant_packed(q[i][j], sc, h);
     u32x4_t out;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) out[b] = reg_h2_to_T<T>(h[b]);
+    for (int b = 0; b < 4; ++b) out[b] = h2_to_T<T>(h[b]);
     return out;
   }
 };

@@ -34,19 +34,10 @@ template <> __device__ __forceinline__ floatx4_t mfma16s<bf16_t>(const u32x4_t& 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-__device__ __forceinline__ u32x4_t ld_stream16(const void* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
-}
 __device__ __forceinline__ u32x2_t ld_stream8(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p));
 }
 __device__ __forceinline__ u32x4_t ld16(const void* p) { return *reinterpret_cast<const u32x4_t*>(p); }
-
-// fp16 pair -> T pair (identity for fp16; fp16 -> fp32 -> bf16 with round-to-nearest-even for bf16)
-template <typename T> __device__ __forceinline__ uint32_t h2_to_T(uint32_t h2) {
-  if constexpr (__is_same(T, f16_t)) return h2;
-  else return pack2<bf16_t>(f16_bits_to_f32(h2 & 0xffffu), f16_bits_to_f32(h2 >> 16));
-}
 
 // ---- per-format weight chunk: 256 reduction elements of one row, as seen by lane (n = lane%16, g = lane/16) ----
 template <int WF> struct SkinnyW;
