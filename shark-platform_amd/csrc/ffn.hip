@@ -164,8 +164,10 @@ static bool reg_loses(int dtype, int wtag, int mode, const GemmParams& p, int64_
   // 8 experts: Zipf 8 and 5 %, -6 .. 29, uniform nothing, -8 .. 15; with 4 experts there is nothing to win)
   if (streams) return !fast && rows < 4 * E && (E >= 16 ? halves <= 256 : E >= 8 && halves < 224);
   // units for a quarter of the CUs and a long reduction, which the prefill kernel cuts in four where it has scratch (4 experts 9 %,
-  // -12 .. 35, 8 experts from 11264 elements on 6 %, -11 .. 27, below that 3 and, under Zipf, -1 %; with 16 nothing)
-  if (!fast && p.split_scratch && E <= 8 && units <= 64 && p.kred > (E <= 4 ? 8192 : 11264) && rows <= 52 * E) return true;
+  // -12 .. 35, 8 experts from 11264 elements on 6 %, -11 .. 27, below that 3 and, under Zipf, -1 %; with 16 nothing; up to 32 units from
+  // 6144 elements on uniform 7 %, -3 .. 19, Zipf 2 %, -20 .. 23, in bf16 and fp8; the fp16 conversions of the other two are faster)
+  const int64_t most = units <= 32 && (dtype == STMOE_BF16 || wtag == WF_FP8_F32D_P) ? 6144 : E <= 4 ? 8192 : 11264;
+  if (!fast && p.split_scratch && E <= 8 && units <= 64 && p.kred > most && rows <= 52 * E) return true;
   if (E < 32 || units <= 224 || units > 256) return false;
   // one round of whole units that is nearly full, over many experts: some have more than 64 rows and spill into a second round
   // (32 and 64 experts 7 %, -6 .. 14) ...

@@ -673,6 +673,7 @@ def _random_weight(fmt, shape, gen, device):
     ("gate_up", "q4_1", torch.bfloat16, 32, 4, 420, 1024, 1024, "ws"),
     # units for a quarter of the CUs and a long reduction; few rows on many experts
     ("down", "fp8", torch.float16, 4, 2, 67, 8448, 1024, "ws"),
+    ("down", "q8_0", torch.bfloat16, 4, 2, 67, 6400, 1024, "ws"),
     ("down", "q4_1", torch.bfloat16, 16, 2, 16, 3328, 1792, "skinny"),
     # inside the lines
     ("gate_up", "q4_1", torch.bfloat16, 32, 4, 300, 1024, 1024, "reg"),
@@ -681,6 +682,8 @@ def _random_weight(fmt, shape, gen, device):
     ("down", "q4_1", torch.float16, 8, 2, 16, 3072, 4096, "reg"),
     ("down", "q4_1", torch.float16, 16, 2, 16, 3328, 1792, "reg"),
     ("down", "q8_0", torch.float16, 8, 2, 100, 9984, 1024, "reg"),
+    ("down", "q8_0", torch.float16, 4, 2, 67, 6400, 1024, "reg"),
+    ("down", "q8_0", torch.bfloat16, 4, 2, 67, 6400, 2304, "reg"),
 ])
 def test_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k, T, kred, n_out, choice):
     """The automatic choice on both sides of the lines around the register kernel, told by the bits: the kernels add in different orders."""
