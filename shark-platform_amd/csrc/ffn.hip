@@ -105,7 +105,8 @@ static constexpr int64_t kSkinnyMaxRowsSingleSplit = 32;
 // rows 63 / 70; 68 / 65, 512 rows 67 / 78; 71 / 75; [8192, 4096] 513 rows 64 / 66; 68 / 65, 1024 rows 70 / 85; 75 / 82; [14336, 6144] 300
 // rows 91 / 89; 99 / 83, 512 rows 95 / 100; 101 / 96; against whole units, which reductions up to 3072 keep, [16384, 2048] 300 rows 38 / 50;
 // 40 / 43.  With equal token tiles of at most 192 rows they pay earlier ([14336, 4096], 128-row tiles / split: 270 rows Q4_1 bf16 57 / 64, Q8_0
-// fp16 55 / 62, fp8 49 / 60, 384 rows Q8_0 59 / 69, fp8 53 / 67).  fp8 takes Q8_0's constant: [14336, 4096] 300 rows 58 / 66, 512 rows 64 / 77, [14336, 6144] 300 rows 83 / 84.
+// fp16 55 / 62, fp8 49 / 60, 384 rows Q8_0 59 / 69, fp8 53 / 67; over 280 matrices of up to 6144 columns that have such tiles the median
+// gains 1 to 12 % by format and none is slower beyond the noise).  fp8 takes Q8_0's constant: [14336, 4096] 300 rows 58 / 66, 512 rows 64 / 77, [14336, 6144] 300 rows 83 / 84.
 static bool narrow_pays(int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (rows <= 128) return false;
   const int64_t features = (mode == MODE_GATEUP ? 32 : 64) * (narrow_wide(mode, p.n_out, rows) ? 2 : 1);

@@ -45,7 +45,8 @@ struct BigTagOff { static constexpr bool value = false; };
 // TJ: 16-row column blocks of a wavefront.  TJ = 3 is for a single matrix whose token tiles, made equal, have at most 192 rows (129 to 192
 // rows, and 257 to 384, which would be a tile of 256 and a rest): the tile's rows are spread over the four token-row groups in multiples
 // of 16 (tile row grp * rpg + i lives in LDS row grp * 64 + i), so that every wavefront has 3 blocks to multiply instead of some four and
-// some none, and the launch, one round, ends with tiles of 150 rows instead of 256.  [14336, 4096] at 300 rows, us: Q4_1 bf16 64 -> 60, fp8
+// some none, and the launch, one round, ends with tiles of 150 rows instead of 256.  (The token loads are not spread: LDS rows grp * 64 +
+// rpg .. + 63 are filled with copies of the group's last row, a quarter of the token stream at 192 rows, and nobody reads them.)  [14336, 4096] at 300 rows, us: Q4_1 bf16 64 -> 60, fp8
 // 58 -> 51, Q8_0 fp16 72 -> 59; [14336, 2048] Q8_0 39 -> 31; [8192, 4096] Q4_1 41 -> 38.  With both counts of blocks in
 // one kernel the full tiles were up to 10 % slower (Q8_0, 256 rows 41 -> 45).
 template <typename T, int WF, int MODE, int WN, int WM, int STAGES, int TI, int TJ>
