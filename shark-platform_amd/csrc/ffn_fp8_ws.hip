@@ -1,12 +1,17 @@
 // Prefill kernel for fp8 (e4m3fn) activations and packed fp8 tensor-scaled weights on the fp8 matrix cores.
 //
 // Neither operand needs a conversion on its way to the matrix cores, so no byte passes through a register before the
-// MFMA reads it: every wavefront sends its share of the next stage global -> LDS directly (global_load_lds_dwordx4) and
+// MFMA reads it: every wavefront sends its share of a later stage global -> LDS directly (global_load_lds_dwordx4) and
 // then only reads LDS operands and issues MFMAs.
 //
 //   256 x 256 workgroup tile (GATEUP: 128 gate + the same 128 up rows), 8 wavefronts of 128 weight rows x 64 token
 //   rows, K stage 64 (one v_mfma_scale_f32_32x32x64_f8f6f4 deep), four stages of 16 KB weights + 16 KB tokens + 2 KB
 //   ride-along tokens = 136 KB, loads issued three stages ahead (four are no faster), one barrier per stage.
+//   order:   the two wavefronts of a SIMD take the halves of a stage in opposite orders.  Behind the barrier of stage s wavefronts 4-7
+//            multiply stage s - 1, whose operands they have in registers, and then read those of stage s; wavefronts 0-3 first read
+//            stage s and then multiply it.  So one of the two always has MFMAs to issue and the other one's LDS latency and load
+//            issue (about 300 cycles each) pass beside the 512 cycles of MFMAs.  All of a stage's operands are in registers
+//            before its first MFMA.
 //   ride-along rows: an expert with a few rows more than c full tiles would need a partial tile for them, whose units load all
 //            256 rows and leave most matrix cores idle; each full tile takes up to 32 of them along instead (tail_rows).
 //   weights: a packed 1 KB piece (16 rows x 64 k; lane 16 g + n holds row n, k = 16 g .. + 15) lands in LDS as it is;
@@ -16,15 +21,19 @@
 //            (row l / 4 of the load's 16 rows, the unit that x_unit maps to position l % 4), so that the gather and the
 //            bank swizzle cost nothing; rows of a partial token tile are spread over the four token-row groups.
 //   results: D[8 (i / 4) + 4 h + i % 4][r] (probed on the hardware: rows are the weight rows, columns the token rows);
-//            both token blocks' operands (16 registers) stay resident while the four weight blocks stream through 8
-//            registers, so every operand byte is read from LDS once per wavefront.
+//            both token blocks' operands (16 registers) and the four weight blocks' (32) are read once per wavefront and stage.
 //   epilogue: the fp32 dot products of the quantised samples are scaled once by scale_x * d_w; the gate/up epilogue can
 //            quantise the gated intermediate to e4m3fn for the down projection.
-//   What bounds it: at 256 flop per operand byte the tile needs 32 KB per stage from L2 / HBM; with the operand loads
-//   alone (no MFMA) the launch takes two thirds of its full time and with the MFMAs alone 60 %, i.e. the two overlap only
-//   partly.  More bytes in flight change nothing (3 or 4 stages of 32 KB ahead).  The barrier of every stage costs a fifth of the compute
-//   side (MFMAs alone 1.03 ms of a 1.33 ms layer, without barriers 0.82): both wavefronts of a SIMD wait for their first operands behind
-//   it.  Reading those ahead of the barrier changed nothing or cost registers that are not there.
+//   What bounds it: power.  4096 tokens, 8 experts of 4096 x 14336, gate/up + down: both wavefronts of a SIMD in the same order
+//            962 + 464 us (1.96 + 0.95 M cycles at 2.04 GHz, the matrix cores busy half of them); in opposite orders 799 + 388
+//            (1.40 + 0.68 M at 1.75, busy 0.69); 1259 instead of 1470 us for the layer, and over 36 layers of 4 to 16 experts,
+//            1024 to 6144 x 1024 to 16384, 0 to 25 % less, 10 on average.  Without any barrier 16 % fewer cycles at a clock 9 %
+//            lower, without loads 703 + 323 us.  A launch with nothing but the loads takes 590 + 300 us, 13 TB/s of the 34 that
+//            these loads reach from L2 without a barrier per stage: one stage in flight is as fast as two, so not latency.
+//            Tried and slower, because something other than MFMAs comes between a wavefront's MFMAs: the loads between them
+//            (+15 %), a load's operands read as soon as the last MFMA has used the register (+15 %), both wavefronts late
+//            (+15 %); loads issued in front of the LDS reads (+20 %) or while the early wavefronts' reads are under way (+7 %):
+//            both go through the CU's one vector-memory path.
 #include "ffn_mfma_common.h"
 
 namespace stmoe {
@@ -47,6 +56,19 @@ __device__ __forceinline__ void f8_load16_to_lds_16_lanes(const void* base, uint
   asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 exec, 0xffff\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(byte_off), "s"(base), "s"(lds_addr),
                "n"(kBaseFromVector)
                : "memory", "m0");
+}
+
+// A wavefront's share of a stage, four loads of a kilobyte: two weight pieces (w + w0, w + w1) and twice 16 token rows (x + x0, x + x1) to
+// LDS address `lds_addr` and the kilobytes after it.  The n-th load's immediate offset of 1024 n counts for the LDS and for the global address.
+__device__ __forceinline__ void f8_load_share(const void* w, uint32_t w0, uint32_t w1, const void* x, uint32_t x0, uint32_t x1, uint32_t lds_addr) {
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile(
+      "s_mov_b32 m0, %6\n\t"
+      "s_nop %7\n\tglobal_load_lds_dwordx4 %0, %4\n\t"
+      "s_nop %7\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\t"
+      "s_nop %7\n\tglobal_load_lds_dwordx4 %2, %5 offset:2048\n\t"
+      "s_nop %7\n\tglobal_load_lds_dwordx4 %3, %5 offset:3072" ::"v"(w0), "v"(w1), "v"(x0), "v"(x1), "s"(w), "s"(x), "s"(lds_addr), "n"(kBaseFromVector)
+      : "memory", "m0");
 }
 
 struct F8Args {
@@ -135,8 +157,9 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(512, 1)
 grouped_fp8_ws_kernel(F8Args args) {
   constexpr int BN = 256, BM = 256, KS = 64;      // K samples (= bytes per row) per stage
-  constexpr int WSTAGE = BN * KS, XSTAGE = BM * KS;  // bytes
-  constexpr int STAGE = WSTAGE + XSTAGE + kF8TailRows * KS, D = 4;  // stages in LDS
+  // A stage: eight shares of two weight pieces (32 weight rows) and 32 token rows, 2 KB each, then the ride-along rows.
+  constexpr int SHARE = 32 * KS + 32 * KS, XSTAGE = 8 * SHARE;
+  constexpr int STAGE = XSTAGE + kF8TailRows * KS, D = 4;  // stages in LDS
   constexpr int kBalance = 1;
   extern __shared__ __align__(16) uint8_t lds8[];
   const GemmParams& p = args.p;
@@ -146,12 +169,18 @@ grouped_fp8_ws_kernel(F8Args args) {
   const int E = p.offsets ? p.E : 1;
   const int lane_off = p.offsets ? big_lane_offsets(p) : (lane == 1 ? (int)p.fixed_rows : 0);
   const int nst = (int)(p.kred >> 6);
-  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds8);
-  const uint32_t w_lds = lds0 + 2 * wave * 1024, x_lds = lds0 + WSTAGE + 32 * wave * KS;
-  const uint32_t t_lds = lds0 + WSTAGE + XSTAGE + 4 * wave * KS;
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds8));
+  const uint32_t w_lds = lds0 + wave * SHARE, t_lds = lds0 + XSTAGE + 4 * wave * KS;
   const uint32_t lane16 = lane * 16;
   // bytes from one K stage of a token row to the next: 64 in a plain row, a whole block of rows in the blocked layout
+  const uint32_t x_row_bytes = p.a_block_rows ? (uint32_t)KS : (uint32_t)p.lda;
   const uint32_t x_stage_bytes = p.a_block_rows ? (uint32_t)(p.a_block_rows * KS) : (uint32_t)KS;
+
+  // This wavefront's two row tiles of 16 weight rows: neighbours in one matrix (GATEUP: wavefronts 0-3 gate, 4-7 up).
+  const WeightView& w_mine = MODE == MODE_GATEUP && wave >= 4 ? p.w1 : p.w0;
+  const uint32_t tile_bytes = (uint32_t)(p.kred * 16);
+  const int64_t w_expert_tiles = w_mine.rows >> 4;
+  const uint8_t* const w_first = reinterpret_cast<const uint8_t*>(uniform_ptr(w_mine.qs + (int64_t)(2 * wave % (MODE == MODE_GATEUP ? BN / 32 : BN / 16)) * tile_bytes));
 
   // Launches without ride-along rows walk their units with an instance that knows nothing of them: their loads and the branches around
   // them cost 4 % (2048 rows of one expert, gate/up 239 -> 249 us).
@@ -162,129 +191,147 @@ grouped_fp8_ws_kernel(F8Args args) {
 
     // ---- operands: lane (r, h) supplies row r, samples 32 h .. 32 h + 31 ------------------------------------
     const int wn = wave & 1, wm = wave >> 1;
+    const bool late = wave >= 4;
     const int r32 = lane & 31, h32 = lane >> 5;
     // weight row r of a 32-row block: piece r / 16, lane position 16 g + r % 16 for g = 2 h, 2 h + 1
-    const uint8_t* const a_rd = lds8 + (MODE == MODE_GATEUP ? wn * 4 : wn * 8) * 1024 + (r32 >> 4) * 1024 + ((32 * h32 + (r32 & 15)) << 4);
+    const uint8_t* const a_rd = lds8 + (MODE == MODE_GATEUP ? wn * 2 : wn * 4) * SHARE + (r32 >> 4) * 1024 + ((32 * h32 + (r32 & 15)) << 4);
     const int xrow = wm * 64 + r32;
-    const uint8_t* const b_rd = lds8 + WSTAGE + xrow * KS;
+    const uint8_t* const b_rd = lds8 + wm * 2 * SHARE + 2048 + r32 * KS;
     const int bu0 = x_unit(xrow, 2 * h32) << 4, bu1 = x_unit(xrow, 2 * h32 + 1) << 4;  // rows xrow and xrow + 32 swizzle alike
     floatx16_t acc[4][2];
     // Ride-along rows.  The four wavefronts that share a weight half (128 rows) take 32 of its rows each against all of the unit's ride-along
     // rows: one MFMA per stage, GATEUP 16 gate rows and the same 16 up rows, so that both sums of a feature meet in one lane.
     floatx16_t tacc;
-    auto compute_tail = [&](int slot) __attribute__((always_inline)) {
-      const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? ((r32 >> 4) * 7 + wm) * 1024 : wm * 2048);
-      const uint8_t* bp = b_rd + slot * STAGE + (BM - wm * 64) * KS;  // (rows BM + r32: swizzled like xrow)
-      const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
-      const intx8_t bf = join8(*reinterpret_cast<const u32x4_t*>(bp + bu0), *reinterpret_cast<const u32x4_t*>(bp + bu1));
-      tacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf, tacc, 0, 0, 0, 127, 0, 127);
-    };
-    auto compute = [&](auto both_tag, int slot) __attribute__((always_inline)) {
+    // A stage's operands, all of them in registers before its first MFMA.
+    u32x4_t a_op[4][2], b_op[2][2], ta_op[2], tb_op[2];
+    auto read_operands = [&](auto both_tag, auto tail_tag, int slot) __attribute__((always_inline)) {
       constexpr bool BOTH = decltype(both_tag)::value;  // rows in both 32-row token blocks
       const uint8_t* bp = b_rd + slot * STAGE;
-      intx8_t bf[2];
 #pragma unroll
-      for (int q = 0; q < (BOTH ? 2 : 1); ++q)
-        bf[q] = join8(*reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu0), *reinterpret_cast<const u32x4_t*>(bp + q * 32 * KS + bu1));
+      for (int q = 0; q < (BOTH ? 2 : 1); ++q) {
+        b_op[q][0] = *reinterpret_cast<const u32x4_t*>(bp + q * SHARE + bu0);
+        b_op[q][1] = *reinterpret_cast<const u32x4_t*>(bp + q * SHARE + bu1);
+      }
 #pragma unroll
       for (int ti = 0; ti < 4; ++ti) {
         // 32-row block ti of the wavefront: GATEUP blocks 0, 1 are gate rows, 2, 3 the matching up rows (pieces 8 ..)
-        const int piece_off = MODE == MODE_GATEUP ? (ti < 2 ? 0 : 8) + (ti & 1) * 2 : ti * 2;
-        const uint8_t* ap = a_rd + slot * STAGE + piece_off * 1024;
-        const intx8_t af = join8(*reinterpret_cast<const u32x4_t*>(ap), *reinterpret_cast<const u32x4_t*>(ap + 256));
+        const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? (ti < 2 ? 0 : 4) + (ti & 1) : ti) * SHARE;
+        a_op[ti][0] = *reinterpret_cast<const u32x4_t*>(ap);
+        a_op[ti][1] = *reinterpret_cast<const u32x4_t*>(ap + 256);
+      }
+      if constexpr (decltype(tail_tag)::value != 0) {
+        // GATEUP: lanes r < 16 take piece wm of the wavefront's four gate pieces, the others of its up pieces; DOWN: its 32-row block wm
+        const uint8_t* ap = a_rd + slot * STAGE + (MODE == MODE_GATEUP ? (wm >> 1) * SHARE + (wm & 1) * 1024 + (r32 >> 4) * (4 * SHARE - 1024) : wm * SHARE);
+        const uint8_t* tp = lds8 + slot * STAGE + XSTAGE + r32 * KS;  // (swizzled like xrow)
+        ta_op[0] = *reinterpret_cast<const u32x4_t*>(ap);
+        ta_op[1] = *reinterpret_cast<const u32x4_t*>(ap + 256);
+        tb_op[0] = *reinterpret_cast<const u32x4_t*>(tp + bu0);
+        tb_op[1] = *reinterpret_cast<const u32x4_t*>(tp + bu1);
+      }
+    };
+    auto multiply = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
+      constexpr bool BOTH = decltype(both_tag)::value;
+#pragma unroll
+      for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
         for (int q = 0; q < (BOTH ? 2 : 1); ++q)
-          acc[ti][q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af, bf[q], acc[ti][q], 0, 0, 0, 127, 0, 127);
-      }
+          acc[ti][q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join8(a_op[ti][0], a_op[ti][1]), join8(b_op[q][0], b_op[q][1]), acc[ti][q], 0, 0, 0, 127, 0, 127);
+      if constexpr (decltype(tail_tag)::value != 0)
+        tacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join8(ta_op[0], ta_op[1]), join8(tb_op[0], tb_op[1]), tacc, 0, 0, 0, 127, 0, 127);
+      // (issued here, not behind the barrier that follows)
+#pragma unroll
+      for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+        for (int q = 0; q < (BOTH ? 2 : 1); ++q) asm volatile("" : "+v"(acc[ti][q]));
+      if constexpr (decltype(tail_tag)::value != 0) asm volatile("" : "+v"(tacc));
     };
 
     // ---- epilogue: scale by the activations' reciprocal scale times the weights' scale ---------------------
-    const float xsc = p.x_scale[0];
-    const float out_rs = p.out_scale ? p.out_scale[0] : 0.0f;
-    // 1 / out_rs once; per element q = v * inv refined by one residual step (fma(-q, rs, v) * inv + q), which is the
-    // correctly rounded quotient except in rare last-bit cases that the following rounding to T absorbs
-    const float out_inv = p.out_scale ? __builtin_amdgcn_rcpf(out_rs) : 0.0f;
-    struct Scales {
-      float s0, s1;
-    };
-    auto scales_of = [&](const F8Unit& un) __attribute__((always_inline)) {
-      return Scales{xsc * reinterpret_cast<const float*>(p.w0.d)[p.w0.d_count > 1 ? un.e : 0],
-                    MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(p.w1.d)[p.w1.d_count > 1 ? un.e : 0] : 0.0f};
-    };
-    // four consecutive features `col`.. of output row `orow_i`: gate and up sums (GATEUP), or the sums `g` (DOWN)
-    auto store_quad = [&](auto act_tag, int64_t orow_i, int64_t col, const float(&g)[4], const float(&u)[4], const Scales& sc) __attribute__((always_inline)) {
-      constexpr int ACT = decltype(act_tag)::value;
-      const int64_t orow = orow_i * p.ldo;
-      if (MODE == MODE_GATEUP) {
-        float gq[4], uq[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          gq[q] = g[q] * sc.s0;
-          uq[q] = u[q] * sc.s1;
-        }
-        if (p.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
-          float t[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[q])));
-            const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[q])));
-            const float q0 = v * out_inv;
-            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
-            t[q] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
-          }
-          int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
-          qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
-          const int64_t at = p.out_block_rows ? ((col >> 6) * p.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
-          *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(p.out) + at) = qv;
-        } else {
-          *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
-        }
-      } else {
-        *reinterpret_cast<uint2*>(reinterpret_cast<T*>(p.out) + orow + col) =
-            make_uint2(pack2<T>(g[0] * sc.s0, g[1] * sc.s0), pack2<T>(g[2] * sc.s0, g[3] * sc.s0));
-      }
-    };
-    auto epilogue = [&](auto tj_tag, auto act_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
-      constexpr int tj = decltype(tj_tag)::value;
-      const Scales sc = scales_of(un);
-      if (tj * 32 + r32 < my_rows) {
-        const int64_t orow_i = out_row(p, un.row_begin + wm * rpg + tj * 32 + r32);
-#pragma unroll
-        for (int ti = 0; ti < (MODE == MODE_GATEUP ? 2 : 4); ++ti)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
-            const int64_t col = (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 2 : BN) + wn * (MODE == MODE_GATEUP ? 64 : 128) + ti * 32 + 8 * b + 4 * h32;
-            const floatx16_t &c = acc[ti][tj], &d = acc[MODE == MODE_GATEUP ? ti + 2 : ti][tj];
-            const float g[4] = {c[4 * b], c[4 * b + 1], c[4 * b + 2], c[4 * b + 3]}, u[4] = {d[4 * b], d[4 * b + 1], d[4 * b + 2], d[4 * b + 3]};
-            store_quad(act_tag, orow_i, col, g, u, sc);
-            __builtin_amdgcn_sched_barrier(0);  // one quad at a time: the accumulators leave no room for more
-          }
-      }
-    };
-    auto tail_epilogue = [&](auto act_tag, const F8Unit& un) __attribute__((always_inline)) {
-      const Scales sc = scales_of(un);
-      if (r32 < un.tail_rows) {
-        const int64_t orow_i = out_row(p, un.tail_begin + r32);
-#pragma unroll
-        for (int b = 0; b < (MODE == MODE_GATEUP ? 2 : 4); ++b) {
-          const int64_t col = MODE == MODE_GATEUP ? (int64_t)un.ntile * (BN / 2) + wn * 64 + wm * 16 + 8 * b + 4 * h32
-                                                  : (int64_t)un.ntile * BN + wn * 128 + wm * 32 + 8 * b + 4 * h32;
-          constexpr int UP = MODE == MODE_GATEUP ? 8 : 0;
-          const float g[4] = {tacc[4 * b], tacc[4 * b + 1], tacc[4 * b + 2], tacc[4 * b + 3]};
-          const float u[4] = {tacc[UP + 4 * b], tacc[UP + 4 * b + 1], tacc[UP + 4 * b + 2], tacc[UP + 4 * b + 3]};
-          store_quad(act_tag, orow_i, col, g, u, sc);
-        }
-      }
-    };
-    auto epilogues = [&](auto both_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
+    // What it needs, the kernel's arguments and the lane's place, is derived here from values that the compiler cannot see through:
+    // in front of the K loops it would hold registers that they don't have to spare.
+    auto epilogues = [&](auto both_tag, auto tail_tag, const F8Unit& un, int rpg, int my_rows) __attribute__((always_inline)) {
       constexpr bool BOTH = decltype(both_tag)::value;
-      if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) {
-        epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
-        if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_SILU>{}, un, rpg, my_rows);
-      } else {
-        epilogue(F8Int<0>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
-        if constexpr (BOTH) epilogue(F8Int<1>{}, EpiAct<STMOE_ACT_GELU_ERF>{}, un, rpg, my_rows);
-      }
+      auto kernarg = __builtin_amdgcn_kernarg_segment_ptr();
+      asm volatile("" : "+s"(kernarg));
+      const GemmParams& q = reinterpret_cast<const F8Args*>((const void*)kernarg)->p;
+      const int l = lane_again(), r32 = l & 31, h32 = l >> 5;
+      const float xsc = q.x_scale[0];
+      const float out_rs = q.out_scale ? q.out_scale[0] : 0.0f;
+      // 1 / out_rs once; per element v * inv refined by one residual step (fma(-q0, rs, v) * inv + q0), which is the
+      // correctly rounded quotient except in rare last-bit cases that the following rounding to T absorbs
+      const float out_inv = q.out_scale ? __builtin_amdgcn_rcpf(out_rs) : 0.0f;
+      const float s0 = xsc * reinterpret_cast<const float*>(q.w0.d)[q.w0.d_count > 1 ? un.e : 0];
+      const float s1 = MODE == MODE_GATEUP ? xsc * reinterpret_cast<const float*>(q.w1.d)[q.w1.d_count > 1 ? un.e : 0] : 0.0f;
+      // four consecutive features `col`.. of output row `orow_i`: gate and up sums (GATEUP), or the sums `g` (DOWN)
+      auto store_quad = [&](auto act_tag, int64_t orow_i, int64_t col, const float(&g)[4], const float(&u)[4]) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_tag)::value;
+        const int64_t orow = orow_i * q.ldo;
+        if (MODE == MODE_GATEUP) {
+          float gq[4], uq[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            gq[i] = g[i] * s0;
+            uq[i] = u[i] * s1;
+          }
+          if (q.out_scale) {  // e4m3fn(clamp(T(v / rscale))) for the next fp8 projection
+            float t[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float a = round_to<T>(act_fast<ACT>(round_to<T>(gq[i])));
+              const float v = round_to<T>(__fmul_rn(a, round_to<T>(uq[i])));
+              const float q0 = v * out_inv;
+              const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, out_rs, v), out_inv, q0);
+              t[i] = fminf(fmaxf(round_to<T>(q1), -448.0f), 448.0f);
+            }
+            int qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], 0, false);  // hardware OCP e4m3fn, round to nearest even
+            qv = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], qv, true);
+            const int64_t at = q.out_block_rows ? ((col >> 6) * q.out_block_rows + orow_i) * KS + (col & 63) : orow + col;
+            *reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(q.out) + at) = qv;
+          } else {
+            *reinterpret_cast<uint2*>(reinterpret_cast<T*>(q.out) + orow + col) = gateup_quad<T, ACT>(gq, uq);
+          }
+        } else {
+          *reinterpret_cast<uint2*>(reinterpret_cast<T*>(q.out) + orow + col) =
+              make_uint2(pack2<T>(g[0] * s0, g[1] * s0), pack2<T>(g[2] * s0, g[3] * s0));
+        }
+      };
+      auto block = [&](auto tj_tag, auto act_tag) __attribute__((always_inline)) {
+        constexpr int tj = decltype(tj_tag)::value;
+        if (tj * 32 + r32 < my_rows) {
+          const int64_t orow_i = out_row(q, un.row_begin + wm * rpg + tj * 32 + r32);
+#pragma unroll
+          for (int ti = 0; ti < (MODE == MODE_GATEUP ? 2 : 4); ++ti)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {  // four consecutive features per 8-row band of the 32 x 32 result
+              const int64_t col = (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 2 : BN) + wn * (MODE == MODE_GATEUP ? 64 : 128) + ti * 32 + 8 * b + 4 * h32;
+              const floatx16_t &c = acc[ti][tj], &d = acc[MODE == MODE_GATEUP ? ti + 2 : ti][tj];
+              const float g[4] = {c[4 * b], c[4 * b + 1], c[4 * b + 2], c[4 * b + 3]}, u[4] = {d[4 * b], d[4 * b + 1], d[4 * b + 2], d[4 * b + 3]};
+              store_quad(act_tag, orow_i, col, g, u);
+              __builtin_amdgcn_sched_barrier(0);  // one quad at a time: the accumulators leave no room for more
+            }
+        }
+      };
+      auto tail = [&](auto act_tag) __attribute__((always_inline)) {
+        if (r32 < un.tail_rows) {
+          const int64_t orow_i = out_row(q, un.tail_begin + r32);
+#pragma unroll
+          for (int b = 0; b < (MODE == MODE_GATEUP ? 2 : 4); ++b) {
+            const int64_t col = MODE == MODE_GATEUP ? (int64_t)un.ntile * (BN / 2) + wn * 64 + wm * 16 + 8 * b + 4 * h32
+                                                    : (int64_t)un.ntile * BN + wn * 128 + wm * 32 + 8 * b + 4 * h32;
+            constexpr int UP = MODE == MODE_GATEUP ? 8 : 0;
+            const float g[4] = {tacc[4 * b], tacc[4 * b + 1], tacc[4 * b + 2], tacc[4 * b + 3]};
+            const float u[4] = {tacc[UP + 4 * b], tacc[UP + 4 * b + 1], tacc[UP + 4 * b + 2], tacc[UP + 4 * b + 3]};
+            store_quad(act_tag, orow_i, col, g, u);
+          }
+        }
+      };
+      auto all = [&](auto act_tag) __attribute__((always_inline)) {
+        block(F8Int<0>{}, act_tag);
+        if constexpr (BOTH) block(F8Int<1>{}, act_tag);
+        if constexpr (decltype(tail_tag)::value != 0) tail(act_tag);
+      };
+      if (MODE == MODE_DOWN || q.act == STMOE_ACT_SILU) all(EpiAct<STMOE_ACT_SILU>{});
+      else all(EpiAct<STMOE_ACT_GELU_ERF>{});
     };
     // Rows per token-row group of 64 LDS rows: the rows of a partial tile are spread over the four groups in multiples of 16.
     auto rows_per_group = [](int rows_here) { return min(64, ((rows_here + 3) / 4 + 15) / 16 * 16); };
@@ -301,76 +348,70 @@ grouped_fp8_ws_kernel(F8Args args) {
       // (the items of later rounds come later in the list: the lanes that hold a unit are lanes 0 .. n_units - 1)
       const int n_units = __builtin_popcountll(__ballot(have));
       if (n_units == 0) return;
-      const int t_en = mine.e | (mine.ntile << 8), t_rb = mine.row_begin, t_re = mine.row_end;
-      const int t_tb = mine.tail_begin, t_tr = mine.tail_rows;
+      // (the table lies behind the stages; every wavefront writes the same values and reads back its own)
+      int* const table = reinterpret_cast<int*>(lds8 + D * STAGE);
+      *reinterpret_cast<int4*>(table + lane * 8) = make_int4(mine.e | (mine.ntile << 8), mine.row_begin, mine.row_end, mine.tail_begin);
+      table[lane * 8 + 4] = mine.tail_rows;
       auto unit_at = [&](int i) {
         F8Unit un;
-        const int en = __builtin_amdgcn_readlane(t_en, i);
+        const int4 t = *reinterpret_cast<const int4*>(table + i * 8);
+        const int en = __builtin_amdgcn_readfirstlane(t.x);
         un.e = en & 0xff;
         un.ntile = en >> 8;
-        un.row_begin = __builtin_amdgcn_readlane(t_rb, i);
-        un.row_end = __builtin_amdgcn_readlane(t_re, i);
-        un.tail_begin = __builtin_amdgcn_readlane(t_tb, i);
-        un.tail_rows = __builtin_amdgcn_readlane(t_tr, i);
+        un.row_begin = __builtin_amdgcn_readfirstlane(t.y);
+        un.row_end = __builtin_amdgcn_readfirstlane(t.z);
+        un.tail_begin = __builtin_amdgcn_readfirstlane(t.w);
+        un.tail_rows = __builtin_amdgcn_readfirstlane(table[i * 8 + 4]);
         return un;
       };
-      const int total = n_units * nst;  // K stages of this batch of units
 
       // ---- the load side: stage `gl` of the batch = stage `sl` of unit `ul` ------------------------------------
-      const uint8_t* wq[2] = {nullptr, nullptr};
-      uint32_t xoff[2] = {0, 0}, toff = 0;
-      int ul = -1, sl = nst, gl = 0;
-      auto issue_next = [&]() __attribute__((always_inline)) {
-        if (sl == nst) {  // first stage of the next unit: its operand addresses
-          ++ul;
-          sl = 0;
-          const F8Unit un = unit_at(ul);
-          const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int rtl = 2 * wave + j;  // row tile of 16 inside the 256 weight rows of the stage
-            int64_t row0;
-            const WeightView* wv;
-            if (MODE == MODE_GATEUP) {
-              const bool up = rtl >= BN / 32;
-              wv = up ? &p.w1 : &p.w0;
-              row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * (BN / 2) + (rtl % (BN / 32)) * 16;
-            } else {
-              wv = &p.w0;
-              row0 = (int64_t)un.e * wv->rows + (int64_t)un.ntile * BN + rtl * 16;
-            }
-            const uint64_t addr = reinterpret_cast<uint64_t>(wv->qs + (row0 >> 4) * (p.kred >> 6) * 1024);  // K block 0 of the row tile
-            // wave-uniform by construction; say so to the compiler (the address goes into scalar registers)
-            // (the builtin returns a signed int: go through uint32_t, or the low half sign-extends into the high one)
-            const uint32_t addr_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
-            const uint32_t addr_hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
-            wq[j] = reinterpret_cast<const uint8_t*>((uint64_t)addr_lo | ((uint64_t)addr_hi << 32));
-            // token rows: lane l fills LDS row 32 wave + 16 j + l / 4 with the 16 bytes that belong at position l % 4
-            // (x_unit is an involution: position -> logical unit); LDS rows without a tile row re-read a valid one
-            const int lr = 32 * wave + 16 * j + (lane >> 2);
-            const int r = min((lr >> 6) * rpg + min(lr & 63, rpg - 1), rows_here - 1);
-            xoff[j] = (uint32_t)((int64_t)(un.row_begin + r) * (p.a_block_rows ? KS : p.lda) + (x_unit(lr, lane & 3) << 4));
-          }
-          if constexpr (TAILS) {  // (a unit without ride-along rows: its own rows again, never used)
-            const int tr = 4 * wave + ((lane & 15) >> 2);
-            const int i = un.tail_rows > 0 ? un.tail_begin + min(tr, un.tail_rows - 1) : un.row_begin + min(tr, rows_here - 1);
-            toff = (uint32_t)((int64_t)i * (p.a_block_rows ? KS : p.lda) + (x_unit(tr, lane & 3) << 4));
-          }
+      // One M0 value serves the share's four loads: an instruction's immediate offset counts for both addresses, which the global
+      // ones below make up for.
+      const uint8_t *wq = nullptr, *xq = nullptr;  // at the stage that is loaded next
+      uint32_t xoff[2] = {0, 0}, toff = 0, load_slot = 0;
+      int ul = -1, left = 0;  // unit, stages of it still to load
+      auto next_unit = [&]() __attribute__((always_inline)) {
+        if (ul + 1 == n_units) {  // past the batch's last stage: that one again, into slots that nobody reads
+          left = 1;
+          wq -= 1024;
+          xq -= x_stage_bytes;
+          return;
         }
-        const uint32_t slot = (uint32_t)(gl % D) * STAGE;
-        vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[0]), lane16 + (uint32_t)sl * 1024, w_lds + slot);
-        vm_load16_to_lds<kBaseFromVector>(uniform_ptr(wq[1]), lane16 + (uint32_t)sl * 1024, w_lds + slot + 1024);
-        vm_load16_to_lds<kBaseFromVector>(p.a, xoff[0] + (uint32_t)sl * x_stage_bytes, x_lds + slot);
-        vm_load16_to_lds<kBaseFromVector>(p.a, xoff[1] + (uint32_t)sl * x_stage_bytes, x_lds + slot + 16 * KS);
-        if constexpr (TAILS) f8_load16_to_lds_16_lanes(p.a, toff + (uint32_t)sl * x_stage_bytes, t_lds + slot);
-        ++sl;
-        ++gl;
+        ++ul;
+        left = nst;
+        const F8Unit un = unit_at(ul);
+        const int rows_here = un.row_end - un.row_begin, rpg = rows_per_group(rows_here);
+        wq = w_first + ((int64_t)un.e * w_expert_tiles + (int64_t)un.ntile * (MODE == MODE_GATEUP ? BN / 32 : BN / 16)) * tile_bytes;
+        xq = reinterpret_cast<const uint8_t*>(p.a) + (int64_t)un.row_begin * x_row_bytes - 3072;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          // token rows: lane l fills LDS row 32 wave + 16 j + l / 4 with the 16 bytes that belong at position l % 4
+          // (x_unit is an involution: position -> logical unit); LDS rows without a tile row re-read a valid one
+          const int lr = 32 * wave + 16 * j + (lane >> 2);
+          const int r = min((lr >> 6) * rpg + min(lr & 63, rpg - 1), rows_here - 1);
+          xoff[j] = (uint32_t)r * x_row_bytes + (x_unit(lr, lane & 3) << 4) + (j == 0 ? 1024 : 0);
+        }
+        if constexpr (TAILS) {  // (a unit without ride-along rows: its own rows again, never used)
+          const int tr = 4 * wave + ((lane & 15) >> 2);
+          const int i = un.tail_rows > 0 ? un.tail_begin - un.row_begin + min(tr, un.tail_rows - 1) : min(tr, rows_here - 1);
+          toff = (uint32_t)i * x_row_bytes + (x_unit(tr, lane & 3) << 4);
+        }
+      };
+      auto issue_next = [&]() __attribute__((always_inline)) {
+        if (left == 0) next_unit();
+        f8_load_share(wq, lane16, lane16 + tile_bytes - 1024, xq, xoff[0], xoff[1], w_lds + load_slot);
+        if constexpr (TAILS) f8_load16_to_lds_16_lanes(xq + 3072, toff, t_lds + load_slot);
+        wq += 1024;
+        xq += x_stage_bytes;
+        --left;
+        load_slot = load_slot == (D - 1) * STAGE ? 0 : load_slot + STAGE;
       };
 
       // every wavefront loads its share of every stage and meets every barrier, with or without token rows of its own
 #pragma unroll 1
-      for (int st = 0; st < min(D - 1, total); ++st) issue_next();
-      int slot = 0, g = 0;
+      for (int st = 0; st < D - 1; ++st) issue_next();
+      int slot = 0;
 #pragma unroll 1
       for (int u = 0; u < n_units; ++u) {
         const F8Unit un = unit_at(u);
@@ -384,52 +425,71 @@ grouped_fp8_ws_kernel(F8Args args) {
             for (int q = 0; q < 16; ++q) acc[a][b][q] = 0.0f;
 #pragma unroll
         for (int q = 0; q < 16; ++q) tacc[q] = 0.0f;
-        auto stages = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
+        // Interval st: everybody's share of stage st has landed, everybody has read the stage before, whose slot is filled again.
+        auto meet = [&]() __attribute__((always_inline)) {
+          vm_wait<(D - 2) * LOADS>();  // the loads of the D - 2 stages after this one may still be in flight
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto stages_early = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
 #pragma unroll 1
-          for (int st = 0; st < nst; ++st, ++g) {
-            // the loads of the D - 2 stages after this one may still be in flight when this stage is needed; the batch's
-            // last stages have nothing behind them to issue
-            if (g + D - 1 < total) {
-              vm_wait<(D - 2) * LOADS>();
-              __syncthreads();  // everybody's loads of this stage have landed; everybody is done with the stage before
-              issue_next();     // into the slot of the stage before
-            } else {
-              vm_wait<0>();
-              __syncthreads();
-            }
-            if constexpr (decltype(both_tag)::value >= 0) compute(both_tag, slot);
-            if constexpr (decltype(tail_tag)::value != 0) compute_tail(slot);
+          for (int st = 0; st < nst; ++st) {
+            meet();
+            if constexpr (decltype(both_tag)::value >= 0) read_operands(both_tag, tail_tag, slot);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            issue_next();
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(both_tag)::value >= 0) multiply(both_tag, tail_tag);
             slot = slot == D - 1 ? 0 : slot + 1;
           }
+        };
+        auto stages_late = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
+          meet();
+          issue_next();
+          if constexpr (decltype(both_tag)::value >= 0) read_operands(both_tag, tail_tag, slot);
+          slot = slot == D - 1 ? 0 : slot + 1;
+#pragma unroll 1
+          for (int st = 1; st < nst; ++st) {
+            meet();
+            if constexpr (decltype(both_tag)::value >= 0) multiply(both_tag, tail_tag);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (decltype(both_tag)::value >= 0) read_operands(both_tag, tail_tag, slot);
+            __builtin_amdgcn_sched_barrier(0);
+            issue_next();
+            slot = slot == D - 1 ? 0 : slot + 1;
+          }
+          if constexpr (decltype(both_tag)::value >= 0) multiply(both_tag, tail_tag);
+        };
+        auto stages = [&](auto both_tag, auto tail_tag) __attribute__((always_inline)) {
+          if (late) stages_late(both_tag, tail_tag);
+          else stages_early(both_tag, tail_tag);
         };
         if (TAILS && un.tail_rows > 0) {
           if constexpr (TAILS) {
             stages(F8Int<1>{}, F8Int<1>{});
-            epilogues(F8Int<1>{}, un, rpg, my_rows);
-            if (MODE == MODE_DOWN || p.act == STMOE_ACT_SILU) tail_epilogue(EpiAct<STMOE_ACT_SILU>{}, un);
-            else tail_epilogue(EpiAct<STMOE_ACT_GELU_ERF>{}, un);
+            epilogues(F8Int<1>{}, F8Int<1>{}, un, rpg, my_rows);
           }
         } else if (my_rows > 32) {
           stages(F8Int<1>{}, F8Int<0>{});
-          epilogues(F8Int<1>{}, un, rpg, my_rows);
+          epilogues(F8Int<1>{}, F8Int<0>{}, un, rpg, my_rows);
         } else if (my_rows > 0) {
           stages(F8Int<0>{}, F8Int<0>{});
-          epilogues(F8Int<0>{}, un, rpg, my_rows);
+          epilogues(F8Int<0>{}, F8Int<0>{}, un, rpg, my_rows);
         } else {
           stages(F8Int<-1>{}, F8Int<0>{});
         }
       }
-      // (a further batch, if the workgroup has more than 64 units, starts with empty LDS stages: every load has landed and
-      // the last barrier is passed by all before the next stage 0 is written... after one more barrier)
+      // (a further batch, if the workgroup has more than 64 units, starts with empty LDS stages: the loads past this one's end have
+      // landed and the last stage has been read by everybody)
+      vm_wait<0>();
       __syncthreads();
     }
   };
   // Ride-along rows save their expert's partial tile and cost the full tiles an MFMA per nine and their loads: a unit that carries them
   // takes 10-15 % longer, every other one of the launch some 4 %.  They are taken along where that saves an eighth of the rounds over the
-  // CUs or more (8 experts of 4096 x 14336, 4096 tokens: gate/up 16 rounds to 14, 1107 / 1050 us, down 3 to 2, 617 / 512).  Over 3500
-  // launches of 4 to 16 experts, 1024 to 6144 x 1024 to 16384, what they save of the whole layer (median, worst): gate/up one round of 2
-  // 15, 7 %; of 4 4, -4 %; of 6 2, -2 %; of 8 2, -3 %; of 9 0, -3 %; of 14 and more -2, -6 %; two of 16 1, -1 %; down one of 2 10, -4 %; of
-  // 3 5, 0 %; of 4 to 6 2 to 4, 1 %.
+  // CUs or more.  44 layers of 4 to 16 experts with 1 to 40 rows more than whole tiles, 1024 to 6144 x 1024 to 16384: 5 % less time than
+  // without them (-1 to 14 %), and the same within 0.1 % as where any round saved decides (single layers 3 % less to 1 % more).
   const int lane_end = __builtin_amdgcn_ds_bpermute(4 * (lane + 1), lane_off);
   const int lane_rows = lane < E ? lane_end - lane_off : 0;
   auto rounds = [&](bool absorb) {
@@ -445,7 +505,7 @@ grouped_fp8_ws_kernel(F8Args args) {
 template <typename T, int MODE>
 static int launch_fp8_ws_m(const GemmParams& p, int64_t max_rows, hipStream_t st) {
   constexpr int BN = 256, BM = 256;
-  constexpr size_t lds_bytes = (size_t)4 * (BN + BM + kF8TailRows) * 64;
+  constexpr size_t lds_bytes = (size_t)4 * (BN + BM + kF8TailRows) * 64 + 64 * 32;  // four stages and the unit table
   static std::atomic<uint64_t> lds_ready{0};
   auto kern = grouped_fp8_ws_kernel<T, MODE>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_ready, "fp8 ws kernel")) return rc;

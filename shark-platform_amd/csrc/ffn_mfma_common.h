@@ -296,6 +296,13 @@ __device__ __forceinline__ void vm_load_u16_to_reg(uint32_t& dst, const void* ba
 }
 template <typename V> __device__ __forceinline__ void vm_landed(V& v) { asm volatile("" : "+v"(v)::"memory"); }
 
+// The number of the lane within its wavefront, computed where it is asked for.
+__device__ __forceinline__ int lane_again() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+  return l;
+}
+
 // Weights that are read once: past the caches' usual replacement.
 __device__ __forceinline__ u32x4_t ld_stream16(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));

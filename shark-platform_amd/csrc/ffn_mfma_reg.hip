@@ -166,12 +166,6 @@ template <> struct RegData<WF_Q4_1_P> {
     return out;
   }
 };
-// The number of the lane within its wavefront, computed where it is asked for.
-__device__ __forceinline__ int lane_again() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
-  return l;
-}
 // 16-byte unit of a token row that lane group g needs for MFMA step s (rows of 256 elements = 32 units)
 template <int WF> __device__ __forceinline__ int reg_x_unit(int s, int g) {
   return IsQ4<WF>::value ? 16 * (s >> 2) + 4 * g + (s & 3) : 8 * (s >> 1) + 2 * g + (s & 1);
