@@ -53,6 +53,7 @@ static int check_weight(const stmoe_weight* w, const char* who, int64_t E, int64
 //         11 256-row tiles of unquantized 16-bit weights, both operands straight into LDS
 //         12 units of 256 weight rows x 64 token rows, weights converted in the registers of the wavefronts that multiply
 //            them (some dozen rows per expert, single matrices of a few hundred rows; packed formats)
+//         13 the same with up to 96 token rows
 // Automatic choice with fp8 weights and static quantizers on both activations: a prefill-sized launch with fp16
 // activations goes to the fp8 matrix cores (variant 5: both operands as bytes, the fp32 dot product scaled once; 1.8 times
 // faster than dequantise-then-multiply, and 6e-3 from it on the layer output at the Mixtral shape, inside the 2e-2 the fp8
@@ -74,7 +75,7 @@ static int effective_variant(int variant, int dtype, int64_t rows, int64_t K, in
 // in all (such launches get no scratch for split reductions, without which the prefill kernel leaves most CUs idle), or
 // when experts get 16 rows or fewer on average (28 with at most 4 experts); everything else goes to the
 // specialised-wavefront prefill kernel.  (On both sides of that line packed formats go to the register kernel where it pays,
-// reg_pays; 16-bit weights to a kernel of their own, dense_pays.)  Measured on the Mixtral layer (top-2, Q8_0 fp16, whole layer, us; streaming /
+// reg_rows; 16-bit weights to a kernel of their own, dense_pays.)  Measured on the Mixtral layer (top-2, Q8_0 fp16, whole layer, us; streaming /
 // prefill kernel with split scratch): 8 experts at 64 / 80 / 96 / 128 / 160 tokens 297 / 340 / 360 / 436 / 559 against
 // 307 / 310 / 315 / 321 / 331 (Q4_1 bf16: 285 / 330 / 358 / 434 / 565 against 332 / 334 / 335 / 339 / 346); 4 experts at
 // 48 / 56 / 64 / 80 tokens 168 / 172 / 235 / 295 against 183 / 184 / 186 / 190; 2 experts at 40 / 64 tokens 171 / 185
@@ -177,20 +178,36 @@ static bool reg_loses(int dtype, int wtag, int mode, const GemmParams& p, int64_
   // 3 and 5 %, -9 .. 27)
   return wtag != WF_Q4_1_P && mode == MODE_GATEUP && p.kred <= 2560;
 }
-static bool reg_pays_grouped(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
+// Token rows of a unit: 64, or up to 96 in the wide kernel (`wide`), or 0 where other kernels are faster.  Units with 65 to 96 rows save the
+// second conversion of an expert's weights, which is what the time goes into (us, kernel chosen without them / with them, gate/up and down,
+// 8 experts of 4096 x 14336): Q4_1 bf16 52 rows per expert 212 / 207 and 106 / 106, 60 rows 259 / 218 and 137 / 110, 76 rows 283 / 239 and
+// 146 / 125, 92 rows 302 / 302 and 158 / 179; Q8_0 fp16 60 rows 239 / 212 and 130 / 107, 76 rows 272 / 236 and 143 / 122; Q4_1 fp16 60 rows
+// 242 / 188 and 123 / 95, 76 rows 260 / 213 and 137 / 111; 64 experts of 2048 x 1536 60 rows Q4_1 bf16 123 / 96 and 62 / 56, Q8_0 fp16
+// 110 / 101 and 56 / 60 (short reductions of the formats that convert fast gain nothing).  Above 80 rows on average some expert has more
+// than 96.  Two tiles of an expert pay again where they fit one round and tiles of 64 do not (8 of [4096, 14336] down 144 rows Q8_0 fp16
+// 204 / 170, Q4_1 bf16 204 / 200; gate/up of 8 x 1024 x 2048 at 144 rows 1.5 to 1.7).  Where tiles of 64 are at most 128 units, which run as
+// halves, they stay.  Over 118 layers of 4 to 64 experts, 1024 to 6144 x 1024 to 16384, those that they change take 8 % less time under a
+// uniform routing (-1 to 27 %) and 5 % under a Zipf routing (-8 to 29 %: there it depends on which experts have a few rows more than tiles).
+static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   const int64_t E = p.E, units = p.n_out / (mode == MODE_GATEUP ? 128 : 256) * E;  // units: with one token tile per expert
   const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||
                        rows <= skinny_max_avg_rows(p.E) * E;
   const int64_t halves = 2 * (units / E) * std::min<int64_t>(E, rows);
-  if (reg_loses(dtype, wtag, mode, p, units, halves, rows, streams)) return false;
-  if (streams) return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * E) || (halves >= 128 && rows > 16 * E));
-  if (p.kred < 1024) return false;
+  if (reg_loses(dtype, wtag, mode, p, units, halves, rows, streams)) return 0;
+  if (streams) return mode == MODE_DOWN && p.kred >= 3072 && ((halves >= 192 && rows >= 2 * E) || (halves >= 128 && rows > 16 * E)) ? kRegUnitRows : 0;
+  if (p.kred < 1024) return 0;
+  // (an expert's rows vary: by a seventh for a uniform routing of this many)
+  const int64_t most = (rows * 8 / 7 + E - 1) / E, narrow = (most + kRegUnitRows - 1) / kRegUnitRows * units,
+                tiles = (most + kRegWideRows - 1) / kRegWideRows, wide = tiles * units;
+  // (129 to 175 whole units leave too many CUs without one: two tiles of 4 experts of 4864 x 7168 at 135 rows, Q4_1 bf16, layer 195 / 207 us)
+  if (narrow > 128 && (wide <= 128 || wide >= 176) && (wtag == WF_Q4_1_P || p.kred >= 2048) &&
+      ((rows > 52 * E && rows <= (p.kred < 2048 ? 72 : 80) * E) || (tiles == 2 && rows >= 120 * E && wide <= 256) || (tiles > 1 && wide <= 128)))
+    return kRegWideRows;
   // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 37
   // rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
-  if (wtag != WF_Q4_1_P && p.kred <= 2048 && units > 256 && rows > 24 * E) return false;
-  if (rows <= 52 * E) return true;
-  // (an expert's rows vary: by a seventh for a uniform routing of this many)
-  return p.kred <= 8192 && (rows * 8 / 7 / E + kRegUnitRows - 1) / kRegUnitRows * units <= 256;
+  if (wtag != WF_Q4_1_P && p.kred <= 2048 && units > 256 && rows > 24 * E) return 0;
+  if (rows <= 52 * E) return kRegUnitRows;
+  return p.kred <= 8192 && narrow <= 256 ? kRegUnitRows : 0;
 }
 // A single matrix: its half units run at the pace of their reduction, whatever their number, where the prefill kernel cuts the reduction
 // in four and the narrow tiles re-read the token rows ([out, in], other kernels / this one, Q8_0 fp16; Q4_1 bf16): [14336, 4096] 33 rows
@@ -201,14 +218,27 @@ static bool reg_pays_grouped(int dtype, int wtag, int mode, const GemmParams& p,
 // (13 / 10 at 300 rows).  Over 1100 products of 33 to 2048 rows, 1024 to 6144 x 1024 to 16384, Q8_0 and Q4_1 in both types, none that comes
 // here is slower; median gain 27 to 56 % by format, at more than 1024 rows (narrow matrices) as at 64.  The gate/up pair of a dense
 // network follows the same line (3600 networks, all formats: none slower by more than 4 %, 2200 faster).
-static bool reg_pays(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
-  if (!reg_takes(dtype, wtag, mode, p, rows)) return false;
-  if (p.E > 1) return p.offsets && reg_pays_grouped(dtype, wtag, mode, p, rows);
+// Where tiles of 64 rows are more than 128 units (which run as halves), tiles of up to 96 rows take over: while they are at most 128 units
+// ([out, in], other kernels / these, Q4_1 bf16; Q8_0 fp16; fp8 bf16: [14336, 4096] 160 rows 38 / 33; 36 / 30; 34 / 29, [8192, 8192] 300 rows
+// 80 / 63; 79 / 58; 78 / 57, 384 rows 84 / 70; 83 / 69; 80 / 66, [4096, 4096] 768 rows 40 / 38; 41 / 37; 38 / 34), and then, as many of them as fit one
+// round, while they have more than 64 rows ([14336, 4096] 300 rows in four tiles of 75 61 / 54; 61 / 48; 51 / 45, 384 rows 61 / 60; 62 / 56;
+// 54 / 52, [6144, 3072] 768 rows 51 / 44; 58 / 40; 56 / 38, [16384, 2048] 300 rows 34 / 33; 36 / 31; 32 / 30; with tiles of 50 to 64 rows the narrow tiles
+// are as fast or faster).  Not for longer reductions, which the prefill kernel cuts ([4096, 14336] 768 rows 114 / 123; 107 / 113; 106 / 107).
+static int reg_rows(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
+  if (!reg_takes(dtype, wtag, mode, p, rows)) return 0;
+  if (p.E > 1) return p.offsets ? reg_rows_grouped(dtype, wtag, mode, p, rows) : 0;
   const int64_t tiles = p.n_out / (mode == MODE_GATEUP ? 128 : 256);  // units per token tile
-  const int64_t units = (rows + kRegUnitRows - 1) / kRegUnitRows * tiles;
-  if (rows <= kSkinnyMaxRowsSingleSplit || p.kred < 1024 || units > 128) return false;
-  if (rows <= 64) return p.kred <= 2048 || (p.kred <= 4096 && tiles >= 32);
-  return rows > 128 ? p.kred > 2048 : p.kred <= 4096;
+  if (rows <= kSkinnyMaxRowsSingleSplit || p.kred < 1024) return 0;
+  if ((rows + kRegUnitRows - 1) / kRegUnitRows * tiles <= 128) {
+    if (rows <= 64) return p.kred <= 2048 || (p.kred <= 4096 && tiles >= 32) ? kRegUnitRows : 0;
+    return (rows > 128 ? p.kred > 2048 : p.kred <= 4096) ? kRegUnitRows : 0;
+  }
+  if (rows <= 64 || (rows > 128 ? p.kred <= 2048 || p.kred > 8192 : p.kred > 4096)) return 0;
+  const int64_t wide = (rows + kRegWideRows - 1) / kRegWideRows;
+  if (wide * tiles <= 128) return (int)((rows + wide - 1) / wide);
+  if (wide * tiles > 256) return 0;
+  const int64_t spread = (rows + 256 / tiles - 1) / (256 / tiles);
+  return spread > kRegUnitRows ? (int)spread : 0;
 }
 // fp8 activations x fp8 weights on the fp8 matrix cores: the 256 x 256 kernel for packed weights and launches with
 // enough rows to fill its tiles (variant 5), the 128 x 128 kernel otherwise (and always with variant 7).
@@ -230,11 +260,12 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     const int rc = launch_skinny(dtype, wtag, mode, p, max_rows, st);
     return rc != STMOE_ERR_UNSUPPORTED ? rc : set_error(STMOE_ERR_UNSUPPORTED, "grouped_ffn: no streaming kernel for a launch that builds its own dispatch");
   }
+  int tile_rows = 0;  // of the register kernel
   if (variant == 0) {
     if (dtype == STMOE_F32) variant = 10;
     // (one matrix, with or without an offsets array around its rows)
     else if (dense_pays(dtype, wtag, mode, p, max_rows)) variant = 11;
-    else if (reg_pays(dtype, wtag, mode, p, max_rows)) variant = 12;
+    else if ((tile_rows = reg_rows(dtype, wtag, mode, p, max_rows)) > 0) variant = 12;
     else if (p.E == 1) variant = max_rows <= (p.split_scratch ? kSkinnyMaxRowsSingleSplit : kSkinnyMaxRowsSingle) ? 3
                                  : narrow_pays(wtag, mode, p, max_rows) ? 9 : 6;
     else if (p.offsets && ((p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) ||
@@ -257,8 +288,9 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     if (rc != STMOE_ERR_UNSUPPORTED) return rc;
     variant = 6;
   }
-  if (variant == 12) {
-    int rc = launch_mfma_reg(dtype, wtag, mode, p, max_rows, st);
+  if (variant == 12 || variant == 13) {
+    if (tile_rows == 0) tile_rows = variant == 13 ? kRegWideRows : kRegUnitRows;
+    int rc = launch_mfma_reg(dtype, wtag, mode, p, max_rows, tile_rows, st);
     if (rc != STMOE_ERR_UNSUPPORTED) return rc;
     variant = 6;
   }

@@ -176,9 +176,10 @@ static inline bool narrow_wide(int mode, int64_t n_out, int64_t rows) {
   return n_out % (2 * features) == 0 && n_out / features * ((rows + 255) / 256) > 256;
 }
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
-static constexpr int kRegUnitRows = 64;  // token rows of a unit of launch_mfma_reg
+static constexpr int kRegUnitRows = 64, kRegWideRows = 96;  // most token rows of a unit of launch_mfma_reg, and of its wide kernel
 bool reg_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows);
-int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
+int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, int tile_rows, hipStream_t st);
+int launch_reg_wide(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, hipStream_t st);
 int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, float* partial, hipStream_t st);
 size_t mfma_ws_partial_bytes();
 size_t mfma_ws_tickets_offset();  // byte offset of the split units' ticket words inside that scratch

@@ -31,6 +31,7 @@ VARIANT_STEP_BY_STEP = 8  # automatic choice among the kernels that round where 
 VARIANT_MFMA_F32 = 10  # fp32 activations on the fp32 matrix cores (chosen automatically)
 VARIANT_DENSE = 11  # 16-bit weights of the activations' type, both operands straight into LDS (chosen automatically where it pays)
 VARIANT_MFMA_REG = 12  # weights converted in the registers of the wavefronts that multiply them (chosen automatically where it pays)
+VARIANT_MFMA_REG_WIDE = 13  # the same with units of up to 96 instead of 64 token rows (chosen automatically where they pay)
 VARIANT_MFMA_NARROW = 9  # 64 x 256 tiles: a single matrix with a few hundred rows (chosen automatically where it pays)
 
 _DTYPE_ENUM = {

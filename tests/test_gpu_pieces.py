@@ -646,6 +646,78 @@ def test_register_kernel_single_matrix_and_scattered_rows(device, fmt, dtype):
         assert worst_row(lambda v: hip.grouped_mmt(a, stacked[0], offsets, perm, T, k, a_per_pair=per_pair, variant=v)) < ulp
 
 
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,act", [(256, 256, "silu"), (2304, 1280, "gelu"), (3072, 768, "silu"), (1024, 1024, "silu")])
+def test_wide_register_kernel(device, fmt, dtype, N, K, act):
+    """The register kernel with units of up to 96 rows, forced: experts on both sides of 64, 80 and 96 rows, of two tiles, and without rows;
+    reductions of 1 to 12 chunks (its two register sets and three LDS stages with every remainder); launches of half units only, of whole
+    ones and of both.  Against the oracle, the worst row as well, and bit for bit against units of 64 rows, which add in the same order."""
+    hip = _hip()
+    from sharktank_amd.ops import device_weight
+
+    rows = [0, 1, 64, 65, 80, 81, 96, 97, 193]
+    E, T = len(rows), sum(rows)
+    tol = 1e-3 if dtype == torch.float16 else 8e-3
+    case = MC.build(MC.Case(T=T, K=K, N=N, E=E, k=1, fmt=fmt, dtype=dtype, act=act, seed=72))
+    order = torch.randperm(T, generator=torch.Generator().manual_seed(73))
+    idx = torch.tensor([e for e, n in enumerate(rows) for _ in range(n)])[order].reshape(T, 1)
+    want = O.grouped_ffn_moe(case.planes["h"], idx, torch.ones(T, 1, dtype=dtype), *MC.dense_weights(case), case.activation)
+    dws = [device_weight(MC.to_inference_tensor(fmt, case.planes[n], shp, n, device), stacked=True, prepack=True)
+           for n, shp in (("gate", [E, N, K]), ("up", [E, N, K]), ("down", [E, K, N]))]
+    _, offsets, perm, inv = hip.dispatch_build(idx.to(torch.int32).to(device), E)
+    act_id = hip.ACT_SILU if act == "silu" else hip.ACT_GELU_ERF
+    wide, narrow = (hip.combine(hip.grouped_ffn(case.planes["h"].to(device), *dws, act_id, offsets, perm, 1, variant=v),
+                                torch.ones(T, 1, dtype=dtype, device=device), inv, T, 1).cpu()
+                    for v in (hip.VARIANT_MFMA_REG_WIDE, hip.VARIANT_MFMA_REG))
+    assert O.rel_l2(wide, want) < tol
+    diff, size = wide.double() - want.double(), want.double().norm(dim=1)
+    assert float((diff.norm(dim=1) / size).max()) < 4 * tol
+    assert torch.equal(wide.view(torch.int16), narrow.view(torch.int16))
+
+
+@pytest.mark.parametrize("mode,fmt,dtype,E,k,T,kred,n_out,choice", [
+    ("gate_up", "q4_1", torch.bfloat16, 8, 2, 260, 1024, 4096, "reg"),   # 65 rows per expert, one round of whole units
+    ("gate_up", "q4_1", torch.bfloat16, 8, 2, 330, 1024, 4096, "ws"),    # 82: some expert has more than 96
+    ("gate_up", "q8_0", torch.float16, 8, 2, 260, 1536, 4096, "ws"),     # a short reduction of a format that converts fast
+    ("down", "q8_0", torch.float16, 8, 2, 560, 3072, 3072, "reg"),       # 140: two tiles, 192 whole units
+    ("down", "q8_0", torch.float16, 8, 2, 560, 9216, 2304, "ws"),        # 144 whole units leave CUs idle
+    ("down", "fp8", torch.bfloat16, 8, 2, 560, 3072, 2048, "reg"),       # 128 units, run as halves
+])
+def test_wide_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k, T, kred, n_out, choice):
+    """The automatic choice on both sides of the lines around units of up to 96 rows, told by the bits."""
+    hip = _hip()
+    gen = torch.Generator(device=device).manual_seed(93)
+    idx = torch.stack([torch.arange(k) + t for t in range(T)]).remainder(E).to(torch.int32).to(device)
+    _, offsets, perm, _ = hip.dispatch_build(idx, E)
+    w = _random_weight(fmt, [E, n_out, kred], gen, device)
+    a = torch.randn(T if mode == "gate_up" else T * k, kred, generator=gen, device=device).to(dtype)
+
+    def run(variant):
+        if mode == "gate_up":
+            return hip.grouped_gate_up(a, w, w, hip.ACT_SILU, offsets, perm, k, variant=variant).view(torch.int16)
+        return hip.grouped_down(a, w, offsets, T, k, variant=variant).view(torch.int16)
+
+    outs = {"reg": run(hip.VARIANT_MFMA_REG_WIDE), "ws": run(hip.VARIANT_MFMA_WS)}
+    auto = run(hip.VARIANT_AUTO)
+    assert not torch.equal(outs["reg"], outs["ws"]) and torch.equal(auto, outs[choice])
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,N,tiles", [(160, 2304, 14336, 2), (300, 2304, 14336, 4), (340, 2304, 14336, 4), (384, 2304, 14336, 4)])
+def test_register_kernel_spreads_the_rows_of_a_single_matrix(device, fmt, dtype, rows, K, N, tiles):
+    """A single matrix whose tiles of 64 rows do not fit: as few tiles of up to 96 as run as halves (112 units), or as many as fit one round
+    (224 units, 75 to 96 rows each).  The automatic choice, bit for bit against units of 64 rows, which add in the same order, and
+    not the other kernels' bits."""
+    hip = _hip()
+    gen = torch.Generator(device=device).manual_seed(94)
+    w = _random_weight(fmt, [1, N, K], gen, device)
+    a = torch.randn(rows, K, generator=gen, device=device).to(dtype)
+    auto, reg, ws = (hip.mmt(a, w, variant=v).view(torch.int16) for v in (hip.VARIANT_AUTO, hip.VARIANT_MFMA_REG, hip.VARIANT_MFMA_WS))
+    assert torch.equal(auto, reg) and not torch.equal(auto, ws)
+
+
 def _random_weight(fmt, shape, gen, device):
     """A packed weight of random planes, made on the device (no reference for it: for launches that are compared with each other)."""
     from sharktank_amd import types as ST
