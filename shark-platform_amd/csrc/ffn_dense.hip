@@ -5,72 +5,110 @@
 // at the rate of a large copy), beyond that the matrix pipe.  Nothing has to be converted, so there are no loader wavefronts:
 // all eight issue their share of the direct loads of a later K step and multiply the current one.
 //
-//   LDS: three weight stages (32 KB each with BN = 256), so that a stage has two K steps to arrive (64 KB in flight per CU cover
-//     the memory latency), and three token stages of 128 or 256 rows; 256 weight rows and 256 token rows leave room for two of
-//     them, whose rows come from L2 and have one K step.  (BN = 128 with two token stages of 256 rows: down projection of 515
-//     tokens 259 us, with three 197.)  Rows of 128 bytes, XOR-swizzled in 16-byte
-//     units (see ffn_mfma_common.h): the direct load puts lane l's 16 bytes at its base + 16 l, so the lanes fetch the units
-//     of a row in swizzled order.
-//   wavefronts: 4 x 2 (64 x 64 of BN = 256) up to 128 rows, 2 x 4 (128 x 64) above; the rows of a unit are spread evenly over
-//     the token groups in multiples of 16 and only the column blocks that hold rows are multiplied.
+//   LDS: as many stages of either operand as 160 KB hold, four at most (three are the least that give a load two K steps to arrive;
+//     64 KB in flight per CU cover the memory latency; over 41 layers eight at most are 0.7 % slower than four: short reductions start
+//     later).  256 weight rows and 256 token rows leave room for three and two.  Rows of 128 bytes, XOR-swizzled in 16-byte units
+//     (see ffn_mfma_common.h): the direct load puts lane l's 16 bytes at its base + 16 l, so the lanes fetch the units of a row in
+//     swizzled order.
+//   units: LDS and loads for 32, 128, 192 or 256 token rows.  With 192 a token row has two steps to arrive, as the weights have, and a
+//     quarter of the loads from L2 goes: gate/up of 515 tokens (129 rows per expert) 416 us with 256 only, 398 so.
+//   last round: units left over after the last whole round over an XCD's CUs are cut into two of 128 weight rows if the halves fit one
+//     round (515 tokens, down: 16 units on 32 CUs, 203 us; 32 halves 194).
+//   wavefronts: 4 x 2 (64 x 64 of BN = 256) up to 128 rows, 2 x 4 (128 x 48 or 64) above; the rows of a unit are spread evenly
+//     over the token groups in multiples of 16 and only the column blocks that hold rows are multiplied.
 //   The reduction runs in the order of the 128 x 128 kernel: the sums are the same bits.
 // Measured (8 experts of 4096 x 14336, top-2, bf16; gate/up + down, us; 128 x 128 kernel / this one): 100 tokens 421 + 279 /
-// 329 + 195, 515 tokens 640 + 313 / 376 + 212 (5 TB/s of weights), 2048 tokens 1916 + 823 / 1025 + 537 (0.92 PFLOP/s; SiLU
+// 329 + 195, 515 tokens 640 + 313 / 398 + 194 (4.8 TB/s of weights), 2048 tokens 1916 + 823 / 1025 + 537 (0.92 PFLOP/s; SiLU
 // by expf and a division, as the 128 x 128 kernel computes it, is 20 us of the 1025: on the hardware exp2 and reciprocal 1002).
+// Slower at 515 tokens, gate/up: weights and tokens sent by different wavefronts 442, both loads behind the first half's products 465,
+// after the step's products 488.
 #include "ffn_mfma_common.h"
 
 namespace stmoe {
 
 template <int V> struct DenseInt { static constexpr int value = V; };
 
-template <typename T, int MODE, int BN>
+// Stages in LDS of a unit of `bn` weight rows and `lds_rows` token rows.  A CU's loads return in the order of their issue, token rows that
+// hit in L2 behind the weights in front of them: one operand further ahead than the other is of no use, so both get as many stages as fit,
+// except that three weight stages are worth two token stages.
+struct DenseStages {
+  int w, x;
+};
+static constexpr int kDenseLds = 160 * 1024;
+static constexpr DenseStages dense_stages(int bn, int lds_rows) {
+  const int both = kDenseLds / ((bn + lds_rows) * 128);
+  return both >= 3 ? DenseStages{both < 4 ? both : 4, both < 4 ? both : 4} : DenseStages{3, 2};
+}
+
+template <typename T, int MODE, int BN_LAUNCH>
 __global__ void __launch_bounds__(512, 1)
 grouped_dense_kernel(GemmParams p, int n_tiles) {
   constexpr int BM = 256;
-  constexpr int WSTAGE = BN * BIG_LS;  // elements
   extern __shared__ __align__(16) uint16_t lds[];
-  BigTile tile;
-  if (!big_tile_id(p, BM, n_tiles, false, tile, false, 2)) return;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, n_in = lane & 15;
+  // The XCD's units; those after the last whole round over its CUs are cut into two of half the weight rows if the halves fit one round.
+  BigTile tile;
+  int half = -1;
+  {
+    const int xcd = blockIdx.x & 7;
+    int item = blockIdx.x >> 3;
+    const BigLanes lanes = big_lanes(p, big_lane_offsets(p), lane, BM, false, 2);
+    const BigPlan plan = big_plan(lanes, n_tiles, xcd, false);
+    if constexpr (BN_LAUNCH == 256) {
+      const int units = plan.whole, rest = units % kBigCusPerXcd, whole = 2 * rest <= kBigCusPerXcd ? units - rest : units;
+      if (item >= whole) {
+        half = (item - whole) & 1;
+        item = whole + (item - whole) / 2;
+        if (item >= units) return;
+      }
+    }
+    if (!big_unit(lanes, BM, n_tiles, plan, item, tile, false)) return;
+  }
   const int row_begin = tile.row_begin, rows_here = tile.row_end - tile.row_begin;
   const int nkt = (int)(p.kred >> 6), last = nkt - 1;
 
-  auto unit = [&](auto groups_tag) {
-    constexpr int GROUPS = decltype(groups_tag)::value;  // token-row groups of 64 LDS rows
-    constexpr int WN = 8 / GROUPS, TI = BN / 16 / WN;    // wavefronts along the features, 16-feature blocks of each
-    constexpr int XSTAGE = GROUPS * 64 * BIG_LS;
-    constexpr bool XEARLY = GROUPS == 2 || BN == 128;    // token rows two K steps ahead (three stages), else one (two stages)
-    constexpr int XSTAGES = XEARLY ? 3 : 2;
-    constexpr int WLOADS = BN / 64, XLOADS = GROUPS;     // direct loads of 8 rows per wavefront and K step
-    const int rpg = min(64, ((rows_here + GROUPS - 1) / GROUPS + 15) / 16 * 16);  // tile row grp * rpg + i <-> LDS row grp * 64 + i
-    uint16_t* const Wbase = lds;               // [3][BN][64]
-    uint16_t* const Xbase = lds + 3 * WSTAGE;  // [XSTAGES][64 GROUPS][64]
+  auto unit = [&](auto bn_tag, auto groups_tag, auto blocks_tag) {
+    constexpr int BN = decltype(bn_tag)::value, WSTAGE = BN * BIG_LS;
+    constexpr int GROUPS = decltype(groups_tag)::value;           // token-row groups
+    constexpr int BLOCKS = decltype(blocks_tag)::value;           // 16-row column blocks of a group
+    constexpr int RPG = 16 * BLOCKS, XROWS = GROUPS * RPG;        // LDS rows of a group, of a token stage
+    constexpr int WN = 8 / GROUPS, TI = BN / 16 / WN;             // wavefronts along the features, 16-feature blocks of each
+    constexpr int XSTAGE = XROWS * BIG_LS;
+    constexpr DenseStages ST = dense_stages(BN, XROWS);
+    constexpr int WA = ST.w - 1, XA = ST.x - 1;                   // K steps ahead
+    constexpr int WLOADS = BN / 64, XLOADS = (XROWS + 63) / 64;   // direct loads of 8 rows per wavefront and K step
+    static_assert((ST.w * BN + ST.x * XROWS) * 128 <= kDenseLds && WA >= 2 && (XA == WA || XA == 1) && WA * (WLOADS + XLOADS) <= 63, "stages and waits");
+    const int ntile = BN == BN_LAUNCH ? tile.ntile : 2 * tile.ntile + half;
+    const int rpg = min(RPG, ((rows_here + GROUPS - 1) / GROUPS + 15) / 16 * 16);  // tile row grp * rpg + i <-> LDS row grp * RPG + i
+    uint16_t* const Wbase = lds;                  // [ST.w][BN][64]
+    uint16_t* const Xbase = lds + ST.w * WSTAGE;  // [ST.x][XROWS][64]
 
     // ---- loads: this wavefront's rows are 64 j + 8 wave .. + 7 of either operand's tile
+    const int unit_off = ((lane & 7) ^ (lane >> 3)) << 4;  // LDS unit lane % 8 of row lane / 8 holds this unit of the row
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)lds);
+    const uint32_t w_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 8 * BIG_LS * 2);
+    const uint32_t x_lds = __builtin_amdgcn_readfirstlane(lds0 + (ST.w * WSTAGE + (XROWS < 64 ? wave & 3 : wave) * 8 * BIG_LS) * 2);
     const char* wsrc[WLOADS];
 #pragma unroll
     for (int j = 0; j < WLOADS; ++j) {
       const int r = 64 * j;  // (a block of 64 rows is all gate or all up)
       const bool up = MODE == MODE_GATEUP && r >= BN / 2;
       const WeightView& wv = up ? p.w1 : p.w0;
-      const int64_t row = (int64_t)tile.e * wv.rows + (MODE == MODE_GATEUP ? (int64_t)tile.ntile * (BN / 2) + (up ? r - BN / 2 : r)
-                                                                           : (int64_t)tile.ntile * BN + r) + wave * 8;
+      const int64_t row = (int64_t)tile.e * wv.rows + (MODE == MODE_GATEUP ? (int64_t)ntile * (BN / 2) + (up ? r - BN / 2 : r)
+                                                                           : (int64_t)ntile * BN + r) + wave * 8;
       wsrc[j] = reinterpret_cast<const char*>(wv.qs) + row * p.kred * 2;
     }
-    const int unit_off = ((lane & 7) ^ (lane >> 3)) << 4;  // LDS unit lane % 8 of row lane / 8 holds this unit of the row
     const uint32_t woff = (uint32_t)((lane >> 3) * (int)p.kred * 2 + unit_off);
     uint32_t xoff[XLOADS];
 #pragma unroll
     for (int j = 0; j < XLOADS; ++j) {
-      // LDS rows that hold no tile row re-read a valid one (their outputs are never stored)
-      const int i = row_begin + min(j * rpg + min(wave * 8 + (lane >> 3), rpg - 1), rows_here - 1);
+      // LDS rows that hold no tile row re-read a valid one (their outputs are never stored); of 32 rows wavefronts 4-7 send the same again
+      const int lr = (64 * j + 8 * wave + (lane >> 3)) % XROWS, grp = lr / RPG, in = lr - grp * RPG;
+      const int i = row_begin + min(grp * rpg + min(in, rpg - 1), rows_here - 1);
       const int64_t src = p.perm ? (int64_t)(p.perm[i] / p.k_top) : (int64_t)i;
       xoff[j] = (uint32_t)(src * p.lda * 2 + unit_off);
     }
-    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint16_t*)lds);
-    const uint32_t w_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 8 * BIG_LS * 2);
-    const uint32_t x_lds = __builtin_amdgcn_readfirstlane(lds0 + (3 * WSTAGE + wave * 8 * BIG_LS) * 2);
     // Requests past the last step read the last step again (into a stage that nobody reads), so that the number of loads in
     // flight is the same at every wait.
     auto load_w = [&](int kt, int stage) {
@@ -83,7 +121,11 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
 #pragma unroll
       for (int j = 0; j < XLOADS; ++j) vm_load16_to_lds(src, xoff[j], x_lds + (uint32_t)((stage * XSTAGE + 64 * j * BIG_LS) * 2));
     };
-
+    // Order of the loads, and what the waits (at most N of a wavefront's loads still in flight, the N youngest) leave:
+    //   as many stages of both: W0 X0 .. | step kt: W, X(kt + WA); behind its wait W, X(kt + 1) have landed: N = (WA - 1) (WLOADS + XLOADS)
+    //   else:                   W0 X0 W1 | step kt: X(kt + 1) W(kt + 2); behind its wait W, X(kt + 1) have landed: N = WLOADS
+    constexpr bool XEARLY = XA == WA;
+    constexpr int INFLIGHT = XEARLY ? (WA - 1) * (WLOADS + XLOADS) : WLOADS;
     // ---- operands
     const int wn = wave % WN, wm = wave / WN;
     const int my_rows = min(rpg, rows_here - wm * rpg);  // rows of this wavefront's group (<= 0: none)
@@ -94,14 +136,14 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
     for (int ks = 0; ks < 2; ++ks) {
       const int u = ((ks * 4 + g) ^ (n_in & 7)) << 3;
       a_rd[ks] = Wbase + ((MODE == MODE_GATEUP ? wn * (BN / 2 / WN) : wn * (BN / WN)) + n_in) * BIG_LS + u;
-      b_rd[ks] = Xbase + (wm * 64 + n_in) * BIG_LS + u;
+      b_rd[ks] = Xbase + (wm * RPG + n_in) * BIG_LS + u;
     }
     auto block_row = [](int ti) { return MODE == MODE_GATEUP ? (ti < TI / 2 ? ti * 16 : BN / 2 + (ti - TI / 2) * 16) : ti * 16; };
-    floatx4_t acc[TI][4];
+    floatx4_t acc[TI][BLOCKS];
 #pragma unroll
     for (int a = 0; a < TI; ++a)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < BLOCKS; ++b) acc[a][b] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
 
     auto compute = [&](auto ntj_tag, int ws, int xs, int ks) {
       constexpr int NTJ = decltype(ntj_tag)::value;
@@ -131,36 +173,33 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
         __builtin_amdgcn_sched_group_barrier(0x008, 2 * NTJ, 0);
       }
     };
-    // Order of the loads, and what the waits (at most N of a wavefront's loads still in flight, the N youngest) leave:
-    //   XEARLY: W0 X0 W1 X1 | step kt: W(kt+2) X(kt+2); behind its wait W, X(kt+1) have landed: N = WLOADS + XLOADS
-    //   else:   W0 X0 W1    | step kt: X(kt+1) W(kt+2); behind its wait W, X(kt+1) have landed: N = WLOADS
     // Step kt overwrites the stages that step kt - 1 read; the barrier at its end lies between.
-    constexpr int INFLIGHT = XEARLY ? WLOADS + XLOADS : WLOADS;
     auto k_loop = [&](auto ntj_tag) {
       int ws = 0, xs = 0;
       for (int kt = 0; kt < nkt; ++kt) {
-        const int ws2 = ws == 0 ? 2 : ws - 1;  // stage of step kt + 2
-        if constexpr (XEARLY) load_w(kt + 2, ws2);
-        else load_x(kt + 1, xs ^ 1);
+        const int wl = ws == 0 ? ST.w - 1 : ws - 1, xl = xs == 0 ? ST.x - 1 : xs - 1;
+        if constexpr (XEARLY) load_w(kt + WA, wl);
+        else load_x(kt + 1, xl);
         compute(ntj_tag, ws, xs, 0);
-        if constexpr (XEARLY) load_x(kt + 2, ws2);
-        else load_w(kt + 2, ws2);
+        if constexpr (XEARLY) load_x(kt + XA, xl);
+        else load_w(kt + WA, wl);
         compute(ntj_tag, ws, xs, 1);
         vm_wait<INFLIGHT>();
         __syncthreads();
-        ws = ws == 2 ? 0 : ws + 1;
-        xs = xs == XSTAGES - 1 ? 0 : xs + 1;
+        ws = ws == ST.w - 1 ? 0 : ws + 1;
+        xs = xs == ST.x - 1 ? 0 : xs + 1;
       }
     };
-    load_w(0, 0);
-    load_x(0, 0);
-    load_w(1, 1);
-    if constexpr (XEARLY) load_x(1, 1);
+#pragma unroll
+    for (int i = 0; i < WA; ++i) {
+      load_w(i, i);
+      if (i < XA) load_x(i, i);
+    }
     vm_wait<INFLIGHT>();
     __syncthreads();
-    if (ntj == 4) k_loop(DenseInt<4>{});
-    else if (ntj == 3) k_loop(DenseInt<3>{});
-    else if (ntj == 2) k_loop(DenseInt<2>{});
+    if (BLOCKS > 3 && ntj == 4) k_loop(DenseInt<BLOCKS < 4 ? 0 : 4>{});
+    else if (BLOCKS > 2 && ntj == 3) k_loop(DenseInt<BLOCKS < 3 ? 0 : 3>{});
+    else if (BLOCKS > 1 && ntj == 2) k_loop(DenseInt<BLOCKS < 2 ? 0 : 2>{});
     else if (ntj == 1) k_loop(DenseInt<1>{});
     else k_loop(DenseInt<0>{});
     vm_wait<0>();  // the requests past the last step: nothing may land in LDS after the workgroup is done
@@ -168,11 +207,11 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
     // ---- results: lane (n_in, g) holds features 4 g .. 4 g + 3 of each block for token row n_in of each column block
     const FakeQuant fq = fq_scale(p);
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
+    for (int tj = 0; tj < BLOCKS; ++tj) {
       if (tj * 16 + n_in >= my_rows) continue;
       T* orow = reinterpret_cast<T*>(p.out) + out_row(p, row_begin + wm * rpg + tj * 16 + n_in) * p.ldo + 4 * g;
       if constexpr (MODE == MODE_GATEUP) {
-        orow += (int64_t)tile.ntile * (BN / 2) + wn * (BN / 2 / WN);
+        orow += (int64_t)ntile * (BN / 2) + wn * (BN / 2 / WN);
 #pragma unroll
         for (int ti = 0; ti < TI / 2; ++ti) {
           const floatx4_t ga = acc[ti][tj], ua = acc[ti + TI / 2][tj];
@@ -182,7 +221,7 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
           else *dst = gateup_quad<T, STMOE_ACT_GELU_ERF>(gq, uq, fq);
         }
       } else {
-        orow += (int64_t)tile.ntile * BN + wn * (BN / WN);
+        orow += (int64_t)ntile * BN + wn * (BN / WN);
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti) {
           const floatx4_t v = acc[ti][tj];
@@ -191,22 +230,26 @@ grouped_dense_kernel(GemmParams p, int n_tiles) {
       }
     }
   };
-  if (rows_here <= BM / 2) unit(DenseInt<2>{});
-  else unit(DenseInt<4>{});
+  auto sized = [&](auto bn_tag) {
+    if (rows_here <= 32) unit(bn_tag, DenseInt<2>{}, DenseInt<1>{});
+    else if (rows_here <= 128) unit(bn_tag, DenseInt<2>{}, DenseInt<4>{});
+    else if (rows_here <= 192) unit(bn_tag, DenseInt<4>{}, DenseInt<3>{});
+    else unit(bn_tag, DenseInt<4>{}, DenseInt<4>{});
+  };
+  if (BN_LAUNCH == 256 && half < 0) sized(DenseInt<BN_LAUNCH>{});
+  else sized(DenseInt<128>{});
 }
 
 template <typename T, int MODE, int BN>
 static int launch_dense_m(const GemmParams& p, int64_t max_rows, hipStream_t st) {
-  // three weight stages and the larger of three token stages of 128 rows and two (BN = 128: three) of 256
-  constexpr size_t lds_bytes = (size_t)(3 * BN + (BN == 128 ? 3 : 2) * 256) * BIG_LS * 2;
-  static_assert(lds_bytes <= 160 * 1024 && 3 * 128 <= 2 * 256, "stages fit a CU's LDS");
+  constexpr size_t lds_bytes = kDenseLds;
   static std::atomic<uint64_t> lds_ready{0};
   auto kern = grouped_dense_kernel<T, MODE, BN>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_ready, "dense kernel")) return rc;
   const int n_tiles = (int)(p.n_out / (MODE == MODE_GATEUP ? BN / 2 : BN));
   const int experts = p.offsets ? p.E : 1;
   const int m_slots = (int)((max_rows + 255) / 256) + experts;
-  kern<<<dim3((unsigned)big_grid(n_tiles, m_slots, false)), 512, lds_bytes, st>>>(p, n_tiles);
+  kern<<<dim3((unsigned)(big_grid(n_tiles, m_slots, false) + (BN == 256 ? 8 * kBigCusPerXcd / 2 : 0))), 512, lds_bytes, st>>>(p, n_tiles);
   return check_launch("grouped_dense");
 }
 // 128 weight rows per unit instead of 256 while 256 would leave CUs without a unit (a unit per 256 features and expert, and half

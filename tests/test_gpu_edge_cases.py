@@ -466,3 +466,24 @@ def test_many_experts_on_the_256_row_kernels(device, E, K, N):
                 size = torch.maximum(want.float().abs(), want.float().pow(2).mean(dim=1, keepdim=True).sqrt())
                 worst = ((got.float() - want.float()).abs() / size).amax(dim=1)
                 assert float(worst.max()) < 4 * 2.0 ** -10, int(worst.argmax())
+
+
+@pytest.mark.parametrize("K,tiles", [(64, 36), (192, 36), (576, 36), (576, 3)])
+def test_unit_sizes_of_the_kernel_of_unquantized_weights(device, K, tiles):
+    """Units at the edges of every token-row size, with reductions of one step, of fewer and of more steps than stages, in launches of 256
+    weight rows per unit whose last round is cut into halves (36 tiles) and of 128: bit for bit against the 128 x 128 kernel."""
+    from sharktank_amd import _hip
+
+    rows = [32, 33, 128, 129, 192, 193, 256, 1]
+    E, T = len(rows), sum(rows)
+    g = torch.Generator(device=device).manual_seed(K + tiles)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=device).to(torch.bfloat16)
+    weight = lambda n: _hip.DeviceWeight(_hip.W_DENSE, E, n, K, draw(E, n, K) / K**0.5, None, None, _hip.BF16)
+    gate, up, down = weight(128 * tiles), weight(128 * tiles), weight(256 * tiles)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(rows)).to(torch.int32)[torch.randperm(T, generator=torch.Generator().manual_seed(K))]
+    _, offsets, perm, _ = _hip.dispatch_build(idx.reshape(T, 1).to(device), E)
+    x = draw(T, K)
+    for run in (lambda v: _hip.grouped_gate_up(x, gate, up, _hip.ACT_SILU, offsets, perm, 1, variant=v),
+                lambda v: _hip.grouped_down(x, down, offsets, T, 1, variant=v)):
+        got, want = run(_hip.VARIANT_DENSE), run(_hip.VARIANT_MFMA_TILE)
+        assert float(want.float().abs().max()) > 0 and torch.equal(got.view(torch.int16), want.view(torch.int16))
