@@ -320,8 +320,10 @@ grouped_mfma_reg_kernel(RegArgs args) {
         // A SIMD serves its older wavefront first: that one went through a chunk at its own pace (3500 cycles of 5900, Q4_1 bf16, 64 rows)
         // and waited, while the younger one finished alone, at half the rate at which a SIMD issues.  In bf16, where issue slots are what
         // runs out, the younger one goes first for half a chunk: 1 to 4 % (8 experts of 4096 x 14336 at 203 tokens 297 -> 292 us, 64 rows of
-        // [14336, 4096] 28.7 -> 27.5).  In fp16 nothing (-1 to 1 %).
-        const bool hand_over = !__is_same(T, f16_t) && wave >= 4;
+        // [14336, 4096] 28.7 -> 27.5).  In fp16 nothing (-1 to 1 %).  (Gate/up of Q8_0 in
+        // the wide kernel has no register left for it: one would go to scratch memory, whose accesses the counted waits do not know.)
+        constexpr bool HAND_OVER = !__is_same(T, f16_t) && !(MT > 4 && WF == WF_Q8_0_P && MODE == MODE_GATEUP);
+        const bool hand_over = HAND_OVER && wave >= 4;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           if (s == 0 && hand_over) __builtin_amdgcn_s_setprio(1);
