@@ -196,6 +196,16 @@ router_topk_kernel(const T* __restrict__ x, const T* __restrict__ wr, int64_t T_
   softmax_topk_store<T, EP>(lg, E, k, t, lane, idx_out, idx64_out, gate_out);
 }
 
+// fp16: a product of two fp16 numbers is exact in fp32 (22 significant bits, exponents far inside the fp32 range), so a
+// fused multiply-add rounds once exactly where the separate multiply and add round: same bits, fewer instructions.  bf16
+// products can fall into the fp32 subnormal range, where the separate multiply would round: they keep both steps.
+template <typename T> __device__ __forceinline__ float mul_add_like_separate(float acc, float a, float b) {
+  if constexpr (__is_same(T, f16_t)) return __fmaf_rn(a, b, acc);
+  else return __fadd_rn(acc, __fmul_rn(a, b));
+}
+
+template <int V> struct RtInt { static constexpr int value = V; };
+
 // ---------------------------------------------------------------------------------------------------
 // router, one workgroup (8 wavefronts) per token, optionally fused with the preceding RMS norm.
 //
@@ -210,8 +220,8 @@ struct SingleTokenDispatch {
   int32_t *counts, *offsets, *perm, *inv;
 };
 
-template <typename T, typename W, bool FUSE_NORM, int PRE>
-__global__ void __launch_bounds__(512, PRE ? 4 : 8)
+template <typename T, typename W, bool FUSE_NORM, int PRE, int MANY = 0>
+__global__ void __launch_bounds__(512, PRE || MANY ? 4 : 8)
 router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float eps, T* __restrict__ xn,
                  const T* __restrict__ wr, int64_t K, int E, int k, T* __restrict__ logits_out,
                  int32_t* __restrict__ idx_out, int64_t* __restrict__ idx64_out, T* __restrict__ gate_out,
@@ -224,7 +234,7 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
   T* xs = reinterpret_cast<T*>(smem);                                  // [K] the (normalised) token row
   float* lg_s = reinterpret_cast<float*>(smem + ((K * sizeof(T) + 15) / 16) * 16);  // [E] logits, then 8 partials
   float* part = lg_s + 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t t = blockIdx.x;
   const T* xr = x + t * K;
 
@@ -233,9 +243,9 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
   // No load here has a condition of its own: past the row's end the last piece is read again and not used.  Loads under
   // separate conditions are waited for one by one, those of a straight line are all in flight together (rows shorter than
   // NC * 512 elements used to pay one memory latency per 512 elements: 7 tokens of 3328, launch 8.7 -> 6.8 us).
-  // PRE = 8 (a whole row of 4096) for launches of at most 64 tokens, 4 up to 512 tokens and wherever a wavefront has several
-  // experts (latency).  Other launches of more tokens, where throughput counts and the prefetch registers held through the norm
-  // would cost half of the workgroups a CU can hold, have PRE = 0 and read the rows in the loop over the chunks.
+  // PRE = 8 (a whole row of 4096) for launches of at most 64 tokens, 4 up to 512 tokens (latency).  Launches of more tokens, where
+  // throughput counts and the prefetch registers held through the norm would cost half of the workgroups a CU can hold, have PRE = 0
+  // and read the rows in the loop over the chunks.  MANY: see below.
   constexpr int NC = 8;
   uint4 wpre[PRE ? PRE : 1];
   auto prefetch = [&](uint4 (&dst)[PRE ? PRE : 1], int e) {
@@ -249,6 +259,41 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
     }
   };
   prefetch(wpre, wave);
+  // MANY > 0 (16-bit rows, more than 8 experts): MANY experts of the wavefront side by side.  The token row is read from LDS and widened
+  // once for all of them, and their chains of additions, none of which may be reordered, run beside one another.  The experts wave +
+  // 8 (MANY n + i), i < MANY, go through the row in blocks of RING chunks of 512; the next block is requested piece by piece while this
+  // one is summed, and the last one requests nothing, so that nothing is waited for in vain.  Experts and pieces past the end read the
+  // last ones again.  The first block is requested behind the token row (16 KB a wavefront in front of it delayed the norm by 1 us).
+  constexpr int RING = 4;
+  uint4 ring[MANY ? RING : 1][MANY ? MANY : 1];
+  const int nch = (int)((K + 511) >> 9);
+  const T* rq_row[MANY ? MANY : 1];
+  int rq_c = 0, rq_e = wave;  // first chunk and first expert of the block that is requested
+  auto rows = [&]() {
+#pragma unroll
+    for (int i = 0; i < MANY; ++i) rq_row[i] = wr + (int64_t)min(rq_e + 8 * i, E - 1) * K;
+  };
+  auto request = [&](uint4 (&dst)[MANY ? MANY : 1], int j) {
+    const uint32_t off = (uint32_t)min((rq_c + j) * 512 + lane * 8, (int)K - 8) * (uint32_t)sizeof(T);
+#pragma unroll
+    for (int i = 0; i < MANY; ++i) dst[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(rq_row[i]) + off);
+  };
+  auto next_block = [&]() {
+    rq_c += RING;
+    if (rq_c >= nch) {
+      rq_c = 0;
+      rq_e += 8 * MANY;
+      rows();
+    }
+  };
+  auto request_first = [&]() {
+    if constexpr (MANY > 0) {
+      rows();
+#pragma unroll
+      for (int j = 0; j < RING; ++j) request(ring[j], j);
+      next_block();
+    }
+  };
   if constexpr (FUSE_NORM) {
     // the row's elements tid + 512 j are read once and kept (NC of them) for the second pass; the norm weights are
     // requested before the reduction
@@ -260,6 +305,9 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
     for (int j = 0; j < NC; ++j) xraw[j] = xr[min(tid + j * 512, (int)K - 1)];
 #pragma unroll
     for (int j = 0; j < NC; ++j) wraw[j] = norm_w[min(tid + j * 512, (int)K - 1)];
+    __builtin_amdgcn_sched_barrier(0);  // (loads return in order: what the norm waits for must not queue behind the router's rows)
+    request_first();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       xv[j] = Cvt<T>::to_f32(xraw[j]);
@@ -298,6 +346,7 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
     for (int64_t i = (int64_t)tid * 8; i < K; i += 512 * 8)
       *reinterpret_cast<uint4*>(reinterpret_cast<unsigned char*>(xs) + i * sizeof(T)) =
           *reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(xr) + i * sizeof(T));
+    request_first();
     if constexpr (sizeof(T) == 4)
       for (int64_t i = (int64_t)tid * 8 + 4; i < K; i += 512 * 8)
         *reinterpret_cast<uint4*>(&xs[i]) = *reinterpret_cast<const uint4*>(&xr[i]);
@@ -341,17 +390,52 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
       if (logits_out) logits_out[t * E + e] = Cvt<T>::from_f32(l);
     }
   };
-  if (E <= 8) {
-    if (wave < E) logit(wave, wpre);
-  } else {
-    // several experts per wavefront: the next one's chunks are on their way while this one's are summed
-    for (int e = wave; e < E; e += 8) {
-      uint4 wnext[PRE ? PRE : 1];
-      prefetch(wnext, e + 8);
-      logit(e, wpre);
+  if constexpr (MANY > 0) {
+    float acc[MANY];
 #pragma unroll
-      for (int j = 0; j < PRE; ++j) wpre[j] = wnext[j];
-    }
+    for (int i = 0; i < MANY; ++i) acc[i] = 0.0f;
+    int c = 0, first = 0;
+    auto block = [&](auto more_tag) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < RING; ++j) {
+        const int k0 = (c + j) * 512 + lane * 8;
+        if (k0 < (int)K) {
+          Vec8<T> xv;
+          xv.load(xs + k0);
+#pragma unroll
+          for (int i = 0; i < MANY; ++i) {
+            Vec8<T> wv;
+            wv.from_raw(ring[j][i]);
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj) acc[i] = mul_add_like_separate<T>(acc[i], xv.v[jj], wv.v[jj]);
+          }
+        }
+        if (decltype(more_tag)::value) request(ring[j], j);
+      }
+      if (decltype(more_tag)::value) next_block();
+      c += RING;
+      if (c < nch) return;
+      float l = 0.0f;  // lane i: of expert first + wave + 8 i
+#pragma unroll
+      for (int i = 0; i < MANY; ++i) {
+        const float sum = wave_xor_sum(acc[i]);
+        l = lane == i ? sum : l;
+        acc[i] = 0.0f;
+      }
+      const int e = first + wave + 8 * lane;
+      if (lane < MANY && e < E) {
+        l = round_to<T>(l);
+        lg_s[e] = l;
+        if (logits_out) logits_out[t * E + e] = Cvt<T>::from_f32(l);
+      }
+      c = 0;
+      first += 8 * MANY;
+    };
+    while (c + RING < nch || first + 8 * MANY < E) block(RtInt<1>{});
+    block(RtInt<0>{});
+  } else {
+    // (several experts per wavefront: fp32 rows, or PRE = 0, which have no chunks of the first one in registers)
+    for (int e = wave; e < E; e += 8) logit(e, wpre);
   }
   __syncthreads();
   if (wave != 0) return;
@@ -425,14 +509,6 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
 // order through the wavefront's own piece of LDS; the normalised row is computed, stored and multiplied in the
 // router's layout again (normalisation is elementwise).  16-bit rows of NCH * 512 elements.
 //
-// fp16: a product of two fp16 numbers is exact in fp32 (22 significant bits, exponents far inside the fp32 range), so a
-// fused multiply-add rounds once exactly where the separate multiply and add round: same bits, fewer instructions.  bf16
-// products can fall into the fp32 subnormal range, where the separate multiply would round: they keep both steps.
-template <typename T> __device__ __forceinline__ float mul_add_like_separate(float acc, float a, float b) {
-  if constexpr (__is_same(T, f16_t)) return __fmaf_rn(a, b, acc);
-  else return __fadd_rn(acc, __fmul_rn(a, b));
-}
-
 template <typename T, typename W, int NCH, int EP>
 __global__ void __launch_bounds__(256)
 norm_router_wave_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float eps, T* __restrict__ xn,
@@ -593,17 +669,20 @@ static int launch_router_wg(const void* x, const void* norm_w, float eps, void* 
                             const float* x_fq = nullptr) {
   const size_t lds = ((K * sizeof(T) + 15) / 16) * 16 + (64 + 8 + 64) * sizeof(float);
   if (lds > 64 * 1024) return set_error(STMOE_ERR_UNSUPPORTED, "router: K=%lld does not fit the per-token LDS row", (long long)K);
-  if (T_tokens <= 64)
-    router_wg_kernel<T, W, FUSE_NORM, 8><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
+  auto launch = [&](auto pre_tag, auto many_tag) {
+    router_wg_kernel<T, W, FUSE_NORM, decltype(pre_tag)::value, decltype(many_tag)::value><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
-  else if (T_tokens <= 512 || E > 16)
-    // (several experts per wavefront: the next one's row is worth its registers at any size.  With the tail on v_readlane 26 tokens of
-    // 2048 with 32 experts take 11 us instead of 25, 400 with 64 experts 17 instead of 51, 2048 with 64 47 instead of 73)
-    router_wg_kernel<T, W, FUSE_NORM, 4><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
-        (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
-  else
-    router_wg_kernel<T, W, FUSE_NORM, 0><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
-        (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
+  };
+  // More than 8 experts, 16-bit rows: several of a wavefront's experts side by side (us, one by one / side by side, norm included, 1, 64, 256,
+  // 400 and 2000 tokens of 2048 elements: 64 experts bf16 13.9, 15.2, 12.7, 15.6, 52.5 / 8.8, 11.3, 11.1, 14.4, 44.1; 32 experts fp16 10.7,
+  // 11.3, 9.4, 12.3, 34.4 / 6.0, 6.8, 7.4, 10.2, 26.6; 12 experts bf16 7.0, 8.7, 6.6, 8.1 / 4.4, 5.6, 6.2, 7.7).  Up to 16 experts, launches
+  // of more than 512 tokens that the wavefront-per-token kernel leaves here keep the form with most workgroups per CU.
+  constexpr bool HALF = sizeof(T) == 2;
+  if (HALF && E > 16) launch(RtInt<0>{}, RtInt<HALF ? 4 : 0>{});
+  else if (HALF && E > 8 && T_tokens <= 512) launch(RtInt<0>{}, RtInt<HALF ? 2 : 0>{});
+  else if (T_tokens <= 64) launch(RtInt<8>{}, RtInt<0>{});
+  else if (T_tokens <= 512) launch(RtInt<4>{}, RtInt<0>{});
+  else launch(RtInt<0>{}, RtInt<0>{});
   return check_launch("router_wg");
 }
 
