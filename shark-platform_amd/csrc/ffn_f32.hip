@@ -6,10 +6,13 @@
 // meet 16, 32 or 64 token rows per sweep.  A workgroup takes one expert and 16 output features (GATEUP: of gate and up; DOWN:
 // 32 features where they divide), its four wavefronts a quarter of the reduction each: a layer of 8 x 1024 x 512 has 512 such
 // items, 2048 wavefronts, whose loads are all in flight after two steps.  The quarters are added through LDS in a fixed order.
-// Measured (8 experts, top-2, gate/up + down, us; general kernel / this one): 64 tokens of 512 x 1024 71 + 33 / 17 + 11; the
-// whole layer 110 / 38 us, of which the host takes 31.  109 tokens of 896 x 1280: layer 325 / 69 us; 101 tokens of 256 x 1152
-// 154 / 47.  At 10 tokens of 768 x 1536 the gate/up launch reads 3.3 TB/s; with 25 rows per expert and more the time goes into the
-// multiplications (32 cycles each for 16 x 16 x 4).  Eight wavefronts per item instead of four: no change.
+// Order of the loads: they return in the order of their issue, so the tokens of an item's rows are requested first, then its weights, then
+// the token rows; two chunks of both are in flight, every load unconditional (a row's ragged end re-reads its last piece and drops it in
+// registers: an instance of its own, TAIL).  With one chunk ahead, each load under its own condition, and the wavefront's number in a vector
+// register, every wait was for all loads in flight: 64 tokens of 512 x 1024 16.3 + 11.7 us; now 14.0 + 9.2.  Layer (8 experts, top-2, us,
+// before / now): 64 tokens of 512 x 1024 37.6 / 31.4, 109 tokens of 896 x 1280 77 / 69, 128 tokens of 1024 x
+// 1536 88 / 76; Q8_0 weights of 1024 x 1024, 2000 tokens 435 / 349; one Q8_0 matrix of [2048, 2048], 60 rows 28.7 / 20.0.  (On the general
+// kernel the first took 110.)  Weights requested in front of the tokens: 34.3.
 // Order of the sums: the matrix instruction rounds after every product, so one running sum per quarter was up to 3.6 times as far
 // from fp64 as the general kernel, whose 64 lanes hold short sums (K = 4096: rms error 9.6 / 2.7 times 2^-24 of the result's rms;
 // K = 512: 3.5 / 1.6).  A chunk of 64 elements is eight sums of 8 products, added in pairs: 1.9 and 1.4, below the general kernel at
@@ -27,23 +30,31 @@ namespace stmoe {
 
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
-// One chunk of 64 reduction elements of one row: value(4 i + r) is the lane's element of MFMA step 4 i + r.
-template <int WF> struct F32Weight {
+// One chunk of 64 reduction elements of one row: value(4 i + r) is the lane's element of MFMA step 4 i + r.  `TAIL`:
+// a row's last chunk may have `blocks` < 4 pieces of 16 elements: the loads read the last one again, drop() puts zeros there.
+template <int WF, bool TAIL> struct F32Weight {
   static constexpr bool kRowContiguous = false;
   Chunk16<WF> c;
-  __device__ __forceinline__ void load(const WeightView& w, int64_t e, int64_t n, int64_t k, int g, bool ok) {
-    if (ok) c.load(w, e, n, k + 16 * g);
-    else c.zero();
+  __device__ __forceinline__ void load(const WeightView& w, int64_t e, int64_t n, int64_t k, int g, int blocks) {
+    c.load(w, e, n, k + 16 * (TAIL ? min(g, blocks - 1) : g));
+  }
+  __device__ __forceinline__ void drop(int g, int blocks) {
+    if (g >= blocks) c.zero();
   }
   __device__ __forceinline__ void values(float (&v)[16]) const { c.to_f32(v); }
 };
-template <> struct F32Weight<WF_DENSE_F32> {
+template <bool TAIL> struct F32Weight<WF_DENSE_F32, TAIL> {
   static constexpr bool kRowContiguous = true;
   floatx4_t q[4];
   __device__ __forceinline__ void load(const WeightView& w, int64_t e, int64_t n, int64_t k, int g, int blocks) {
     const float* p = reinterpret_cast<const float*>(w.qs) + (e * w.rows + n) * w.cols + k + 4 * g;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) q[i] = i < blocks ? *reinterpret_cast<const floatx4_t*>(p + 16 * i) : (floatx4_t){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const floatx4_t*>(p + 16 * (TAIL ? min(i, blocks - 1) : i));
+  }
+  __device__ __forceinline__ void drop(int, int blocks) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i >= blocks) q[i] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
   }
   __device__ __forceinline__ void values(float (&v)[16]) const {
 #pragma unroll
@@ -51,47 +62,73 @@ template <> struct F32Weight<WF_DENSE_F32> {
   }
 };
 
-template <int WF, int MODE, int NT, int MT>
-__device__ __forceinline__ void f32_pass(const GemmParams& p, int e, const int64_t (&wrow)[NT], int tile, int r0, int re, int lane, int wave,
-                                         floatx4_t (*red)[64]) {
-  constexpr bool ROWC = F32Weight<WF>::kRowContiguous;
-  const int g = lane >> 4, n_in = lane & 15;
-  const int nch = (int)((p.kred + 63) >> 6), c_begin = nch * wave / 4, c_end = nch * (wave + 1) / 4;
-  const float* xrow[MT];
+// A wavefront's quarter of the reduction, [begin, end) in chunks, and its weight rows.
+template <int WF, int MODE, int NT, bool TAIL> struct F32Quarter {
+  int begin, end;
+  int64_t wrow[NT];
+  F32Weight<WF, TAIL> w[2][NT];
+  // (the reduction length is a multiple of 16: a chunk's 16-element pieces are whole)
+  static __device__ __forceinline__ int blocks_of(const GemmParams& p, int c) { return (int)min((int64_t)4, (p.kred - (int64_t)c * 64) >> 4); }
+  __device__ __forceinline__ void load(const GemmParams& p, int e, int g, int slot, int c) {
+    const int blocks = blocks_of(p, c);
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int i = min(r0 + mt * 16 + n_in, re - 1);  // rows past the end re-read the last one (never stored)
-    const int64_t src = p.perm ? (int64_t)(p.perm[i] / p.k_top) : (int64_t)i;
-    xrow[mt] = reinterpret_cast<const float*>(p.a) + src * p.lda;
+    for (int t = 0; t < NT; ++t) w[slot][t].load(MODE == MODE_GATEUP && t == 1 ? p.w1 : p.w0, e, wrow[t], (int64_t)c * 64, g, blocks);
   }
+  __device__ __forceinline__ void load_first(const GemmParams& p, int e, int g) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) load(p, e, g, j, max(min(begin + j, end - 1), 0));
+  }
+};
+
+template <int WF, int MODE, int NT, bool TAIL, int MT>
+__device__ __forceinline__ void f32_pass(const GemmParams& p, int e, F32Quarter<WF, MODE, NT, TAIL>& quarter, int tile, int r0, int re, int lane, int wave,
+                                         floatx4_t (*red)[64]) {
+  constexpr bool ROWC = F32Weight<WF, TAIL>::kRowContiguous;
+  const int g = lane >> 4, n_in = lane & 15;
+  const int c_begin = quarter.begin, c_end = quarter.end;
+  const float* xrow[MT];
+  int src[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) src[mt] = min(r0 + mt * 16 + n_in, re - 1);  // rows past the end re-read the last one (never stored)
+  if (p.perm) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) src[mt] = p.perm[src[mt]];
+  }
+  // The weights are on their way while the tokens of the rows and then the token rows are fetched.  (Behind the tokens: loads return in order.)
+  __builtin_amdgcn_sched_barrier(0);
+  quarter.load_first(p, e, g);
+  __builtin_amdgcn_sched_barrier(0);
+  if (p.perm) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) src[mt] /= p.k_top;
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) xrow[mt] = reinterpret_cast<const float*>(p.a) + (int64_t)src[mt] * p.lda;
   floatx4_t acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[mt][t] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
 
-  // (the reduction length is a multiple of 16: a chunk's 16-element pieces are whole, those past the end read as zeros)
-  auto blocks_of = [&](int c) { return (int)min((int64_t)4, (p.kred - (int64_t)c * 64) >> 4); };
-  auto load_w = [&](F32Weight<WF> (&w)[NT], int c) {
-    const int blocks = blocks_of(c);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const WeightView& wv = MODE == MODE_GATEUP && t == 1 ? p.w1 : p.w0;
-      if constexpr (ROWC) w[t].load(wv, e, wrow[t], (int64_t)c * 64, g, blocks);
-      else w[t].load(wv, e, wrow[t], (int64_t)c * 64, g, g < blocks);
-    }
-  };
   auto load_x = [&](floatx4_t (&x)[MT][4], int c) {
-    const int blocks = blocks_of(c);
+    const int blocks = quarter.blocks_of(p, c);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bool ok = ROWC ? i < blocks : g < blocks;
-        x[mt][i] = ok ? *reinterpret_cast<const floatx4_t*>(xrow[mt] + (int64_t)c * 64 + (ROWC ? 16 * i + 4 * g : 16 * g + 4 * i)) : (floatx4_t){0.f, 0.f, 0.f, 0.f};
-      }
+      for (int i = 0; i < 4; ++i)
+        x[mt][i] = *reinterpret_cast<const floatx4_t*>(xrow[mt] + (int64_t)c * 64 + (ROWC ? 16 * (TAIL ? min(i, blocks - 1) : i) + 4 * g : 16 * (TAIL ? min(g, blocks - 1) : g) + 4 * i));
   };
-  auto multiply = [&](const F32Weight<WF> (&w)[NT], const floatx4_t (&x)[MT][4]) {
+  auto multiply = [&](F32Weight<WF, TAIL> (&w)[NT], floatx4_t (&x)[MT][4], int c) {
+    const int blocks = quarter.blocks_of(p, c);
+    if (TAIL && blocks < 4) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) w[t].drop(g, blocks);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if ((ROWC ? i : g) >= blocks) x[mt][i] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+    }
     float v[NT][16];
 #pragma unroll
     for (int t = 0; t < NT; ++t) w[t].values(v[t]);
@@ -116,30 +153,38 @@ __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, const int64
         asm volatile("" : "+v"(acc[mt][t]));
       }
   };
-  if (c_begin < c_end) {
-    // Both operands one chunk ahead while the registers allow it (four token tiles: the weights only).  Requests are
-    // unconditional (past the end the last chunk again), so that no wait covers a younger one.
-    F32Weight<WF> w0[NT], w1[NT];
-    floatx4_t x0[MT][4], x1[MT <= 2 ? MT : 1][4];
-    load_w(w0, c_begin);
-    load_x(x0, c_begin);
-    // (one copy of the 64 to 256 multiplications: two alternating buffers doubled the code and measured up to a fifth slower)
+  // No request is under a condition of its own: such loads were waited for one by one.
+  if (MT > 2 && c_begin < c_end) {
+    // The weights two chunks ahead (for more token rows there are no registers).  One copy of the 128 to 256 multiplications: two
+    // alternating buffers doubled the code and measured up to a fifth slower.
+    floatx4_t x[MT][4];
 #pragma unroll 1
     for (int c = c_begin; c < c_end; ++c) {
-      const int c1 = min(c + 1, c_end - 1);
-      load_w(w1, c1);
-      if constexpr (MT <= 2) load_x(x1, c1);
-      multiply(w0, x0);
-      if constexpr (MT > 2) load_x(x0, c1);
+      load_x(x, c);
+      multiply(quarter.w[0], x, c);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) w0[t] = w1[t];
-      if constexpr (MT <= 2) {
+      for (int t = 0; t < NT; ++t) quarter.w[0][t] = quarter.w[1][t];
+      quarter.load(p, e, g, 1, min(c + 2, c_end - 1));
+    }
+  }
+  if (MT <= 2 && c_begin < c_end) {
+    // Both operands two chunks ahead; none is requested that nobody reads, except that an odd last chunk is requested twice.
+    floatx4_t x[2][MT][4];
+    load_x(x[0], c_begin);
+    load_x(x[1], min(c_begin + 1, c_end - 1));
+    int c = c_begin;
+#pragma unroll 1
+    for (; c + 2 < c_end; c += 2) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) x0[mt][i] = x1[mt][i];
+      for (int j = 0; j < 2; ++j) {
+        multiply(quarter.w[j], x[j], c + j);
+        const int ahead = min(c + j + 2, c_end - 1);
+        quarter.load(p, e, g, j, ahead);
+        load_x(x[j], ahead);
       }
     }
+    multiply(quarter.w[0], x[0], c);
+    if (c + 1 < c_end) multiply(quarter.w[1], x[1], c + 1);
   }
 
   // the four quarters, ((0 + 1) + (2 + 3)); wavefront w finishes token tile w
@@ -184,22 +229,25 @@ __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, const int64
 }
 
 // grid: (feature tiles, experts, passes in flight)
-template <int WF, int MODE, int NT>
+template <int WF, int MODE, int NT, bool TAIL>
 __global__ void __launch_bounds__(256, 2) grouped_f32_kernel(GemmParams p) {
   __shared__ floatx4_t red[4 * NT * 4][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int e = blockIdx.y, tile = blockIdx.x;
-  int rb, re;
-  expert_range(p, e, rb, re);
-  int64_t wrow[NT];
+  const int nch = (int)((p.kred + 63) >> 6);
+  F32Quarter<WF, MODE, NT, TAIL> quarter;
+  quarter.begin = nch * wave / 4;
+  quarter.end = nch * (wave + 1) / 4;
 #pragma unroll
   for (int t = 0; t < NT; ++t)  // features past the end re-read the last one (never stored)
-    wrow[t] = min((int64_t)tile * (MODE == MODE_GATEUP ? 16 : 16 * NT) + (MODE == MODE_GATEUP ? 0 : 16 * t) + (lane & 15), p.n_out - 1);
+    quarter.wrow[t] = min((int64_t)tile * (MODE == MODE_GATEUP ? 16 : 16 * NT) + (MODE == MODE_GATEUP ? 0 : 16 * t) + (lane & 15), p.n_out - 1);
+  int rb, re;
+  expert_range(p, e, rb, re);
   for (int r0 = rb + 64 * (int)blockIdx.z; r0 < re; r0 += 64 * (int)gridDim.z) {
     const int left = re - r0;
-    if (left <= 16) f32_pass<WF, MODE, NT, 1>(p, e, wrow, tile, r0, re, lane, wave, red);
-    else if (left <= 32) f32_pass<WF, MODE, NT, 2>(p, e, wrow, tile, r0, re, lane, wave, red);
-    else f32_pass<WF, MODE, NT, 4>(p, e, wrow, tile, r0, min(re, r0 + 64), lane, wave, red);
+    if (left <= 16) f32_pass<WF, MODE, NT, TAIL, 1>(p, e, quarter, tile, r0, re, lane, wave, red);
+    else if (left <= 32) f32_pass<WF, MODE, NT, TAIL, 2>(p, e, quarter, tile, r0, re, lane, wave, red);
+    else f32_pass<WF, MODE, NT, TAIL, 4>(p, e, quarter, tile, r0, min(re, r0 + 64), lane, wave, red);
   }
 }
 
@@ -211,7 +259,9 @@ static int launch_f32_nt(const GemmParams& p, int64_t max_rows, hipStream_t st) 
   const int64_t rows = p.expert_rows_bound > 0 && p.expert_rows_bound < max_rows ? p.expert_rows_bound : max_rows;
   const int64_t passes = std::min<int64_t>((rows + 63) / 64, std::max<int64_t>(1, 8192 / (tiles * experts)));
   if (experts > 65535 || tiles >= ((int64_t)1 << 31)) return set_error(STMOE_ERR_UNSUPPORTED, "f32 kernel: %lld experts exceed its grid", (long long)experts);
-  grouped_f32_kernel<WF, MODE, NT><<<dim3((unsigned)tiles, (unsigned)experts, (unsigned)passes), 256, 0, st>>>(p);
+  const dim3 grid((unsigned)tiles, (unsigned)experts, (unsigned)passes);
+  if (p.kred % 64 == 0) grouped_f32_kernel<WF, MODE, NT, false><<<grid, 256, 0, st>>>(p);
+  else grouped_f32_kernel<WF, MODE, NT, true><<<grid, 256, 0, st>>>(p);
   return check_launch("grouped_f32");
 }
 template <int WF>

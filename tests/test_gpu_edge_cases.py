@@ -487,3 +487,33 @@ def test_unit_sizes_of_the_kernel_of_unquantized_weights(device, K, tiles):
                 lambda v: _hip.grouped_down(x, down, offsets, T, 1, variant=v)):
         got, want = run(_hip.VARIANT_DENSE), run(_hip.VARIANT_MFMA_TILE)
         assert float(want.float().abs().max()) > 0 and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt", ["dense", "q8_0"])
+@pytest.mark.parametrize("K", [16, 64, 80, 320, 560, 1024])  # part of a chunk, one, one and a piece, 1 to 4 chunks of a wavefront
+def test_fp32_kernel_reduction_and_row_edges(device, fmt, K):
+    """fp32 activations: rows at the edges of the token tiles, reductions with an odd number of chunks per wavefront or a ragged end.  The
+    bound on a sum of K products is that of any order of additions."""
+    from sharktank_amd import _hip
+    from sharktank_amd.ops import device_weight
+
+    rows = [1, 16, 17, 32, 33, 64, 65, 0]
+    E, T, N = len(rows), sum(rows), 72 if fmt == "dense" else 64
+    K = K if fmt == "dense" else (K + 31) // 32 * 32
+    g = torch.Generator().manual_seed(K)
+    x, offsets = torch.randn(T, K, generator=g), torch.tensor([0, *torch.tensor(rows).cumsum(0).tolist()], dtype=torch.int32)
+    if fmt == "dense":
+        w = torch.randn(E, N, K, generator=g)
+        w[1, 3, K - 1] = float("inf")  # (the piece that a ragged end reads again)
+        dw = _hip.DeviceWeight(_hip.W_DENSE, E, N, K, w.to(device), None, None, _hip.F32)
+    else:
+        case = MC.build(MC.Case(T=4, K=K, N=N, E=E, k=1, fmt=fmt, dtype=torch.float32, seed=K))
+        w = MC.dense_weights(case)[0].float()
+        dw = device_weight(MC.to_inference_tensor(fmt, case.planes["gate"], [E, N, K], "gate", device), stacked=True)
+    got = _hip.grouped_down(x.to(device), dw, offsets.to(device), T, 1).cpu()
+    for e in range(E):
+        a, b, xe = offsets[e], offsets[e + 1], x[offsets[e]:offsets[e + 1]].double()
+        want, size = xe @ w[e].double().T, xe.abs() @ w[e].double().abs().T
+        inf = want.isinf()
+        assert torch.equal(got[a:b][inf], want[inf].float())
+        assert bool(((got[a:b] - want).abs()[~inf] <= K * 2.0 ** -24 * size[~inf]).all()), e
