@@ -294,7 +294,9 @@ struct SkinnyExperts {
 template <typename T, int WF, int MODE, int MT, int KS, int NT>
 __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExperts& experts, const int64_t (&wrow)[NT], int tile,
                                             int r0, int re, int64_t nch_total, int lane, bool pin_prefetch) {
-  const int kw = KS > 1 ? (int)(threadIdx.x >> 6) : 0;
+  // (a scalar: from a vector register it made the loop's bounds and every prefetch's condition execution masks.  Layers of 8 experts, us: 1 token
+  // of 4096 x 14336, Q4_1 bf16 70.4 -> 69.3, 2 tokens of 4096 x 1024, fp16 48.6 -> 44.5)
+  const int kw = KS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int64_t c_begin = KS > 1 ? nch_total * kw / KS : 0;
   const int64_t nch = KS > 1 ? nch_total * (kw + 1) / KS : nch_total;  // end of this wavefront's chunk range
   const int g = lane >> 4, n_in = lane & 15;
@@ -459,7 +461,7 @@ grouped_skinny_kernel(GemmParams p, int tiles_per_expert, int total_waves, bool 
   static_assert(MODE == MODE_DOWN || NT == 2, "gate and up");
   const int lane = threadIdx.x & 63;
   const int n_in = lane & 15;
-  const int wave_global = KS > 1 ? (int)blockIdx.x : (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int wave_global = KS > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int64_t nch = p.kred >> 8;
   // experts that received rows, in increasing id
   SkinnyExperts experts;
