@@ -203,11 +203,9 @@ static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, 
   if (narrow > 128 && (wide <= 128 || wide >= 176) && (wtag == WF_Q4_1_P || p.kred >= 2048) &&
       ((rows > 52 * E && rows <= (p.kred < 2048 ? 72 : 80) * E) || (tiles == 2 && rows >= 120 * E && wide <= 256) || (tiles > 1 && wide <= 128)))
     return kRegWideRows;
-  // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 47
-  // rows, where some expert has more than 64, 101 / 115 us, down 55 / 70; Q4_1 104 / 92 and 57 / 55.  With 2048 elements and up to 40 rows they
-  // gain: 38 rows 98.6 / 94.4, fp16 90.4 / 87.5; over 16 widths with 32 to 64 experts, 26 to 38 rows, uniform and 1 / sqrt(rank) routings, the mean
-  // of each format and routing 5 to 17 %, extremes -13 and 44; with 1792 elements 0 to 14 %, with 1536 -6 to 8)
-  if (wtag != WF_Q4_1_P && units > 256 && (p.kred < 2048 ? rows > 24 * E : p.kred == 2048 && rows > 40 * E)) return 0;
+  // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 37
+  // rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
+  if (wtag != WF_Q4_1_P && p.kred <= 2048 && units > 256 && rows > 24 * E) return 0;
   if (rows <= 52 * E) return kRegUnitRows;
   return p.kred <= 8192 && narrow <= 256 ? kRegUnitRows : 0;
 }

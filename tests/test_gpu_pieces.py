@@ -696,9 +696,10 @@ def test_wide_register_kernel(device, fmt, dtype, N, K, act):
     ("down", "q8_0", torch.float16, 8, 2, 560, 3072, 3072, "reg"),       # 140: two tiles, 192 whole units
     ("down", "q8_0", torch.float16, 8, 2, 560, 9216, 2304, "ws"),        # 144 whole units leave CUs idle
     ("down", "fp8", torch.bfloat16, 8, 2, 560, 3072, 2048, "reg"),       # 128 units, run as halves
-    ("gate_up", "q8_0", torch.bfloat16, 33, 2, 660, 2048, 1024, "reg"),  # several rounds of units with 2048 elements: 40 rows per expert
-    ("gate_up", "q8_0", torch.bfloat16, 33, 2, 661, 2048, 1024, "ws"),   # ... and more
-    ("gate_up", "q8_0", torch.float16, 33, 2, 400, 1792, 1024, "ws"),    # shorter, more than 24 rows
+    ("gate_up", "q8_0", torch.bfloat16, 33, 2, 396, 2048, 1024, "reg"),  # several rounds of units: 24 rows per expert with up to 2048 elements
+    ("gate_up", "q8_0", torch.bfloat16, 33, 2, 397, 2048, 1024, "ws"),   # ... and more
+    ("gate_up", "q8_0", torch.bfloat16, 33, 2, 660, 2048, 1024, "ws"),
+    ("gate_up", "q8_0", torch.float16, 33, 2, 400, 1792, 1024, "ws"),
 ])
 def test_wide_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k, T, kred, n_out, choice):
     """The automatic choice on both sides of the lines around units of up to 96 rows, told by the bits."""
