@@ -364,6 +364,15 @@ size_t stmoe_mmt_workspace_bytes(int64_t M);
 int stmoe_mmt(const void* a, int dtype, int64_t M, const stmoe_weight* w, void* out, void* workspace /*nullable*/,
               size_t workspace_bytes, int workspace_ready, int variant, stmoe_stream_t stream);
 
+/* Which work units the automatic choice makes of one projection (nothing is launched; tests and tuning): the most token rows of a unit
+ * of the kernel that converts packed weights in the registers of the wavefronts that multiply them, 64 or up to 96, or 0 where
+ * another kernel takes the call.  `w`: format, dtype and sizes (its planes are not read); gate_up != 0: the pair of projections of
+ * stmoe_grouped_gate_up, else one matrix per expert; T tokens of k (token, slot) pairs each.  counts (nullable): the rows of each
+ * of w->experts experts, which that kernel looks at where the choice leaves two sizes open.  has_scratch: whether the call brings
+ * scratch for split reductions (stmoe_grouped_ffn of more than 128 pairs has it, stmoe_grouped_mmt has not). */
+int stmoe_register_unit_rows(int dtype, const stmoe_weight* w, int gate_up, int64_t T, int k, const int64_t* counts /*host, nullable*/,
+                             int has_scratch);
+
 #ifdef __cplusplus
 }
 #endif

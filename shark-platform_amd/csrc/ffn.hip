@@ -200,14 +200,17 @@ static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, 
   const int64_t most = (rows * 8 / 7 + E - 1) / E, narrow = (most + kRegUnitRows - 1) / kRegUnitRows * units,
                 tiles = (most + kRegWideRows - 1) / kRegWideRows, wide = tiles * units;
   // (129 to 175 whole units leave too many CUs without one: two tiles of 4 experts of 4864 x 7168 at 135 rows, Q4_1 bf16, layer 195 / 207 us)
-  if (narrow > 128 && (wide <= 128 || wide >= 176) && (wtag == WF_Q4_1_P || p.kred >= 2048) &&
+  // (one such tile per expert that nearly fills a round, of few experts or of very many: an expert with more than 96 rows spills into a second
+  // round.  4 experts from 61 rows on under uneven routings 0 % on average, -25 to 43, uniform ones gain 13 %; 32 and 64 experts from 73 rows on -20 to 24)
+  const bool spills = tiles == 1 && wide <= 256 && ((E <= 4 && wide > 192 && rows > 60 * E) || (E >= 32 && wide > 240 && rows > 72 * E));
+  if (narrow > 128 && (wide <= 128 || wide >= 176) && !spills && (wtag == WF_Q4_1_P || p.kred >= 2048) &&
       ((rows > 52 * E && rows <= (p.kred < 2048 ? 72 : 80) * E) || (tiles == 2 && rows >= 120 * E && wide <= 256) || (tiles > 1 && wide <= 128)))
     return kRegWideRows;
   // (short reductions over several rounds of units: the formats that convert faster gain less: 64 experts of 2048 x 1536, Q8_0 bf16 37
   // rows 98 / 102 and 55 / 60 us, Q4_1 47 rows 104 / 92 and 57 / 55)
   if (wtag != WF_Q4_1_P && p.kred <= 2048 && units > 256 && rows > 24 * E) return 0;
   if (rows <= 52 * E) return kRegUnitRows;
-  return p.kred <= 8192 && narrow <= 256 ? kRegUnitRows : 0;
+  return p.kred <= 8192 && (rows * 8 / 7 / E + kRegUnitRows - 1) / kRegUnitRows * units <= 256 ? kRegUnitRows : 0;
 }
 // A single matrix: its half units run at the pace of their reduction, whatever their number, where the prefill kernel cuts the reduction
 // in four and the narrow tiles re-read the token rows ([out, in], other kernels / this one, Q8_0 fp16; Q4_1 bf16): [14336, 4096] 33 rows
@@ -240,6 +243,11 @@ static int reg_rows(int dtype, int wtag, int mode, const GemmParams& p, int64_t 
   const int64_t spread = (rows + 256 / tiles - 1) / (256 / tiles);
   return spread > kRegUnitRows ? (int)spread : 0;
 }
+// The other unit size of a launch of several experts that the automatic choice gives 96 rows, 0 for none: the kernel, which knows the experts'
+// rows, takes whichever needs fewer rounds.  With 96 rows always, 14 % of 5000 launches (4 to 64 experts, uniform and Zipf routings) were slower
+// by more than 3 % than on the kernels they came from (extreme 1.44, mean 0.871 of the time); now 3 % (1.3, where an expert spills into a
+// second round; mean 0.843).  Layer of 8 experts of 5120 x 2048, Q4_1 fp16, 129 tokens of four experts each, Zipf, us: 64 / 96 / this 94.8 / 106 / 94.8.
+static int reg_fewer_rows(const GemmParams& p, int tile_rows) { return tile_rows == kRegWideRows && p.E > 1 ? kRegUnitRows : 0; }
 // fp8 activations x fp8 weights on the fp8 matrix cores: the 256 x 256 kernel for packed weights and launches with
 // enough rows to fill its tiles (variant 5), the 128 x 128 kernel otherwise (and always with variant 7).
 // Whether the 256 x 256 kernel takes a projection (its token rows must come without a gather: see fp8_ws_takes' caller).
@@ -289,8 +297,9 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     variant = 6;
   }
   if (variant == 12 || variant == 13) {
+    const int fewer_rows = reg_fewer_rows(p, tile_rows);
     if (tile_rows == 0) tile_rows = variant == 13 ? kRegWideRows : kRegUnitRows;
-    int rc = launch_mfma_reg(dtype, wtag, mode, p, max_rows, tile_rows, st);
+    int rc = launch_mfma_reg(dtype, wtag, mode, p, max_rows, tile_rows, fewer_rows, st);
     if (rc != STMOE_ERR_UNSUPPORTED) return rc;
     variant = 6;
   }
@@ -543,6 +552,29 @@ extern "C" int stmoe_mmt(const void* a, int dtype, int64_t M, const stmoe_weight
     p.split_tickets_zeroed = workspace_ready != 0;
   }
   return run_projection(variant, dtype, weight_tag(w), MODE_DOWN, p, M, as_stream(stream));
+}
+
+extern "C" int stmoe_register_unit_rows(int dtype, const stmoe_weight* w, int gate_up, int64_t T, int k, const int64_t* counts, int has_scratch) {
+  if (!w || T < 1 || k < 1 || w->experts < 1 || w->experts > 0x7fffffff || weight_tag(w) < 0) return 0;
+  GemmParams p{};
+  static const int32_t some = 0;  // (that there are offsets, or scratch, is all that the choice looks at)
+  float scratch_there = 0.0f;
+  p.E = (int32_t)w->experts;
+  p.offsets = p.E > 1 ? &some : nullptr;
+  p.k_top = k;
+  p.n_out = p.ldo = w->rows;
+  p.kred = p.lda = w->cols;
+  p.expert_rows_bound = T;
+  p.split_scratch = has_scratch ? &scratch_there : nullptr;
+  const int rows = reg_rows(dtype, weight_tag(w), gate_up ? MODE_GATEUP : MODE_DOWN, p, T * k), fewer = reg_fewer_rows(p, rows);
+  if (!counts || fewer == 0) return rows;
+  const int64_t n_tiles = p.n_out / (gate_up ? 128 : 256);
+  auto half_rounds = [&](int tile_rows) {
+    int64_t tiles = 0;
+    for (int e = 0; e < p.E; ++e) tiles += (counts[e] + tile_rows - 1) / tile_rows;
+    return reg_half_rounds((int)(tiles * n_tiles));
+  };
+  return half_rounds(fewer) <= half_rounds(rows) ? fewer : rows;
 }
 
 extern "C" int stmoe_grouped_mmt(const void* a, int dtype, int64_t T, int k, int a_per_pair, const stmoe_weight* w,

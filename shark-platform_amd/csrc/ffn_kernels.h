@@ -177,9 +177,15 @@ static inline bool narrow_wide(int mode, int64_t n_out, int64_t rows) {
 }
 int launch_mfma_narrow(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 static constexpr int kRegUnitRows = 64, kRegWideRows = 96;  // most token rows of a unit of launch_mfma_reg, and of its wide kernel
+static constexpr int kRegWgsPerXcd = 32;
+// Half rounds over an XCD's workgroups that `units` units of that kernel take: what is left after the last whole round runs as halves if they fit.
+static __host__ __device__ inline int reg_half_rounds(int units) {
+  const int n = (units + 7) / 8, rest = n % kRegWgsPerXcd;
+  return n / kRegWgsPerXcd * 2 + (rest == 0 ? 0 : 2 * rest <= kRegWgsPerXcd ? 1 : 2);
+}
 bool reg_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows);
-int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, int tile_rows, hipStream_t st);
-int launch_reg_wide(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, hipStream_t st);
+int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, int tile_rows, int fewer_rows, hipStream_t st);
+int launch_reg_wide(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, int fewer_rows, hipStream_t st);
 int launch_mfma_ws(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, float* partial, hipStream_t st);
 size_t mfma_ws_partial_bytes();
 size_t mfma_ws_tickets_offset();  // byte offset of the split units' ticket words inside that scratch

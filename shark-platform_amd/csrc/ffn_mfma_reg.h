@@ -41,6 +41,7 @@ struct RegArgs {
   int n_tiles;      // units per token tile: 256 weight rows each
   int wgs_per_xcd;  // grid size / 8
   int tile_rows;    // most token rows of a unit, at most 16 MT
+  int fewer_rows;   // wide kernel: most token rows of a unit where the launch takes no more rounds with so many (0: always tile_rows)
 };
 
 // Register sets of weights, LDS stages of token rows in a kernel whose units have up to `mt` 16-row token tiles.
@@ -215,8 +216,17 @@ grouped_mfma_reg_kernel(RegArgs args) {
     rows = lane < p.E ? end - off : 0;
     if (!p.offsets) { begin = 0; rows = lane == 0 ? (int)p.fixed_rows : 0; }
   }
-  const int main = (rows + args.tile_rows - 1) / args.tile_rows;
-  const int main_end = wave_inclusive_sum(main);
+  int main = (rows + args.tile_rows - 1) / args.tile_rows;
+  int main_end = wave_inclusive_sum(main);
+  if constexpr (MT > 4) {
+    if (args.fewer_rows > 0) {
+      const int main2 = (rows + args.fewer_rows - 1) / args.fewer_rows, end2 = wave_inclusive_sum(main2);
+      if (reg_half_rounds(__builtin_amdgcn_readlane(end2, 63) * n_tiles) <= reg_half_rounds(__builtin_amdgcn_readlane(main_end, 63) * n_tiles)) {
+        main = main2;
+        main_end = end2;
+      }
+    }
+  }
   const int U = __builtin_amdgcn_readlane(main_end, 63) * n_tiles;
   const int f0 = (int)((int64_t)U * xcd / 8), f1 = (int)((int64_t)U * (xcd + 1) / 8), n_units = f1 - f0;
   const int rest = n_units % wgs;
@@ -457,17 +467,17 @@ grouped_mfma_reg_kernel(RegArgs args) {
 
 // `tile_rows`: most token rows of a unit.
 template <typename T, int WF, int MODE, int MT>
-static int launch_reg_m(const GemmParams& p, int tile_rows, hipStream_t st) {
+static int launch_reg_m(const GemmParams& p, int tile_rows, int fewer_rows, hipStream_t st) {
   constexpr size_t lds_bytes = (size_t)reg_stages(MT) * 16 * MT * 512;
   static std::atomic<uint64_t> lds_ready{0};
   auto kern = grouped_mfma_reg_kernel<T, WF, MODE, MT>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kern), lds_bytes, lds_ready, "mfma reg kernel")) return rc;
   const int n_tiles = (int)(MODE == MODE_GATEUP ? p.n_out / 128 : p.n_out / 256);
-  kern<<<dim3(256), 512, lds_bytes, st>>>(RegArgs{p, n_tiles, 32, tile_rows});
+  kern<<<dim3(8 * kRegWgsPerXcd), 512, lds_bytes, st>>>(RegArgs{p, n_tiles, kRegWgsPerXcd, tile_rows, fewer_rows});
   return check_launch("grouped_mfma_reg");
 }
-template <int MT> static int launch_reg_mt(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, hipStream_t st) {
-#define STMOE_REG(T, WF) (mode == MODE_GATEUP ? launch_reg_m<T, WF, MODE_GATEUP, MT>(p, tile_rows, st) : launch_reg_m<T, WF, MODE_DOWN, MT>(p, tile_rows, st))
+template <int MT> static int launch_reg_mt(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, int fewer_rows, hipStream_t st) {
+#define STMOE_REG(T, WF) (mode == MODE_GATEUP ? launch_reg_m<T, WF, MODE_GATEUP, MT>(p, tile_rows, fewer_rows, st) : launch_reg_m<T, WF, MODE_DOWN, MT>(p, tile_rows, fewer_rows, st))
   if (act_dtype == STMOE_F16) {
     if (wtag == WF_Q8_0_P) return STMOE_REG(f16_t, WF_Q8_0_P);
     if (wtag == WF_Q4_1_P) return STMOE_REG(f16_t, WF_Q4_1_P);

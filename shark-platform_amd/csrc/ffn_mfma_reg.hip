@@ -13,14 +13,14 @@ bool reg_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t m
   const int64_t src_rows = p.perm ? (max_rows + p.k_top - 1) / p.k_top : max_rows;
   return src_rows * p.lda * 2 < (int64_t)1 << 32;
 }
-int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, int tile_rows, hipStream_t st) {
+int launch_mfma_reg(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, int tile_rows, int fewer_rows, hipStream_t st) {
   if (max_rows == 0) return STMOE_OK;
   if (!reg_takes(act_dtype, wtag, mode, p, max_rows))
     return set_error(STMOE_ERR_UNSUPPORTED, "mfma reg kernel: needs packed weights, 16-bit activations, at most 64 experts, K %% 256 == 0 and output features in whole tiles");
   if (tile_rows < 1 || tile_rows > kRegWideRows)
     return set_error(STMOE_ERR_SHAPE, "mfma reg kernel: units of %d token rows", tile_rows);
-  if (tile_rows > kRegUnitRows) return launch_reg_wide(act_dtype, wtag, mode, p, tile_rows, st);
-  return launch_reg_mt<kRegUnitRows / 16>(act_dtype, wtag, mode, p, tile_rows, st);
+  if (tile_rows > kRegUnitRows) return launch_reg_wide(act_dtype, wtag, mode, p, tile_rows, fewer_rows, st);
+  return launch_reg_mt<kRegUnitRows / 16>(act_dtype, wtag, mode, p, tile_rows, 0, st);
 }
 
 }  // namespace stmoe

@@ -3,8 +3,8 @@
 
 namespace stmoe {
 
-int launch_reg_wide(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, hipStream_t st) {
-  return launch_reg_mt<kRegWideRows / 16>(act_dtype, wtag, mode, p, tile_rows, st);
+int launch_reg_wide(int act_dtype, int wtag, int mode, const GemmParams& p, int tile_rows, int fewer_rows, hipStream_t st) {
+  return launch_reg_mt<kRegWideRows / 16>(act_dtype, wtag, mode, p, tile_rows, fewer_rows, st);
 }
 
 }  // namespace stmoe

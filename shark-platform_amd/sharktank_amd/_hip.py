@@ -115,6 +115,7 @@ SIGNATURES = {
                                          c_void_p, c_void_p, c_int, c_void_p]),
     "stmoe_mmt_workspace_bytes": (c_size_t, [c_int64]),
     "stmoe_mmt": (c_int, [c_void_p, c_int, c_int64, POINTER(StmoeWeight), c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p]),
+    "stmoe_register_unit_rows": (c_int, [c_int, POINTER(StmoeWeight), c_int, c_int64, c_int, POINTER(c_int64), c_int]),
     "stmoe_probe_mfma": (c_int, [c_int, c_int, c_int, c_void_p, POINTER(ctypes.c_double), c_void_p]),
 }
 STATIC_SCRATCH_BYTES = 17 << 20  # STMOE_STATIC_SCRATCH_BYTES

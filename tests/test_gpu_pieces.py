@@ -689,6 +689,25 @@ def test_wide_register_kernel(device, fmt, dtype, N, K, act):
     assert torch.equal(wide.view(torch.int16), narrow.view(torch.int16))
 
 
+@pytest.mark.parametrize("fmt", ["q8_0", "q4_1", "fp8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("counts", [
+    [65, 65, 65, 65, 64, 64, 64, 64], [129, 129, 129, 49, 40, 20, 10, 10], [97, 97, 97, 97, 97, 10, 10, 11], [172, 172, 172, 0, 0, 0, 0, 0],
+    [1, 1, 1, 1, 1, 1, 255, 255]])
+def test_wide_register_kernel_picks_its_units(device, fmt, dtype, counts):
+    """A launch chosen for units of up to 96 rows whose kernel picks between 96 and 64 from the experts' rows: both ways, with units of one
+    row and with experts without rows, every output the bits of units of 64 rows, which add in the same order."""
+    hip = _hip()
+    gen = torch.Generator(device=device).manual_seed(95)
+    E, T, K, N = 8, 129, 2048, 2048
+    w = _random_weight(fmt, [E, N, K], gen, device)
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(516, generator=torch.Generator().manual_seed(96))]
+    _, offsets, perm, _ = hip.dispatch_build(idx.to(torch.int32).reshape(T, 4).to(device), E)
+    a = torch.randn(T, K, generator=gen, device=device).to(dtype)
+    auto, narrow = (hip.grouped_gate_up(a, w, w, hip.ACT_SILU, offsets, perm, 4, variant=v).view(torch.int16) for v in (hip.VARIANT_AUTO, hip.VARIANT_MFMA_REG))
+    assert torch.equal(auto, narrow)
+
+
 @pytest.mark.parametrize("mode,fmt,dtype,E,k,T,kred,n_out,choice", [
     ("gate_up", "q4_1", torch.bfloat16, 8, 2, 260, 1024, 4096, "reg"),   # 65 rows per expert, one round of whole units
     ("gate_up", "q4_1", torch.bfloat16, 8, 2, 330, 1024, 4096, "ws"),    # 82: some expert has more than 96
