@@ -268,6 +268,10 @@ static int run_projection(int variant, int dtype, int wtag, int mode, const Gemm
     const int rc = launch_skinny(dtype, wtag, mode, p, max_rows, st);
     return rc != STMOE_ERR_UNSUPPORTED ? rc : set_error(STMOE_ERR_UNSUPPORTED, "grouped_ffn: no streaming kernel for a launch that builds its own dispatch");
   }
+  // An empty reduction, with the variants that the rest of this function takes (gate/up has elements to reduce: grouped_ffn_impl).
+  if (p.kred <= 0 && mode == MODE_DOWN && variant >= 0 && variant <= 13 && variant != 5 && variant != 7 && variant != 8 &&
+      (variant != 10 || dtype == STMOE_F32) && (variant != 1 || max_rows <= 65535))
+    return launch_empty_reduction(dtype, p, max_rows, st);
   int tile_rows = 0;  // of the register kernel
   if (variant == 0) {
     if (dtype == STMOE_F32) variant = 10;

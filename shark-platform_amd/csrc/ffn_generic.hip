@@ -106,6 +106,24 @@ static int launch_generic_t(int wtag, int mode, const GemmParams& p, int64_t max
   }
 }
 
+// A reduction of no elements: zeros, without a look at operands that have none.  (The kernels request a first chunk before they know that there
+// is one, or clamp past the last one.)
+template <typename U>
+__global__ void __launch_bounds__(256) empty_reduction_kernel(GemmParams p, int64_t max_rows) {
+  const int64_t rows = min(p.offsets ? (int64_t)p.offsets[p.E] : p.fixed_rows, max_rows);
+  for (int64_t i = blockIdx.x; i < rows; i += gridDim.x) {
+    U* o = reinterpret_cast<U*>(p.out) + out_row(p, (int)i) * p.ldo;
+    for (int64_t n = threadIdx.x; n < p.n_out; n += 256) o[n] = 0;
+  }
+}
+int launch_empty_reduction(int act_dtype, const GemmParams& p, int64_t max_rows, hipStream_t st) {
+  if (max_rows == 0 || p.n_out <= 0) return STMOE_OK;
+  const dim3 grid((unsigned)(max_rows < 4096 ? max_rows : 4096));
+  if (act_dtype == STMOE_F32) empty_reduction_kernel<uint32_t><<<grid, 256, 0, st>>>(p, max_rows);
+  else empty_reduction_kernel<uint16_t><<<grid, 256, 0, st>>>(p, max_rows);
+  return check_launch("empty_reduction");
+}
+
 int launch_generic(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   if (max_rows > 65535) return set_error(STMOE_ERR_UNSUPPORTED, "generic kernel: %lld rows exceed its 65535-row grid", (long long)max_rows);
   switch (act_dtype) {

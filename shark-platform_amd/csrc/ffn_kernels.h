@@ -164,6 +164,7 @@ namespace stmoe {
 // Launchers (one per kernel family).  `act_dtype` is the activation dtype enum, `wtag` a WF_* tag,
 // `max_rows` an upper bound of the sorted row count known on the host (T*k).  Each returns
 // STMOE_ERR_UNSUPPORTED when the family has no instantiation for the combination.
+int launch_empty_reduction(int act_dtype, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_generic(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 int launch_f32(int wtag, int mode, const GemmParams& p, int64_t max_rows, hipStream_t st);
 bool dense_takes(int act_dtype, int wtag, int mode, const GemmParams& p, int64_t max_rows);

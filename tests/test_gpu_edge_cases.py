@@ -517,3 +517,34 @@ def test_fp32_kernel_reduction_and_row_edges(device, fmt, K):
         inf = want.isinf()
         assert torch.equal(got[a:b][inf], want[inf].float())
         assert bool(((got[a:b] - want).abs()[~inf] <= K * 2.0 ** -24 * size[~inf]).all()), e
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("fmt", ["W_DENSE", "W_Q8_0", "W_Q4_1", "W_FP8", "W_Q8_0_PACKED", "W_Q4_1_PACKED", "W_FP8_PACKED"])
+def test_empty_reduction_is_zero(device, dtype, fmt):
+    """Weights of no columns: every output is zero, whichever kernel is asked for, and nothing is read from planes that have no element."""
+    import ctypes
+
+    from sharktank_amd import _hip as hip
+
+    lib, E, rows, T, k = hip.load_library(), 3, 48, 70000, 1
+    plane = torch.zeros(64, dtype=torch.uint8, device=device)
+    desc = lambda e: ctypes.byref(hip.StmoeWeight(  # noqa: E731
+        format=getattr(hip, fmt), dtype=hip.dtype_enum(dtype) if fmt == "W_DENSE" else hip.F32 if "FP8" in fmt else 0, experts=e, rows=rows, cols=0,
+        qs=plane.data_ptr(), d=plane.data_ptr(), m=plane.data_ptr() if "Q4" in fmt else None, d_count=1))
+    stream = torch.cuda.current_stream().cuda_stream
+    offsets = torch.tensor([0, 5, 5, T * k], dtype=torch.int32, device=device)
+    perm = torch.randperm(T * k, device=device).to(torch.int32)
+    for variant in [0, 1, 2, 3, 4, 6, 9, 11, 12, 13] + [10] * (dtype == torch.float32):
+        out = torch.full((T * k, rows), float("nan"), dtype=dtype, device=device)
+        assert lib.stmoe_mmt(plane.data_ptr(), hip.dtype_enum(dtype), 33, desc(1), out.data_ptr(), None, 0, 0, variant, stream) == 0
+        assert bool((out[:33] == 0).all()) and bool(out[33:].isnan().all())
+        rc = lib.stmoe_grouped_mmt(plane.data_ptr(), hip.dtype_enum(dtype), T, k, 0, desc(E), offsets.data_ptr(), perm.data_ptr(), out.data_ptr(),
+                                   variant, stream)
+        if variant == 1:  # (the general kernel takes 65535 rows)
+            assert rc != 0
+        else:
+            assert rc == 0 and bool((out == 0).all())
+    out = torch.empty(1, rows, dtype=dtype, device=device)
+    for variant in [-1, 5, 7, 8, 14] + [10] * (dtype != torch.float32):
+        assert lib.stmoe_mmt(plane.data_ptr(), hip.dtype_enum(dtype), 1, desc(1), out.data_ptr(), None, 0, 0, variant, stream) != 0
