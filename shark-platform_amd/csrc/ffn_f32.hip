@@ -7,12 +7,16 @@
 // 32 features where they divide), its four wavefronts a quarter of the reduction each: a layer of 8 x 1024 x 512 has 512 such
 // items, 2048 wavefronts, whose loads are all in flight after two steps.  The quarters are added through LDS in a fixed order.
 // Order of the loads: they return in the order of their issue, so the tokens of an item's rows are requested first, then its weights, then
-// the token rows; two chunks of both are in flight, every load unconditional (a row's ragged end re-reads its last piece and drops it in
-// registers: an instance of its own, TAIL).  With one chunk ahead, each load under its own condition, and the wavefront's number in a vector
+// the token rows; two chunks of both are in flight up to 32 rows, of the weights alone from 33 rows on, every load unconditional (a row's
+// ragged end re-reads its last piece and drops it in registers: an instance of its own, TAIL).  With one chunk ahead, each load under its own condition, and the wavefront's number in a vector
 // register, every wait was for all loads in flight: 64 tokens of 512 x 1024 16.3 + 11.7 us; now 14.0 + 9.2.  Layer (8 experts, top-2, us,
 // before / now): 64 tokens of 512 x 1024 37.6 / 31.4, 109 tokens of 896 x 1280 77 / 69, 128 tokens of 1024 x
 // 1536 88 / 76; Q8_0 weights of 1024 x 1024, 2000 tokens 435 / 349; one Q8_0 matrix of [2048, 2048], 60 rows 28.7 / 20.0.  (On the general
 // kernel the first took 110.)  Weights requested in front of the tokens: 34.3.
+// Registers: all 256 are in use, and a register in scratch memory comes back through the same in-order path as the loads ahead of it.  So
+// a weight row is converted and multiplied with all token rows before the next one is (with both in any order ten of 54 instances
+// kept 12 to 44 bytes a lane in scratch memory: 3000 launches of 1 to 16 experts, 256 to 2048 x 128 to 2048, 1 to 100 rows per expert, plain
+// and quantized weights, take 0.872 of the time of the first order of loads with it and 0.843 without, slower by more than 3 % 1.8 and 0.3 %).
 // Order of the sums: the matrix instruction rounds after every product, so one running sum per quarter was up to 3.6 times as far
 // from fp64 as the general kernel, whose 64 lanes hold short sums (K = 4096: rms error 9.6 / 2.7 times 2^-24 of the result's rms;
 // K = 512: 3.5 / 1.6).  A chunk of 64 elements is eight sums of 8 products, added in pairs: 1.9 and 1.4, below the general kernel at
@@ -84,6 +88,8 @@ template <int WF, int MODE, int NT, bool TAIL, int MT>
 __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, F32Quarter<WF, MODE, NT, TAIL>& quarter, int tile, int r0, int re, int lane, int wave,
                                          floatx4_t (*red)[64]) {
   constexpr bool ROWC = F32Weight<WF, TAIL>::kRowContiguous;
+  // (plain fp32 weights: the lane's addresses are computed in each pass; kept for all three, seven registers went to scratch memory)
+  if (ROWC) asm volatile("" : "+v"(lane));
   const int g = lane >> 4, n_in = lane & 15;
   const int c_begin = quarter.begin, c_end = quarter.end;
   const float* xrow[MT];
@@ -129,13 +135,12 @@ __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, F32Quarter<
         for (int i = 0; i < 4; ++i)
           if ((ROWC ? i : g) >= blocks) x[mt][i] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
     }
-    float v[NT][16];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) w[t].values(v[t]);
     // A chunk's sixteen instructions are eight chains of two, which start at zero and are added in pairs; the chunk's sum then
     // goes to the running one.
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < NT; ++t) {
+      float v[16];
+      w[t].values(v);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         floatx4_t half[2];
@@ -143,15 +148,17 @@ __device__ __forceinline__ void f32_pass(const GemmParams& p, int e, F32Quarter<
         for (int h = 0; h < 2; ++h) {
           floatx4_t c[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][8 * h + 2 * i], x[mt][2 * h + (i >> 1)][(2 * i) & 3], (floatx4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[8 * h + 2 * i], x[mt][2 * h + (i >> 1)][(2 * i) & 3], (floatx4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][8 * h + 2 * i + 1], x[mt][2 * h + (i >> 1)][(2 * i + 1) & 3], c[i], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) c[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[8 * h + 2 * i + 1], x[mt][2 * h + (i >> 1)][(2 * i + 1) & 3], c[i], 0, 0, 0);
           half[h] = (c[0] + c[1]) + (c[2] + c[3]);
         }
         acc[mt][t] += half[0] + half[1];
         // (finished here: sunk behind the next chunk's loads, the adds would keep the chains of all tiles in registers)
         asm volatile("" : "+v"(acc[mt][t]));
+        if (mt == MT - 1) __builtin_amdgcn_sched_barrier(0);  // (see the head: no register may go to scratch memory)
       }
+    }
   };
   // No request is under a condition of its own: such loads were waited for one by one.
   if (MT > 2 && c_begin < c_end) {

@@ -108,6 +108,11 @@ def test_hand_scheduled_kernels_get_no_scratch_accesses_from_the_compiler():
         assert r["VGPRs Spill"] == "0", (n, r)
         if "grouped_mfma_ws_kernel" in n:
             assert int(r["VGPRs"]) <= 168, (n, r)  # 12 wavefronts per CU
+    # The fp32 kernel keeps two chunks of loads in flight by their order alone; a register in scratch memory would come back behind them.
+    f32 = {n: r for n, r in kernels.items() if "grouped_f32_kernel" in n}
+    assert len(f32) == 9 * 3 * 2, sorted(f32)  # weight formats x (gate/up, down of 32 and of 16 features) x whole or ragged reductions
+    for n, r in f32.items():
+        assert r["ScratchSize [bytes/lane]"] == "0", (n, r)
 
 
 def test_hand_issued_loads_wait_for_their_base(tmp_path):
