@@ -294,9 +294,12 @@ struct SkinnyExperts {
 template <typename T, int WF, int MODE, int MT, int KS, int NT>
 __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExperts& experts, const int64_t (&wrow)[NT], int tile,
                                             int r0, int re, int64_t nch_total, int lane, bool pin_prefetch) {
-  // (a scalar: from a vector register it made the loop's bounds and every prefetch's condition execution masks.  Layers of 8 experts, us: 1 token
-  // of 4096 x 14336, Q4_1 bf16 70.4 -> 69.3, 2 tokens of 4096 x 1024, fp16 48.6 -> 44.5)
-  const int kw = KS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+  // (a scalar: from a vector register it makes the loop's bounds and every prefetch's condition execution masks.  Over 5000 launches of 1 to 8
+  // experts, 1 to 32 rows, time with / without by form and type: Q8_0 and fp8, one token tile 0.91 to 1.0, two 0.95 to 1.01; Q4_1, whose nibbles
+  // take more registers, 0.99 to 1.04 and, with two token tiles of a long reduction, up to 1.09, except the down projection of two weight tiles in
+  // bf16: means of 0.97 to 1.01 by form, one token of 8 experts of 4096 x 14336 69.4 us for the layer instead of 70.0.)
+  constexpr bool SCALAR = !IsQ4<WF>::value || (MODE == MODE_DOWN && NT == 2 && !__is_same(T, f16_t));
+  const int kw = KS > 1 ? (SCALAR ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)(threadIdx.x >> 6)) : 0;
   const int64_t c_begin = KS > 1 ? nch_total * kw / KS : 0;
   const int64_t nch = KS > 1 ? nch_total * (kw + 1) / KS : nch_total;  // end of this wavefront's chunk range
   const int g = lane >> 4, n_in = lane & 15;
