@@ -234,7 +234,10 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
   T* xs = reinterpret_cast<T*>(smem);                                  // [K] the (normalised) token row
   float* lg_s = reinterpret_cast<float*>(smem + ((K * sizeof(T) + 15) / 16) * 16);  // [E] logits, then 8 partials
   float* part = lg_s + 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63;
+  // (a scalar where the first expert's row is prefetched whole or several are in flight: 8 experts, 64 tokens 4.8 -> 4.0 us.  In the other forms it
+  // cost 4 to 8 %: 8 experts of 256 elements, 400 tokens 3.9 -> 4.2 us)
+  const int wave = MANY || PRE == 8 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int64_t t = blockIdx.x;
   const T* xr = x + t * K;
 
@@ -434,8 +437,11 @@ router_wg_kernel(const T* __restrict__ x, const W* __restrict__ norm_w, float ep
     while (c + RING < nch || first + 8 * MANY < E) block(RtInt<1>{});
     block(RtInt<0>{});
   } else {
-    // (several experts per wavefront: fp32 rows, or PRE = 0, which have no chunks of the first one in registers)
-    for (int e = wave; e < E; e += 8) logit(e, wpre);
+    if (E <= 8) {
+      if (wave < E) logit(wave, wpre);
+    } else {  // (several experts per wavefront: fp32 rows, or PRE = 0, which have no chunks of the first one in registers)
+      for (int e = wave; e < E; e += 8) logit(e, wpre);
+    }
   }
   __syncthreads();
   if (wave != 0) return;
@@ -673,12 +679,17 @@ static int launch_router_wg(const void* x, const void* norm_w, float eps, void* 
     router_wg_kernel<T, W, FUSE_NORM, decltype(pre_tag)::value, decltype(many_tag)::value><<<dim3((unsigned)T_tokens), 512, lds, st>>>(
         (const T*)x, (const W*)norm_w, eps, (T*)xn, (const T*)wr, K, E, k, (T*)logits, idx, idx64, (T*)gate, disp, x_fq);
   };
-  // More than 8 experts, 16-bit rows: several of a wavefront's experts side by side (us, one by one / side by side, norm included, 1, 64, 256,
+  // More than 8 experts, 16-bit rows: several of a wavefront's experts side by side, in groups whose last one has few places without an expert
+  // (a place without one reads and sums like the others.  One by one / groups of four / these, without the norm, us: 48 experts of 1024 elements,
+  // bf16, 400 and 600 tokens 9.0, 12.3 / 9.5, 15.4 / 8.4, 9.7; 33 experts of 4096, 400 tokens 11.4 / 15.4 / 11.5; 24 experts of 2048, 600 tokens
+  // 9.8 / 10.8 / 7.4; groups of five from 513 tokens on 0 to 25 % slower than of three).  (Us, one by one / side by side, norm included, 1, 64, 256,
   // 400 and 2000 tokens of 2048 elements: 64 experts bf16 13.9, 15.2, 12.7, 15.6, 52.5 / 8.8, 11.3, 11.1, 14.4, 44.1; 32 experts fp16 10.7,
   // 11.3, 9.4, 12.3, 34.4 / 6.0, 6.8, 7.4, 10.2, 26.6; 12 experts bf16 7.0, 8.7, 6.6, 8.1 / 4.4, 5.6, 6.2, 7.7).  Up to 16 experts, launches
   // of more than 512 tokens that the wavefront-per-token kernel leaves here keep the form with most workgroups per CU.
   constexpr bool HALF = sizeof(T) == 2;
-  if (HALF && E > 16) launch(RtInt<0>{}, RtInt<HALF ? 4 : 0>{});
+  if (HALF && E > 32 && E <= 40 && T_tokens <= 512) launch(RtInt<0>{}, RtInt<HALF ? 5 : 0>{});
+  else if (HALF && E > 16 && (E <= 24 || (E > 32 && E <= 48))) launch(RtInt<0>{}, RtInt<HALF ? 3 : 0>{});
+  else if (HALF && E > 16) launch(RtInt<0>{}, RtInt<HALF ? 4 : 0>{});
   else if (HALF && E > 8 && T_tokens <= 512) launch(RtInt<0>{}, RtInt<HALF ? 2 : 0>{});
   else if (T_tokens <= 64) launch(RtInt<8>{}, RtInt<0>{});
   else if (T_tokens <= 512) launch(RtInt<4>{}, RtInt<0>{});

@@ -135,11 +135,11 @@ def test_router_bit_exact(device, dtype, T, K, E, k):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K", [8, 504, 2048, 2056, 4096 + 512])  # part of a chunk, four chunks and one more, several blocks of four
-@pytest.mark.parametrize("E", [9, 16, 17, 32, 33, 64])
-def test_router_experts_side_by_side(device, dtype, K, E):
+@pytest.mark.parametrize("T,E", [*((5, E) for E in (9, 16, 17, 24, 25, 32, 33, 40, 41, 48, 49, 64)), (513, 33), (513, 40)])
+def test_router_experts_side_by_side(device, dtype, K, T, E):
     """Several experts of a wavefront side by side: every logit keeps the bits of the documented order."""
     g = torch.Generator().manual_seed(K + E)
-    x, wr = torch.randn(5, K, generator=g).to(dtype), torch.randn(E, K, generator=g) * 0.02
+    x, wr = torch.randn(T, K, generator=g).to(dtype), torch.randn(E, K, generator=g) * 0.02
     idx, _, logits = _hip().router_topk(x.to(device), wr.to(dtype).to(device), 4, want_logits=True)
     want = O.router_logits_ordered(x, wr)
     assert torch.equal(logits.cpu().view(torch.int16), want.view(torch.int16))
