@@ -246,8 +246,10 @@ __global__ void __launch_bounds__(256, 2) grouped_f32_kernel(GemmParams p) {
   quarter.begin = nch * wave / 4;
   quarter.end = nch * (wave + 1) / 4;
 #pragma unroll
-  for (int t = 0; t < NT; ++t)  // features past the end re-read the last one (never stored)
-    quarter.wrow[t] = min((int64_t)tile * (MODE == MODE_GATEUP ? 16 : 16 * NT) + (MODE == MODE_GATEUP ? 0 : 16 * t) + (lane & 15), p.n_out - 1);
+  for (int t = 0; t < NT; ++t)
+    // Features past the end re-read the last one (never stored).  A quarter without a chunk (fewer than 256 elements) requests one all the
+    // same, and all its lanes the same row's: down projection of 64 elements, 87 tokens of 6 of 56 experts, 4064 features 67 -> 43 us.
+    quarter.wrow[t] = min((int64_t)tile * (MODE == MODE_GATEUP ? 16 : 16 * NT) + (MODE == MODE_GATEUP ? 0 : 16 * t) + (quarter.begin < quarter.end ? lane & 15 : 0), p.n_out - 1);
   int rb, re;
   expert_range(p, e, rb, re);
   for (int r0 = rb + 64 * (int)blockIdx.z; r0 < re; r0 += 64 * (int)gridDim.z) {
