@@ -226,7 +226,10 @@ static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, 
 // 80 / 63; 79 / 58; 78 / 57, 384 rows 84 / 70; 83 / 69; 80 / 66, [4096, 4096] 768 rows 40 / 38; 41 / 37; 38 / 34), and then, as many of them as fit one
 // round, while they have more than 64 rows ([14336, 4096] 300 rows in four tiles of 75 61 / 54; 61 / 48; 51 / 45, 384 rows 61 / 60; 62 / 56;
 // 54 / 52, [6144, 3072] 768 rows 51 / 44; 58 / 40; 56 / 38, [16384, 2048] 300 rows 34 / 33; 36 / 31; 32 / 30; with tiles of 50 to 64 rows the narrow tiles
-// are as fast or faster).  Not for longer reductions, which the prefill kernel cuts ([4096, 14336] 768 rows 114 / 123; 107 / 113; 106 / 107).
+// are as fast or faster).  Not for longer reductions, which the prefill kernel cuts ([4096, 14336] 768 rows 114 / 123; 107 / 113; 106 / 107), in
+// Q8_0 bf16, which converts slowest, from 6145 elements on ([13568, 7680] 272 rows 83 / 92; 93 such launches 0.96 of the time, 17 % of them
+// slower by more than 3 %).  Over 4000 matrices and gate/up pairs of 65 to 2000 rows, 1024 to 10240 x 1024 to 16384, the launches that tiles
+// of more than 64 rows take need 0.83 of the time, 0.4 % are slower by more than 3 % (worst 1.09, tiles of a few rows more than 64 or 80).
 static int reg_rows(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   if (!reg_takes(dtype, wtag, mode, p, rows)) return 0;
   if (p.E > 1) return p.offsets ? reg_rows_grouped(dtype, wtag, mode, p, rows) : 0;
@@ -239,7 +242,7 @@ static int reg_rows(int dtype, int wtag, int mode, const GemmParams& p, int64_t 
   if (rows <= 64 || (rows > 128 ? p.kred <= 2048 || p.kred > 8192 : p.kred > 4096)) return 0;
   const int64_t wide = (rows + kRegWideRows - 1) / kRegWideRows;
   if (wide * tiles <= 128) return (int)((rows + wide - 1) / wide);
-  if (wide * tiles > 256) return 0;
+  if (wide * tiles > 256 || (wtag == WF_Q8_0_P && dtype == STMOE_BF16 && p.kred > 6144)) return 0;
   const int64_t spread = (rows + 256 / tiles - 1) / (256 / tiles);
   return spread > kRegUnitRows ? (int)spread : 0;
 }

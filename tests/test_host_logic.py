@@ -270,3 +270,49 @@ def test_nearly_full_rounds_of_wide_units(E, k, T, n_out, rows):
 def test_one_unit_per_expert_up_to_56_rows():
     """226 pairs on 4 experts, 136 units: a seventh more than the average is 64.57 rows, which counts as one unit of 64."""
     assert _unit_rows("fp8", torch.float16, True, 4, 2, 113, 2048, 4352) == 64
+
+
+@pytest.mark.parametrize("fmt,dtype,gate_up,T,kred,n_out,rows", [
+    ("q8_0", torch.float16, False, 160, 4096, 14336, 80),    # 168 units of 64 rows; 112 of 80 run as halves
+    ("q8_0", torch.float16, False, 300, 4096, 14336, 75),    # 280; 224 of 75 fit one round
+    ("q8_0", torch.float16, False, 256, 4096, 14336, 0),     # 224 of 64
+    ("q8_0", torch.float16, False, 385, 4096, 14336, 0),     # 280 of 96
+    ("q8_0", torch.float16, False, 100, 4096, 14336, 64),    # 112 of 64
+    ("q4_1", torch.bfloat16, True, 130, 4096, 8192, 65),     # gate/up: 192 of 64; 128 of 65
+    ("q8_0", torch.float16, False, 272, 8192, 13568, 68),
+    ("q8_0", torch.float16, False, 272, 8448, 13568, 0),     # reductions that the prefill kernel cuts
+    ("q8_0", torch.bfloat16, False, 272, 6144, 13568, 68),
+    ("q8_0", torch.bfloat16, False, 272, 6400, 13568, 0),    # ... from shorter ones on where the conversion is slowest
+    ("q4_1", torch.bfloat16, False, 272, 8192, 13568, 68),
+    ("q8_0", torch.bfloat16, False, 160, 8192, 14336, 80),   # (halves: all formats)
+    ("q8_0", torch.float16, False, 160, 2048, 14336, 0),     # from 129 rows on, more than 2048 elements
+    ("q8_0", torch.float16, False, 128, 2048, 14336, 64),
+])
+def test_units_of_a_single_matrix(fmt, dtype, gate_up, T, kred, n_out, rows):
+    """One matrix on both sides of the lines around tiles of 64 and of up to 96 rows: as few tiles as run as halves, or as many as fit one round."""
+    assert _unit_rows(fmt, dtype, gate_up, 1, 1, T, kred, n_out) == rows
+
+
+@pytest.mark.parametrize("fmt,dtype,gate_up,E,k,T,kred,n_out,scratch,rows", [
+    ("q4_1", torch.bfloat16, True, 8, 2, 208, 1024, 8192, True, 64),    # 52 rows per expert
+    ("q4_1", torch.bfloat16, True, 8, 2, 212, 1024, 8192, True, 96),    # 53: some expert has more than 64
+    ("q4_1", torch.bfloat16, True, 8, 2, 288, 1024, 8192, True, 96),    # 72 ...
+    ("q4_1", torch.bfloat16, True, 8, 2, 292, 1024, 8192, True, 0),
+    ("q4_1", torch.bfloat16, True, 8, 2, 320, 2048, 8192, True, 96),    # ... and 80 with 2048 elements
+    ("q4_1", torch.bfloat16, True, 8, 2, 324, 2048, 8192, True, 0),
+    ("q8_0", torch.float16, True, 8, 2, 240, 1792, 4096, True, 0),      # a short reduction of a format that converts fast
+    ("q8_0", torch.float16, True, 8, 2, 240, 2048, 4096, True, 96),
+    ("q8_0", torch.float16, False, 8, 2, 560, 3072, 3072, True, 96),    # two tiles of 140 rows: 192 units
+    ("q8_0", torch.float16, False, 8, 2, 560, 9216, 2304, True, 0),     # 144 leave CUs idle
+    ("fp8", torch.bfloat16, False, 8, 2, 560, 3072, 2048, True, 96),    # 128 run as halves
+    ("q8_0", torch.bfloat16, True, 33, 2, 396, 2048, 1024, True, 64),   # several rounds: 24 rows per expert with up to 2048 elements
+    ("q8_0", torch.bfloat16, True, 33, 2, 397, 2048, 1024, True, 0),
+    ("q8_0", torch.bfloat16, True, 33, 2, 397, 2304, 1024, True, 64),
+    ("fp8", torch.bfloat16, False, 4, 2, 67, 8448, 1024, True, 0),      # units for a quarter of the CUs, a reduction that can be cut
+    ("fp8", torch.bfloat16, False, 4, 2, 67, 8448, 1024, False, 64),    # ... where there is scratch
+    ("q4_1", torch.bfloat16, False, 8, 2, 16, 3072, 4096, True, 64),    # streamed launches
+    ("q8_0", torch.float16, True, 8, 2, 16, 4096, 14336, True, 0),
+])
+def test_units_of_grouped_launches(fmt, dtype, gate_up, E, k, T, kred, n_out, scratch, rows):
+    """Several experts on both sides of the lines."""
+    assert _unit_rows(fmt, dtype, gate_up, E, k, T, kred, n_out, scratch=scratch) == rows
