@@ -291,14 +291,14 @@ struct SkinnyExperts {
 // One pass of one work item: rows [r0, min(r0 + 16*MT, re)) of expert rows against the item's two weight tiles.
 // KS > 1: the KS wavefronts of a workgroup share the item, each takes a contiguous 1/KS of the chunks, and the partial
 // sums are added through LDS in a fixed order ((w0 + w1) + (w2 + w3)) by wavefront 0, which then writes the result.
-template <typename T, int WF, int MODE, int MT, int KS, int NT>
+// SCALAR: the wavefront's number in a scalar register.  From a vector register it makes the loop's bounds and every prefetch's condition execution
+// masks.  Over 5000 launches of 1 to 8 experts, 1 to 32 rows, time with / without, mean by form and type: Q8_0 and fp8, one token tile 0.91 to
+// 1.0, two 0.95 to 1.01; Q4_1, whose nibbles take more registers, 0.99 to 1.04 and, with two token tiles of a long reduction, up to 1.09
+// (plane order, 16 features: 1.16), except down projections of two weight tiles and one token tile in bf16: 0.97 and 1.0, one token of 8 experts of
+// 4096 x 14336 69.0 us for the layer instead of 70.0.
+template <typename T, int WF, int MODE, int MT, int KS, int NT, bool SCALAR>
 __device__ __forceinline__ void skinny_pass(const GemmParams& p, const SkinnyExperts& experts, const int64_t (&wrow)[NT], int tile,
                                             int r0, int re, int64_t nch_total, int lane, bool pin_prefetch) {
-  // (a scalar: from a vector register it makes the loop's bounds and every prefetch's condition execution masks.  Over 5000 launches of 1 to 8
-  // experts, 1 to 32 rows, time with / without by form and type: Q8_0 and fp8, one token tile 0.91 to 1.0, two 0.95 to 1.01; Q4_1, whose nibbles
-  // take more registers, 0.99 to 1.04 and, with two token tiles of a long reduction, up to 1.09, except the down projection of two weight tiles in
-  // bf16: means of 0.97 to 1.01 by form, one token of 8 experts of 4096 x 14336 69.4 us for the layer instead of 70.0.)
-  constexpr bool SCALAR = !IsQ4<WF>::value || (MODE == MODE_DOWN && NT == 2 && !__is_same(T, f16_t));
   const int kw = KS > 1 ? (SCALAR ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)(threadIdx.x >> 6)) : 0;
   const int64_t c_begin = KS > 1 ? nch_total * kw / KS : 0;
   const int64_t nch = KS > 1 ? nch_total * (kw + 1) / KS : nch_total;  // end of this wavefront's chunk range
@@ -458,7 +458,7 @@ template <int WF> struct SkinnyOcc { static constexpr int value = 2; };
 // KS == 1: `total_workers` wavefronts, one item each at a time.  KS > 1: `total_workers` workgroups, the KS
 // wavefronts of a workgroup split the reduction of one item (for launches with too few items to fill the chip).
 // NT: weight tiles of an item (GATEUP 2: gate and up of 16 features; DOWN 2 or 1 of 16 features each).
-template <typename T, int WF, int MODE, int KS, int NT>
+template <typename T, int WF, int MODE, int KS, int NT, bool SCALAR = !IsQ4<WF>::value>
 __global__ void __launch_bounds__(256, SkinnyOcc<WF>::value)
 grouped_skinny_kernel(GemmParams p, int tiles_per_expert, int total_waves, bool pin_prefetch) {
   static_assert(MODE == MODE_DOWN || NT == 2, "gate and up");
@@ -486,9 +486,9 @@ grouped_skinny_kernel(GemmParams p, int tiles_per_expert, int total_waves, bool 
     }
     // up to 16 rows: one 16-row token tile; otherwise passes of two tiles (one pass up to 32 rows)
     if (re - rb <= 16) {
-      skinny_pass<T, WF, MODE, 1, KS, NT>(p, experts, wrow, tile, rb, re, nch, lane, pin_prefetch);
+      skinny_pass<T, WF, MODE, 1, KS, NT, SCALAR>(p, experts, wrow, tile, rb, re, nch, lane, pin_prefetch);
     } else {
-      for (int r0 = rb; r0 < re; r0 += 32) skinny_pass<T, WF, MODE, 2, KS, NT>(p, experts, wrow, tile, r0, re, nch, lane, false);
+      for (int r0 = rb; r0 < re; r0 += 32) skinny_pass<T, WF, MODE, 2, KS, NT, SCALAR>(p, experts, wrow, tile, r0, re, nch, lane, false);
     }
   }
 }
@@ -695,7 +695,15 @@ static int launch_skinny_t(int mode, const GemmParams& p, int64_t max_rows, hipS
     if (mode == MODE_GATEUP) grouped_skinny_kernel<T, WF, MODE_GATEUP, 4, 2><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
     else if (items_bound <= 128)
       grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 1><<<dim3((unsigned)items_bound * 2), 256, 0, st>>>(p, tiles * 2, (int)items_bound * 2, pin);
-    else grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 2><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
+    else {
+      if constexpr (IsQ4<WF>::value && !__is_same(T, f16_t)) {
+        if (rows_bound <= 16) {  // (see skinny_pass)
+          grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 2, true><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
+          return check_launch("grouped_skinny(split)");
+        }
+      }
+      grouped_skinny_kernel<T, WF, MODE_DOWN, 4, 2><<<grid, 256, 0, st>>>(p, tiles, (int)items_bound, pin);
+    }
     return check_launch("grouped_skinny(split)");
   }
   // gate/up launches of up to 1024 items and one token tile per expert: a wavefront per item (one round)

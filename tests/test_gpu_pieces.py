@@ -754,6 +754,26 @@ def test_register_kernel_spreads_the_rows_of_a_single_matrix(device, fmt, dtype,
     assert torch.equal(auto, reg) and not torch.equal(auto, ws)
 
 
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(1024, 4128), (2304, 6144)])  # 129 and 192 items of 32 features, four and nine chunks for four wavefronts
+def test_streaming_kernel_shared_reductions_of_q4_1(device, packed, dtype, rows, K, N):
+    """A down projection whose items four wavefronts share, on both sides of one token tile (in bf16 an instance of its own), against fp64 over the
+    weights as the kernel rounds them: a sum of K products in fp32 and one rounding to the output type."""
+    hip = _hip()
+    from sharktank_amd.ops import device_weight
+
+    case = MC.build(MC.Case(T=4, K=K, N=N, E=1, k=1, fmt="q4_1", dtype=dtype, seed=K + rows))
+    dw = device_weight(MC.to_inference_tensor("q4_1", case.planes["gate"], [1, N, K], "gate", device), stacked=True, prepack=packed)
+    assert dw.is_packed == packed
+    x = torch.randn(rows, K, generator=torch.Generator().manual_seed(rows)).to(dtype)
+    got = hip.mmt(x.to(device), dw, variant=hip.VARIANT_SKINNY).cpu().double()
+    w = MC.dense_weights(case)[0][0].to(dtype).double()
+    want, size = x.double() @ w.T, x.double().abs() @ w.abs().T
+    assert bool(((got - want).abs() <= K * 2.0 ** -24 * size + 2.0 ** (-11 if dtype == torch.float16 else -8) * want.abs() + 2.0 ** -24).all())
+
+
 def _random_weight(fmt, shape, gen, device):
     """A packed weight of random planes, made on the device (no reference for it: for launches that are compared with each other)."""
     from sharktank_amd import types as ST
