@@ -143,3 +143,15 @@ def oracle_block(case: Case, formulation: str = "grouped", ordered_logits: bool 
         case.activation, out_norm_w=case.planes["out_norm"], formulation=formulation, ordered_logits=ordered_logits,
         x_rscale=case.planes["x_rscale"], z_rscale=case.planes["z_rscale"],
     )
+
+
+def unit_rows(fmt, dtype, gate_up, E, k, T, kred, n_out, counts=None, scratch=True):
+    """Most token rows of a unit if the automatic choice sends a projection to the register kernel, 0 if another kernel takes it."""
+    import ctypes
+
+    from sharktank_amd import _hip
+
+    packed = {"q8_0": _hip.W_Q8_0_PACKED, "q4_1": _hip.W_Q4_1_PACKED, "fp8": _hip.W_FP8_PACKED}[fmt]
+    w = _hip.StmoeWeight(format=packed, dtype=_hip.F32 if fmt == "fp8" else 0, experts=E, rows=n_out, cols=kred, d_count=1)
+    c = (ctypes.c_int64 * E)(*counts) if counts else None
+    return _hip.load_library().stmoe_register_unit_rows(_hip.dtype_enum(dtype), ctypes.byref(w), int(gate_up), T, k, c, int(scratch))

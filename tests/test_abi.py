@@ -84,7 +84,7 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
 
 
 def test_hand_scheduled_kernels_get_no_scratch_accesses_from_the_compiler():
-    """The prefill and register kernels issue loads by hand and wait for them with counted `s_waitcnt vmcnt(N)`.  That count only
+    """The prefill and register kernels and the one of unquantized weights issue loads by hand and wait for them with counted `s_waitcnt vmcnt(N)`.  That count only
     holds while the compiler adds no vector-memory instruction of its own to those wavefronts: a register spilled to scratch
     memory would be one (and a spill of a register with a load in flight would read it too early).  The build keeps the
     compiler's per-kernel resource report beside the library; every instance of those kernels must show no scratch and no
@@ -101,8 +101,15 @@ def test_hand_scheduled_kernels_get_no_scratch_accesses_from_the_compiler():
             kernels[name] = {}
         elif name is not None:
             kernels[name][key] = value
-    hand = {n: r for n, r in kernels.items() if any(k in n for k in ("grouped_mfma_ws_kernel", "grouped_mfma_reg_kernel", "grouped_fp8_ws_kernel"))}
-    assert len(hand) >= 2 * 12 + 4, sorted(hand)  # two kernels of 2 dtypes x 3 formats x 2 modes, and the fp8 x fp8 kernel (2 dtypes x 2 modes)
+    instances = {
+        "grouped_mfma_ws_kernel": 2 * 3 * 2,  # types x formats x (gate/up, down)
+        "grouped_mfma_reg_kernel": 2 * 3 * 2 * 2,  # ... x units of up to 64 and of up to 96 rows
+        "grouped_fp8_ws_kernel": 2 * 2,
+        "grouped_dense_kernel": 2 * 2 * 2,  # types x (gate/up, down) x 128 or 256 weight rows
+    }
+    hand = {n: r for n, r in kernels.items() if any(k in n for k in instances)}
+    for kernel, count in instances.items():
+        assert sum(kernel in n for n in hand) == count, (kernel, sorted(hand))
     for n, r in hand.items():
         assert r["ScratchSize [bytes/lane]"] == "0", (n, r)
         assert r["VGPRs Spill"] == "0", (n, r)

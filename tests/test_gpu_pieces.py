@@ -721,7 +721,8 @@ def test_wide_register_kernel_picks_its_units(device, fmt, dtype, counts):
     ("gate_up", "q8_0", torch.float16, 33, 2, 400, 1792, 1024, "ws"),
 ])
 def test_wide_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, E, k, T, kred, n_out, choice):
-    """The automatic choice on both sides of the lines around units of up to 96 rows, told by the bits."""
+    """The automatic choice on both sides of the lines around units of up to 96 rows: the register kernel or the prefill kernel, told by the bits.
+    (Which units the register kernel makes the bits do not tell: test_units_of_grouped_launches.)"""
     hip = _hip()
     gen = torch.Generator(device=device).manual_seed(93)
     idx = torch.stack([torch.arange(k) + t for t in range(T)]).remainder(E).to(torch.int32).to(device)
@@ -744,12 +745,13 @@ def test_wide_register_kernel_is_chosen_where_it_pays(device, mode, fmt, dtype, 
 @pytest.mark.parametrize("rows,K,N,tiles", [(160, 2304, 14336, 2), (300, 2304, 14336, 4), (340, 2304, 14336, 4), (384, 2304, 14336, 4)])
 def test_register_kernel_spreads_the_rows_of_a_single_matrix(device, fmt, dtype, rows, K, N, tiles):
     """A single matrix whose tiles of 64 rows do not fit: as few tiles of up to 96 as run as halves (112 units), or as many as fit one round
-    (224 units, 75 to 96 rows each).  The automatic choice, bit for bit against units of 64 rows, which add in the same order, and
-    not the other kernels' bits."""
+    (224 units, 75 to 96 rows each).  The automatic choice, bit for bit against units of 64
+    rows, which add in the same order, and not the other kernels' bits."""
     hip = _hip()
     gen = torch.Generator(device=device).manual_seed(94)
     w = _random_weight(fmt, [1, N, K], gen, device)
     a = torch.randn(rows, K, generator=gen, device=device).to(dtype)
+    assert -(-rows // MC.unit_rows(fmt, dtype, False, 1, 1, rows, K, N)) == tiles
     auto, reg, ws = (hip.mmt(a, w, variant=v).view(torch.int16) for v in (hip.VARIANT_AUTO, hip.VARIANT_MFMA_REG, hip.VARIANT_MFMA_WS))
     assert torch.equal(auto, reg) and not torch.equal(auto, ws)
 

@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+import moe_cases as MC
 from sharktank_amd import ops
 from sharktank_amd import types as ST
 from sharktank_amd.ops._registry import AllOfType, AnyOfType, overridable
@@ -228,17 +229,6 @@ def test_padded_layers_that_fitted_the_built_in_workspace_still_do():
                     assert need((n + 255) // 256 * 256) <= _hip.STATIC_SCRATCH_BYTES, (T, k, K, n)
 
 
-def _unit_rows(fmt, dtype, gate_up, E, k, T, kred, n_out, counts=None, scratch=True):
-    import ctypes
-
-    from sharktank_amd import _hip
-
-    packed = {"q8_0": _hip.W_Q8_0_PACKED, "q4_1": _hip.W_Q4_1_PACKED, "fp8": _hip.W_FP8_PACKED}[fmt]
-    w = _hip.StmoeWeight(format=packed, dtype=_hip.F32 if fmt == "fp8" else 0, experts=E, rows=n_out, cols=kred, d_count=1)
-    c = (ctypes.c_int64 * E)(*counts) if counts else None
-    return _hip.load_library().stmoe_register_unit_rows(_hip.dtype_enum(dtype), ctypes.byref(w), int(gate_up), T, k, c, int(scratch))
-
-
 @pytest.mark.parametrize("counts,rows", [
     ([65, 65, 65, 65, 64, 64, 64, 64], 96),      # 192 units of 64 rows: one round; 128 of 96: half a round
     ([129, 129, 129, 49, 40, 20, 10, 10], 64),   # 224 and 176: one round either way
@@ -250,8 +240,8 @@ def test_units_of_the_register_kernel_follow_the_rows_of_the_experts(counts, row
     """A launch that the automatic choice gives units of up to 96 rows takes them only where they save half a round; the sizes alone (8 experts
     of 1024 x 2048, 516 pairs) do not tell."""
     assert sum(counts) == 516
-    assert _unit_rows("q4_1", torch.float16, True, 8, 4, 129, 1024, 2048) == 96
-    assert _unit_rows("q4_1", torch.float16, True, 8, 4, 129, 1024, 2048, counts) == rows
+    assert MC.unit_rows("q4_1", torch.float16, True, 8, 4, 129, 1024, 2048) == 96
+    assert MC.unit_rows("q4_1", torch.float16, True, 8, 4, 129, 1024, 2048, counts) == rows
 
 
 @pytest.mark.parametrize("E,k,T,n_out,rows", [
@@ -264,12 +254,12 @@ def test_units_of_the_register_kernel_follow_the_rows_of_the_experts(counts, row
 ])
 def test_nearly_full_rounds_of_wide_units(E, k, T, n_out, rows):
     """Where one unit per expert and feature tile nearly fills a round of the CUs and the experts are few or very many."""
-    assert _unit_rows("q4_1", torch.bfloat16, True, E, k, T, 4096, n_out) == rows
+    assert MC.unit_rows("q4_1", torch.bfloat16, True, E, k, T, 4096, n_out) == rows
 
 
 def test_one_unit_per_expert_up_to_56_rows():
     """226 pairs on 4 experts, 136 units: a seventh more than the average is 64.57 rows, which counts as one unit of 64."""
-    assert _unit_rows("fp8", torch.float16, True, 4, 2, 113, 2048, 4352) == 64
+    assert MC.unit_rows("fp8", torch.float16, True, 4, 2, 113, 2048, 4352) == 64
 
 
 @pytest.mark.parametrize("fmt,dtype,gate_up,T,kred,n_out,rows", [
@@ -290,7 +280,7 @@ def test_one_unit_per_expert_up_to_56_rows():
 ])
 def test_units_of_a_single_matrix(fmt, dtype, gate_up, T, kred, n_out, rows):
     """One matrix on both sides of the lines around tiles of 64 and of up to 96 rows: as few tiles as run as halves, or as many as fit one round."""
-    assert _unit_rows(fmt, dtype, gate_up, 1, 1, T, kred, n_out) == rows
+    assert MC.unit_rows(fmt, dtype, gate_up, 1, 1, T, kred, n_out) == rows
 
 
 @pytest.mark.parametrize("fmt,dtype,gate_up,E,k,T,kred,n_out,scratch,rows", [
@@ -315,4 +305,4 @@ def test_units_of_a_single_matrix(fmt, dtype, gate_up, T, kred, n_out, rows):
 ])
 def test_units_of_grouped_launches(fmt, dtype, gate_up, E, k, T, kred, n_out, scratch, rows):
     """Several experts on both sides of the lines."""
-    assert _unit_rows(fmt, dtype, gate_up, E, k, T, kred, n_out, scratch=scratch) == rows
+    assert MC.unit_rows(fmt, dtype, gate_up, E, k, T, kred, n_out, scratch=scratch) == rows
