@@ -7,19 +7,21 @@
 //
 //   LDS: as many stages of either operand as 160 KB hold, four at most (three are the least that give a load two K steps to arrive;
 //     64 KB in flight per CU cover the memory latency; over 41 layers eight at most are 0.7 % slower than four: short reductions start
-//     later).  256 weight rows and 256 token rows leave room for three and two.  Rows of 128 bytes, XOR-swizzled in 16-byte units
+//     later).  256 weight rows and 192 or 256 token rows leave room for three and two.  Rows of 128 bytes, XOR-swizzled in 16-byte units
 //     (see ffn_mfma_common.h): the direct load puts lane l's 16 bytes at its base + 16 l, so the lanes fetch the units of a row in
 //     swizzled order.
-//   units: LDS and loads for 32, 128, 192 or 256 token rows.  With 192 a token row has two steps to arrive, as the weights have, and a
-//     quarter of the loads from L2 goes: gate/up of 515 tokens (129 rows per expert) 416 us with 256 only, 398 so.
+//   units: LDS and loads for 32, 128, 192 or 256 token rows.  With 192 a quarter of the loads from L2 goes (and of 128 weight rows a token row
+//     has as many steps to arrive as the weights): gate/up of 515 tokens (129 rows per expert) 416 us with 256 only, 398 so.
 //   last round: units left over after the last whole round over an XCD's CUs are cut into two of 128 weight rows if the halves fit one
-//     round (515 tokens, down: 16 units on 32 CUs, 203 us; 32 halves 194).
+//     round (with whole units / halves, us: gate/up of 515 tokens, three rounds and 16 units, 387 / 371; to 6144 features, one and 16, 187 / 169;
+//     down of 2048 tokens, two and 16, 510 / 456).  The halves of less than a round take what units of 128 weight rows take: [4096, 8192] at 400
+//     tokens, 16 units, 133 and 133 (whole 162).
 //   wavefronts: 4 x 2 (64 x 64 of BN = 256) up to 128 rows, 2 x 4 (128 x 48 or 64) above; the rows of a unit are spread evenly
 //     over the token groups in multiples of 16 and only the column blocks that hold rows are multiplied.
 //   The reduction runs in the order of the 128 x 128 kernel: the sums are the same bits.
-// Measured (8 experts of 4096 x 14336, top-2, bf16; gate/up + down, us; 128 x 128 kernel / this one): 100 tokens 421 + 279 /
-// 329 + 195, 515 tokens 640 + 313 / 398 + 194 (4.8 TB/s of weights), 2048 tokens 1916 + 823 / 1025 + 537 (0.92 PFLOP/s; SiLU
-// by expf and a division, as the 128 x 128 kernel computes it, is 20 us of the 1025: on the hardware exp2 and reciprocal 1002).
+// Measured (8 experts of 4096 x 14336, top-2, bf16; gate/up + down, us; 128 x 128 kernel / this one): 100 tokens 425 + 272 /
+// 331 + 170, 515 tokens 675 + 317 / 371 to 398 + 200 (4.8 to 5.1 TB/s of weights; where the pages lie moves it), 2048 tokens 1936 + 835 /
+// 1004 + 456 (0.96 PFLOP/s; SiLU by expf and a division, as the 128 x 128 kernel computes it, is some 20 us of the gate/up launch).
 // Slower at 515 tokens, gate/up: weights and tokens sent by different wavefronts 442, both loads behind the first half's products 465,
 // after the step's products 488.
 #include "ffn_mfma_common.h"
@@ -253,9 +255,12 @@ static int launch_dense_m(const GemmParams& p, int64_t max_rows, hipStream_t st)
   return check_launch("grouped_dense");
 }
 // 128 weight rows per unit instead of 256 while 256 would leave CUs without a unit (a unit per 256 features and expert, and half
-// a unit more per 256 rows).  Measured (8 experts, top-2, bf16, us, 256 / 128): gate/up of 1024 features 300 tokens 17 / 12, 2048
-// tokens 36 / 32; of 4096 features 80 tokens 43 / 46; of 14336 515 tokens 374 / 406.  Down to 4096 features from 14336: 515 tokens
-// 267 / 197, 1024 tokens 346 / 422; to 2048 from 4096, 1500 tokens 98 / 58.
+// a unit more per 256 rows).  Measured (8 experts, top-2, bf16, us, 256 / 128): gate/up of 1024 features from 1024, 300 tokens 12.6 / 12.5, 2048
+// tokens 35 / 30; of 6144 from 4096, 515 tokens 169 / 177; of 14336 515 tokens 371 / 403.  Down to 4096 features from 14336: 515 tokens
+// 198 / 200, 1024 tokens 334 / 421; to 2048 from 4096, 1500 tokens 58 / 59.  Over 12900 launches of 1 to 64 experts, 512 to 14336 x 512 to
+// 14336, 2 to 2500 rows per expert, by this measure of units: up to 96 the same (halves), 96 to 128 256 rows take 0.99 of the time, 128 to 192 0.92 (up to
+// 1.49: launches of just over half a round), beyond 0.9 to 0.95 (up to 1.4, from 512 on 1.2).  On the line at 192 a launch takes 1.02 of the
+// better choice, at 128 1.01.
 template <typename T>
 static int launch_dense_t(int mode, const GemmParams& p, int64_t max_rows, hipStream_t st) {
   const int64_t wide = mode == MODE_GATEUP ? 128 : 256, experts = p.offsets ? std::min<int64_t>(p.E, max_rows) : 1;

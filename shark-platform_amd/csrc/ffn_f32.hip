@@ -9,10 +9,10 @@
 // Order of the loads: they return in the order of their issue, so the tokens of an item's rows are requested first, then its weights, then
 // the token rows; two chunks of both are in flight up to 32 rows, of the weights alone from 33 rows on, every load unconditional (a row's
 // ragged end re-reads its last piece and drops it in registers: an instance of its own, TAIL).  With one chunk ahead, each load under its own condition, and the wavefront's number in a vector
-// register, every wait was for all loads in flight: 64 tokens of 512 x 1024 16.3 + 11.7 us; now 14.0 + 9.2.  Layer (8 experts, top-2, us,
-// before / now): 64 tokens of 512 x 1024 37.6 / 31.4, 109 tokens of 896 x 1280 77 / 69, 128 tokens of 1024 x
-// 1536 88 / 76; Q8_0 weights of 1024 x 1024, 2000 tokens 435 / 349; one Q8_0 matrix of [2048, 2048], 60 rows 28.7 / 20.0.  (On the general
-// kernel the first took 110.)  Weights requested in front of the tokens: 34.3.
+// register, every wait was for all loads in flight: 64 tokens of 512 x 1024 16.8 + 12.0 us; now 12.6 + 8.3.  Layer (8 experts, top-2, us,
+// before / now): 64 tokens of 512 x 1024 37.0 / 29.5, 109 tokens of 896 x 1280 74 / 66, 128 tokens of 1024 x
+// 1536 85 / 75; Q8_0 weights of 1024 x 1024, 2000 tokens 432 / 342; one Q8_0 matrix of [2048, 2048], 60 rows 28.7 / 19.0.  (On the general
+// kernel the first took 110.)  Weights requested in front of the tokens: 3 us more.
 // Registers: all 256 are in use, and a register in scratch memory comes back through the same in-order path as the loads ahead of it.  So
 // a weight row is converted and multiplied with all token rows before the next one is (with both in any order ten of 54 instances
 // kept 12 to 44 bytes a lane in scratch memory: 3000 launches of 1 to 16 experts, 256 to 2048 x 128 to 2048, 1 to 100 rows per expert, plain

@@ -6,7 +6,7 @@
 //
 //   256 x 256 workgroup tile (GATEUP: 128 gate + the same 128 up rows), 8 wavefronts of 128 weight rows x 64 token
 //   rows, K stage 64 (one v_mfma_scale_f32_32x32x64_f8f6f4 deep), four stages of 16 KB weights + 16 KB tokens + 2 KB
-//   ride-along tokens = 136 KB, loads issued three stages ahead (four are no faster), one barrier per stage.
+//   ride-along tokens = 136 KB, loads issued three stages ahead (more stages do not fit), one barrier per stage.
 //   order:   the two wavefronts of a SIMD take the halves of a stage in opposite orders.  Behind the barrier of stage s wavefronts 4-7
 //            multiply stage s - 1, whose operands they have in registers, and then read those of stage s; wavefronts 0-3 first read
 //            stage s and then multiply it.  So one of the two always has MFMAs to issue and the other one's LDS latency and load
@@ -20,16 +20,18 @@
 //   tokens:  quantised rows, 64 bytes per stage; lane l of a load fetches the 16 bytes that belong at LDS position l
 //            (row l / 4 of the load's 16 rows, the unit that x_unit maps to position l % 4), so that the gather and the
 //            bank swizzle cost nothing; rows of a partial token tile are spread over the four token-row groups.  (A swizzle
-//            under which two rows of a cycle shared their banks: 799 + 388 us for the launches below, this one 770 + 369.)
+//            under which two rows of a cycle shared their banks: 4 to 5 % more for the launches below.)
 //   results: D[8 (i / 4) + 4 h + i % 4][r] (probed on the hardware: rows are the weight rows, columns the token rows);
 //            both token blocks' operands (16 registers) and the four weight blocks' (32) are read once per wavefront and stage.
 //   epilogue: the fp32 dot products of the quantised samples are scaled once by scale_x * d_w; the gate/up epilogue can
 //            quantise the gated intermediate to e4m3fn for the down projection.
-//   What bounds it: power.  4096 tokens, 8 experts of 4096 x 14336, gate/up + down: both wavefronts of a SIMD in the same order
-//            962 + 464 us (1.96 + 0.95 M cycles at 2.04 GHz, the matrix cores busy half of them); in opposite orders 770 + 369
-//            (1.33 + 0.63 M at 1.73, busy 0.73); 1225 instead of 1456 us for the layer, and over 36 layers of 4 to 16 experts,
-//            1024 to 6144 x 1024 to 16384, 0 to 25 % less, 10 on average.  An early build of it without any barrier took 16 % fewer
-//            cycles at a clock 9 % lower, without loads 703 + 323 us.  A launch with nothing but the loads takes 590 + 300 us, 13 TB/s of the 34 that
+//   What bounds it: power.  4096 tokens, 8 experts of 4096 x 14336, gate/up + down, both sides traced on one box: both wavefronts of a SIMD in the
+//            same order 1032 + 496 us of 1608 for the layer, in opposite orders 820 + 394 of 1301 (without the profiler 1499 and 1205; the rest
+//            are router, dispatch, the rows' quantizer and combine).  Counters: 1.96 + 0.95 M cycles at 1.98 GHz, the matrix cores busy
+//            0.48 of them; 1.35 + 0.66 M at 1.73 and 1.69, busy 0.69 and 0.71.  Over 1800 layers of 1 to 32 experts, 1024 to 6144 x 1024 to 16384,
+//            8 % less time on average, nine of them more by 2 to 10 % (16 experts of 4096 columns and more with one tile of 100 to 260 rows each).
+//            An early build of it without any barrier took 16 % fewer
+//            cycles at a clock 9 % lower.  A launch with nothing but the loads takes 590 + 300 us, 13 TB/s of the 34 that
 //            these loads reach from L2 without a barrier per stage: one stage in flight is as fast as two, so not latency.
 //            Tried and slower, because something other than MFMAs comes between a wavefront's MFMAs: the loads between them
 //            (+15 %), a load's operands read as soon as the last MFMA has used the register (+15 %), both wavefronts late
