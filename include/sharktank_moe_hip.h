@@ -352,10 +352,11 @@ int stmoe_probe_mfma(int kind, int random_operands, int iters, float* sink, doub
  * a [M,K], out [M,rows], both `dtype`; fp32 accumulation.
  * `workspace` (nullable; stmoe_mmt_workspace_bytes(M) bytes, 16-byte aligned): scratch for reductions split over several
  * workgroups, which lets a launch of a few hundred rows (too few 256 x 256 units for 256 CUs) use the whole chip; without
- * it the result is the same up to the grouping of the fp32 sums, the launch only slower.  (Two kinds of launch use no
+ * it the result is the same up to the grouping of the fp32 sums, the launch only slower.  (Three kinds of launch use no
  * workspace: those of 129 rows and more whose tiles of 64 output features x 256 rows fit the 256 CUs, which run on such tiles,
- * and most of 33 rows and more that make at most 128 units of 256 output features x 64 rows, which run on those: a matrix of
- * 14336 features up to 128 rows, one of 1024 features up to 2048.)  The workspace ends in a few counters that elect the
+ * most of 33 rows and more that make at most 128 units of 256 output features x 64 rows, which run on those: a matrix of
+ * 14336 features up to 128 rows, one of 1024 features up to 2048; and most of more rows that make at most 256 units of 65 to
+ * 96 rows, or 128 of up to 96: that of 14336 features up to 192 rows and from 257 to 384.)  The workspace ends in a few counters that elect the
  * workgroup which adds a split unit's chunks; every call leaves them at zero.
  * `workspace_ready` != 0: the caller vouches that the workspace was zero-filled before its first use and has since been
  * written only by calls of this function (on one stream at a time); 0: the counters are cleared first, one small launch

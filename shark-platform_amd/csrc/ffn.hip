@@ -187,7 +187,7 @@ static bool reg_loses(int dtype, int wtag, int mode, const GemmParams& p, int64_
 // than 96.  Two tiles of an expert pay again where they fit one round and tiles of 64 do not (8 of [4096, 14336] down 144 rows Q8_0 fp16
 // 204 / 170, Q4_1 bf16 204 / 200; gate/up of 8 x 1024 x 2048 at 144 rows 1.5 to 1.7).  Where tiles of 64 are at most 128 units, which run as
 // halves, they stay.  Over 118 layers of 4 to 64 experts, 1024 to 6144 x 1024 to 16384, those that they change take 8 % less time under a
-// uniform routing (-1 to 27 %) and 5 % under a Zipf routing (-8 to 29 %: there it depends on which experts have a few rows more than tiles).
+// uniform routing (-1 to 27 %) and 5 % under a Zipf routing (-8 to 29 %) with units of 96 throughout; which units a launch gets: reg_fewer_rows.
 static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, int64_t rows) {
   const int64_t E = p.E, units = p.n_out / (mode == MODE_GATEUP ? 128 : 256) * E;  // units: with one token tile per expert
   const bool streams = (p.expert_rows_bound > 0 && p.expert_rows_bound <= kSkinnyMaxRowsPerExpert) || rows <= kSkinnyMaxRows ||

@@ -18,6 +18,7 @@
 //             gate/up 259 -> 218 us, down 137 -> 110; 300 rows of [14336, 4096] in four tiles of 75: 61 -> 53 us).  112 rows spill; units
 //             of 128 weight rows x 160 token rows (half as many conversions, twice the operand reads) gave 49 and 46 us for those 300
 //             rows in Q4_1 bf16 and Q8_0 fp16, where this one takes 53 and 48, and lost elsewhere.
+//             A launch of several experts takes units of up to 64 rows here instead where they need no more rounds (fewer_rows).
 //   half unit the units after the last whole round over the workgroups are cut into two of 128 weight rows if the halves fit one round
 //             (a tile per wavefront): 8 experts of [4096, 14336] are 128 units, 256 halves.
 //
@@ -449,7 +450,7 @@ grouped_mfma_reg_kernel(RegArgs args) {
     };
     auto sized = [&](auto nt_tag) {
       const int tiles = (row_end - row_begin + 15) >> 4;
-      if constexpr (MT > 4) {  // (chosen where units have more than 64 rows)
+      if constexpr (MT > 4) {  // (units of up to 64 rows where they take no more rounds: 0.99 of the time of the narrow kernel's, with their three sets)
         if (tiles <= 4) unit(nt_tag, RgInt<4>{});
         else if (tiles == 5) unit(nt_tag, RgInt<5>{});
         else unit(nt_tag, RgInt<6>{});
