@@ -29,7 +29,7 @@
 //            same order 1032 + 496 us of 1608 for the layer, in opposite orders 820 + 394 of 1301 (without the profiler 1499 and 1205; the rest
 //            are router, dispatch, the rows' quantizer and combine).  Counters: 1.96 + 0.95 M cycles at 1.98 GHz, the matrix cores busy
 //            0.48 of them; 1.35 + 0.66 M at 1.73 and 1.69, busy 0.69 and 0.71.  Over 1800 layers of 1 to 32 experts, 1024 to 6144 x 1024 to 16384,
-//            8 % less time on average, nine of them more by 2 to 10 % (16 experts of 4096 columns and more with one tile of 100 to 260 rows each).
+//            8 % less time on average (nine took 2 to 10 % more in that run; 24 layers around the worst of them, 12 to 20 experts with one tile each, 5 to 10 % less).
 //            An early build of it without any barrier took 16 % fewer
 //            cycles at a clock 9 % lower.  A launch with nothing but the loads takes 590 + 300 us, 13 TB/s of the 34 that
 //            these loads reach from L2 without a barrier per stage: one stage in flight is as fast as two, so not latency.
