@@ -201,8 +201,8 @@ static int reg_rows_grouped(int dtype, int wtag, int mode, const GemmParams& p, 
                 tiles = (most + kRegWideRows - 1) / kRegWideRows, wide = tiles * units;
   // (129 to 175 whole units leave too many CUs without one: two tiles of 4 experts of 4864 x 7168 at 135 rows, Q4_1 bf16, layer 195 / 207 us)
   // (one such tile per expert that nearly fills a round, of few experts or of very many: an expert with more than 96 rows spills into a second
-  // round.  4 experts from 61 rows on under uneven routings 0 % on average, -25 to 43, uniform ones gain 13 %; 32 and 64 experts from 73 rows on -20 to 24)
-  const bool spills = tiles == 1 && wide <= 256 && ((E <= 4 && wide > 192 && rows > 60 * E) || (E >= 32 && wide > 240 && rows > 72 * E));
+  // round.  4 experts from 61 rows on under uneven routings 0 % on average, -25 to 43, uniform ones gain 13 %; 32 and 64 experts from 77 rows on 1 % slower on average, -15 to 38, from 65 to 76 rows 10 % faster, -20 to 31)
+  const bool spills = tiles == 1 && wide <= 256 && ((E <= 4 && wide > 192 && rows > 60 * E) || (E >= 32 && wide > 240 && rows > 76 * E));
   if (narrow > 128 && (wide <= 128 || wide >= 176) && !spills && (wtag == WF_Q4_1_P || p.kred >= 2048) &&
       ((rows > 52 * E && rows <= (p.kred < 2048 ? 72 : 80) * E) || (tiles == 2 && rows >= 120 * E && wide <= 256) || (tiles > 1 && wide <= 128)))
     return kRegWideRows;

@@ -249,8 +249,8 @@ def test_units_of_the_register_kernel_follow_the_rows_of_the_experts(counts, row
     (4, 2, 121, 7168, 0),     # from 61 on an expert of an uneven routing spills into a second round too often
     (4, 2, 160, 6144, 96),    # 192 units
     (8, 2, 310, 3584, 96),    # eight experts
-    (32, 4, 576, 1024, 96),   # 72 rows on each of 32 experts, 256 units
-    (32, 4, 577, 1024, 0),
+    (32, 4, 608, 1024, 96),   # 76 rows on each of 32 experts, 256 units
+    (32, 4, 609, 1024, 0),
 ])
 def test_nearly_full_rounds_of_wide_units(E, k, T, n_out, rows):
     """Where one unit per expert and feature tile nearly fills a round of the CUs and the experts are few or very many."""
